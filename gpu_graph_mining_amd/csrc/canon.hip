@@ -384,7 +384,11 @@ __global__ void __launch_bounds__(64) k_canon_level(CanonArgs c) {
     __syncthreads();
     const int res = canon_core(L, len + 1, nv, lane);
     // answer + 1, so that a record the kernel did not reach reads as 0
-    if (lane == 0) f[1] = (f[1] & 0xFFFFFFFFull) | ((unsigned long long)(res + 1) << 32);
+    if (lane == 0) {
+      const unsigned long long w = (f[1] & 0xFFFFFFFFull) | ((unsigned long long)(res + 1) << 32);
+      f[1] = w;
+      if (c.down && slot < c.down_cap) c.down[4ull * slot + 1] = w;
+    }
   }
 }
 

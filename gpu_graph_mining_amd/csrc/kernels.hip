@@ -761,17 +761,25 @@ __global__ void __launch_bounds__(64) k_level_fix(StepArgs a) {
 // Sum every key's replicas; keys reaching their job's min support go to the
 // frequent list as (key, support, embeddings, item sum), in key order, and
 // keep their replicas (k_cursors splits the children's rows by them, then
-// clears them); the other keys' replicas are cleared here.  Three kernels:
-// k_reduce counts the frequent keys of each tile of kReduceTile keys,
-// k_reduce_scan turns the counts into the tiles' first slots (and the
-// list's length), k_reduce_list writes each tile's records in key order.
+// clears them); the other keys' replicas are cleared here.  Two kernels:
+// k_reduce counts the frequent keys of each tile of a.tile_keys keys;
+// k_reduce_list adds up the tiles before its own (at most kReduceTiles
+// counts, a few loads per lane) and writes its records in key order, to the
+// device's list and to the host's mapped copy of its head.
+//
+// What bounds them is the latency of the replica loads (8-byte loads one
+// replica apart, a few thousand keys): G groups of lanes share a key's
+// replicas (G = 4 from 8 replicas on), and in k_reduce_list and k_cursors
+// `rep` lanes take one frequent key's replicas together and scan them.  One
+// lane walking 64 replicas measured 16-26 us (k_reduce), 14-24 us (list)
+// and 18-46 us (k_cursors) per level of the 10,000- and 100,000-transaction
+// workloads.
 constexpr int kReduceThreads = 256;
-constexpr int kReduceSteps = kReduceTile / kReduceThreads;
-static_assert(kReduceSteps * kReduceThreads == kReduceTile, "reduce tile");
 
 template <bool ROOT>
 __device__ __forceinline__ bool reduce_frequent(const StepArgs &a, int64_t i, int32_t s) {
   if (s <= 0) return false;
+  if (!a.minsup_job) return s >= a.minsup_one;
   const int64_t p = i / a.K + a.p_base;
   const int32_t owner = ROOT ? (int32_t)p : meta_at(a.meta, a.S, p)->job;
   return s >= a.minsup_job[owner];
@@ -790,99 +798,140 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t x, uint32_t *s_part) {
   return t;
 }
 
-template <bool ROOT>
+template <bool ROOT, int G>
 __global__ void __launch_bounds__(kReduceThreads) k_reduce(StepArgs a) {
+  constexpr int KS = kReduceThreads / G;  // keys of a step
   __shared__ uint32_t s_part[kReduceThreads / 64];
-  const int64_t n_tiles = reduce_tiles(a.nkeys);
-  for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    uint32_t hits = 0;
-    for (int j = 0; j < kReduceSteps; ++j) {
-      const int64_t i = t * kReduceTile + (int64_t)j * kReduceThreads + threadIdx.x;
-      if (i >= a.nkeys) continue;
-      unsigned long long v = 0;
-      for (int r = 0; r < a.rep; ++r) v += a.acc[(int64_t)r * a.nkeys + i];
-      const int32_t s = (int32_t)(v >> kSupShift);
-      a.sup[i] = s;
-      const bool hit = reduce_frequent<ROOT>(a, i, s);
-      hits += hit ? 1u : 0u;
-      if (v && !hit)
-        for (int r = 0; r < a.rep; ++r) {
-          a.acc[(int64_t)r * a.nkeys + i] = 0;
-          a.accb[(int64_t)r * a.nkeys + i] = 0;
-        }
+  __shared__ unsigned long long s_v[G > 1 ? kReduceThreads : 1];
+  const int kt = threadIdx.x % KS, g = threadIdx.x / KS;
+  const int64_t t = blockIdx.x;
+  uint32_t hits = 0;
+  for (int64_t j = 0; j < a.tile_keys; j += KS) {
+    const int64_t i = t * a.tile_keys + j + kt;
+    const bool in = i < a.nkeys;
+    unsigned long long v = 0;
+    if (in) {
+#pragma unroll 8
+      for (int r = g; r < a.rep; r += G) v += a.acc[(int64_t)r * a.nkeys + i];
     }
-    hits = block_sum(hits, s_part);
-    if (threadIdx.x == 0) a.tile_count[t] = hits;
+    unsigned long long own = v;
+    if constexpr (G > 1) {
+      s_v[threadIdx.x] = v;
+      __syncthreads();
+      v = 0;
+#pragma unroll
+      for (int q = 0; q < G; ++q) v += s_v[q * KS + kt];
+      __syncthreads();
+    }
+    if (!in) continue;
+    const int32_t s = (int32_t)(v >> kSupShift);
+    const bool hit = reduce_frequent<ROOT>(a, i, s);
+    if (g == 0) {
+      a.sup[i] = s;
+      hits += hit ? 1u : 0u;
+    }
+    if (own && !hit)
+      for (int r = g; r < a.rep; r += G) {
+        a.acc[(int64_t)r * a.nkeys + i] = 0;
+        a.accb[(int64_t)r * a.nkeys + i] = 0;
+      }
   }
+  hits = block_sum(hits, s_part);
+  if (threadIdx.x == 0) a.tile_count[t] = hits;
 }
 
-// One workgroup: exclusive scan of the tile counts in place; the total is
-// the list's length.
-__global__ void __launch_bounds__(1024) k_reduce_scan(StepArgs a) {
-  __shared__ uint32_t s_wave[16];
-  const int64_t n = reduce_tiles(a.nkeys);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t carry = 0;
-  for (int64_t b = 0; b < n; b += 1024) {
-    const int64_t i = b + threadIdx.x;
-    const uint32_t x = i < n ? a.tile_count[i] : 0u;
-    uint32_t wt;
-    const uint32_t ex = wave_exclusive_scan<uint32_t>(x, wt);
-    if (lane == 0) s_wave[wave] = wt;
-    __syncthreads();
-    uint32_t before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      before += w < wave ? s_wave[w] : 0u;
-      total += s_wave[w];
-    }
-    if (i < n) a.tile_count[i] = carry + before + ex;
-    carry += total;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *a.freq_count = carry;
+// x summed over aligned groups of `width` lanes (a power of two), read by
+// every lane of the group
+template <class T>
+__device__ __forceinline__ T group_sum(T x, int width) {
+  for (int o = width >> 1; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+  return x;
 }
 
 template <bool ROOT>
 __global__ void __launch_bounds__(kReduceThreads) k_reduce_list(StepArgs a) {
   __shared__ uint32_t s_part[kReduceThreads / 64];
-  const int64_t n_tiles = reduce_tiles(a.nkeys);
+  __shared__ uint32_t s_hit[kReduceThreads];  // the step's frequent keys, relative to its first
+  const int64_t n_tiles = reduce_tiles(a);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-    uint32_t next = a.tile_count[t];  // the tile's first slot
-    for (int j = 0; j < kReduceSteps; ++j) {
-      const int64_t i = t * kReduceTile + (int64_t)j * kReduceThreads + threadIdx.x;
-      const int32_t s = i < a.nkeys ? a.sup[i] : 0;
-      const bool hit = i < a.nkeys && reduce_frequent<ROOT>(a, i, s);
-      // rank among the tile's keys of this step, in key order
-      const uint64_t m = __ballot(hit);
-      if (lane == 0) s_part[wave] = (uint32_t)__popcll(m);
-      __syncthreads();
-      uint32_t before = 0, step = 0;
-#pragma unroll
-      for (int w = 0; w < kReduceThreads / 64; ++w) {
-        before += w < wave ? s_part[w] : 0u;
-        step += s_part[w];
-      }
-      __syncthreads();
-      if (hit) {
-        const uint32_t slot = next + before + (uint32_t)__popcll(m & lanes_below(lane));
-        if (slot < a.freq_cap) {
-          unsigned long long v = 0, bs = 0;
-          for (int r = 0; r < a.rep; ++r) {
-            v += a.acc[(int64_t)r * a.nkeys + i];
-            bs += a.accb[(int64_t)r * a.nkeys + i];
-          }
-          unsigned long long *f = a.freq + 4 * (int64_t)slot;
-          f[0] = (unsigned long long)i;
-          f[1] = (unsigned long long)s;
-          f[2] = v & ((1ull << kSupShift) - 1);
-          f[3] = bs;
-        }
-      }
-      next += step;
+  const int64_t t = blockIdx.x;
+  // the tile's first slot: the frequent keys of the tiles before it
+  uint32_t x = 0;
+  for (int64_t q = threadIdx.x; q < t; q += kReduceThreads) x += a.tile_count[q];
+  uint32_t next = block_sum(x, s_part);
+  if (a.down && t == 0) {
+    // the level's counters (complete: k_level and k_level_fix are done),
+    // but for the list's length, which the last tile's workgroup stores
+    const unsigned long long *src = a.counters;
+    for (int i = threadIdx.x; i < kCounterWords; i += kReduceThreads) {
+      if (i == 0) reinterpret_cast<uint32_t *>(a.down)[1] = reinterpret_cast<const uint32_t *>(src)[1];
+      else a.down[i] = src[i];
     }
   }
+  if (t == n_tiles - 1 && threadIdx.x == 0) {
+    const uint32_t total = next + a.tile_count[t];
+    *a.freq_count = total;
+    if (a.down) *reinterpret_cast<uint32_t *>(a.down) = total;
+  }
+  if (a.tile_count[t] == 0) return;
+  for (int64_t j = 0; j < a.tile_keys; j += kReduceThreads) {
+    const int64_t i0 = t * a.tile_keys + j, i = i0 + threadIdx.x;
+    const bool in = j + threadIdx.x < a.tile_keys && i < a.nkeys;
+    const bool hit = in && reduce_frequent<ROOT>(a, i, a.sup[i]);
+    // rank among the tile's keys of this step, in key order
+    const uint64_t m = __ballot(hit);
+    if (lane == 0) s_part[wave] = (uint32_t)__popcll(m);
+    __syncthreads();
+    uint32_t before = 0, step = 0;
+#pragma unroll
+    for (int w = 0; w < kReduceThreads / 64; ++w) {
+      before += w < wave ? s_part[w] : 0u;
+      step += s_part[w];
+    }
+    if (hit) s_hit[before + (uint32_t)__popcll(m & lanes_below(lane))] = (uint32_t)threadIdx.x;
+    __syncthreads();
+    // `rep` lanes per frequent key sum its replicas
+    const int per = 64 / a.rep, sub = lane / a.rep, r = lane % a.rep;
+    for (uint32_t h0 = (uint32_t)(wave * per); h0 < step; h0 += (uint32_t)(per * (kReduceThreads / 64))) {
+      const uint32_t h = h0 + (uint32_t)sub, slot = next + h;
+      const bool ok = h < step && slot < a.freq_cap;
+      const int64_t key = i0 + (ok ? s_hit[h] : 0u);
+      unsigned long long v = 0, bs = 0;
+      if (ok) {
+        v = a.acc[(int64_t)r * a.nkeys + key];
+        bs = a.accb[(int64_t)r * a.nkeys + key];
+      }
+      v = group_sum(v, a.rep);
+      bs = group_sum(bs, a.rep);
+      if (ok && r == 0) {
+        const unsigned long long rec[4] = {(unsigned long long)key, v >> kSupShift, v & ((1ull << kSupShift) - 1), bs};
+        unsigned long long *f = a.freq + 4 * (int64_t)slot;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) f[q] = rec[q];
+        if (a.down && slot < a.down_cap) {
+          unsigned long long *d = a.down + kCounterWords + 4 * (int64_t)slot;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) d[q] = rec[q];
+        }
+      }
+    }
+    next += step;
+    __syncthreads();  // the next step rewrites the shared counts and keys
+  }
+}
+
+// The level's counters start from zero: frequent-key count, failure list,
+// errors and spread statistics but the written-row slots, which keep
+// counting across levels (the host compares their total with the rows it
+// asked for).
+__device__ __forceinline__ void clear_counters(const StepArgs &a) {
+  if (threadIdx.x == 0) {
+    *a.freq_count = 0;
+    *a.fail_count = 0;
+    *a.error_flag = 0;
+  }
+  for (int i = threadIdx.x; i < kSpread * kSpreadStride; i += blockDim.x)
+    if (i % kSpreadStride != kSpreadWritten) a.spread[i] = 0;
 }
 
 // After the host chose the children: frequent key i (the key of record i of
@@ -890,33 +939,45 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_list(StepArgs a) {
 // entry points at the child, and
 // every (child, replica) gets its first row and list entry -- the child's
 // bases plus the earlier replicas' embeddings and item sums -- and a zero
-// reservation cursor; the frequent keys' replicas are cleared.  Also copies
-// the children's upload.
-__global__ void k_cursors(StepArgs a, unsigned long long *dst, const unsigned long long *src, int64_t n,
-                          const int32_t *fchild, const unsigned long long *row_base, const unsigned long long *list_base,
-                          int64_t F) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+// reservation cursor; the frequent keys' replicas are cleared.  `rep` lanes
+// take one key's replicas and scan their counts.  The first workgroup clears
+// the next level's counters (the host has read this level's).
+__global__ void __launch_bounds__(256) k_cursors(StepArgs a, const int32_t *fchild, const unsigned long long *row_base,
+                                                 const unsigned long long *list_base, int64_t F) {
+  if (blockIdx.x == 0) clear_counters(a);
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int64_t i = t; i < n; i += stride) dst[i] = src[i];
-  for (int64_t i = t; i < F; i += stride) {
-    const int64_t key = (int64_t)a.freq[4 * i];
-    const int32_t ch = fchild[i];
-    unsigned long long re = ch >= 0 ? row_base[ch] : 0ull, rl = ch >= 0 ? list_base[ch] : 0ull;
-    if (ch >= 0) a.sup[key] = -(ch + 1);
-    for (int r = 0; r < a.rep; ++r) {
-      const int64_t at = (int64_t)r * a.nkeys + key;
-      const unsigned long long v = a.acc[at], bs = a.accb[at];
-      if (ch >= 0) {
-        a.cur_rows[(int64_t)ch * a.rep + r] = re;
-        a.cur_list[(int64_t)ch * a.rep + r] = rl;
-        a.cursor[(int64_t)ch * a.rep + r] = 0;
-        re += v & ((1ull << kSupShift) - 1);
-        rl += bs;
-      }
-      a.acc[at] = 0;
-      a.accb[at] = 0;
+  const int64_t i = t / a.rep;
+  const int r = (int)(t % a.rep);
+  const bool ok = i < F;
+  int64_t key = 0, at = 0;
+  int32_t ch = -1;
+  unsigned long long v = 0, bs = 0;
+  if (ok) {
+    key = (int64_t)a.freq[4 * i];
+    at = (int64_t)r * a.nkeys + key;
+    ch = fchild[i];
+    v = a.acc[at];
+    bs = a.accb[at];
+  }
+  // exclusive scans over the key's replicas
+  unsigned long long rows = v & ((1ull << kSupShift) - 1), sr = rows, sb = bs;
+  for (int o = 1; o < a.rep; o <<= 1) {
+    const unsigned long long yr = __shfl_up(sr, o, 64), yb = __shfl_up(sb, o, 64);
+    if (r >= o) {
+      sr += yr;
+      sb += yb;
     }
   }
+  if (!ok) return;
+  if (ch >= 0) {
+    if (r == 0) a.sup[key] = -(ch + 1);
+    const int64_t c = (int64_t)ch * a.rep + r;
+    a.cur_rows[c] = row_base[ch] + (sr - rows);
+    a.cur_list[c] = list_base[ch] + (sb - bs);
+    a.cursor[c] = 0;
+  }
+  a.acc[at] = 0;
+  a.accb[at] = 0;
 }
 
 // ------------------------------------------------------------------ WRITE
@@ -1254,17 +1315,7 @@ __global__ void k_fill8(unsigned long long *dst, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = 0ull;
 }
 
-__global__ void __launch_bounds__(256) k_clear_counters(StepArgs a) {
-  if (threadIdx.x == 0) {
-    *a.freq_count = 0;
-    *a.fail_count = 0;
-    *a.error_flag = 0;
-  }
-  // the written-row slots keep counting across levels (the host compares
-  // their total with the rows it asked for)
-  for (int i = threadIdx.x; i < kSpread * kSpreadStride; i += blockDim.x)
-    if (i % kSpreadStride != kSpreadWritten) a.spread[i] = 0;
-}
+__global__ void __launch_bounds__(256) k_clear_counters(StepArgs a) { clear_counters(a); }
 
 template <bool ROOT>
 hipError_t level_tw(const StepArgs &a, hipStream_t s, size_t lds) {
@@ -1312,19 +1363,22 @@ hipError_t launch_level_fix(const StepArgs &a, bool root, hipStream_t s) {
   return hipGetLastError();
 }
 
+namespace {
+template <bool ROOT>
+hipError_t reduce_of(const StepArgs &a, hipStream_t s) {
+  const unsigned g = (unsigned)reduce_tiles(a);
+  if (a.rep >= kReduceSplitRep)
+    hipLaunchKernelGGL((k_reduce<ROOT, 4>), dim3(g), dim3(kReduceThreads), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_reduce<ROOT, 1>), dim3(g), dim3(kReduceThreads), 0, s, a);
+  hipLaunchKernelGGL(k_reduce_list<ROOT>, dim3(g), dim3(kReduceThreads), 0, s, a);
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_reduce(const StepArgs &a, bool root, hipStream_t s) {
   if (a.nkeys <= 0) return hipSuccess;
-  const unsigned g = (unsigned)std::min<int64_t>(reduce_tiles(a.nkeys), 8192);
-  if (root)
-    hipLaunchKernelGGL(k_reduce<true>, dim3(g), dim3(kReduceThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_reduce<false>, dim3(g), dim3(kReduceThreads), 0, s, a);
-  hipLaunchKernelGGL(k_reduce_scan, dim3(1), dim3(1024), 0, s, a);
-  if (root)
-    hipLaunchKernelGGL(k_reduce_list<true>, dim3(g), dim3(kReduceThreads), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_reduce_list<false>, dim3(g), dim3(kReduceThreads), 0, s, a);
-  return hipGetLastError();
+  return root ? reduce_of<true>(a, s) : reduce_of<false>(a, s);
 }
 
 hipError_t launch_write(const StepArgs &a, bool root, hipStream_t s) {
@@ -1360,15 +1414,12 @@ hipError_t launch_copy8(void *dst, const void *src, size_t bytes, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_cursors(const StepArgs &a, void *dst, const void *src, size_t bytes, const int32_t *fchild,
-                          const unsigned long long *row_base, const unsigned long long *list_base, int64_t F,
-                          hipStream_t s) {
-  if (bytes % 8) return hipErrorInvalidValue;
-  const int64_t n = (int64_t)(bytes / 8);
-  if (n == 0 && F == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_cursors, dim3(copy_grid(std::max(n, F))), dim3(256), 0, s, a,
-                     static_cast<unsigned long long *>(dst), static_cast<const unsigned long long *>(src), n, fchild,
-                     row_base, list_base, F);
+hipError_t launch_cursors(const StepArgs &a, const int32_t *fchild, const unsigned long long *row_base,
+                          const unsigned long long *list_base, int64_t F, hipStream_t s) {
+  if (F <= 0) return hipSuccess;
+  const int64_t lanes = F * a.rep;
+  hipLaunchKernelGGL(k_cursors, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, a, fchild, row_base, list_base,
+                     F);
   return hipGetLastError();
 }
 

@@ -31,6 +31,8 @@ constexpr int kSpreadStart = 4;    // ~(earliest start) of the extension + suppo
 constexpr int kSpreadEnd = 5;      // latest end of the stage (atomicMax); device wall clock
 constexpr int kSpreadWritten = 6;  // child rows written by k_write
 constexpr int kSpreadFailed = 7;   // chunks recounted by k_level_fix
+// the counter block: 8 words (frequent keys, failed chunks, error bits), then the spread lines
+constexpr int kCounterWords = 8 + kSpread * kSpreadStride;
 
 // One chunk of a level's rows: [start, end) after alignment to segment
 // starts (a segment is the rows of one pattern in one graph; at the root,
@@ -100,11 +102,19 @@ struct StepArgs {
   // k_reduce: supports (>= 0), then child ids (-(child + 1)) once chosen
   int32_t *sup;
   int64_t nkeys;
-  const int32_t *minsup_job;
+  const int32_t *minsup_job;  // per job; null: every job's is minsup_one
+  int32_t minsup_one;
   unsigned long long *freq;  // (key, support, embeddings, item sum) of frequent keys, in key order
   uint32_t *freq_count;
   uint32_t freq_cap;
-  uint32_t *tile_count;  // k_reduce: frequent keys per tile of kReduceTile keys, then the tiles' first slots
+  uint32_t *tile_count;  // k_reduce: frequent keys per tile of tile_keys keys
+  int64_t tile_keys;
+  // the counter block (kCounterWords words, freq right behind it) and its
+  // mapped host copy, which k_reduce_list fills with the counters and the
+  // first down_cap records (null: no mapped copy)
+  const unsigned long long *counters;
+  unsigned long long *down;
+  uint32_t down_cap;
   // k_write: child rows; cur_rows / cur_list[c * rep + r] are the first row
   // and the first list entry of child c for the chunks of replica r, and
   // cursor[c * rep + r] = rows << 32 | list entries reserved so far
@@ -127,26 +137,30 @@ hipError_t launch_level(const StepArgs &a, bool root, hipStream_t s);
 // none failed).
 hipError_t launch_level_fix(const StepArgs &a, bool root, hipStream_t s);
 // The level's supports and its frequent-key list in key order: a pass that
-// counts the frequent keys of each tile of kReduceTile keys (and clears the
-// other keys' replicas), a scan of the tile counts, and a pass that writes
-// each tile's records from its first slot on.  tile_count holds
-// reduce_tiles(nkeys) entries.
-constexpr int kReduceTile = 256;
-__host__ __device__ inline int64_t reduce_tiles(int64_t nkeys) { return (nkeys + kReduceTile - 1) / kReduceTile; }
+// counts the frequent keys of each tile of a.tile_keys keys (and clears the
+// other keys' replicas), and a pass that writes each tile's records behind
+// those of the tiles before it.  At most kReduceTiles tiles (the second pass
+// adds their counts up), each a whole number of the workgroup's steps.
+constexpr int64_t kReduceTiles = 1024;
+constexpr int kReduceSplitRep = 8;  // replicas from which four lane groups share a key's
+inline int64_t reduce_tile_keys(int64_t nkeys, int rep) {
+  const int64_t step = rep >= kReduceSplitRep ? 64 : 256;
+  const int64_t steps = (nkeys + step * kReduceTiles - 1) / (step * kReduceTiles);
+  return step * (steps > 0 ? steps : 1);
+}
+__host__ __device__ inline int64_t reduce_tiles(const StepArgs &a) { return (a.nkeys + a.tile_keys - 1) / a.tile_keys; }
 hipError_t launch_reduce(const StepArgs &a, bool root, hipStream_t s);
 // Children of every chunk in chunks[0, n_chunks) (the whole level).
 hipError_t launch_write(const StepArgs &a, bool root, hipStream_t s);
 // Copy `bytes` (a multiple of 8) between device memory and mapped pinned
 // host memory with a kernel on stream s.
 hipError_t launch_copy8(void *dst, const void *src, size_t bytes, hipStream_t s);
-// Copy the children's upload (bytes, a multiple of 8) and, for the F
-// frequent keys (the keys of the frequent list a.freq, in its order):
-// sup[key] = -(fchild[i] + 1) for the chosen ones (fchild >= 0), their
-// (child, replica) cursors from row_base / list_base[child] and the
-// replicas' counts, and clear the keys' replicas.
-hipError_t launch_cursors(const StepArgs &a, void *dst, const void *src, size_t bytes, const int32_t *fchild,
-                          const unsigned long long *row_base, const unsigned long long *list_base, int64_t F,
-                          hipStream_t s);
+// For the F frequent keys (the keys of the frequent list a.freq, in its
+// order): sup[key] = -(fchild[i] + 1) for the chosen ones (fchild >= 0),
+// their (child, replica) cursors from row_base / list_base[child] and the
+// replicas' counts; the keys' replicas and the level's counters are cleared.
+hipError_t launch_cursors(const StepArgs &a, const int32_t *fchild, const unsigned long long *row_base,
+                          const unsigned long long *list_base, int64_t F, hipStream_t s);
 // Gather selected graphs of a resident packed database into a new one
 // (k_gather_graphs): per selected graph t, its source graph, first vertex
 // and first adjacency entry in the output, and its job.
@@ -181,6 +195,10 @@ struct CanonArgs {
   unsigned long long *freq;
   const uint32_t *freq_count;
   uint32_t freq_cap;
+  // mapped host copy of the first down_cap records' support words (record i
+  // at down[4 * i + 1]); null: none
+  unsigned long long *down;
+  uint32_t down_cap;
   // the level's patterns: nv from meta, len tuples each packed from | to << 8
   // | elabel << 16 | tolabel << 24 (dense labels), S vertex labels each
   // (S: the level's tuple stride; meta_bytes(S) bytes of metadata each)

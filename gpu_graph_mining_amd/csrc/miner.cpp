@@ -577,7 +577,7 @@ struct Counters {
   unsigned long long pad[6];
   unsigned long long spread[kSpread * kSpreadStride];
 };
-static_assert(sizeof(Counters) == 64 + 8 * kSpread * kSpreadStride, "counter block layout");
+static_assert(sizeof(Counters) == 8 * kCounterWords, "counter block layout");
 
 // Grow a workspace buffer; the stream is drained first because the old
 // allocation may still be in use by queued kernels.
@@ -659,9 +659,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   }
   w.acc_zero = false;  // until this call ends normally
 
-  grow(w.minsup, sizeof(int32_t) * opt.minsup.size(), s);
-  hip_check(hipMemcpyAsync(w.minsup.p, opt.minsup.data(), sizeof(int32_t) * opt.minsup.size(),
-                           hipMemcpyHostToDevice, s), "upload min supports");
+  if (opt.minsup.size() > 1) {  // a single job's goes with the kernel arguments
+    grow(w.minsup, sizeof(int32_t) * opt.minsup.size(), s);
+    hip_check(hipMemcpyAsync(w.minsup.p, opt.minsup.data(), sizeof(int32_t) * opt.minsup.size(),
+                             hipMemcpyHostToDevice, s), "upload min supports");
+  }
 
   double ext_ms = 0, dev_sec = 0, canon_sec = 0, ev_stage_ms = 0;
   uint64_t ext_launches = 0;
@@ -692,6 +694,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   Arr<uint64_t> nproj;    // per child: embeddings reported
   bool stopped = false;
   unsigned long long written_expect = 0;  // child rows asked of every k_write so far
+  bool written_pending = false;           // the last k_write's rows are not compared with it yet
   uint32_t last_fcount = 0;
   int table_bits = opt.table_bits > 0 ? opt.table_bits : 8;
   const int max_chunk_rows = opt.chunk_rows > 0 ? opt.chunk_rows : kChunkRows;
@@ -727,6 +730,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   };
   std::vector<DFS> orig;  // a reported code in the database's own labels
   bool counters_fresh = true;  // the counter block must be zeroed (first level, or it moved)
+  bool counters_clear = false;  // the level's counters are zero (k_cursors of the level before cleared them)
 
   // The levels being mined, the current one last.  A level is normally
   // expanded whole: its children become the next level and it is dropped.
@@ -836,7 +840,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     while (!w.arena && rep < 64 && (int64_t)rep * 2 * nkeys * 16 <= (64ll << 20) && (int64_t)rep * 2 * 32 <= total_chunks)
       rep *= 2;
     grow(w.sup, sizeof(int32_t) * std::max<int64_t>(nkeys, 1), s);
-    grow(w.tiles, sizeof(uint32_t) * std::max<int64_t>(reduce_tiles(nkeys), 1), s);
+    grow(w.tiles, sizeof(uint32_t) * kReduceTiles, s);
     grow_zero(w.acc, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
     grow_zero(w.accb, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
     grow(w.chunks, sizeof(ChunkInfo) * std::max<int64_t>(total_chunks, 1), s);
@@ -872,7 +876,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         // written rows of an earlier level live in the old block: checked already
         hip_check(launch_fill8(dctr, sizeof(Counters), s), "clear counters");
         written_expect = 0;
+        written_pending = false;
         counters_fresh = false;
+        counters_clear = true;
       }
       dctr_last = dctr;
       a.rccnt = w.rccnt.as<uint16_t>();
@@ -893,11 +899,21 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.nkeys = nkeys;
       a.p_base = (int32_t)p_begin;
       a.K = K;
-      a.minsup_job = w.minsup.as<int32_t>();
+      a.minsup_job = opt.minsup.size() > 1 ? w.minsup.as<int32_t>() : nullptr;
+      a.minsup_one = opt.minsup[0];
       a.freq = reinterpret_cast<unsigned long long *>(dctr + 1);
       a.freq_cap = fcap;
       a.freq_count = &dctr->fcount;
       a.tile_count = w.tiles.as<uint32_t>();
+      a.tile_keys = reduce_tile_keys(nkeys, rep);
+      // counters and (most often all of) the frequent keys come down with
+      // the list pass: into the mapped buffer
+      guess = std::min<uint32_t>(fcap, std::max<uint32_t>(1024, 2 * last_fcount));
+      const size_t head = sizeof(Counters) + sizeof(Freq) * guess;
+      hbuf = static_cast<const char *>(w.down.ensure(head));
+      a.counters = reinterpret_cast<const unsigned long long *>(dctr);
+      a.down = w.arena ? nullptr : static_cast<unsigned long long *>(w.down.dev);
+      a.down_cap = guess;
       a.pid = root ? nullptr : w.row(cur).pid.as<int32_t>();
       a.rgraph = root ? nullptr : w.row(cur).rgraph.as<int32_t>();
       a.vt = root ? nullptr : w.row(cur).vt.as<uint8_t>();
@@ -908,7 +924,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.mask_stride = root ? 0 : mask_stride;
       a.pmask = a.mask_stride ? reinterpret_cast<const unsigned long long *>(w.row(cur).upl.as<char>() + mask_off)
                               : nullptr;
-      hip_check(launch_clear_counters(a, s), "clear counters");
+      if (!counters_clear) hip_check(launch_clear_counters(a, s), "clear counters");
+      counters_clear = false;
       const bool time_stage = opt.stage_events && !root && !w.arena;
       if (time_stage) {
         for (hipEvent_t &e : w.ev)
@@ -942,6 +959,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         c.freq = a.freq;
         c.freq_count = a.freq_count;
         c.freq_cap = fcap;
+        c.down = a.down ? a.down + kCounterWords : nullptr;
+        c.down_cap = a.down_cap;
         c.meta = a.meta;
         c.p_base = (int32_t)p_begin;
         c.pcode = reinterpret_cast<const uint32_t *>(w.row(cur).upl.as<char>() + code_off);
@@ -955,11 +974,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         const int64_t grid = std::min<int64_t>(fcap, std::max<int64_t>(256, std::min<int64_t>(8192, 2 * (int64_t)last_fcount)));
         hip_check(launch_canon_level(c, (int)grid, s), "k_canon_level");
       }
-      // counters and (most often all of) the frequent keys in one copy
-      guess = std::min<uint32_t>(fcap, std::max<uint32_t>(1024, 2 * last_fcount));
-      const size_t head = sizeof(Counters) + sizeof(Freq) * guess;
-      hbuf = static_cast<const char *>(w.down.ensure(head));
-      stage_down(w, w.down, dctr, head, s);
+      if (!a.down) stage_down(w, w.down, dctr, head, s);
       hip_check(hipStreamSynchronize(s), "k_level");
       std::memcpy(&cnt, hbuf, sizeof(cnt));
       if (cnt.err) throw Error(GM_E_DEVICE, "internal: level step error " + std::to_string(cnt.err));
@@ -978,6 +993,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       if (written != written_expect)
         throw Error(GM_E_DEVICE, "child rows written (" + std::to_string(written) +
                                      ") differ from the embedding counts (" + std::to_string(written_expect) + ")");
+      written_pending = false;
       t_start = ~t_start;
       ms = (t_end > t_start && t_start != ~0ull) ? (double)(t_end - t_start) / wall_khz : 0.0;
       if (time_stage) {
@@ -1281,9 +1297,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     if (F > 0) stage_up(w, w.up, fc_off, masks_off - fc_off, s);  // child ids, bases
     if (F > 0 && C == 0) {  // nothing to write: the frequent keys' replicas are cleared
       const char *su = static_cast<const char *>(w.up.dev);
-      hip_check(launch_cursors(a, nullptr, nullptr, 0, reinterpret_cast<const int32_t *>(su + fc_off), nullptr, nullptr,
-                               F, s),
-                "k_cursors");
+      hip_check(launch_cursors(a, reinterpret_cast<const int32_t *>(su + fc_off), nullptr, nullptr, F, s), "k_cursors");
+      counters_clear = true;
     }
     if (C > 0) {
       // The embedding counts size the child level exactly; k_write reserves
@@ -1329,12 +1344,14 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.n_chunks = total_chunks;
       // child ids and cursors, then the write pass (launched back to back:
       // the device does not wait on the host between)
-      hip_check(launch_cursors(a, du, su, 0, reinterpret_cast<const int32_t *>(su + fc_off),
+      hip_check(launch_cursors(a, reinterpret_cast<const int32_t *>(su + fc_off),
                                reinterpret_cast<const unsigned long long *>(su + rb_off),
                                reinterpret_cast<const unsigned long long *>(su + lb_off), F, s),
                 "k_cursors");
       hip_check(launch_write(a, root, s), "k_write");
       written_expect += (unsigned long long)child_rows;
+      written_pending = true;
+      counters_clear = true;
       us_host = t_host.sec() * 1e6;
 
       // while the device writes the children: the canonical check of the
@@ -1563,8 +1580,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       cf.codes_ready = want_codes;
     }
   }
-  // the last write's row count
-  if (written_expect) {
+  // the last write's row count, when no level after it compared it
+  if (written_pending) {
     Counters c;
     hip_check(hipMemcpyAsync(&c, w.freq.p, sizeof(c), hipMemcpyDeviceToHost, s), "download counters");
     hip_check(hipStreamSynchronize(s), "mining");
