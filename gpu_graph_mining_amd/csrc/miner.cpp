@@ -1262,8 +1262,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     const size_t lb_off = rb_off + sizeof(unsigned long long) * C;
     // path masks of the children with >= 2 edges: a forward and a
     // backward word per rightmost-path vertex (at most max_nv of them)
-    // (a 2-edge level written in pieces leaves no complete path table)
-    if (new_len == 2 && !(p_begin == 0 && p_end == P && key_lo == 0 && key_cut == ~0ull)) t2_partial = true;
+    // (a 2-edge level written in pieces leaves no complete path table, nor
+    // does a job's root level cut by key: each piece's children have only
+    // their own 2-edge patterns)
+    const bool keys_whole = key_lo == 0 && key_cut == ~0ull;
+    if ((new_len == 1 && !keys_whole) || (new_len == 2 && !(p_begin == 0 && p_end == P && keys_whole))) t2_partial = true;
     const bool masks = prune && !t2_partial && new_len >= 2 && C > 0;
     const int mstride = masks ? max_nv : 0;
     const size_t masks_off = lb_off + sizeof(unsigned long long) * C;
