@@ -26,7 +26,7 @@ ARCH = os.environ.get("GM_OFFLOAD_ARCH", "gfx950")
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-parameter", f"-I{PKG.parent / 'include'}"]
 
-DEVICE_SOURCES = ["kernels.hip", "canon.hip"]
+DEVICE_SOURCES = ["kernels.hip", "compact.hip", "canon.hip"]
 HOST_SOURCES = ["capi.cpp", "miner.cpp", "canonical.cpp", "host_db.cpp", "generators.cpp"]
 
 

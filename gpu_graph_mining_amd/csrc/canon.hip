@@ -352,7 +352,7 @@ __global__ void __launch_bounds__(64) k_canon_level(CanonArgs c) {
     const unsigned long long key = f[0];
     const int64_t p = (int64_t)(key / (unsigned long long)c.K) + c.p_base;
     const int64_t x = (int64_t)(key % (unsigned long long)c.K);
-    const int nvp = meta_at(c.meta, c.S, p)->nv;
+    const int nvp = meta_at(c.meta, c.meta_stride, p)->nv;
     const int len = c.len;
     __syncthreads();  // the previous key's LDS is no longer read
     for (int t = lane; t < len && t < kCE; t += 64) {

@@ -1,0 +1,756 @@
+// compact.hip -- level-step kernels of the compact databases (gfx950, wave64).
+//
+// A database is compact when every graph has at most 64 vertices, its label
+// alphabets are small (NEL * (NVL + 1) <= 63) and a graph's vertices fit 255
+// groups (below): transactions, molecules, random graphs of the common
+// sizes.  The kernels of kernels.hip mine the others, and all databases under
+// the entry point that allocates nothing.
+//
+// Layout.  A vertex is one 8-byte *group* at vgrp[g + u] (g the graph's first
+// group, u the local id): four items (neighbour 6 bits, label pair
+// edge label * NVL + neighbour label 6 bits) of 12 bits, two per word, and in
+// the top byte of the first word the place (relative to g) of a further group
+// when the vertex has more than four neighbours.  One gather per rightmost-path
+// source fetches all of the common vertices' neighbours; nothing depends on an
+// offset read first.  (With a 4-byte offset and 4-byte entries a row's sources
+// touched 4-5 lines of 128 bytes per segment, in two dependent steps.)
+//
+// Rows are {g, tuple} of 1 + TW words (tuple bytes past the pattern's vertices
+// repeat vertex 0's, so that the visited set is an OR over all bytes),
+// pattern-major; a chunk is a run of
+// whole segments (rows of one graph) of ONE pattern, so everything about the
+// pattern is wave-uniform: the sources are walked in a scalar loop, and the
+// label rules of a source (order rule, minimum label, 2-edge path masks) are a
+// 64-bit mask over label pairs that the host prepares.  An item is tested with
+// two shifts: its label pair against the mask, its neighbour against the
+// row's visited set.
+//
+// Per block of up to 64 rows and per source, the passing items are counted,
+// ranked over the wave and appended to the chunk's dense list
+//   key << 20 | neighbour << 14 | row of the chunk
+// (4 bytes a candidate; entry key 0xFFF moves the row base on by kMarkRows).
+// Counts live in LDS tables indexed by the key itself (K <= 4032; no hashing,
+// no overflow).  A key names its source, and within a source the list is in
+// row order, so every key's entries are in row order: k_cwrite can place the
+// children's rows graph-contiguously in list order.
+//
+// What bounds them: vector instruction issue and the group gathers' latency;
+// k_level of kernels.hip spends about 2,500 vector instructions on a 64-row
+// block of 8-byte tuples with half of its lanes idle.
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <type_traits>
+
+#include "device.hpp"
+#include "kernels.hpp"
+#include "wave.hpp"
+
+namespace gm {
+namespace {
+
+constexpr uint32_t kNone32 = 0xFFFFFFFFu;
+constexpr uint32_t kMarkKey = 0xFFFu;
+constexpr int kMarkRows = 8192;
+
+// (lambdas used several times must not become calls: a call needs scratch)
+#define GM_INLINE __attribute__((always_inline))
+
+// wave-uniform read-only data through the scalar cache
+typedef const uint32_t __attribute__((address_space(4))) *ConstWords;
+template <class T>
+__device__ __forceinline__ T cload(ConstWords c) {
+  uint32_t w[sizeof(T) / 4];
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(T) / 4); ++i) w[i] = c[i];
+  T t;
+  __builtin_memcpy(&t, w, sizeof(t));
+  return t;
+}
+template <class T>
+__device__ __forceinline__ T cload(const void *p) {
+  return cload<T>((ConstWords)(uintptr_t)p);
+}
+
+// A kernel argument read where it is used (from the argument segment,
+// through the scalar cache) instead of held in scalar registers from the
+// kernel's start on: k_clevel uses some thirty of them, most of them once.
+#define GM_ARG(field) arg_at<decltype(StepArgs::field), offsetof(StepArgs, field)>()
+template <class T, size_t kOffset>
+__device__ __forceinline__ T arg_at() {
+  ConstWords c = (ConstWords)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(c));
+  return cload<T>(c + kOffset / 4);
+}
+
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// lanes below this one in a ballot
+__device__ __forceinline__ uint32_t below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+template <int TW>
+struct CRow {
+  uint32_t x[1 + TW];
+};
+
+// The graph vertex at pattern vertex i (wave-uniform).  Masks, not selects:
+// the compiler turns a chain of selects into an indexed array in scratch.
+template <int TW>
+__device__ __forceinline__ uint32_t image(const CRow<TW> &t, int i) {
+  uint32_t x = 0;
+#pragma unroll
+  for (int q = 0; q < TW; ++q) x |= t.x[1 + q] & (0u - (uint32_t)((i >> 2) == q));
+  return (x >> ((i & 3) * 8)) & 0xFFu;
+}
+
+// Groups are held as 64-bit values: items at bits 0, 12, 32 and 44, the next
+// group's place at bits 24-31.
+typedef unsigned long long Group;
+constexpr Group kEmptyGroup = (Group)(kEmptyItem | kEmptyItem << 12) << 32 | (kEmptyItem | kEmptyItem << 12);
+__device__ __forceinline__ uint32_t next_of(Group g) { return (uint32_t)g >> 24; }
+// item i (0..7) of a vertex's first two groups
+__device__ __forceinline__ uint32_t item(Group p, Group o, int i) {
+  const Group g = (i & 4) ? o : p;
+  return (uint32_t)(g >> ((i & 1) * 12 + (i & 2) * 16)) & 0xFFFu;
+}
+
+// The chunk's candidate list: extents of entries, the first at
+// chunk * page, further ones from the pool (64 slices with a cursor each on a
+// line of its own).  An extent starts with {entries, next extent or kNone32};
+// extents are named in units of kListUnit entries.
+struct ListOut {
+  uint32_t *ext;
+  uint32_t used, cap;
+  bool off;  // the pool ran out: the stage runs again with a larger one
+};
+
+template <bool ROOT, int TW, bool M32>
+__global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_clevel(StepArgs) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
+  const int K = (int)GM_ARG(K);
+  unsigned long long *const kmask = reinterpret_cast<unsigned long long *>(dyn);  // segments of the block, by head lane
+  uint32_t *const ksup = dyn + 2 * K, *const kemb = dyn + 3 * K;
+  const int lane = threadIdx.x;
+  const uint32_t gci = blockIdx.x;
+  if (gci < (uint32_t)kSpread) stamp_start(GM_ARG(spread), gci);
+
+  // the chunk: pattern p, nominal rows [nom0, nom1) of the pattern's pend
+  // (relative to its first row: a pattern has fewer than 2^32), moved
+  // forward to segment starts
+  constexpr int RW = 1 + TW;
+  int p;
+  uint32_t nom0, pend;
+  uint64_t first;
+  const char *meta = nullptr;
+  CMetaHead H = {};
+  const uint32_t nom = (uint32_t)GM_ARG(nom);
+  if constexpr (ROOT) {
+    const uint4 ct = cload<uint4>(GM_ARG(rtab) + GM_ARG(tab0) + gci);
+    p = (int)ct.x;
+    first = ct.z;
+    pend = ct.w;
+    nom0 = ct.y * nom;
+  } else {
+    const uint2 ct = cload<uint2>(GM_ARG(ctab) + GM_ARG(tab0) + gci);
+    p = uniform((int)ct.x);
+    meta = reinterpret_cast<const char *>(GM_ARG(meta)) + (int64_t)p * GM_ARG(meta_stride);
+    H = cload<CMetaHead>(meta);
+    first = H.row0;
+    pend = (uint32_t)H.nrows;
+    nom0 = (uint32_t)uniform((int)ct.y) * nom;
+  }
+  const uint32_t nom1 = pend - nom0 <= nom ? pend : nom0 + nom;
+  const uint32_t *const rows = GM_ARG(crow) + first * RW;
+  uint32_t b = nom0;
+  bool empty = !ROOT && (H.flags & kPatDead);
+  if (!empty && nom0 > 0) {
+    for (uint64_t base = nom0;; base += 64) {
+      if (base >= nom1) {
+        empty = true;
+        break;
+      }
+      const uint64_t r = base + (uint32_t)lane;
+      const bool f = r < pend && rows[r * RW] != rows[(r - 1) * RW];
+      const uint64_t m = __ballot(f);
+      if (m) {
+        b = (uint32_t)base + (uint32_t)__ffsll((long long)m) - 1u;
+        empty = b >= nom1;
+        break;
+      }
+    }
+  }
+  if (empty) {
+    if (lane == 0) GM_ARG(cchunks)[gci] = CChunk{0, 0, 0u};
+    return;
+  }
+  const uint32_t start = b;
+  for (int i = lane; i < K; i += 64) {
+    kmask[i] = 0;
+    ksup[i] = 0;
+    kemb[i] = 0;
+  }
+  wave_sync();
+
+  const uint32_t page = GM_ARG(page);
+  ListOut L{GM_ARG(clist) + (uint64_t)gci * page, 2u, page, false};
+  // room for n entries in one extent: their place in it
+  auto reserve = [&](uint32_t n) GM_INLINE -> uint32_t {
+    if (L.used + n > L.cap) {
+      const uint32_t units = (max(page, n + 2u) + kListUnit - 1) / kListUnit;
+      uint32_t at = kNone32;
+      if (lane == 0 && !L.off) {
+        unsigned long long *const spread = GM_ARG(spread);
+        const uint32_t sub_size = GM_ARG(pool_sub), pool0 = GM_ARG(pool0);
+        for (uint32_t t = 0; t < (uint32_t)kSpread && at == kNone32; ++t) {
+          const uint32_t sub = (gci + t) & (kSpread - 1);
+          const unsigned long long o = atomicAdd(&spread[sub * kSpreadStride + kSpreadPool], (unsigned long long)units);
+          if (o + units <= (unsigned long long)sub_size) at = pool0 + sub * sub_size + (uint32_t)o;
+        }
+        L.ext[0] = L.used - 2u;
+        L.ext[1] = at;
+        if (at == kNone32) atomicOr(GM_ARG(error_flag), kErrListPool);
+      }
+      at = (uint32_t)uniform((int)at);
+      L.off = L.off || at == kNone32;
+      if (!L.off) L.ext = GM_ARG(clist) + (uint64_t)at * kListUnit;
+      L.used = 2u;
+      L.cap = L.off ? kNone32 - 1u : units * kListUnit;
+    }
+    const uint32_t pos = L.used;
+    L.used += n;
+    return pos;
+  };
+
+  uint32_t n_pruned = 0;
+  unsigned long long listed = 0;
+  bool carry = false;   // the block's first rows may go on with the last block's segment
+  uint32_t carry_g = 0;  // of this graph
+  uint32_t rowbase = 0;  // rows of the chunk before the list's current row base
+  for (;;) {
+    const int ws = (int)min(64u, pend - b);
+    CRow<TW> t;
+    {
+      const uint32_t *src = rows + ((uint64_t)b + (uint32_t)min(lane, ws - 1)) * RW;
+      __builtin_memcpy(&t, src, sizeof(t));
+    }
+    const uint32_t g = t.x[0];
+    const uint32_t pg = __shfl_up(g, 1, 64);
+    const uint64_t diff = __ballot(lane < ws && (lane == 0 ? !carry || g != carry_g : pg != g));
+    if (carry && (diff & 1ull)) {  // it ended with the last block: its keys' marks are done with
+      for (int i = lane; i < K; i += 64) {
+        ksup[i] &= 0x7FFFFFFFu;
+        kmask[i] = 0;
+      }
+      wave_sync();
+    }
+    // the block: up to the first segment start at or past nom1 (none of the
+    // window's rows when a carried segment ended with the last block there),
+    // to the pattern's end, or to the window's last segment start (its segment may
+    // go on); a window that is one segment is taken whole and carried on
+    int nb;
+    bool last = true, carry_out = false;
+    {
+      uint64_t after = 0;
+      if (nom1 < pend && (nom1 <= b || nom1 - b < 64)) after = diff & (nom1 <= b ? ~0ull : ~0ull << (nom1 - b));
+      const uint64_t later = diff & ~1ull;
+      if (after) {
+        nb = __ffsll((long long)after) - 1;
+      } else if (pend - b == (uint32_t)ws) {
+        nb = ws;
+      } else {
+        last = false;
+        if (later) {
+          nb = 63 - __clzll((long long)later);
+        } else {
+          nb = 64;
+          carry_out = true;
+        }
+      }
+    }
+    const bool live = lane < nb;
+    const uint64_t starts = nb == 64 ? diff : diff & ((1ull << nb) - 1ull);
+    const unsigned long long hbit = 1ull << head_lane(starts, lane);
+    while (b - start - rowbase >= (uint32_t)kMarkRows) {  // (rows of a block stay below kMarkRows + 64 < 2^14)
+      const uint32_t pos = reserve(1);
+      if (lane == 0 && !L.off) L.ext[pos] = kMarkKey << 20;
+      rowbase += kMarkRows;
+    }
+    const uint32_t rowrel = b - start - rowbase + (uint32_t)lane;
+
+    // the row's visited vertices
+    unsigned long long used = 0;
+    if constexpr (ROOT) {
+      used = 1ull << (t.x[1] & 63u);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4 * TW; ++i)
+        used |= 1ull << ((t.x[1 + i / 4] >> ((i & 3) * 8)) & 63u);
+    }
+
+    const Group *const vgrp = GM_ARG(vgrp);
+    auto load_group = [&](uint32_t off) GM_INLINE -> Group { return vgrp[(uint64_t)g + off]; };
+    const int nsrc = ROOT ? 1 : H.nsrc;
+    const char *srcs = meta + sizeof(CMetaHead);
+    auto load_src = [&](int j) GM_INLINE -> Group {
+      if (!live) return kEmptyGroup;
+      if constexpr (ROOT) return load_group(t.x[1] & 63u);
+      return load_group(image<TW>(t, cload<int>(srcs + j * (int)sizeof(CSource) + 16)));
+    };
+    auto load_next = [&](Group q) GM_INLINE -> Group {
+      Group o = kEmptyGroup;
+      if (next_of(q)) o = load_group(next_of(q));
+      return o;
+    };
+    // a lane's items past its first two groups, one group at a time
+    auto walk_on = [&](Group o, auto &&fn) GM_INLINE {
+      uint32_t nx = next_of(o);
+      while (nx) {
+        const Group c = load_group(nx);
+        for (int i = 0; i < 4; ++i) fn(item(c, c, i));
+        nx = next_of(c);
+      }
+    };
+    auto emit = [&](uint32_t pos, uint32_t key, uint32_t w) GM_INLINE {
+      if (!L.off) L.ext[pos] = key << 20 | w << 14 | rowrel;
+      atomicOr(&kmask[key], hbit);
+      atomicAdd(&kemb[key], 1u);
+    };
+
+    Group P = load_src(0), Pn = nsrc > 1 ? load_src(1) : kEmptyGroup;
+    Group O = load_next(P);
+    for (int j = 0; j < nsrc; ++j) {
+      // the groups of the next two sources are in flight while this one's
+      // items are tested
+      const Group Pnn = j + 2 < nsrc ? load_src(j + 2) : kEmptyGroup;
+      const Group On = j + 1 < nsrc ? load_next(Pn) : kEmptyGroup;
+      const bool deep = __ballot(next_of(O) != 0) != 0;  // some vertex has more than eight neighbours
+
+      // backward: from the rightmost vertex (source 0) to the images of the
+      // path vertices the host lists
+      if constexpr (!ROOT) {
+        if (j == 0 && H.nback) {
+          const char *backs = srcs + nsrc * (int)sizeof(CSource);
+          unsigned long long bset = 0;
+          for (int q = 0; q < H.nback; ++q)
+            bset |= 1ull << image<TW>(t, cload<int>(backs + q * (int)sizeof(CSource) + 16));
+          uint32_t hit = 0;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const uint32_t x = item(P, O, i);
+            hit |= (uint32_t)(bset >> (x & 63u)) & (x >> 6 != 63u ? 1u : 0u);
+          }
+          if (deep || __ballot(hit != 0)) {
+            for (int q = 0; q < H.nback; ++q) {
+              const CSource bk = cload<CSource>(backs + q * (int)sizeof(CSource));
+              const uint32_t v = image<TW>(t, bk.from);
+              uint32_t lab = 63;
+              auto match = [&](uint32_t x) GM_INLINE { lab = (x & 63u) == v ? min(lab, x >> 6) : lab; };
+#pragma unroll
+              for (int i = 0; i < 8; ++i) match(item(P, O, i));
+              walk_on(O, match);
+              const bool ok = live && ((bk.rule >> lab) & 1ull), kept = ok && ((bk.keep >> lab) & 1ull);
+              n_pruned += ok && !kept ? 1u : 0u;
+              const uint64_t m = __ballot(kept);
+              if (m) {
+                const uint32_t pos = reserve((uint32_t)__popcll(m)) + below(m);
+                listed += (unsigned long long)__popcll(m);
+                if (kept) emit(pos, (uint32_t)bk.kbase + ((lab * GM_ARG(inv_nvl)) >> 16), 0u);
+              }
+            }
+          }
+        }
+      }
+
+      // forward to unvisited neighbours whose label pair the source's rule
+      // lets through
+      typedef typename std::conditional<M32, uint32_t, unsigned long long>::type Mask;
+      Mask rule, keep;
+      uint32_t kbase;
+      bool masked = false;
+      if constexpr (ROOT) {
+        // from a vertex to neighbours of its label or a larger one
+        const uint32_t lu = (t.x[1] >> 8) & 0xFFu;
+        const unsigned long long nl = ((1ull << GM_ARG(NVL)) - 1ull) & (~0ull << lu);
+        rule = keep = (Mask)(nl * GM_ARG(lab_rep));
+        kbase = lu * (uint32_t)GM_ARG(AR);
+      } else {
+        const CSource sc = cload<CSource>(srcs + j * (int)sizeof(CSource));
+        rule = (Mask)sc.rule;
+        keep = (Mask)sc.keep;
+        masked = sc.keep != sc.rule;
+        kbase = (uint32_t)sc.kbase;
+      }
+      auto passes = [&](uint32_t x) GM_INLINE -> uint32_t {
+        return (uint32_t)(rule >> (x >> 6 & (M32 ? 31u : 63u))) & ~(uint32_t)(used >> (x & 63u)) & 1u;
+      };
+      auto keeps = [&](uint32_t x) GM_INLINE -> uint32_t { return (uint32_t)(keep >> (x >> 6 & (M32 ? 31u : 63u))) & 1u; };
+      uint32_t m = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m |= passes(item(P, O, i)) << i;
+      if (__ballot(next_of(P) != 0)) {
+#pragma unroll
+        for (int i = 4; i < 8; ++i) m |= passes(item(P, O, i)) << i;
+      }
+      if (masked) {
+        uint32_t k = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) k |= keeps(item(P, O, i)) << i;
+        n_pruned += (uint32_t)__popc(m & ~k);
+        m &= k;
+      }
+      uint32_t total, off;
+      if (!deep) {
+        const uint32_t c = (uint32_t)__popc(m);
+        const uint64_t b0 = __ballot(c & 1u), b1 = __ballot(c & 2u), b2 = __ballot(c & 4u), b3 = __ballot(c & 8u);
+        total = (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2) + 8 * __popcll(b3));
+        off = below(b0) + 2u * below(b1) + 4u * below(b2) + 8u * below(b3);
+      } else {
+        uint32_t c = (uint32_t)__popc(m);
+        walk_on(O, [&](uint32_t x) GM_INLINE {
+          const uint32_t ok = passes(x), kp = ok & keeps(x);
+          n_pruned += ok & ~kp;
+          c += kp;
+        });
+        off = wave_exclusive_scan<uint32_t>(c, total);
+        total = (uint32_t)uniform((int)total);
+      }
+      if (total) {
+        listed += total;
+        uint32_t pos = reserve(total) + off;
+        while (m) {
+          const int i = __ffs((int)m) - 1;
+          m &= m - 1;
+          const uint32_t x = item(P, O, i);
+          emit(pos++, kbase + (x >> 6), x & 63u);
+        }
+        if (deep)
+          walk_on(O, [&](uint32_t x) GM_INLINE {
+            if (passes(x) & keeps(x)) emit(pos++, kbase + (x >> 6), x & 63u);
+          });
+      }
+      P = Pn;
+      O = On;
+      Pn = Pnn;
+    }
+    wave_sync();
+    // support: one per segment of the block that holds the key, less a
+    // segment carried in; a carried-out segment keeps its bit (head lane 0)
+    // and is marked as counted in bit 31
+    for (int i = lane; i < K; i += 64) {
+      const unsigned long long m = kmask[i];
+      if (m) {
+        const uint32_t sv = ksup[i];
+        const uint32_t kp = carry_out ? (uint32_t)(m & 1ull) : 0u;
+        ksup[i] = ((sv & 0x7FFFFFFFu) + (uint32_t)__popcll(m) - (sv >> 31)) | (kp << 31);
+        kmask[i] = kp;
+      }
+    }
+    wave_sync();
+    if (last) break;
+    b += (uint32_t)nb;
+    carry = carry_out;
+    carry_g = (uint32_t)uniform((int)g);  // (a carried block is one segment)
+  }
+  // close the list, commit the counts to the chunk's replica and keep the
+  // chunk's {key, embeddings} records behind the list
+  uint32_t nrec = 0;
+  for (int i0 = 0; i0 < K; i0 += 64) nrec += (uint32_t)__popcll(__ballot(i0 + lane < K && kemb[min(i0 + lane, K - 1)] != 0));
+  uint32_t *const ext0 = L.ext;
+  const uint32_t n0 = L.used - 2u;
+  uint32_t at = 0;
+  if (nrec) {
+    at = reserve(2u * nrec);
+    const uint32_t n = L.ext == ext0 ? n0 : 0u;  // a new extent for the records closed the old one
+    if (lane == 0 && !L.off) {
+      L.ext[0] = n;
+      L.ext[1] = kNone32;
+    }
+  }
+  unsigned long long *const acc = GM_ARG(acc) + (int64_t)(gci & (uint32_t)(GM_ARG(rep) - 1)) * GM_ARG(nkeys) +
+                                  (int64_t)(p - GM_ARG(p_base)) * K;
+  uint32_t w = at;
+  for (int i0 = 0; i0 < K; i0 += 64) {
+    const int i = i0 + lane;
+    const uint32_t e = i < K ? kemb[i] : 0u;
+    const uint64_t m = __ballot(e != 0);
+    if (e) {
+      atomicAdd(&acc[i], ((unsigned long long)ksup[i] << kSupShift) | (unsigned long long)e);
+      if (!L.off) {
+        const uint32_t q = w + 2u * below(m);
+        L.ext[q] = (uint32_t)i;
+        L.ext[q + 1] = e;
+      }
+    }
+    w += 2u * (uint32_t)__popcll(m);
+  }
+  const unsigned long long w_pruned = wave_sum((unsigned long long)n_pruned);
+  if (lane == 0) {
+    GM_ARG(cchunks)[gci] = CChunk{(int64_t)(first + start), (uint64_t)(L.ext - GM_ARG(clist)) + at, L.off ? 0u : nrec};
+    unsigned long long *const spread = GM_ARG(spread), *const line = spread + (gci & (kSpread - 1)) * kSpreadStride;
+    if (listed + w_pruned) atomicAdd(&line[kSpreadCand], listed + w_pruned);
+    if (w_pruned) atomicAdd(&line[kSpreadPruned], w_pruned);
+    atomicMax(&line[kSpreadFill], (unsigned long long)nrec);
+    stamp_end(spread, gci);
+  }
+}
+
+// ------------------------------------------------------------------ WRITE
+// One wave per chunk: the records name the chunk's keys; those that became
+// children get a small index and a run of the child's rows (one atomic on
+// the (child, replica) cursor), then the list is taken 64 entries at a time:
+// an entry's child index comes from an LDS map of its key, its position is
+// the child's run plus its rank among the window's entries of the same child
+// (one ballot per index bit: a chunk's pattern has one to a few children),
+// and the parent's row is read with the new vertex put in.  Chunks without
+// children read no list.
+constexpr int kWinUnroll = 2;  // windows whose loads are issued together
+
+template <bool ROOT, int TW>
+__global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
+  const int K = (int)a.K;
+  unsigned long long *const cbase = reinterpret_cast<unsigned long long *>(dyn);
+  uint32_t *const crun = dyn + 2 * K;
+  uint16_t *const cmap = reinterpret_cast<uint16_t *>(dyn + 3 * K);
+  const int lane = threadIdx.x;
+  const uint32_t gci = blockIdx.x;
+  const CChunk c = cload<CChunk>(a.cchunks + gci);
+  if (c.nrec == 0) return;
+  const int p = ROOT ? (int)cload<uint4>(a.rtab + a.tab0 + gci).x : (int)cload<uint2>(a.ctab + a.tab0 + gci).x;
+  for (int i = lane; i < K; i += 64) cmap[i] = 0;
+  wave_sync();
+  const int64_t kb = (int64_t)(p - a.p_base) * K;
+  const int64_t rsel = (int64_t)(gci & (uint32_t)(a.rep - 1));
+  int nchild = 0;
+  for (uint32_t i0 = 0; i0 < c.nrec; i0 += 64) {
+    const uint32_t i = i0 + lane;
+    int32_t ch = -1;
+    uint32_t key = 0, n = 0;
+    if (i < c.nrec) {
+      key = a.clist[c.rec + 2u * i];
+      n = a.clist[c.rec + 2u * i + 1u];
+      const int32_t v = a.sup[kb + key];
+      ch = v < 0 ? -v - 1 : -1;
+    }
+    const uint64_t m = __ballot(ch >= 0);
+    if (ch >= 0) {
+      const int ix = nchild + (int)below(m);
+      cmap[key] = (uint16_t)(ix + 1);
+      cbase[ix] = atomicAdd(&a.cursor[(int64_t)ch * a.rep + rsel], (unsigned long long)n);
+      crun[ix] = 0;
+    }
+    nchild += __popcll(m);
+  }
+  if (nchild == 0) return;
+  wave_sync();
+  const int bits = nchild > 1 ? 32 - __clz(nchild - 1) : 0;
+  constexpr int RW = 1 + TW;
+  const int CW = a.CS >> 2;
+  const int nvp = ROOT ? 1 : (int)cload<CMetaHead>(reinterpret_cast<const char *>(a.meta) + (int64_t)p * a.meta_stride).nv;
+  const uint32_t SB = (uint32_t)(a.S * a.NEL);  // first forward key
+  unsigned long long written = 0;
+  uint32_t rowbase = 0;
+  for (const uint32_t *ext = a.clist + (uint64_t)gci * a.page;;) {
+    const uint32_t n = (uint32_t)uniform((int)ext[0]), next = (uint32_t)uniform((int)ext[1]);
+    const uint32_t *list = ext + 2;
+    for (uint32_t j0 = 0; j0 < n; j0 += 64 * kWinUnroll) {
+      uint32_t e[kWinUnroll];
+      int ix[kWinUnroll];
+      CRow<TW> t[kWinUnroll];
+#pragma unroll
+      for (int u = 0; u < kWinUnroll; ++u) {
+        const uint32_t j = j0 + u * 64 + lane;
+        e[u] = j < n ? list[j] : kNone32;
+      }
+#pragma unroll
+      for (int u = 0; u < kWinUnroll; ++u) {
+        const uint32_t key = e[u] >> 20;
+        // entries past the end read as marks too, at the lanes behind all others
+        const uint64_t marks = __ballot(key == kMarkKey);
+        uint32_t row = rowbase + (e[u] & 0x3FFFu);
+        if (marks) {
+          row += (uint32_t)kMarkRows * below(marks);
+          rowbase += (uint32_t)kMarkRows * (uint32_t)__popcll(__ballot(key == kMarkKey && e[u] != kNone32));
+        }
+        ix[u] = key < (uint32_t)K ? (int)cmap[key] - 1 : -1;
+        if (ix[u] >= 0) {
+          const uint32_t *src = a.crow + (c.start + (int64_t)row) * RW;
+          __builtin_memcpy(&t[u], src, sizeof(t[u]));
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kWinUnroll; ++u) {
+        const bool sel = ix[u] >= 0;
+        const uint64_t active = __ballot(sel);
+        if (!active) continue;
+        written += (unsigned long long)__popcll(active);
+        const uint32_t h = sel ? (uint32_t)ix[u] : 0u;
+        uint64_t peers = active;
+        for (int bit = 0; bit < bits; ++bit) {
+          const bool hb = (h >> bit) & 1u;
+          const uint64_t m = __ballot(sel && hb);
+          peers &= hb ? m : ~m;
+        }
+        const uint32_t rank = below(peers);
+        const uint32_t run = sel ? crun[h] : 0u;
+        wave_sync();
+        if (sel && rank == 0) crun[h] = run + (uint32_t)__popcll(peers);
+        wave_sync();
+        if (sel) {
+          const unsigned long long pos = cbase[h] + (unsigned long long)run + rank;
+          const uint32_t key = e[u] >> 20, w = (e[u] >> 14) & 63u;
+          if ((int64_t)pos < a.ccap) {
+            uint32_t out[2 + TW];
+            out[0] = t[u].x[0];
+            const uint32_t v0 = t[u].x[1] & 0xFFu;
+            const uint32_t fill = v0 * 0x01010101u;  // past the pattern's vertices: vertex 0 again
+            if constexpr (ROOT) {
+              out[1] = (fill & 0xFFFF00FFu) | w << 8;
+              out[2] = fill;
+            } else {
+              const uint32_t put = w << ((nvp & 3) * 8), clear = ~(0xFFu << ((nvp & 3) * 8));
+#pragma unroll
+              for (int q = 0; q <= TW; ++q) {
+                const uint32_t word = q < TW ? t[u].x[q < TW ? 1 + q : 1] : fill;
+                out[1 + q] = key >= SB && (nvp >> 2) == q ? (word & clear) | put : word;
+              }
+            }
+            uint32_t *dst = a.crow_out + pos * (unsigned long long)(1 + CW);
+            if (CW == 1) {
+              __builtin_memcpy(dst, out, 8);
+            } else if (TW >= 1 && CW == 2) {
+              __builtin_memcpy(dst, out, 12);
+            } else {
+#pragma unroll
+              for (int q = 0; q < 2 + TW; ++q)
+                if (q <= CW) dst[q] = out[q];
+              for (int q = 2 + TW; q <= CW; ++q) dst[q] = fill;
+            }
+          }
+        }
+      }
+    }
+    if (next == kNone32) break;
+    ext = a.clist + (uint64_t)next * kListUnit;
+  }
+  if (lane == 0 && written)
+    atomicAdd(&a.spread[(gci & (kSpread - 1)) * kSpreadStride + kSpreadWritten], written);
+}
+
+// After the host chose the children (see k_cursors): every (child, replica)'s
+// cursor starts at its first row, and the children's chunk table is filled
+// ({child, chunk of the child}).  `rep` lanes take one frequent key.
+__global__ void __launch_bounds__(256) k_ccursors(StepArgs a, const int32_t *fchild, const unsigned long long *row_base,
+                                                  const uint32_t *chunk_base, int64_t F) {
+  if (blockIdx.x == 0) clear_counters(a);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = t / a.rep;
+  const int r = (int)(t % a.rep);
+  const bool ok = i < F;
+  int64_t key = 0, at = 0;
+  int32_t ch = -1;
+  unsigned long long rows = 0;
+  if (ok) {
+    key = (int64_t)a.freq[4 * i];
+    at = (int64_t)r * a.nkeys + key;
+    ch = fchild[i];
+    rows = a.acc[at] & ((1ull << kSupShift) - 1);
+  }
+  unsigned long long sr = rows;  // inclusive scan over the key's replicas
+  for (int o = 1; o < a.rep; o <<= 1) {
+    const unsigned long long y = __shfl_up(sr, o, 64);
+    if (r >= o) sr += y;
+  }
+  const unsigned long long all = __shfl(sr, ((threadIdx.x & 63) | (a.rep - 1)), 64);
+  if (!ok) return;
+  a.acc[at] = 0;
+  if (ch < 0) return;
+  if (r == 0) a.sup[key] = -(ch + 1);
+  a.cursor[(int64_t)ch * a.rep + r] = row_base[ch] + (sr - rows);
+  const uint32_t n = (uint32_t)((all + (unsigned long long)a.child_nom - 1) / (unsigned long long)a.child_nom);
+  uint2 *tab = a.child_tab + chunk_base[ch];
+  for (uint32_t k = (uint32_t)r; k < n; k += (uint32_t)a.rep) tab[k] = make_uint2((uint32_t)ch, k);
+}
+
+// A compact database of selected graphs gathered from a resident one: one
+// workgroup per selected graph t copies its groups (their links are relative)
+// and its root rows, rebased to the new first group dgb[t].
+__global__ void __launch_bounds__(64) k_cgather(CGatherArgs g) {
+  const int64_t t = blockIdx.x;
+  const int32_t src = g.sel[t];
+  const uint32_t b0 = g.ggb[src], nb = g.ggb[src + 1] - b0, d0 = g.dgb[t];
+  const int32_t v0 = g.gvbase[src], nv = g.gvbase[src + 1] - v0, dv = g.dvb[t];
+  for (uint32_t i = threadIdx.x; i < nb; i += blockDim.x) g.out_vgrp[d0 + i] = g.vgrp[b0 + i];
+  for (int32_t i = threadIdx.x; i < nv; i += blockDim.x)
+    g.out_rrows[dv + i] = make_uint2(d0, g.rrows[v0 + i].y);
+}
+
+template <bool ROOT, int TW>
+hipError_t level_of(const StepArgs &a, hipStream_t s) {
+  const size_t lds = clevel_lds_bytes(a.K);
+  if (a.AR <= 31)  // label pairs fit a 32-bit mask (bit 31 is the empty item's)
+    hipLaunchKernelGGL((k_clevel<ROOT, TW, true>), dim3((unsigned)a.n_chunks), dim3(64), lds, s, a);
+  else
+    hipLaunchKernelGGL((k_clevel<ROOT, TW, false>), dim3((unsigned)a.n_chunks), dim3(64), lds, s, a);
+  return hipGetLastError();
+}
+
+template <bool ROOT, int TW>
+hipError_t write_of(const StepArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL((k_cwrite<ROOT, TW>), dim3((unsigned)a.n_chunks), dim3(64), (size_t)a.K * 14 + 16, s, a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_clevel(const StepArgs &a, bool root, hipStream_t s) {
+  if (a.n_chunks <= 0) return hipSuccess;
+  if (root) return level_of<true, 1>(a, s);
+  switch (a.S >> 2) {
+    case 1: return level_of<false, 1>(a, s);
+    case 2: return level_of<false, 2>(a, s);
+    case 3: return level_of<false, 3>(a, s);
+    case 4: return level_of<false, 4>(a, s);
+    case 5: return level_of<false, 5>(a, s);
+    case 6: return level_of<false, 6>(a, s);
+    case 7: return level_of<false, 7>(a, s);
+    case 8: return level_of<false, 8>(a, s);
+    case 16: return level_of<false, 16>(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_cwrite(const StepArgs &a, bool root, hipStream_t s) {
+  if (a.n_chunks <= 0) return hipSuccess;
+  if (root) return write_of<true, 1>(a, s);
+  switch (a.S >> 2) {
+    case 1: return write_of<false, 1>(a, s);
+    case 2: return write_of<false, 2>(a, s);
+    case 3: return write_of<false, 3>(a, s);
+    case 4: return write_of<false, 4>(a, s);
+    case 5: return write_of<false, 5>(a, s);
+    case 6: return write_of<false, 6>(a, s);
+    case 7: return write_of<false, 7>(a, s);
+    case 8: return write_of<false, 8>(a, s);
+    case 16: return write_of<false, 16>(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_ccursors(const StepArgs &a, const int32_t *fchild, const unsigned long long *row_base,
+                           const uint32_t *chunk_base, int64_t F, hipStream_t s) {
+  if (F <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_ccursors, dim3((unsigned)((F * a.rep + 255) / 256)), dim3(256), 0, s, a, fchild, row_base,
+                     chunk_base, F);
+  return hipGetLastError();
+}
+
+hipError_t launch_cgather(const CGatherArgs &g, hipStream_t s) {
+  if (g.n_sel <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_cgather, dim3((unsigned)g.n_sel), dim3(64), 0, s, g);
+  return hipGetLastError();
+}
+
+}  // namespace gm

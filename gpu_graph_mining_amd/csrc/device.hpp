@@ -76,9 +76,10 @@ static_assert(sizeof(PatMeta) == 192 && sizeof(PatMetaWide) == 352, "PatMeta lay
 // bytes per pattern of the metadata of a level of tuple stride S
 __host__ __device__ constexpr int meta_bytes(int S) { return S > kNarrowPatV ? (int)sizeof(PatMetaWide) : (int)sizeof(PatMeta); }
 // The first 16 bytes (job, nv, nrm, labels, low mask half, flags) of
-// pattern p's metadata in a level of tuple stride S, either layout.
-__host__ __device__ inline const PatMeta *meta_at(const PatMeta *m, int S, int64_t p) {
-  return reinterpret_cast<const PatMeta *>(reinterpret_cast<const char *>(m) + p * meta_bytes(S));
+// pattern p's metadata at `stride` bytes a pattern, either layout (job and nv
+// are at the same place in the compact layout's CMetaHead too).
+__host__ __device__ inline const PatMeta *meta_at(const PatMeta *m, int stride, int64_t p) {
+  return reinterpret_cast<const PatMeta *>(reinterpret_cast<const char *>(m) + p * stride);
 }
 
 // Extension key of one pattern at a level whose tuple stride is S:
@@ -89,5 +90,41 @@ struct KeySpace {
   int32_t S, NEL, NVL;
   int64_t K() const { return (int64_t)S * NEL * (NVL + 1); }
 };
+
+// ---- compact databases (compact.hip)
+//
+// When every graph has at most kCompactV vertices, NEL * (NVL + 1) is at most
+// kCompactLabels and a graph needs at most 255 groups:
+//   vgrp[g + u]   vertex u of the graph whose first group is g: four 12-bit
+//                 items (neighbour | label pair << 6; label pair = edge label *
+//                 NVL + neighbour's label), two per 32-bit word, unused ones
+//                 kEmptyItem; bits 24-31 of the first word: the place,
+//                 relative to g, of the vertex's next group (0: none), after
+//                 the graph's vertices
+//   rrows[v]      the root level's row of global vertex v: {g, local id |
+//                 label << 8}
+//   rtab[c]       the root level's chunk c: {job, chunk of the job, the job's
+//                 first vertex, its vertices}
+// Rows of later levels are {g, tuple} of 1 + S / 4 words.
+constexpr int kCompactV = 64;
+constexpr int kCompactLabels = 63;  // label pairs stay below 63 and keys at 64 vertices below 4096
+constexpr uint32_t kEmptyItem = 63u << 6;
+
+// A pattern of a compact level: the head, then nsrc sources (the rightmost
+// vertex first), then nback backward targets.  A source's rule has the bits
+// of the label pairs that the extension rules let through from it, keep those
+// that the 2-edge path rule leaves; a backward target's likewise for the edge
+// from the rightmost vertex to it (the pair's label is the target's own).
+struct alignas(8) CMetaHead {
+  int32_t job;
+  uint8_t nv, nsrc, nback, flags;  // flags: kPatDead
+  uint64_t row0, nrows;            // the pattern's rows
+};
+struct alignas(8) CSource {
+  uint64_t rule, keep;
+  int32_t from;   // pattern vertex
+  int32_t kbase;  // first key: forward, of (from, label pair 0); backward, of (target, edge label 0)
+};
+__host__ __device__ constexpr int cmeta_bytes(int max_nv) { return (int)sizeof(CMetaHead) + 2 * max_nv * (int)sizeof(CSource); }
 
 }  // namespace gm

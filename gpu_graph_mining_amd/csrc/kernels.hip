@@ -66,13 +66,13 @@
 
 #include "device.hpp"
 #include "kernels.hpp"
+#include "wave.hpp"
 
 namespace gm {
 
 namespace {
 
 constexpr uint32_t kEmpty32 = 0xFFFFFFFFu;
-constexpr int kSupShift = 40;  // packed counters: support << 40 | embeddings
 // k_write: children per chunk in one pass.  A chunk with more frequent
 // children than that is counted again in passes split by child residue;
 // the small table (1.75 KB with its row and list bases; 4 KB of LDS per
@@ -85,55 +85,7 @@ constexpr int kWriteTableBits = 6;
 constexpr int kWriteTableBitsRoot = 8;
 constexpr int kFixTableBits = 11;   // k_level_fix: (segment, key) pairs per pass
 
-// ----------------------------------------------------------- wave helpers
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-template <class T>
-__device__ __forceinline__ T wave_exclusive_scan(T x, T &total) {
-  const int lane = threadIdx.x & 63;
-  T v = x;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const T y = __shfl_up(v, o, 64);
-    if (lane >= o) v += y;
-  }
-  total = __shfl(v, 63, 64);
-  return v - x;
-}
-
-template <class T>
-__device__ __forceinline__ T wave_sum(T x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
-}
-
-__device__ __forceinline__ int wave_max(int x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = max(x, __shfl_xor(x, o, 64));
-  return x;
-}
-
-__device__ __forceinline__ uint64_t lanes_below(int lane) { return (1ull << lane) - 1ull; }
-
 __device__ __forceinline__ uint32_t hash_slot32(uint32_t k, int bits) { return (k * 0x9E3779B1u) >> (32 - bits); }
-
-// Wall-clock stamps of the extension + support stage: the first chunks
-// record ~start (the max of complements is the earliest start), every
-// chunk its end; the host reads them from the spread lines.
-__device__ __forceinline__ void stamp_start(const StepArgs &a, int64_t ci) {
-  if (ci < kSpread && threadIdx.x == 0)
-    atomicMax(&a.spread[ci * kSpreadStride + kSpreadStart], ~(unsigned long long)__builtin_amdgcn_s_memrealtime());
-}
-__device__ __forceinline__ void stamp_end(const StepArgs &a, int64_t ci) {
-  if (threadIdx.x == 0)
-    atomicMax(&a.spread[(ci & (kSpread - 1)) * kSpreadStride + kSpreadEnd],
-              (unsigned long long)__builtin_amdgcn_s_memrealtime());
-}
 
 // Candidate list entries: {code, child item count}.
 //   root codes   key | w << 24          (key < 255^3 < 2^24)
@@ -218,13 +170,6 @@ __device__ __forceinline__ int block_rows(const StepArgs &a, int64_t b, int64_t 
   if (later) return 63 - __clzll((long long)later);
   carry = true;
   return ws;
-}
-
-// Lane t's segment head within the block: the last segment start at or
-// before t (0 when the segment began in an earlier block).
-__device__ __forceinline__ int head_lane(uint64_t starts, int lane) {
-  const uint64_t upto = starts & (lane == 63 ? ~0ull : ((2ull << lane) - 1ull));
-  return upto ? 63 - __clzll((long long)upto) : 0;
 }
 
 // ----------------------------------------------------------- tuples
@@ -343,7 +288,7 @@ __global__ void __launch_bounds__(64, (TW <= 2 ? 6 : TW <= 8 ? 5 : 4)) k_level(S
   __shared__ int s_scal[2];
   const int lane = threadIdx.x;
   const int64_t ci = blockIdx.x;
-  stamp_start(a, ci);
+  stamp_start(a.spread, ci);
   int64_t start, end;
   chunk_bounds<ROOT>(a, ci, start, end);
   ChunkInfo *info = a.chunks + a.chunk0 + ci;
@@ -627,7 +572,7 @@ __global__ void __launch_bounds__(64, (TW <= 2 ? 6 : TW <= 8 ? 5 : 4)) k_level(S
     atomicMax(&line[kSpreadFill], (unsigned long long)s_scal[0]);
     if (failed) atomicAdd(&line[kSpreadFailed], 1ull);
   }
-  stamp_end(a, ci);
+  stamp_end(a.spread, ci);
 }
 
 // ------------------------------------------------------------- LEVEL FIX
@@ -754,7 +699,7 @@ __global__ void __launch_bounds__(64) k_level_fix(StepArgs a) {
       wave_sync();
     }
   }
-  if (blockIdx.x < (unsigned)kSpread) stamp_end(a, blockIdx.x);
+  if (blockIdx.x < (unsigned)kSpread) stamp_end(a.spread, blockIdx.x);
 }
 
 // ----------------------------------------------------------------- REDUCE
@@ -781,7 +726,7 @@ __device__ __forceinline__ bool reduce_frequent(const StepArgs &a, int64_t i, in
   if (s <= 0) return false;
   if (!a.minsup_job) return s >= a.minsup_one;
   const int64_t p = i / a.K + a.p_base;
-  const int32_t owner = ROOT ? (int32_t)p : meta_at(a.meta, a.S, p)->job;
+  const int32_t owner = ROOT ? (int32_t)p : meta_at(a.meta, a.meta_stride, p)->job;
   return s >= a.minsup_job[owner];
 }
 
@@ -833,7 +778,7 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce(StepArgs a) {
     if (own && !hit)
       for (int r = g; r < a.rep; r += G) {
         a.acc[(int64_t)r * a.nkeys + i] = 0;
-        a.accb[(int64_t)r * a.nkeys + i] = 0;
+        if (a.accb) a.accb[(int64_t)r * a.nkeys + i] = 0;
       }
   }
   hits = block_sum(hits, s_part);
@@ -899,7 +844,7 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_list(StepArgs a) {
       unsigned long long v = 0, bs = 0;
       if (ok) {
         v = a.acc[(int64_t)r * a.nkeys + key];
-        bs = a.accb[(int64_t)r * a.nkeys + key];
+        if (a.accb) bs = a.accb[(int64_t)r * a.nkeys + key];
       }
       v = group_sum(v, a.rep);
       bs = group_sum(bs, a.rep);
@@ -918,20 +863,6 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_list(StepArgs a) {
     next += step;
     __syncthreads();  // the next step rewrites the shared counts and keys
   }
-}
-
-// The level's counters start from zero: frequent-key count, failure list,
-// errors and spread statistics but the written-row slots, which keep
-// counting across levels (the host compares their total with the rows it
-// asked for).
-__device__ __forceinline__ void clear_counters(const StepArgs &a) {
-  if (threadIdx.x == 0) {
-    *a.freq_count = 0;
-    *a.fail_count = 0;
-    *a.error_flag = 0;
-  }
-  for (int i = threadIdx.x; i < kSpread * kSpreadStride; i += blockDim.x)
-    if (i % kSpreadStride != kSpreadWritten) a.spread[i] = 0;
 }
 
 // After the host chose the children: frequent key i (the key of record i of
@@ -1164,7 +1095,7 @@ __global__ void __launch_bounds__(64, (ROOT ? 5 : TW <= 8 ? 8 : 6)) k_write(Step
           p = a.pid[r];
           g = a.rgraph[r];
           if (n) {
-            nvp = meta_at(a.meta, a.S, p)->nv;
+            nvp = meta_at(a.meta, a.meta_stride, p)->nv;
             const uint32_t *src = reinterpret_cast<const uint32_t *>(a.vt + r * a.S);
 #pragma unroll
             for (int q = 0; q < TW; ++q) s_tup[lane * TW + q] = src[q];

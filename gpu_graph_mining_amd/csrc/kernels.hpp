@@ -25,7 +25,7 @@ constexpr int kSpread = 64;
 constexpr int kSpreadStride = 16;  // 64-bit words per line
 constexpr int kSpreadCand = 0;     // extension candidates enumerated (listed + pruned)
 constexpr int kSpreadFill = 1;     // largest count-table fill of a chunk (atomicMax)
-// (slot 2 unused)
+constexpr int kSpreadPool = 2;     // compact levels: list entries taken from the slice's pool
 constexpr int kSpreadPruned = 3;   // candidates dropped by the 2-edge path rule
 constexpr int kSpreadStart = 4;    // ~(earliest start) of the extension + support stage (atomicMax)
 constexpr int kSpreadEnd = 5;      // latest end of the stage (atomicMax); device wall clock
@@ -44,6 +44,15 @@ struct alignas(16) ChunkInfo {
   int32_t p_lo;    // their keys are (pattern - p_lo) * K + key
   uint32_t pad;
 };
+// A chunk of a compact level: its first row and its {key, embeddings}
+// records, nrec of them at entry rec of the list buffer.
+struct alignas(16) CChunk {
+  int64_t start;
+  uint64_t rec;
+  uint32_t nrec;
+};
+constexpr uint32_t kListUnit = 16;  // list extents start at multiples of this many entries (64 bytes)
+constexpr int kErrListPool = 16;  // error bit: a compact level's list pool ran out (the stage runs again)
 constexpr uint32_t kChunkFailed = 1;  // the LDS count table overflowed; k_level_fix counted it
 
 // Everything the level-step kernels read or write.  Plain device pointers.
@@ -65,7 +74,8 @@ struct StepArgs {
   const uint32_t *rbound;
   const unsigned long long *rlist;
   int32_t S;  // tuple stride in bytes
-  const PatMeta *meta;  // meta_bytes(S) bytes per pattern (the wide layout when S = 64)
+  const PatMeta *meta;  // meta_stride bytes per pattern (the wide layout when S = 64; compact levels: CMetaHead)
+  int32_t meta_stride;
   // path pruning masks (2 * mask_stride words per pattern; 0: none):
   // fwd[0] new arms at the rightmost vertex, fwd[1 + i] at rm[i].from
   // (bit elabel * NVL + label), bwd[1 + i] backward edges to rm[i].from (bit
@@ -126,7 +136,42 @@ struct StepArgs {
   unsigned long long *crlist;
   int32_t CS;  // child tuple stride
   int64_t ccap;
+  // ---- compact levels (compact.hip)
+  const unsigned long long *vgrp;
+  const uint32_t *crow;   // the rows (root: rrows)
+  uint32_t *crow_out;     // the children's rows
+  const uint4 *rtab;      // root chunks
+  const uint2 *ctab;      // later levels' chunks: {pattern, chunk of the pattern}
+  int64_t tab0;           // first chunk of the piece in its table
+  int32_t nom;            // nominal rows of a chunk
+  CChunk *cchunks;
+  uint32_t *clist;        // chunk c's first extent at c * page; then 64 pool slices of pool_sub units from unit pool0
+  uint32_t page, pool0, pool_sub;
+  int32_t AR;             // label pairs: NEL * NVL
+  uint32_t inv_nvl;       // (x * inv_nvl) >> 16 = x / NVL for x < 64
+  unsigned long long lab_rep;  // bit el * NVL for every edge label
+  uint2 *child_tab;       // the children's chunk table, child_nom rows a chunk
+  int32_t child_nom;
 };
+// Compact levels: dynamic LDS of k_clevel, and the launches (see the general
+// ones below).
+inline size_t clevel_lds_bytes(int64_t K) { return (size_t)16 * (size_t)K; }
+hipError_t launch_clevel(const StepArgs &a, bool root, hipStream_t s);
+hipError_t launch_cwrite(const StepArgs &a, bool root, hipStream_t s);
+hipError_t launch_ccursors(const StepArgs &a, const int32_t *fchild, const unsigned long long *row_base,
+                           const uint32_t *chunk_base, int64_t F, hipStream_t s);
+struct CGatherArgs {
+  const unsigned long long *vgrp;
+  const uint2 *rrows;
+  const uint32_t *ggb;
+  const int32_t *gvbase;
+  const int32_t *sel, *dvb;
+  const uint32_t *dgb;
+  int64_t n_sel;
+  unsigned long long *out_vgrp;
+  uint2 *out_rrows;
+};
+hipError_t launch_cgather(const CGatherArgs &g, hipStream_t s);
 
 // Dynamic LDS of k_level for table_bits, and the per-chunk key records its
 // table leaves at most.
@@ -203,6 +248,7 @@ struct CanonArgs {
   // | elabel << 16 | tolabel << 24 (dense labels), S vertex labels each
   // (S: the level's tuple stride; meta_bytes(S) bytes of metadata each)
   const PatMeta *meta;
+  int32_t meta_stride;
   int32_t p_base;  // record keys are (pattern - p_base) * K + key
   const uint32_t *pcode;
   const uint8_t *pvlab;

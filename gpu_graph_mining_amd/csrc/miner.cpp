@@ -126,6 +126,59 @@ void upload(DevBuf &b, const std::vector<T> &v, hipStream_t s) {
 
 int64_t round4(int64_t x) { return (x + 3) & ~int64_t(3); }
 
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The compact layout's groups of one graph (vertices [v0, v0 + n) of the
+// packed adjacency), appended to pk; false when they do not fit 255.
+bool pack_groups(PackedDB &pk, int32_t v0, int32_t n, int32_t a_end, int32_t NVL) {
+  constexpr unsigned long long kEmpty =
+      (unsigned long long)(kEmptyItem | kEmptyItem << 12) << 32 | (kEmptyItem | kEmptyItem << 12);
+  const size_t base = pk.vgrp.size();
+  pk.vgrp.resize(base + n, kEmpty);
+  for (int32_t v = 0; v < n; ++v) {
+    const int32_t a0 = pk.vadj[v0 + v], a1 = v + 1 < n ? pk.vadj[v0 + v + 1] : a_end;
+    size_t at = base + v;
+    for (int32_t x = a0; x < a1; ++x) {
+      const int i = (x - a0) & 3;
+      if (i == 0 && x > a0) {  // a further group, linked from the last one
+        const size_t next = pk.vgrp.size() - base;
+        if (next > 255) return false;
+        pk.vgrp[at] |= (unsigned long long)next << 24;
+        pk.vgrp.push_back(kEmpty);
+        at = base + next;
+      }
+      const uint32_t e = pk.adj[x], lab = ((e >> 8) & 0xFF) * (uint32_t)NVL + ((e >> 16) & 0xFF);
+      const int sh = (i & 1) * 12 + (i & 2) * 16;
+      pk.vgrp[at] = (pk.vgrp[at] & ~(0xFFFull << sh)) | (unsigned long long)((e & 0xFF) | lab << 6) << sh;
+    }
+  }
+  for (int32_t v = 0; v < n; ++v) pk.rrows.push_back(make_uint2((uint32_t)base, (uint32_t)v | (uint32_t)pk.vlab[v0 + v] << 8));
+  return true;
+}
+
+// Nominal rows of a compact chunk of about `blocks` blocks of 64 rows whose
+// segments have avg_seg rows: a block ends at a segment start and the last
+// one has to reach the first start past the nominal end, so each gives up
+// about a segment.  (With nominal lengths of whole blocks every chunk ended
+// in a block of a few rows.)
+int32_t chunk_nominal(int blocks, double avg_seg) {
+  if (avg_seg >= 32) return 64 * blocks;
+  return std::max<int32_t>(32, (int32_t)(blocks * (63.0 - avg_seg)));
+}
+
+// The root level's chunks of every job (a compact database's rows are its
+// vertices).
+void root_chunks(DeviceDB &out, std::vector<uint4> &tab) {
+  out.root_nom = chunk_nominal(2, out.n_graphs > 0 ? (double)out.n_vertices / out.n_graphs : 1.0);
+  out.root_chunk0.assign(1, 0);
+  for (int32_t j = 0; j < out.n_jobs; ++j) {
+    const int64_t v0 = out.job_first_vertex[j], n = out.job_first_vertex[j + 1] - v0;
+    const int64_t k = ceil_div(n, out.root_nom);
+    for (int64_t c = 0; c < k; ++c) tab.push_back(make_uint4((uint32_t)j, (uint32_t)c, (uint32_t)v0, (uint32_t)n));
+    out.root_chunk0.push_back((int64_t)tab.size());
+  }
+}
+
 }  // namespace
 
 int32_t QueryTrie::add(const std::vector<DFS> &code, int32_t query) {
@@ -153,15 +206,53 @@ int32_t QueryTrie::child(int32_t node, const DFS &t) const {
   return -1;
 }
 
+namespace {
+
+// The distinct values of the databases' labels, ascending, and their places.
+// Labels within a range of 2^16 are marked in a table (a sort of every label
+// of 100,000 transactions took about a third of the packing); others sorted.
+struct LabelIds {
+  std::vector<int32_t> values;  // distinct, ascending
+  std::vector<int32_t> table;   // label - lo -> place
+  int64_t lo = 0;
+  LabelIds(const std::vector<const HostDB *> &dbs, const std::vector<int32_t> HostDB::*labels) {
+    int64_t hi = INT32_MIN;
+    lo = INT32_MAX;
+    for (const HostDB *db : dbs)
+      for (int32_t l : db->*labels) {
+        lo = std::min<int64_t>(lo, l);
+        hi = std::max<int64_t>(hi, l);
+      }
+    if (hi < lo) return;
+    if (hi - lo < (1 << 16)) {
+      table.assign((size_t)(hi - lo + 1), 0);
+      for (const HostDB *db : dbs)
+        for (int32_t l : db->*labels) table[(size_t)(l - lo)] = 1;
+      for (size_t i = 0; i < table.size(); ++i)
+        if (table[i]) {
+          table[i] = (int32_t)values.size();
+          values.push_back((int32_t)(lo + (int64_t)i));
+        }
+      return;
+    }
+    for (const HostDB *db : dbs) values.insert(values.end(), (db->*labels).begin(), (db->*labels).end());
+    std::sort(values.begin(), values.end());
+    values.erase(std::unique(values.begin(), values.end()), values.end());
+  }
+  int32_t at(int32_t l) const {
+    if (!table.empty()) return table[(size_t)(l - lo)];
+    return (int32_t)(std::lower_bound(values.begin(), values.end(), l) - values.begin());
+  }
+};
+
+}  // namespace
+
 void pack_db(const std::vector<const HostDB *> &dbs, DeviceDB &out, PackedDB &pk) {
   out.n_jobs = (int32_t)dbs.size();
-  std::vector<int32_t> vls, els;
   int64_t nv = 0, ne = 0;
   int64_t ng = 0;
   for (const HostDB *db : dbs) {
     db->check_consistent();
-    vls.insert(vls.end(), db->vlabel.begin(), db->vlabel.end());
-    els.insert(els.end(), db->elabel.begin(), db->elabel.end());
     nv += db->n_vertices();
     ne += db->n_edges();
     ng += db->n_graphs;
@@ -169,23 +260,25 @@ void pack_db(const std::vector<const HostDB *> &dbs, DeviceDB &out, PackedDB &pk
   if (ng > INT32_MAX - 1 || nv > INT32_MAX - 1 || 2 * ne > INT32_MAX - 1)
     throw Error(GM_E_UNSUPPORTED, "database too large for 32-bit offsets");
   if (ng >= (1ll << 24)) throw Error(GM_E_UNSUPPORTED, "more than 16777215 graphs (24-bit support counters)");
-  std::sort(vls.begin(), vls.end());
-  vls.erase(std::unique(vls.begin(), vls.end()), vls.end());
-  std::sort(els.begin(), els.end());
-  els.erase(std::unique(els.begin(), els.end()), els.end());
+  const LabelIds vids(dbs, &HostDB::vlabel), eids(dbs, &HostDB::elabel);
+  const std::vector<int32_t> &vls = vids.values, &els = eids.values;
   if (vls.size() > 255 || els.size() > 255)
     throw Error(GM_E_UNSUPPORTED, "more than 255 distinct vertex or edge labels");
   out.vl_values = vls;
   out.el_values = els;
   out.NVL = std::max<int32_t>(1, (int32_t)vls.size());
   out.NEL = std::max<int32_t>(1, (int32_t)els.size());
-  auto vmap = [&](int32_t l) { return (int32_t)(std::lower_bound(vls.begin(), vls.end(), l) - vls.begin()); };
-  auto emap = [&](int32_t l) { return (int32_t)(std::lower_bound(els.begin(), els.end(), l) - els.begin()); };
+  auto vmap = [&](int32_t l) { return vids.at(l); };
+  auto emap = [&](int32_t l) { return eids.at(l); };
 
   std::vector<int32_t> &gvbase = pk.gvbase, &vadj = pk.vadj, &gjob = pk.gjob, &vgraph = pk.vgraph;
   std::vector<uint32_t> &adj = pk.adj;
   std::vector<uint8_t> &vlab = pk.vlab;
   pk.max_graph_v = pk.max_graph_adj = 0;
+  pk.vgrp.clear();
+  pk.rrows.clear();
+  out.compact = (int64_t)out.NEL * (out.NVL + 1) <= kCompactLabels;
+  out.ggb.assign(1, 0);
   gvbase.clear();
   vadj.clear();
   gjob.clear();
@@ -201,7 +294,7 @@ void pack_db(const std::vector<const HostDB *> &dbs, DeviceDB &out, PackedDB &pk
   out.job_first_graph.assign(1, 0);
   out.job_first_vertex.assign(1, 0);
   std::vector<int32_t> deg, fill, dl;
-  std::vector<std::pair<int32_t, int32_t>> pairs;
+  std::vector<uint64_t> seen;  // bit (smaller * n + larger) of a graph's vertex pairs
   int32_t job = 0;
   for (const HostDB *db : dbs) {
     for (int32_t g = 0; g < db->n_graphs; ++g) {
@@ -209,15 +302,16 @@ void pack_db(const std::vector<const HostDB *> &dbs, DeviceDB &out, PackedDB &pk
       const int32_t e0 = db->ebegin[g], e1 = db->ebegin[g + 1];
       if (n > kMaxGraphV)
         throw Error(GM_E_UNSUPPORTED, "graph " + std::to_string(g) + " has more than 256 vertices");
-      pairs.clear();
+      seen.assign(((size_t)n * n + 63) / 64, 0);
+      bool parallel = false;
       for (int32_t e = e0; e < e1; ++e) {
-        int32_t a = db->efrom[e], b = db->eto[e];
+        const int32_t a = db->efrom[e], b = db->eto[e];
         if (a == b) throw Error(GM_E_UNSUPPORTED, "self-loop in graph " + std::to_string(g));
-        pairs.emplace_back(std::min(a, b), std::max(a, b));
+        const size_t bit = (size_t)std::min(a, b) * n + (size_t)std::max(a, b);
+        parallel = parallel || ((seen[bit >> 6] >> (bit & 63)) & 1);
+        seen[bit >> 6] |= 1ull << (bit & 63);
       }
-      std::sort(pairs.begin(), pairs.end());
-      if (std::adjacent_find(pairs.begin(), pairs.end()) != pairs.end())
-        throw Error(GM_E_UNSUPPORTED, "parallel edges in graph " + std::to_string(g));
+      if (parallel) throw Error(GM_E_UNSUPPORTED, "parallel edges in graph " + std::to_string(g));
       gvbase.push_back((int32_t)vlab.size());
       gjob.push_back(job);
       dl.resize(n);
@@ -252,6 +346,9 @@ void pack_db(const std::vector<const HostDB *> &dbs, DeviceDB &out, PackedDB &pk
         adj[abase + fill[a]++] = (uint32_t)b | (el << 8) | ((uint32_t)dl[b] << 16) | ((uint32_t)deg[b] << 24);
         adj[abase + fill[b]++] = (uint32_t)a | (el << 8) | ((uint32_t)dl[a] << 16) | ((uint32_t)deg[a] << 24);
       }
+      if (out.compact)
+        out.compact = n <= kCompactV && pack_groups(pk, (int32_t)vlab.size() - n, n, (int32_t)adj.size(), out.NVL);
+      out.ggb.push_back((uint32_t)pk.vgrp.size());
     }
     ++job;
     out.job_first_graph.push_back((int32_t)gvbase.size());
@@ -264,6 +361,12 @@ void pack_db(const std::vector<const HostDB *> &dbs, DeviceDB &out, PackedDB &pk
   out.n_adj = (int64_t)adj.size();
   out.max_graph_v = pk.max_graph_v;
   out.max_graph_adj = pk.max_graph_adj;
+  if (!out.compact) {
+    pk.vgrp.clear();
+    pk.rrows.clear();
+    out.ggb.clear();
+  }
+  out.n_groups = (int64_t)pk.vgrp.size();
 }
 
 void upload_db(const PackedDB &pk, DeviceDB &out, hipStream_t s) {
@@ -273,9 +376,17 @@ void upload_db(const PackedDB &pk, DeviceDB &out, hipStream_t s) {
   upload(out.vlab, pk.vlab, s);
   upload(out.gjob, pk.gjob, s);
   upload(out.vgraph, pk.vgraph, s);
+  std::vector<uint4> tab;
+  if (out.compact) {
+    root_chunks(out, tab);
+    upload(out.vgrp, pk.vgrp, s);
+    upload(out.rrows, pk.rrows, s);
+    upload(out.rtab, tab, s);
+    upload(out.dggb, out.ggb, s);
+  }
   hip_check(hipStreamSynchronize(s), "upload database");
   out.bytes = 4 * pk.gvbase.size() + 4 * pk.vadj.size() + 4 * pk.adj.size() + pk.vlab.size() + 4 * pk.gjob.size() +
-              4 * pk.vgraph.size();
+              4 * pk.vgraph.size() + 8 * pk.vgrp.size() + 8 * pk.rrows.size() + 16 * tab.size();
 }
 
 void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32_t *begin, const int32_t *ids,
@@ -283,7 +394,8 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
   if (n_jobs < 1 || begin[0] != 0) throw Error(GM_E_ARG, "job ranges must start at 0");
   const int32_t n_sel = begin[n_jobs];
   std::vector<int32_t> sel(n_sel), dvb(n_sel), dab(n_sel), djob(n_sel);
-  int64_t nv = 0, na = 0;
+  std::vector<uint32_t> dgb(src.compact ? n_sel : 0);
+  int64_t nv = 0, na = 0, ngr = 0;
   int32_t max_v = 0, max_a = 0;
   out.n_jobs = n_jobs;
   out.job_first_graph.assign(1, 0);
@@ -298,6 +410,10 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
       dvb[t] = (int32_t)nv;
       dab[t] = (int32_t)na;
       djob[t] = j;
+      if (src.compact) {
+        dgb[t] = (uint32_t)ngr;
+        ngr += src.ggb[g + 1] - src.ggb[g];
+      }
       nv += n;
       na += a;
       max_v = std::max(max_v, n);
@@ -316,6 +432,41 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
   out.NEL = src.NEL;
   out.vl_values = src.vl_values;
   out.el_values = src.el_values;
+  if (src.compact) {
+    // only the compact layout: a gathered database is mined by gm_batch_mine
+    // alone, which takes it
+    if (nv > INT32_MAX - 1 || ngr >= (1ll << 32)) throw Error(GM_E_UNSUPPORTED, "database too large for 32-bit offsets");
+    out.compact = true;
+    out.n_groups = ngr;
+    std::vector<uint4> tab;
+    root_chunks(out, tab);
+    upload(out.rtab, tab, s);
+    out.vgrp.ensure(8 * (size_t)std::max<int64_t>(ngr, 1));
+    out.rrows.ensure(8 * (size_t)std::max<int64_t>(nv, 1));
+    out.bytes = 8 * (size_t)ngr + 8 * (size_t)nv + 16 * tab.size();
+    DevBuf idx;  // sel, dvb, dgb
+    idx.ensure(12 * (size_t)std::max<int32_t>(n_sel, 1));
+    int32_t *d = idx.as<int32_t>();
+    if (n_sel > 0) {
+      hip_check(hipMemcpyAsync(d, sel.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
+      hip_check(hipMemcpyAsync(d + n_sel, dvb.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
+      hip_check(hipMemcpyAsync(d + 2 * (size_t)n_sel, dgb.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
+    }
+    CGatherArgs g;
+    g.vgrp = src.vgrp.as<unsigned long long>();
+    g.rrows = src.rrows.as<uint2>();
+    g.ggb = src.dggb.as<uint32_t>();
+    g.gvbase = src.gvbase.as<int32_t>();
+    g.sel = d;
+    g.dvb = d + n_sel;
+    g.dgb = reinterpret_cast<const uint32_t *>(d + 2 * (size_t)n_sel);
+    g.n_sel = n_sel;
+    g.out_vgrp = out.vgrp.as<unsigned long long>();
+    g.out_rrows = out.rrows.as<uint2>();
+    hip_check(launch_cgather(g, s), "k_cgather");
+    hip_check(hipStreamSynchronize(s), "k_cgather");  // before the index buffer is freed
+    return;
+  }
   out.gvbase.ensure(4 * (size_t)(n_sel + 1));
   out.vadj.ensure(4 * (size_t)(nv + 1));
   out.adj.ensure(4 * (size_t)std::max<int64_t>(na, 1));
@@ -394,10 +545,12 @@ struct Level {
   Arr<int32_t> node;   // query mode: trie node of the code
   Arr<uint8_t> alive;  // the code is minimal (a dead pattern's rows are not extended)
   Arr<int64_t> row0;   // n + 1: pattern i's rows are [row0[i], row0[i + 1]) (pattern-major rows)
+  Arr<int64_t> chunk0; // n + 1 (compact levels): pattern i's chunks
   void resize(int64_t k, int l) {
     n = k;
     len = l;
     row0.resize(k + 1);
+    chunk0.resize(k + 1);
     code.resize(k * l);
     vlab.resize(k * kMaxPatV);
     nv.resize(k);
@@ -444,6 +597,79 @@ PatMetaT<V> make_meta(const DFS *code, int len, const uint8_t *vlab, int nv, int
   m.bwd_from = (uint32_t)bwd_from;
   m.bwd_from_hi = (uint32_t)(bwd_from >> 32);
   return m;
+}
+
+// The label rules of a database's compact levels (device.hpp: CSource).
+struct LabelRules {
+  int NEL, NVL, AR;
+  uint64_t rep = 0;  // bit el * NVL for every edge label
+  LabelRules(int nel, int nvl) : NEL(nel), NVL(nvl), AR(nel * nvl) {
+    if (AR < 64)
+      for (int e = 0; e < NEL; ++e) rep |= 1ull << (e * NVL);
+  }
+  // neighbour labels >= from
+  uint64_t labels(int from) const { return from >= NVL ? 0 : ((1ull << NVL) - 1) & (~0ull << from); }
+  // label pairs (e, l) with l >= minlabel and (e1 < e or (e1 == e and l1 <= l))
+  uint64_t after(int minlabel, int e1, int l1) const {
+    const uint64_t above = e1 + 1 < NEL ? (labels(minlabel) * rep) & (~0ull << ((e1 + 1) * NVL)) : 0;
+    return above | labels(std::max(minlabel, l1)) << (e1 * NVL);
+  }
+};
+
+// A compact level's pattern: its head, sources and backward targets into
+// dst.  Sources no label pair gets through from are left out (but the
+// rightmost vertex's, which the backward targets need).
+void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv, int32_t job, uint64_t row0,
+                uint64_t nrows, bool dead, int S, const LabelRules &lr) {
+  const PatMetaWide m = make_meta<kMaxPatV>(code, len, vlab, nv, job);
+  CMetaHead h;
+  std::memset(&h, 0, sizeof(h));
+  h.job = job;
+  h.nv = (uint8_t)nv;
+  h.flags = dead ? (uint8_t)kPatDead : 0;
+  h.row0 = row0;
+  h.nrows = nrows;
+  CSource *out = reinterpret_cast<CSource *>(dst + sizeof(CMetaHead));
+  const int SB = S * lr.NEL;
+  auto add = [&](uint64_t rule, int from, int kbase) {
+    out->rule = out->keep = rule;
+    out->from = from;
+    out->kbase = kbase;
+    ++out;
+  };
+  const int rv = nv - 1;
+  const uint64_t bwd = (uint64_t)m.bwd_mask_hi << 32 | m.bwd_mask;
+  CSource back[kMaxPatV];
+  int nback = 0;
+  for (int q = 1; q < m.nrm; ++q) {
+    const int f = (int)(m.rm[q] & 0xFF), e1 = (int)((m.rm[q] >> 8) & 0xFF), l1 = (int)((m.rm[q] >> 16) & 0xFF);
+    if ((bwd >> f) & 1) continue;  // the edge is in the pattern already
+    // pairs (e, label of f) with e1 < e or (e1 == e and l1 <= maxlabel)
+    const int e0 = l1 <= m.maxlabel ? e1 : e1 + 1;
+    const uint64_t rule = e0 < lr.NEL ? (lr.rep & (~0ull << (e0 * lr.NVL))) << vlab[f] : 0;
+    if (!rule) continue;
+    back[nback].rule = back[nback].keep = rule;
+    back[nback].from = f;
+    back[nback].kbase = f * lr.NEL;
+    ++nback;
+  }
+  const uint64_t own = lr.labels(m.minlabel) * lr.rep;
+  int nsrc = 0;
+  if (own || nback) {
+    add(own, rv, SB + rv * lr.AR);
+    ++nsrc;
+  }
+  for (int q = 0; q < m.nrm; ++q) {
+    const int f = (int)(m.rm[q] & 0xFF);
+    const uint64_t rule = lr.after(m.minlabel, (int)((m.rm[q] >> 8) & 0xFF), (int)((m.rm[q] >> 16) & 0xFF));
+    if (!rule) continue;
+    add(rule, f, SB + f * lr.AR);
+    ++nsrc;
+  }
+  for (int q = 0; q < nback; ++q) *out++ = back[q];
+  h.nsrc = (uint8_t)nsrc;
+  h.nback = (uint8_t)nback;
+  std::memcpy(dst, &h, sizeof(h));
 }
 
 // One frequent key as k_reduce appends it: key, support, embeddings, and
@@ -617,8 +843,6 @@ void stage_up(Workspace &w, HostBuf &hb, size_t off, size_t bytes, hipStream_t s
   }
 }
 
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
 // Division by a run-time constant d with one 64 x 64 -> 128-bit multiply by
 // M = ceil(2^64 / d) (Lemire, Kaser and Kurz, "Faster remainder by direct
 // computation", 2019), exact for every dividend below 2^32; larger ones
@@ -658,6 +882,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     if (w.accb.p) hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");
   }
   w.acc_zero = false;  // until this call ends normally
+  // The compact kernels mine every database that has their layout, but for
+  // the entry point that allocates nothing, whose 64 MiB and out-of-memory
+  // answers are defined by the general buffers.
+  const bool compact = db.compact && !w.arena;
+  const LabelRules rules(NEL, NVL);
 
   if (opt.minsup.size() > 1) {  // a single job's goes with the kernel arguments
     grow(w.minsup, sizeof(int32_t) * opt.minsup.size(), s);
@@ -679,6 +908,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   a.vgraph = db.vgraph.as<int32_t>();
   a.NEL = NEL;
   a.NVL = NVL;
+  a.vgrp = db.vgrp.as<unsigned long long>();
+  a.rtab = db.rtab.as<uint4>();
+  a.AR = NEL * NVL;
+  a.inv_nvl = (65536u + (uint32_t)NVL - 1) / (uint32_t)NVL;
+  a.lab_rep = rules.rep;
   int dev = 0, wall_khz = 1;
   hip_check(hipGetDevice(&dev), "hipGetDevice");
   hip_check(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, dev), "hipDeviceGetAttribute");
@@ -753,13 +987,22 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     uint64_t key_next = 0;   // first key (relative to p_next) not written: a pattern split over pieces
     int64_t p_counted = 0;   // patterns whose candidates are in e_cand
     int64_t p_end_next = 0;  // > 0: the next piece ends there (its children were measured)
+    int32_t nom = 0;         // compact levels: nominal rows of a chunk
+    int32_t meta_stride = 0; // bytes of a pattern's metadata
   };
   std::deque<Frame> frames(1);
-  frames.back().list_cap = (uint64_t)std::max<int64_t>(db.n_adj, 1);  // root lists: 2E
+  // Compact lists are written as they come (4 bytes a candidate), not sized
+  // exactly beforehand: seven 8-byte words a row stand for them in the budget
+  // (pages of a little over 4 entries a row and a pool of 8).
+  auto compact_words = [](uint64_t rows) { return std::max<uint64_t>(1, 7 * rows); };
+  frames.back().list_cap =
+      compact ? compact_words((uint64_t)db.n_vertices) : (uint64_t)std::max<int64_t>(db.n_adj, 1);  // root lists: 2E
+  frames.back().nom = db.root_nom;
   const int64_t budget = w.arena ? 0 : opt.mem_budget;
   double piece_bytes_per_row = 0;  // child bytes per parent row of the last piece (estimate)
   // device bytes a level's rows take (rows with their counts) and a list entry
-  auto rows_bytes = [](int64_t rows, int S_) { return (int64_t)rows * (22 + S_); };
+  auto rows_bytes = [&](int64_t rows, int S_) { return (int64_t)rows * ((compact ? 4 : 22) + S_); };
+  int64_t pool_units = 0;  // compact: list pool of the level step (grown when a level overflows it)
 
   for (;;) {
     if (frames.empty()) break;
@@ -826,11 +1069,16 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     const int64_t prow_lo = prow(p_begin), prow_hi = prow(p_end);
     // chunk length: kChunkRows, or shorter so that the piece has about
     // kLevelWaves chunks (a power of two, at least one block)
+    // (compact levels: their chunk table was laid out with the rows)
     int chunk_rows = max_chunk_rows;
     while (chunk_rows > kMinChunkRows && (prow_hi - prow_lo) / chunk_rows < kLevelWaves) chunk_rows /= 2;
     int64_t total_chunks = 0;
-    for (int64_t lo = p_begin; lo < p_end; lo += prange)
-      total_chunks += ceil_div(prow(std::min<int64_t>(p_end, lo + prange)) - prow(lo), chunk_rows);
+    const int64_t ctab0 = !compact ? 0 : root ? db.root_chunk0[p_begin] : L.chunk0[p_begin];
+    if (compact)
+      total_chunks = (root ? db.root_chunk0[p_end] : L.chunk0[p_end]) - ctab0;
+    else
+      for (int64_t lo = p_begin; lo < p_end; lo += prange)
+        total_chunks += ceil_div(prow(std::min<int64_t>(p_end, lo + prange)) - prow(lo), chunk_rows);
     // counter replicas: chunk i counts into replica i mod rep, so that the
     // keys every chunk hits (the root's) are not one hot address (atomics
     // on one address serialise at ~100 ns each); up to 64 MB of them
@@ -842,12 +1090,22 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     grow(w.sup, sizeof(int32_t) * std::max<int64_t>(nkeys, 1), s);
     grow(w.tiles, sizeof(uint32_t) * kReduceTiles, s);
     grow_zero(w.acc, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
-    grow_zero(w.accb, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
-    grow(w.chunks, sizeof(ChunkInfo) * std::max<int64_t>(total_chunks, 1), s);
-    grow(w.fail, sizeof(uint32_t) * std::max<int64_t>(total_chunks, 1), s);
-    grow(w.chunk_keys, sizeof(uint4) * level_chunk_keys(table_bits) * std::max<int64_t>(total_chunks, 1), s);
-    grow(w.rccnt, sizeof(uint16_t) * std::max<int64_t>(rows_now, 1), s);
-    grow(w.cand, sizeof(uint2) * std::max<uint64_t>(list_cap, 1), s);
+    // compact: a page of 256 list entries per 64 nominal rows, records included
+    const uint32_t page = 256u * (uint32_t)std::max(1, (Fr.nom + 63) / 64);
+    if (compact) {
+      grow(w.chunks, sizeof(CChunk) * std::max<int64_t>(total_chunks, 1), s);
+    } else {
+      grow_zero(w.accb, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
+      grow(w.chunks, sizeof(ChunkInfo) * std::max<int64_t>(total_chunks, 1), s);
+      grow(w.fail, sizeof(uint32_t) * std::max<int64_t>(total_chunks, 1), s);
+      grow(w.chunk_keys, sizeof(uint4) * level_chunk_keys(table_bits) * std::max<int64_t>(total_chunks, 1), s);
+      grow(w.rccnt, sizeof(uint16_t) * std::max<int64_t>(rows_now, 1), s);
+      grow(w.cand, sizeof(uint2) * std::max<uint64_t>(list_cap, 1), s);
+    }
+    // the pool of further list extents: eight entries a row (the levels
+    // measured list 2 to 6), at least 512 units (8,192 entries, more than one
+    // source of a block can list) a slice
+    pool_units = std::max<int64_t>(kSpread * 512, (prow_hi - prow_lo) * 8 / kListUnit);
     uint32_t fcap = (uint32_t)std::min<int64_t>(std::max<int64_t>(nkeys, 1), std::max<int64_t>(1 << 16, (p_end - p_begin) * 64));
     // the children would pass max_edges: none is kept
     const bool past_max = opt.max_edges > 0 && (root ? 1 : L.len + 1) > opt.max_edges;
@@ -865,6 +1123,22 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     uint32_t guess = 0;  // frequent keys in the first download
     // the stage; rerun with a longer frequent-key list when it overflowed
     for (int attempt = 0;; ++attempt) {
+      if (compact) {
+        const int64_t pages = total_chunks * (int64_t)(page / kListUnit);  // units
+        const int64_t sub = ceil_div(pool_units, kSpread);
+        if (pages + sub * kSpread >= 0xFFFFFFFFll)
+          throw Error(GM_E_OOM, "candidate lists of a level step need more than 256 GiB");
+        grow(w.cand, sizeof(uint32_t) * (size_t)(pages + sub * kSpread) * kListUnit, s);
+        a.clist = w.cand.as<uint32_t>();
+        a.page = page;
+        a.pool0 = (uint32_t)pages;
+        a.pool_sub = (uint32_t)sub;
+        a.cchunks = w.chunks.as<CChunk>();
+        a.crow = root ? db.rrows.as<uint32_t>() : w.row(cur).vt.as<uint32_t>();
+        a.ctab = root ? nullptr : w.row(cur).ctab.as<uint2>();
+        a.tab0 = ctab0;
+        a.nom = Fr.nom;
+      }
       const size_t freq_bytes = sizeof(Counters) + sizeof(Freq) * fcap;
       {
         // a new block (the allocator may hand back the address it freed)
@@ -887,7 +1161,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.fail_list = w.fail.as<uint32_t>();
       a.fail_count = &dctr->nfail;
       a.acc = w.acc.as<unsigned long long>();
-      a.accb = w.accb.as<unsigned long long>();
+      a.accb = compact ? nullptr : w.accb.as<unsigned long long>();
       a.rep = rep;
       a.table_bits = table_bits;
       a.chunk_rows = chunk_rows;
@@ -921,6 +1195,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.rlist = root ? nullptr : w.row(cur).rlist.as<unsigned long long>();
       a.S = S;
       a.meta = root ? nullptr : reinterpret_cast<const PatMeta *>(w.row(cur).upl.as<char>());
+      a.meta_stride = root ? 0 : Fr.meta_stride;
       a.mask_stride = root ? 0 : mask_stride;
       a.pmask = a.mask_stride ? reinterpret_cast<const unsigned long long *>(w.row(cur).upl.as<char>() + mask_off)
                               : nullptr;
@@ -933,7 +1208,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         hip_check(hipEventRecord(w.ev[0], s), "hipEventRecord");
       }
       int64_t chunk0 = 0;
-      for (int64_t lo = p_begin; lo < p_end; lo += prange) {
+      for (int64_t lo = p_begin; lo < p_end && !compact; lo += prange) {
         const int64_t hi = std::min<int64_t>(p_end, lo + prange);
         a.p_lo = (int32_t)lo;
         a.p_hi = (int32_t)hi;
@@ -950,7 +1225,10 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.row_hi = prow_hi;
       a.chunk0 = 0;
       a.n_chunks = total_chunks;
-      hip_check(launch_level_fix(a, root, s), "k_level_fix");
+      if (compact)
+        hip_check(launch_clevel(a, root, s), "k_clevel");
+      else
+        hip_check(launch_level_fix(a, root, s), "k_level_fix");
       if (time_stage) hip_check(hipEventRecord(w.ev[1], s), "hipEventRecord");
       hip_check(launch_reduce(a, root, s), "k_reduce");
       if (canon_dev) {
@@ -962,6 +1240,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         c.down = a.down ? a.down + kCounterWords : nullptr;
         c.down_cap = a.down_cap;
         c.meta = a.meta;
+        c.meta_stride = a.meta_stride;
         c.p_base = (int32_t)p_begin;
         c.pcode = reinterpret_cast<const uint32_t *>(w.row(cur).upl.as<char>() + code_off);
         c.pvlab = reinterpret_cast<const uint8_t *>(w.row(cur).upl.as<char>() + vlab_off);
@@ -977,6 +1256,14 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       if (!a.down) stage_down(w, w.down, dctr, head, s);
       hip_check(hipStreamSynchronize(s), "k_level");
       std::memcpy(&cnt, hbuf, sizeof(cnt));
+      if (cnt.err == kErrListPool) {
+        // the lists outgrew the pool: the stage is run again with a larger
+        // one, from cleared counters
+        pool_units = std::max<int64_t>(pool_units * 4, kSpread * 512);
+        hip_check(launch_fill8(w.acc.p, w.acc.cap, s), "clear counters");
+        attempt = -1;
+        continue;
+      }
       if (cnt.err) throw Error(GM_E_DEVICE, "internal: level step error " + std::to_string(cnt.err));
       ecand = max_fill = pruned = failed = 0;
       unsigned long long written = 0, t_start = 0, t_end = 0;
@@ -1008,7 +1295,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       if (attempt > 0) throw Error(GM_E_DEVICE, "internal: frequent-key count changed between runs");
       fcap = cnt.fcount;
       hip_check(launch_fill8(w.acc.p, w.acc.cap, s), "clear counters");
-      hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");
+      if (!compact) hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");
     }
     if (!root) {
       ext_ms += ms;
@@ -1049,7 +1336,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     uint64_t key_cut = ~0ull;  // keys [key_lo, key_cut) become children
     if (budget > 0 && !past_max && F > 0) {
       const int CSb = tuple_stride(root ? 2 : std::min(L.max_nv + 1, kMaxPatV));
-      auto kbytes = [&](int64_t i) { return rows_bytes((int64_t)fr[i].proj, CSb) + (int64_t)fr[i].items * 8; };
+      auto kbytes = [&](int64_t i) {
+        return rows_bytes((int64_t)fr[i].proj, CSb) + (int64_t)(compact ? compact_words(fr[i].proj) : fr[i].items) * 8;
+      };
       int64_t total = 0;
       for (int64_t i = 0; i < F; ++i)
         if (fr[i].key >= key_lo) total += kbytes(i);
@@ -1075,7 +1364,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
           Fr.p_end_next = std::max<int64_t>(p_cut, p_begin + 1);
           if (measured_again && Fr.p_end_next >= p_end) throw Error(GM_E_DEVICE, "internal: piece did not shrink");
           hip_check(launch_fill8(w.acc.p, w.acc.cap, s), "clear counters");
-          hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");
+          if (!compact) hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");
           continue;
         }
         if (p_end == p_begin + 1) {
@@ -1233,17 +1522,27 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     st.n_candidates += root ? 0 : F;
 
     // children in key order; child c's rows are [row0[c], row0[c + 1])
-    int64_t C = 0, child_rows = 0;
+    int64_t C = 0, child_rows = 0, child_segs = 0;
     int max_nv = 0;
     for (int64_t i = 0; i < F; ++i) {
       if (kidx[i] < 0) continue;
       kidx[i] = C++;
       child_rows += (int64_t)fr[i].proj;
+      child_segs += (int64_t)(fr[i].sup & 0xFFFFFFFFull);  // (bits 32-39 hold the device check's answer)
       if (!late_decode) max_nv = std::max(max_nv, (int)knv[i]);
     }
     if (late_decode) max_nv = max_nv_exact;
     const int CS = C > 0 ? tuple_stride(max_nv) : 4;  // the children's tuple stride
     const bool wide = CS > kNarrowPatV;                 // and metadata layout
+    const int child_stride = compact ? cmeta_bytes(std::max(max_nv, 1)) : meta_bytes(CS);
+    // compact: blocks of a chunk, as many as leave enough chunks (at most four)
+    int child_nom = 0;
+    if (compact) {
+      const double seg = (double)child_rows / (double)std::max<int64_t>(1, child_segs);
+      int blocks = std::max(1, std::min(4, max_chunk_rows / 64));
+      while (blocks > 1 && child_rows / chunk_nominal(blocks, seg) < kLevelWaves) blocks /= 2;
+      child_nom = chunk_nominal(blocks, seg);
+    }
     N.resize(C, new_len);
     nproj.resize(C);
     double us_host = 0, us_overlap = 0;
@@ -1256,7 +1555,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     // dropped), per child its first row and first list entry, then the
     // children's path masks.  Child c's rows follow the earlier children's
     // (embedding counts), its list entries likewise (item sums).
-    const size_t meta_all = (size_t)meta_bytes(CS) * C;
+    const size_t meta_all = (size_t)child_stride * C;
     const size_t fc_off = (meta_all + 7) & ~size_t(7);
     const size_t rb_off = (fc_off + sizeof(int32_t) * F + 7) & ~size_t(7);
     const size_t lb_off = rb_off + sizeof(unsigned long long) * C;
@@ -1268,7 +1567,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     const bool keys_whole = key_lo == 0 && key_cut == ~0ull;
     if ((new_len == 1 && !keys_whole) || (new_len == 2 && !(p_begin == 0 && p_end == P && keys_whole))) t2_partial = true;
     const bool masks = prune && !t2_partial && new_len >= 2 && C > 0;
-    const int mstride = masks ? max_nv : 0;
+    const int mstride = masks && !compact ? max_nv : 0;  // (compact: the masks are in the metadata)
     const size_t masks_off = lb_off + sizeof(unsigned long long) * C;
     // then per child its packed code (from | to << 8 | elabel << 16 |
     // tolabel << 24 per tuple) and its vertex labels, for the next level's
@@ -1281,26 +1580,38 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       int32_t *hfc = reinterpret_cast<int32_t *>(hu + fc_off);
       unsigned long long *hrb = reinterpret_cast<unsigned long long *>(hu + rb_off);
       unsigned long long *hlb = reinterpret_cast<unsigned long long *>(hu + lb_off);
-      int64_t run = 0;
+      uint32_t *hcb = reinterpret_cast<uint32_t *>(hlb);  // compact: the children's first chunks
+      int64_t run = 0, chunks = 0;
       for (int64_t i = 0; i < F; ++i) {
         const int64_t c = kidx[i];
         hfc[i] = (int32_t)c;
         if (c < 0) continue;
         hrb[c] = (unsigned long long)run;
-        hlb[c] = (unsigned long long)child_items;
         N.row0[c] = run;
         run += (int64_t)fr[i].proj;
-        child_items += fr[i].items;
+        if (compact) {
+          hcb[c] = (uint32_t)chunks;
+          N.chunk0[c] = chunks;
+          chunks += ceil_div((int64_t)fr[i].proj, child_nom);
+        } else {
+          hlb[c] = (unsigned long long)child_items;
+          child_items += fr[i].items;
+        }
         // k_write reserves rows << 32 | list entries in one 64-bit atomic
         if (fr[i].proj >= (1ull << 32) || fr[i].items >= (1ull << 32))
           throw Error(GM_E_UNSUPPORTED, "a pattern with 2^32 or more embeddings or candidate-list entries");
       }
       N.row0[C] = run;
+      N.chunk0[C] = chunks;
+      if (compact) child_items = compact_words((uint64_t)child_rows);
+      if (chunks > INT32_MAX) throw Error(GM_E_OOM, "more than 2^31 chunks of rows");
     }
     if (F > 0) stage_up(w, w.up, fc_off, masks_off - fc_off, s);  // child ids, bases
     if (F > 0 && C == 0) {  // nothing to write: the frequent keys' replicas are cleared
       const char *su = static_cast<const char *>(w.up.dev);
-      hip_check(launch_cursors(a, reinterpret_cast<const int32_t *>(su + fc_off), nullptr, nullptr, F, s), "k_cursors");
+      const int32_t *fc = reinterpret_cast<const int32_t *>(su + fc_off);
+      hip_check(compact ? launch_ccursors(a, fc, nullptr, nullptr, F, s) : launch_cursors(a, fc, nullptr, nullptr, F, s),
+                "k_cursors");
       counters_clear = true;
     }
     if (C > 0) {
@@ -1325,13 +1636,21 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       PatMetaWide *hmw = reinterpret_cast<PatMetaWide *>(hu);
       char *du = static_cast<char *>(grow(w.row(nxt).upl, up_bytes, s));
       const char *su = static_cast<const char *>(w.up.dev);
-      grow(w.row(nxt).pid, sizeof(int32_t) * std::max<int64_t>(child_rows, 1), s);
-      grow(w.row(nxt).rgraph, sizeof(int32_t) * std::max<int64_t>(child_rows, 1), s);
-      grow(w.row(nxt).vt, (size_t)CS * std::max<int64_t>(child_rows, 1), s);
-      grow(w.row(nxt).rbound, sizeof(uint32_t) * std::max<int64_t>(child_rows, 1), s);
-      grow(w.row(nxt).rlist, sizeof(unsigned long long) * std::max<int64_t>(child_rows, 1), s);
-      grow(w.cur_rows, sizeof(unsigned long long) * C * rep, s);
-      grow(w.cur_list, sizeof(unsigned long long) * C * rep, s);
+      if (compact) {
+        grow(w.row(nxt).vt, (size_t)(4 + CS) * std::max<int64_t>(child_rows, 1), s);
+        grow(w.row(nxt).ctab, sizeof(uint2) * std::max<int64_t>(N.chunk0[C], 1), s);
+        a.crow_out = w.row(nxt).vt.as<uint32_t>();
+        a.child_tab = w.row(nxt).ctab.as<uint2>();
+        a.child_nom = child_nom;
+      } else {
+        grow(w.row(nxt).pid, sizeof(int32_t) * std::max<int64_t>(child_rows, 1), s);
+        grow(w.row(nxt).rgraph, sizeof(int32_t) * std::max<int64_t>(child_rows, 1), s);
+        grow(w.row(nxt).vt, (size_t)CS * std::max<int64_t>(child_rows, 1), s);
+        grow(w.row(nxt).rbound, sizeof(uint32_t) * std::max<int64_t>(child_rows, 1), s);
+        grow(w.row(nxt).rlist, sizeof(unsigned long long) * std::max<int64_t>(child_rows, 1), s);
+        grow(w.cur_rows, sizeof(unsigned long long) * C * rep, s);
+        grow(w.cur_list, sizeof(unsigned long long) * C * rep, s);
+      }
       grow(w.cursor, sizeof(unsigned long long) * C * rep, s);
       a.cur_rows = w.cur_rows.as<unsigned long long>();
       a.cur_list = w.cur_list.as<unsigned long long>();
@@ -1347,11 +1666,16 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.n_chunks = total_chunks;
       // child ids and cursors, then the write pass (launched back to back:
       // the device does not wait on the host between)
-      hip_check(launch_cursors(a, reinterpret_cast<const int32_t *>(su + fc_off),
-                               reinterpret_cast<const unsigned long long *>(su + rb_off),
-                               reinterpret_cast<const unsigned long long *>(su + lb_off), F, s),
-                "k_cursors");
-      hip_check(launch_write(a, root, s), "k_write");
+      const int32_t *fc = reinterpret_cast<const int32_t *>(su + fc_off);
+      const unsigned long long *rb = reinterpret_cast<const unsigned long long *>(su + rb_off);
+      if (compact) {
+        hip_check(launch_ccursors(a, fc, rb, reinterpret_cast<const uint32_t *>(su + lb_off), F, s), "k_ccursors");
+        hip_check(launch_cwrite(a, root, s), "k_cwrite");
+      } else {
+        hip_check(launch_cursors(a, fc, rb, reinterpret_cast<const unsigned long long *>(su + lb_off), F, s),
+                  "k_cursors");
+        hip_check(launch_write(a, root, s), "k_write");
+      }
       written_expect += (unsigned long long)child_rows;
       written_pending = true;
       counters_clear = true;
@@ -1386,7 +1710,10 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         N.node[c] = knode[i];
         N.alive[c] = kalive[i];
         nproj[c] = fr[i].proj;
-        if (wide) {
+        if (compact) {
+          make_cmeta(hu + (size_t)c * child_stride, cc, new_len, cv, cnv, N.job[c], (uint64_t)N.row0[c], fr[i].proj,
+                     !kalive[i], CS, rules);
+        } else if (wide) {
           hmw[c] = make_meta<kMaxPatV>(cc, new_len, cv, cnv, N.job[c]);
           if (!kalive[i]) hmw[c].flags |= kPatDead;
         } else {
@@ -1403,12 +1730,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       };
       auto mask_child = [&](int64_t c) {
         if (!N.alive[c]) return;  // dead patterns' rows are never extended
-        uint64_t *fw = hmask + (size_t)c * 2 * mstride, *bw = fw + mstride;
         const DFS *cc = N.c(c);
         const uint8_t *cv = N.vl(c);
-        // nv, nrm and the rightmost path's from vertices, either layout
-        const int m_nv = N.nv[c], m_nrm = wide ? hmw[c].nrm : hm[c].nrm;
-        const uint32_t *m_rm = wide ? hmw[c].rm : hm[c].rm;
+        const int m_nv = N.nv[c];
         const uint64_t *tj = &t2[(size_t)N.job[c] * NVL * AR];
         // per vertex: the arms that form a frequent path with every
         // pattern edge at it (one pass over the edges)
@@ -1420,6 +1744,24 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
           vm[v] &= tj[(size_t)cv[v] * AR + e + cv[u]];
         }
         const int rv = m_nv - 1;
+        if (compact) {
+          const CMetaHead *h = reinterpret_cast<const CMetaHead *>(hu + (size_t)c * child_stride);
+          CSource *src = reinterpret_cast<CSource *>(hu + (size_t)c * child_stride + sizeof(CMetaHead));
+          for (int k = 0; k < h->nsrc; ++k, ++src) src->keep = src->rule & vm[src->from];
+          // backward rv -> t (a pair's label is t's): a new arm at both ends
+          for (int k = 0; k < h->nback; ++k, ++src) {
+            const int t = src->from;
+            uint64_t b = 0;
+            for (int el = 0; el < NEL; ++el)
+              b |= ((vm[rv] >> (el * NVL + cv[t])) & (vm[t] >> (el * NVL + cv[rv])) & 1ull) << (el * NVL + cv[t]);
+            src->keep = src->rule & b;
+          }
+          return;
+        }
+        // nrm and the rightmost path's from vertices, either layout
+        uint64_t *fw = hmask + (size_t)c * 2 * mstride, *bw = fw + mstride;
+        const int m_nrm = wide ? hmw[c].nrm : hm[c].nrm;
+        const uint32_t *m_rm = wide ? hmw[c].rm : hm[c].rm;
         fw[0] = vm[rv];
         bw[0] = 0;
         for (int i = 0; i < m_nrm; ++i) {
@@ -1576,6 +1918,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       cf.S = CS;
       cf.n_rows = child_rows;
       cf.list_cap = std::max<uint64_t>(child_items, 1);  // the children's lists: exactly their item counts
+      cf.nom = child_nom;
+      cf.meta_stride = child_stride;
       cf.mask_off = child_mask_off;
       cf.mask_stride = child_mask_stride;
       cf.code_off = child_code_off;

@@ -80,8 +80,9 @@ struct HostBuf {
 // (metadata, path masks, codes).
 struct RowSet {
   DevBuf pid, rgraph, vt, rbound, rlist, upl;
-  std::vector<DevBuf *> bufs() { return {&pid, &rgraph, &vt, &rbound, &rlist, &upl}; }
-  size_t bytes() const { return pid.cap + rgraph.cap + vt.cap + rbound.cap + rlist.cap + upl.cap; }
+  DevBuf ctab;  // compact levels: the chunk table (their rows, {graph, tuple}, are in vt)
+  std::vector<DevBuf *> bufs() { return {&pid, &rgraph, &vt, &rbound, &rlist, &upl, &ctab}; }
+  size_t bytes() const { return pid.cap + rgraph.cap + vt.cap + rbound.cap + rlist.cap + upl.cap + ctab.cap; }
 };
 
 // Device buffers of the level steps, kept across mining calls on one
@@ -161,6 +162,13 @@ struct DeviceDB {
   std::vector<int32_t> job_first_graph;       // n_jobs + 1
   std::vector<int64_t> job_first_vertex;      // n_jobs + 1 (the root level's rows of each job)
   DevBuf gvbase, vadj, adj, vlab, gjob, vgraph;
+  // compact layout beside it (device.hpp), where the database qualifies
+  bool compact = false;
+  int64_t n_groups = 0;
+  int32_t root_nom = 0;              // nominal rows of a root chunk
+  std::vector<uint32_t> ggb;         // first group of each graph, n_graphs + 1
+  std::vector<int64_t> root_chunk0;  // n_jobs + 1: first root chunk of each job
+  DevBuf vgrp, rrows, rtab, dggb;
   size_t bytes = 0;
   // mining state; one mining call at a time per database
   std::unique_ptr<Workspace> ws;
@@ -173,6 +181,9 @@ struct PackedDB {
   std::vector<int32_t> gvbase, vadj, gjob, vgraph;
   std::vector<uint32_t> adj;
   std::vector<uint8_t> vlab;
+  // compact layout (device.hpp); empty when the database does not qualify
+  std::vector<unsigned long long> vgrp;
+  std::vector<uint2> rrows;
 };
 
 // Validate the databases (one job each) for the device path and pack them:

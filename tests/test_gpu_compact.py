@@ -1,0 +1,105 @@
+"""The compact level kernels (graphs of at most 64 vertices, small label
+alphabets) at the edges of their layout, against the oracle: patterns,
+supports, |Proj(P)|, E_child and E_cand, all whole numbers, exactly equal.
+
+A vertex's neighbours come in groups of four, the first two of which are
+tested in registers; a block is up to 64 rows of whole segments (rows of one
+graph), longer segments are carried from block to block; a chunk's list names
+rows up to 8,192 from a base; label pairs are tested in 32 bits below 32 of
+them."""
+import random
+
+import pytest
+
+import gpu_graph_mining_amd as gm
+from oracle import py_oracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+def star(leaves, vlab=0, elab=0):
+    return [vlab] * (leaves + 1), [(0, v, elab) for v in range(1, leaves + 1)]
+
+
+def clique(n, elab=0):
+    return [0] * n, [(a, b, elab) for a in range(n) for b in range(a + 1, n)]
+
+
+def paths(k):
+    """k disjoint paths of three equal vertices: 4 k rows of the 1-edge
+    pattern, 2 k of the path's."""
+    return [0] * (3 * k), [e for i in range(k) for e in ((3 * i, 3 * i + 1, 0), (3 * i + 1, 3 * i + 2, 0))]
+
+
+def tree(rng, n, nvl, nel, extra=0):
+    labels = [rng.randrange(nvl) for _ in range(n)]
+    pairs = {(rng.randrange(v), v) for v in range(1, n)}
+    while extra:
+        a, b = sorted(rng.sample(range(n), 2))
+        extra -= (a, b) not in pairs
+        pairs.add((a, b))
+    return labels, [(a, b, rng.randrange(nel)) for a, b in sorted(pairs)]
+
+
+def all_labels(nvl, nel):
+    """A graph that holds every label, so that the alphabets have these sizes."""
+    n = max(nvl, nel + 1)
+    return [v % nvl for v in range(n)], [(v, v + 1, v % nel) for v in range(n - 1)]
+
+
+def mixed(nvl, nel, sizes, extra=3):
+    rng = random.Random(17 * nvl + nel)
+    return [all_labels(nvl, nel)] + [tree(rng, n, nvl, nel, min(extra, n * (n - 1) // 2 - (n - 1))) for n in sizes]
+
+
+CASES = {
+    # one to four groups a vertex (4 | 5, 8 | 9 neighbours); segments of 11,880 rows
+    "stars": ([star(n) for n in (1, 3, 4, 5, 8, 9, 12, 12)], 1, 4),
+    # backward edges among a vertex's third group
+    "cliques": ([clique(n) for n in (3, 5, 6, 9, 10)], 1, 3),
+    # segments of exactly 64, 32, 60, 68, 84 and 4 rows, whole blocks of them
+    "paths": ([paths(k) for k in (16, 16, 8, 8, 15, 17, 1, 21, 16)] + [paths(16)] * 9, 1, 0),
+    # the largest graphs, two of them with 64 rows in one segment
+    "64_vertices": (mixed(3, 2, [64, 64, 63, 64, 2, 1, 33]) + [star(63)], 1, 3),
+    # 25 label pairs (32-bit masks), 31, and 42 and 56 (64-bit masks; 56 = 7 edge labels x 8, the largest keys)
+    "labels_5x5": (mixed(5, 5, [20] * 40), 2, 4),
+    "labels_31x1": (mixed(31, 1, [30] * 30), 2, 4),
+    "labels_6x7": (mixed(6, 7, [25] * 40), 2, 4),
+    "labels_8x7": (mixed(8, 7, [40] * 30), 2, 4),
+    # one past the compact alphabets: the general kernels
+    "labels_8x8": (mixed(8, 8, [40] * 30), 2, 4),
+    # graphs without edges or vertices between the others
+    "empty_graphs": ([([], []), star(3), ([0], []), clique(4), ([], []), star(3)], 1, 0),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_compact_levels_match_the_oracle(name):
+    graphs, minsup, max_edges = CASES[name]
+    db = gm.GraphDB.from_graphs(graphs)
+    opats, ost = po.mine_arrays(db.arrays(), minsup, max_edges=max_edges)
+    want = {po.normalize(c): (s, n) for c, s, n in opats}
+    print("case", name, len(want), "patterns", flush=True)
+    for kw in ({}, {"path_pruning": False, "speculate": 2}, {"mem_budget": 20000}, {"canon_host": 2, "chunk_rows": 64}):
+        if kw.get("mem_budget") and len(want) > 2000:
+            continue  # (a level step per piece)
+        print("options", kw, flush=True)
+        pats, st = gm.mine(db, minsup, max_edges=max_edges, collect_proj=True, **kw)
+        assert {po.normalize(c): (s, n) for c, s, n in pats} == want and len(pats) == len(want)
+        assert (st["e_child"], st["e_cand"]) == (ost["e_child"], ost["e_cand"])
+
+
+def test_subsets_of_a_compact_database():
+    """Gathered groups and root rows: each subset's patterns are the oracle's
+    on the same graphs, in a batch of several subsets (one of them empty)."""
+    graphs = mixed(4, 3, [3, 9, 30, 17, 1, 25, 40, 12] * 6)
+    db = gm.GraphDB.from_graphs(graphs)
+    db.upload()
+    rng = random.Random(3)
+    subsets = [rng.sample(range(len(graphs)), 20), list(range(len(graphs))), [], [5, 5, 5], [0]]
+    batch = gm.Batch.from_subsets(db, subsets)
+    res, _ = batch.mine([4, 6, 1, 3, 1], collect_proj=True)
+    for ids, minsup, pats in zip(subsets, [4, 6, 1, 3, 1], res):
+        arrays = gm.GraphDB.from_graphs([graphs[i] for i in ids]).arrays() if ids else None
+        opats = po.mine_arrays(arrays, minsup)[0] if ids else []
+        assert {po.normalize(c): (s, n) for c, s, n in pats} == {po.normalize(c): (s, n) for c, s, n in opats}
