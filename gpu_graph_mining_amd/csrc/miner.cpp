@@ -618,9 +618,11 @@ struct LabelRules {
 
 // A compact level's pattern: its head, sources and backward targets into
 // dst.  Sources no label pair gets through from are left out (but the
-// rightmost vertex's, which the backward targets need).
+// rightmost vertex's, which the backward targets need).  In query mode only
+// the tuples in `want` (the trie node's continuations) get through: the other
+// extensions are neither enumerated nor listed.
 void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv, int32_t job, uint64_t row0,
-                uint64_t nrows, bool dead, int S, const LabelRules &lr) {
+                uint64_t nrows, bool dead, int S, const LabelRules &lr, const std::vector<std::pair<DFS, int32_t>> *want) {
   const PatMetaWide m = make_meta<kMaxPatV>(code, len, vlab, nv, job);
   CMetaHead h;
   std::memset(&h, 0, sizeof(h));
@@ -629,6 +631,16 @@ void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv
   h.flags = dead ? (uint8_t)kPatDead : 0;
   h.row0 = row0;
   h.nrows = nrows;
+  // the label pairs wanted from pattern vertex f, forward or backward to it
+  auto wanted = [&](int f, bool forward) -> uint64_t {
+    if (!want) return ~uint64_t(0);
+    uint64_t w = 0;
+    for (const auto &k : *want) {
+      const DFS &t = k.first;
+      if ((t.from < t.to) == forward && (forward ? t.from : t.to) == f) w |= 1ull << (t.elabel * lr.NVL + t.tolabel);
+    }
+    return w;
+  };
   CSource *out = reinterpret_cast<CSource *>(dst + sizeof(CMetaHead));
   const int SB = S * lr.NEL;
   auto add = [&](uint64_t rule, int from, int kbase) {
@@ -646,14 +658,14 @@ void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv
     if ((bwd >> f) & 1) continue;  // the edge is in the pattern already
     // pairs (e, label of f) with e1 < e or (e1 == e and l1 <= maxlabel)
     const int e0 = l1 <= m.maxlabel ? e1 : e1 + 1;
-    const uint64_t rule = e0 < lr.NEL ? (lr.rep & (~0ull << (e0 * lr.NVL))) << vlab[f] : 0;
+    const uint64_t rule = e0 < lr.NEL ? (lr.rep & (~0ull << (e0 * lr.NVL))) << vlab[f] & wanted(f, false) : 0;
     if (!rule) continue;
     back[nback].rule = back[nback].keep = rule;
     back[nback].from = f;
     back[nback].kbase = f * lr.NEL;
     ++nback;
   }
-  const uint64_t own = lr.labels(m.minlabel) * lr.rep;
+  const uint64_t own = lr.labels(m.minlabel) * lr.rep & wanted(rv, true);
   int nsrc = 0;
   if (own || nback) {
     add(own, rv, SB + rv * lr.AR);
@@ -661,7 +673,8 @@ void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv
   }
   for (int q = 0; q < m.nrm; ++q) {
     const int f = (int)(m.rm[q] & 0xFF);
-    const uint64_t rule = lr.after(m.minlabel, (int)((m.rm[q] >> 8) & 0xFF), (int)((m.rm[q] >> 16) & 0xFF));
+    const uint64_t rule =
+        lr.after(m.minlabel, (int)((m.rm[q] >> 8) & 0xFF), (int)((m.rm[q] >> 16) & 0xFF)) & wanted(f, true);
     if (!rule) continue;
     add(rule, f, SB + f * lr.AR);
     ++nsrc;
@@ -1712,7 +1725,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         nproj[c] = fr[i].proj;
         if (compact) {
           make_cmeta(hu + (size_t)c * child_stride, cc, new_len, cv, cnv, N.job[c], (uint64_t)N.row0[c], fr[i].proj,
-                     !kalive[i], CS, rules);
+                     !kalive[i], CS, rules, opt.queries ? &opt.queries->nodes[knode[i]].kids : nullptr);
         } else if (wide) {
           hmw[c] = make_meta<kMaxPatV>(cc, new_len, cv, cnv, N.job[c]);
           if (!kalive[i]) hmw[c].flags |= kPatDead;
