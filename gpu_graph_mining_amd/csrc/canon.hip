@@ -388,6 +388,8 @@ __global__ void __launch_bounds__(64) k_canon_level(CanonArgs c) {
       const unsigned long long w = (f[1] & 0xFFFFFFFFull) | ((unsigned long long)(res + 1) << 32);
       f[1] = w;
       if (c.down && slot < c.down_cap) c.down[4ull * slot + 1] = w;
+      if (c.spread && res != kCanonNotMin)
+        atomicMax(&c.spread[(slot & (kSpread - 1)) * kSpreadStride + kSpreadNv], (unsigned long long)nv);
     }
   }
 }

@@ -39,6 +39,7 @@
 // block of 8-byte tuples with half of its lanes idle.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <type_traits>
 
@@ -145,8 +146,9 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
   uint64_t first;
   const char *meta = nullptr;
   CMetaHead H = {};
-  const uint32_t nom = (uint32_t)GM_ARG(nom);
+  uint32_t nom;
   if constexpr (ROOT) {
+    nom = (uint32_t)GM_ARG(nom);
     const uint4 ct = cload<uint4>(GM_ARG(rtab) + GM_ARG(tab0) + gci);
     p = (int)ct.x;
     first = ct.z;
@@ -159,6 +161,7 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
     H = cload<CMetaHead>(meta);
     first = H.row0;
     pend = (uint32_t)H.nrows;
+    nom = H.nom;
     nom0 = (uint32_t)uniform((int)ct.y) * nom;
   }
   const uint32_t nom1 = pend - nom0 <= nom ? pend : nom0 + nom;
@@ -639,13 +642,13 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
     atomicAdd(&a.spread[(gci & (kSpread - 1)) * kSpreadStride + kSpreadWritten], written);
 }
 
-// After the host chose the children (see k_cursors): every (child, replica)'s
+// ------------------------------------------------------------- CHILDREN
+// After the children were chosen (see k_cursors): every (child, replica)'s
 // cursor starts at its first row, and the children's chunk table is filled
-// ({child, chunk of the child}).  `rep` lanes take one frequent key.
-__global__ void __launch_bounds__(256) k_ccursors(StepArgs a, const int32_t *fchild, const unsigned long long *row_base,
-                                                  const uint32_t *chunk_base, int64_t F) {
-  if (blockIdx.x == 0) clear_counters(a);
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// ({child, chunk of the child}).  `rep` lanes take one frequent key; t is the
+// lane's index over all of them.
+__device__ __forceinline__ void cursors_of(const StepArgs &a, int64_t t, const int32_t *fchild,
+                                           const unsigned long long *row_base, const uint32_t *chunk_base, int64_t F) {
   const int64_t i = t / a.rep;
   const int r = (int)(t % a.rep);
   const bool ok = i < F;
@@ -663,15 +666,278 @@ __global__ void __launch_bounds__(256) k_ccursors(StepArgs a, const int32_t *fch
     const unsigned long long y = __shfl_up(sr, o, 64);
     if (r >= o) sr += y;
   }
-  const unsigned long long all = __shfl(sr, ((threadIdx.x & 63) | (a.rep - 1)), 64);
   if (!ok) return;
   a.acc[at] = 0;
   if (ch < 0) return;
   if (r == 0) a.sup[key] = -(ch + 1);
   a.cursor[(int64_t)ch * a.rep + r] = row_base[ch] + (sr - rows);
-  const uint32_t n = (uint32_t)((all + (unsigned long long)a.child_nom - 1) / (unsigned long long)a.child_nom);
+  const unsigned long long all = a.freq[4 * i + 2];
+  const uint32_t n =
+      chunk_count((uint32_t)all, chunk_nominal((uint32_t)a.child_blocks, (uint32_t)all, (uint32_t)a.freq[4 * i + 1]));
   uint2 *tab = a.child_tab + chunk_base[ch];
   for (uint32_t k = (uint32_t)r; k < n; k += (uint32_t)a.rep) tab[k] = make_uint2((uint32_t)ch, k);
+}
+
+__global__ void __launch_bounds__(256) k_ccursors(StepArgs a, const int32_t *fchild, const unsigned long long *row_base,
+                                                  const uint32_t *chunk_base, int64_t F) {
+  if (blockIdx.x == 0) clear_counters(a);
+  cursors_of(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, fchild, row_base, chunk_base, F);
+}
+
+// The children, chosen on the device: a tile of 1,024 records per workgroup,
+// which adds up the records before its tile itself (a pass over at most a few
+// ten thousand of them, cheaper than a launch for their sums).  The last
+// tile's workgroup has the totals.  When the host chose, it read the list,
+// numbered the children and sent ids, bases and metadata back: 100-350 us
+// between k_reduce_list and the next k_clevel on the 100,000-transaction
+// levels of 5,000-11,000 records; the host now waits for four words.
+constexpr int kSelThreads = 1024;
+
+struct SelSums {
+  unsigned long long rows, dropped;
+  uint32_t n, chunks, undecided;
+  __device__ __forceinline__ void add(const SelSums &x) {
+    rows += x.rows;
+    dropped += x.dropped;
+    n += x.n;
+    chunks += x.chunks;
+    undecided += x.undecided;
+  }
+};
+
+template <bool ROOT>
+__device__ __forceinline__ SelSums sel_of(const StepArgs &a, uint32_t i) {
+  const unsigned long long w = a.freq[4ull * i + 1], rows = a.freq[4ull * i + 2];
+  const uint32_t answer = (uint32_t)(w >> 32) & 0xFFu;  // k_canon_level's, + 1
+  const bool sel = ROOT || answer == kCanonMin + 1;
+  SelSums s;
+  s.n = sel ? 1u : 0u;
+  s.rows = sel ? rows : 0ull;
+  s.dropped = sel ? 0ull : rows;
+  s.chunks =
+      sel ? chunk_count((uint32_t)rows, chunk_nominal((uint32_t)a.child_blocks, (uint32_t)rows, (uint32_t)w)) : 0u;
+  s.undecided = !ROOT && answer != kCanonMin + 1 && answer != kCanonNotMin + 1 ? 1u : 0u;
+  return s;
+}
+
+__device__ __forceinline__ SelSums wave_total(const SelSums &x) {
+  return SelSums{wave_sum(x.rows), wave_sum(x.dropped), wave_sum(x.n), wave_sum(x.chunks), wave_sum(x.undecided)};
+}
+
+template <bool ROOT>
+__global__ void __launch_bounds__(kSelThreads) k_cselect(StepArgs a, CSelect c) {
+  constexpr int kWaves = kSelThreads / 64;
+  __shared__ SelSums s_before[kWaves], s_own[kWaves];
+  const uint32_t F = min(*a.freq_count, a.freq_cap);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t tiles = F > 0 ? (F + kSelThreads - 1) / kSelThreads : 1u;
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    SelSums b{0, 0, 0, 0, 0};  // the lane's share of the records before the tile
+    for (uint32_t i = threadIdx.x; i < tile * kSelThreads; i += kSelThreads) b.add(sel_of<ROOT>(a, i));
+    const uint32_t i = tile * kSelThreads + threadIdx.x;
+    const SelSums x = i < F ? sel_of<ROOT>(a, i) : SelSums{0, 0, 0, 0, 0};
+    const SelSums wb = wave_total(b), wx = wave_total(x);
+    if (lane == 0) {
+      s_before[wave] = wb;
+      s_own[wave] = wx;
+    }
+    __syncthreads();
+    SelSums base{0, 0, 0, 0, 0};  // everything before this wave's records
+#pragma unroll 1
+    for (int q = 0; q < kWaves; ++q) {
+      base.add(s_before[q]);
+      if (q < wave) base.add(s_own[q]);
+    }
+    if (tile == tiles - 1 && wave == kWaves - 1) {  // base and this wave's own: the totals
+      unsigned long long nv = 2;
+      if (!ROOT) {
+        nv = a.spread[lane * kSpreadStride + kSpreadNv];
+        for (int o = 32; o > 0; o >>= 1) nv = max(nv, __shfl_xor(nv, o, 64));
+      }
+      if (lane == 0) {
+        a.down[kTotChildren] = (unsigned long long)(base.n + wx.n) | (unsigned long long)(base.undecided + wx.undecided) << 32;
+        a.down[kTotRows] = base.rows + wx.rows;
+        a.down[kTotChunks] = (unsigned long long)(base.chunks + wx.chunks) | nv << 32;
+        a.down[kTotDropped] = base.dropped + wx.dropped;
+      }
+    }
+    unsigned long long tr;
+    uint32_t tn, tc;
+    const unsigned long long er = wave_exclusive_scan<unsigned long long>(x.rows, tr);
+    const uint32_t en = wave_exclusive_scan<uint32_t>(x.n, tn), ec = wave_exclusive_scan<uint32_t>(x.chunks, tc);
+    if (i < F) c.fchild[i] = x.n ? (int32_t)(base.n + en) : -1;
+    if (x.n) {
+      const uint32_t ch = base.n + en;
+      c.crec[ch] = i;
+      c.row_base[ch] = base.rows + er;
+      c.chunk_base[ch] = base.chunks + ec;
+    }
+    __syncthreads();
+  }
+}
+
+// A frequent key as the tuple it adds to pattern p of nv vertices.
+struct NewTuple {
+  int from, to, el, tl;  // tl: the to vertex's label; root: of vertex 1
+  int fl;                // root: of vertex 0
+  bool forward;
+};
+template <bool ROOT>
+__device__ __forceinline__ NewTuple tuple_of(const StepArgs &a, uint32_t x, int nv) {
+  NewTuple t{0, 1, 0, 0, 0, true};
+  const uint32_t NEL = (uint32_t)a.NEL, NVL = (uint32_t)a.NVL, SB = (uint32_t)a.S * NEL;
+  if (ROOT || x >= SB) {
+    const uint32_t y = ROOT ? x : x - SB, y1 = y / NVL;
+    t.tl = (int)(y - y1 * NVL);
+    const uint32_t f = y1 / NEL;
+    t.el = (int)(y1 - f * NEL);
+    if (ROOT) {
+      t.fl = (int)f;
+    } else {
+      t.from = (int)f;
+      t.to = nv;
+    }
+  } else {
+    t.forward = false;
+    t.from = nv - 1;
+    t.to = (int)(x / NEL);
+    t.el = (int)(x - (uint32_t)t.to * NEL);
+  }
+  return t;
+}
+
+// The 2-edge children's arms: (0,1,a,e1,b) then (1,2,b,e2,c) is the path with
+// centre b, or (0,2,a,e2,c) with centre a.
+__global__ void __launch_bounds__(256) k_ct2(StepArgs a, CMetaArgs m) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= m.C) return;
+  const uint32_t key = (uint32_t)a.freq[4ull * m.crec[c]], p = key / (uint32_t)a.K;
+  const CMetaHead H = *reinterpret_cast<const CMetaHead *>(reinterpret_cast<const char *>(a.meta) + (int64_t)p * a.meta_stride);
+  const NewTuple t = tuple_of<false>(a, key - p * (uint32_t)a.K, H.nv);
+  const uint32_t w = m.pcode[p];
+  const int l0 = m.pvlab[(int64_t)p * a.S], l1 = m.pvlab[(int64_t)p * a.S + 1], e1 = (int)(w >> 16 & 0xFF);
+  const bool at1 = t.from == 1;
+  const int centre = at1 ? l1 : l0, arm1 = e1 * a.NVL + (at1 ? l0 : l1), arm2 = t.el * a.NVL + t.tl;
+  unsigned long long *row = m.t2 + ((int64_t)H.job * a.NVL + centre) * a.AR;
+  atomicOr(&row[arm1], 1ull << arm2);
+  atomicOr(&row[arm2], 1ull << arm1);
+}
+
+// Cursors and chunk table (the first blocks), then the children's metadata,
+// one wave per child: the child's code is its parent's plus the new tuple; the
+// rightmost path follows the forward tuples from the last vertex to the root;
+// a path vertex's rule (CSource) is a lane's.  The same facts as the host's
+// make_cmeta.
+struct ChildLds {
+  unsigned long long vm[kCompactV];  // arms that go with every pattern edge at a vertex (path rule)
+  unsigned long long bwd;            // vertices the rightmost one has an edge to
+  uint32_t code[64];
+  uint8_t lab[kCompactV], found[kCompactV], path[kCompactV];  // label; its forward tuple; rightmost path's tuples
+};
+
+template <bool ROOT>
+__global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaArgs m, int64_t F, int64_t cursor_blocks) {
+  __shared__ ChildLds lds[4];
+  if ((int64_t)blockIdx.x < cursor_blocks) {
+    if (blockIdx.x == 0) clear_counters(a);
+    cursors_of(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, c.fchild, c.row_base, c.chunk_base, F);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  ChildLds &L = lds[threadIdx.x >> 6];
+  const int64_t ci = ((int64_t)blockIdx.x - cursor_blocks) * 4 + (threadIdx.x >> 6);
+  if (ci >= m.C) return;
+  const unsigned long long *f = a.freq + 4ull * m.crec[ci];
+  const uint32_t key = (uint32_t)f[0], p = key / (uint32_t)a.K;  // below 2^26: one piece
+  int job = (int)p, nv = 2;
+  if constexpr (!ROOT) {
+    const CMetaHead H = *reinterpret_cast<const CMetaHead *>(reinterpret_cast<const char *>(a.meta) + (int64_t)p * a.meta_stride);
+    job = H.job;
+    nv = H.nv;
+  }
+  NewTuple t = tuple_of<ROOT>(a, key - p * (uint32_t)a.K, nv);
+  const int cnv = !ROOT && t.forward ? nv + 1 : nv, n = m.len + 1;  // the child's vertices and tuples (n <= 64)
+  // labels and code
+  if (lane < a.CS) {
+    int l = 0;
+    if (lane < cnv) {
+      if (ROOT)
+        l = lane == 0 ? t.fl : t.tl;
+      else
+        l = lane < nv ? (int)m.pvlab[(int64_t)p * a.S + lane] : t.tl;
+    }
+    L.lab[lane] = (uint8_t)l;
+    m.vlab[ci * a.CS + lane] = (uint8_t)l;
+  }
+  L.vm[lane] = ~0ull;
+  if (lane == 0) L.bwd = 0;
+  wave_sync();
+  if (lane < n) {
+    const int tl = ROOT || t.forward ? t.tl : (int)L.lab[t.to];
+    const uint32_t w = lane < m.len ? m.pcode[(int64_t)p * m.len + lane]
+                                    : (uint32_t)t.from | (uint32_t)t.to << 8 | (uint32_t)t.el << 16 | (uint32_t)tl << 24;
+    L.code[lane] = w;
+    m.code[ci * n + lane] = w;
+    const int u = (int)(w & 0xFF), v = (int)(w >> 8 & 0xFF);
+    if (u < v) L.found[v] = (uint8_t)lane;
+    else if (u == cnv - 1) atomicOr(&L.bwd, 1ull << v);
+    if (m.masks) {
+      const int e = (int)(w >> 16 & 0xFF) * a.NVL;
+      const unsigned long long *tj = m.t2 + (int64_t)job * a.NVL * a.AR;
+      atomicAnd(&L.vm[u], tj[L.lab[u] * a.AR + e + L.lab[v]]);
+      atomicAnd(&L.vm[v], tj[L.lab[v] * a.AR + e + L.lab[u]]);
+    }
+  }
+  wave_sync();
+  int nrm = 0;
+  for (int v = cnv - 1; v > 0;) {
+    const int k = L.found[v];
+    if (lane == 0) L.path[nrm] = (uint8_t)k;
+    ++nrm;
+    v = (int)(L.code[k] & 0xFF);
+  }
+  wave_sync();
+  // lane q: the rightmost path's edge q and its from vertex f
+  const uint32_t w = lane < nrm ? L.code[L.path[lane]] : 0u;
+  const int fv = (int)(w & 0xFF), e1 = (int)(w >> 16 & 0xFF), l1 = lane < nrm ? (int)L.lab[w >> 8 & 0xFF] : 0;
+  const int lf = (int)L.lab[fv], rv = cnv - 1, minlabel = (int)L.lab[0], maxlabel = (int)L.lab[rv];
+  const unsigned long long all = (1ull << a.NVL) - 1ull;
+  auto from_label = [&](int x) GM_INLINE -> unsigned long long { return all & (~0ull << x); };
+  // forward from f: (e, l) with l >= minlabel and (e1 < e or (e1 == e and l1 <= l))
+  unsigned long long fr = 0, br = 0;
+  if (lane < nrm) {
+    if (e1 + 1 < a.NEL) fr = (from_label(minlabel) * a.lab_rep) & (~0ull << ((e1 + 1) * a.NVL));
+    fr |= from_label(max(minlabel, l1)) << (e1 * a.NVL);
+    // backward to f: (e, label of f) with e1 < e or (e1 == e and l1 <= maxlabel)
+    const int e0 = l1 <= maxlabel ? e1 : e1 + 1;
+    if (lane > 0 && !((L.bwd >> fv) & 1ull) && e0 < a.NEL) br = (a.lab_rep & (~0ull << (e0 * a.NVL))) << lf;
+  }
+  const uint64_t mf = __ballot(fr != 0), mb = __ballot(br != 0);
+  const unsigned long long own = from_label(minlabel) * a.lab_rep;
+  const int has_own = own || mb ? 1 : 0, nsrc = has_own + __popcll(mf), nback = __popcll(mb);
+  const int SB = a.CS * a.NEL;
+  char *out = m.meta + ci * m.meta_stride;
+  CSource *src = reinterpret_cast<CSource *>(out + sizeof(CMetaHead));
+  if (lane == 0) {
+    CMetaHead h;
+    h.job = job;
+    h.nv = (uint8_t)cnv;
+    h.nsrc = (uint8_t)nsrc;
+    h.nback = (uint8_t)nback;
+    h.flags = 0;
+    h.row0 = c.row_base[ci];
+    h.nrows = f[2];
+    h.nom = chunk_nominal((uint32_t)a.child_blocks, (uint32_t)f[2], (uint32_t)f[1]);
+    h.pad = 0;
+    *reinterpret_cast<CMetaHead *>(out) = h;
+    if (has_own) src[0] = CSource{own, own & L.vm[rv], rv, SB + rv * a.AR};
+  }
+  if (fr) src[has_own + (int)below(mf)] = CSource{fr, fr & L.vm[fv], fv, SB + fv * a.AR};
+  if (br) {
+    // a new arm at both ends: (e, label of f) at the rightmost vertex, (e, its label) at f
+    const unsigned long long both = (L.vm[rv] >> lf) & (L.vm[fv] >> maxlabel) & a.lab_rep;
+    src[nsrc + (int)below(mb)] = CSource{br, m.masks ? br & (both << lf) : br, fv, fv * a.NEL};
+  }
 }
 
 // A compact database of selected graphs gathered from a resident one: one
@@ -744,6 +1010,34 @@ hipError_t launch_ccursors(const StepArgs &a, const int32_t *fchild, const unsig
   if (F <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_ccursors, dim3((unsigned)((F * a.rep + 255) / 256)), dim3(256), 0, s, a, fchild, row_base,
                      chunk_base, F);
+  return hipGetLastError();
+}
+
+hipError_t launch_cselect(const StepArgs &a, const CSelect &c, bool root, uint32_t expect, hipStream_t s) {
+  // a workgroup per tile of the records expected, any number covers them
+  const unsigned g = std::max(1u, std::min(256u, (expect + kSelThreads - 1) / kSelThreads));
+  if (root)
+    hipLaunchKernelGGL(k_cselect<true>, dim3(g), dim3(kSelThreads), 0, s, a, c);
+  else
+    hipLaunchKernelGGL(k_cselect<false>, dim3(g), dim3(kSelThreads), 0, s, a, c);
+  return hipGetLastError();
+}
+
+hipError_t launch_cchildren(const StepArgs &a, const CSelect &c, const CMetaArgs &m, bool root, int64_t F, hipStream_t s) {
+  if (F <= 0) return hipSuccess;
+  if (m.C > 0 && m.len + 1 > 64) return hipErrorInvalidValue;
+  const int64_t cb = (F * a.rep + 255) / 256;
+  const unsigned g = (unsigned)(cb + (m.C + 3) / 4);
+  if (root)
+    hipLaunchKernelGGL(k_cchildren<true>, dim3(g), dim3(256), 0, s, a, c, m, F, cb);
+  else
+    hipLaunchKernelGGL(k_cchildren<false>, dim3(g), dim3(256), 0, s, a, c, m, F, cb);
+  return hipGetLastError();
+}
+
+hipError_t launch_ct2(const StepArgs &a, const CMetaArgs &m, hipStream_t s) {
+  if (m.C <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_ct2, dim3((unsigned)((m.C + 255) / 256)), dim3(256), 0, s, a, m);
   return hipGetLastError();
 }
 

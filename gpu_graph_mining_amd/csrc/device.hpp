@@ -119,12 +119,24 @@ struct alignas(8) CMetaHead {
   int32_t job;
   uint8_t nv, nsrc, nback, flags;  // flags: kPatDead
   uint64_t row0, nrows;            // the pattern's rows
+  uint32_t nom, pad;               // nominal rows of its chunks
 };
 struct alignas(8) CSource {
   uint64_t rule, keep;
   int32_t from;   // pattern vertex
   int32_t kbase;  // first key: forward, of (from, label pair 0); backward, of (target, edge label 0)
 };
+// Nominal rows of a chunk of about `blocks` blocks of 64 rows, for `rows` rows
+// in `segs` segments: a block ends at a segment start and the last one has to
+// reach the first start past the nominal end, so each gives up about a
+// segment.  (With nominal lengths of whole blocks every chunk ended in a block
+// of a few rows.)
+// (A pattern has fewer than 2^32 rows: 32-bit divisions.)
+__host__ __device__ inline uint32_t chunk_nominal(uint32_t blocks, uint32_t rows, uint32_t segs) {
+  const uint32_t seg = segs > 0 && rows > 0 ? (rows - 1) / segs + 1 : 1;
+  return seg >= 32 ? 64 * blocks : blocks * (63 - seg);
+}
+__host__ __device__ inline uint32_t chunk_count(uint32_t rows, uint32_t nom) { return rows > 0 ? (rows - 1) / nom + 1 : 0; }
 __host__ __device__ constexpr int cmeta_bytes(int max_nv) { return (int)sizeof(CMetaHead) + 2 * max_nv * (int)sizeof(CSource); }
 
 }  // namespace gm

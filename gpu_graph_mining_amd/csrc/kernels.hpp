@@ -31,8 +31,12 @@ constexpr int kSpreadStart = 4;    // ~(earliest start) of the extension + suppo
 constexpr int kSpreadEnd = 5;      // latest end of the stage (atomicMax); device wall clock
 constexpr int kSpreadWritten = 6;  // child rows written by k_write
 constexpr int kSpreadFailed = 7;   // chunks recounted by k_level_fix
+constexpr int kSpreadNv = 8;       // most vertices of a child that k_canon_level let through (atomicMax)
 // the counter block: 8 words (frequent keys, failed chunks, error bits), then the spread lines
 constexpr int kCounterWords = 8 + kSpread * kSpreadStride;
+// words of the block that k_cselect fills: children | undecided records << 32,
+// their rows, their chunks | most vertices << 32, the dropped records' rows
+constexpr int kTotChildren = 2, kTotRows = 3, kTotChunks = 4, kTotDropped = 5;
 
 // One chunk of a level's rows: [start, end) after alignment to segment
 // starts (a segment is the rows of one pattern in one graph; at the root,
@@ -143,15 +147,31 @@ struct StepArgs {
   const uint4 *rtab;      // root chunks
   const uint2 *ctab;      // later levels' chunks: {pattern, chunk of the pattern}
   int64_t tab0;           // first chunk of the piece in its table
-  int32_t nom;            // nominal rows of a chunk
+  int32_t nom;            // nominal rows of a root chunk (later levels': in their metadata)
   CChunk *cchunks;
   uint32_t *clist;        // chunk c's first extent at c * page; then 64 pool slices of pool_sub units from unit pool0
   uint32_t page, pool0, pool_sub;
   int32_t AR;             // label pairs: NEL * NVL
   uint32_t inv_nvl;       // (x * inv_nvl) >> 16 = x / NVL for x < 64
   unsigned long long lab_rep;  // bit el * NVL for every edge label
-  uint2 *child_tab;       // the children's chunk table, child_nom rows a chunk
-  int32_t child_nom;
+  uint2 *child_tab;       // the children's chunk table
+  int32_t child_blocks;   // blocks of a child's chunk (chunk_nominal)
+};
+// The children's metadata built on the device (k_cchildren), from the level's
+// codes and labels: len tuples and S labels a pattern (root: none).
+struct CMetaArgs {
+  const uint32_t *pcode;
+  const uint8_t *pvlab;
+  int32_t len;
+  const uint32_t *crec;  // child -> record of the frequent list
+  int64_t C;
+  // path rule: arms t2[(job * NVL + centre) * AR + arm]; null: none
+  unsigned long long *t2;
+  int32_t masks;         // the table is complete: the sources' keep masks follow it
+  char *meta;            // out: meta_stride bytes a child
+  int32_t meta_stride;
+  uint32_t *code;        // out: len + 1 tuples a child
+  uint8_t *vlab;         // out: CS labels a child
 };
 // Compact levels: dynamic LDS of k_clevel, and the launches (see the general
 // ones below).
@@ -160,6 +180,20 @@ hipError_t launch_clevel(const StepArgs &a, bool root, hipStream_t s);
 hipError_t launch_cwrite(const StepArgs &a, bool root, hipStream_t s);
 hipError_t launch_ccursors(const StepArgs &a, const int32_t *fchild, const unsigned long long *row_base,
                            const uint32_t *chunk_base, int64_t F, hipStream_t s);
+// Choose the children on the device: the frequent records whose code is
+// minimal (root: all), in key order; their ids, first rows and first chunks,
+// and the totals for the host (kTot* words of a.down).
+struct CSelect {
+  int32_t *fchild;                // per record
+  uint32_t *crec;                 // per child
+  unsigned long long *row_base;   // per child
+  uint32_t *chunk_base;           // per child
+};
+hipError_t launch_cselect(const StepArgs &a, const CSelect &c, bool root, uint32_t expect, hipStream_t s);
+// k_ccursors and the children's metadata (m.C of them) in one launch.
+hipError_t launch_cchildren(const StepArgs &a, const CSelect &c, const CMetaArgs &m, bool root, int64_t F, hipStream_t s);
+// The arms of the 2-edge children (m.t2, cleared by the caller).
+hipError_t launch_ct2(const StepArgs &a, const CMetaArgs &m, hipStream_t s);
 struct CGatherArgs {
   const unsigned long long *vgrp;
   const uint2 *rrows;
@@ -255,6 +289,7 @@ struct CanonArgs {
   int32_t len;
   int64_t K;
   int32_t S, NEL, NVL;
+  unsigned long long *spread;  // (level check) kSpreadNv lines; null: not wanted
   // explicit codes: n codes of len (from, to, fromlabel, elabel, tolabel)
   // tuples; out[i] gets the answer (kCanonBad: a malformed tuple)
   const int32_t *codes;

@@ -156,24 +156,14 @@ bool pack_groups(PackedDB &pk, int32_t v0, int32_t n, int32_t a_end, int32_t NVL
   return true;
 }
 
-// Nominal rows of a compact chunk of about `blocks` blocks of 64 rows whose
-// segments have avg_seg rows: a block ends at a segment start and the last
-// one has to reach the first start past the nominal end, so each gives up
-// about a segment.  (With nominal lengths of whole blocks every chunk ended
-// in a block of a few rows.)
-int32_t chunk_nominal(int blocks, double avg_seg) {
-  if (avg_seg >= 32) return 64 * blocks;
-  return std::max<int32_t>(32, (int32_t)(blocks * (63.0 - avg_seg)));
-}
-
 // The root level's chunks of every job (a compact database's rows are its
 // vertices).
 void root_chunks(DeviceDB &out, std::vector<uint4> &tab) {
-  out.root_nom = chunk_nominal(2, out.n_graphs > 0 ? (double)out.n_vertices / out.n_graphs : 1.0);
+  out.root_nom = (int32_t)chunk_nominal(2, (uint32_t)out.n_vertices, (uint32_t)out.n_graphs);
   out.root_chunk0.assign(1, 0);
   for (int32_t j = 0; j < out.n_jobs; ++j) {
     const int64_t v0 = out.job_first_vertex[j], n = out.job_first_vertex[j + 1] - v0;
-    const int64_t k = ceil_div(n, out.root_nom);
+    const int64_t k = chunk_count((uint32_t)n, (uint32_t)out.root_nom);
     for (int64_t c = 0; c < k; ++c) tab.push_back(make_uint4((uint32_t)j, (uint32_t)c, (uint32_t)v0, (uint32_t)n));
     out.root_chunk0.push_back((int64_t)tab.size());
   }
@@ -622,7 +612,7 @@ struct LabelRules {
 // the tuples in `want` (the trie node's continuations) get through: the other
 // extensions are neither enumerated nor listed.
 void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv, int32_t job, uint64_t row0,
-                uint64_t nrows, bool dead, int S, const LabelRules &lr, const std::vector<std::pair<DFS, int32_t>> *want) {
+                uint64_t nrows, uint32_t nom, bool dead, int S, const LabelRules &lr, const std::vector<std::pair<DFS, int32_t>> *want) {
   const PatMetaWide m = make_meta<kMaxPatV>(code, len, vlab, nv, job);
   CMetaHead h;
   std::memset(&h, 0, sizeof(h));
@@ -631,6 +621,7 @@ void make_cmeta(char *dst, const DFS *code, int len, const uint8_t *vlab, int nv
   h.flags = dead ? (uint8_t)kPatDead : 0;
   h.row0 = row0;
   h.nrows = nrows;
+  h.nom = nom;
   // the label pairs wanted from pattern vertex f, forward or backward to it
   auto wanted = [&](int f, bool forward) -> uint64_t {
     if (!want) return ~uint64_t(0);
@@ -976,6 +967,23 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     return !nd.kids.empty();
   };
   std::vector<DFS> orig;  // a reported code in the database's own labels
+  // the path table of a level of 2-edge patterns: (0,1,a,e1,b) then
+  // (1,2,b,e2,c) (centre b) or (0,2,a,e2,c) (centre a)
+  auto build_t2 = [&](const Level &L) {
+    t2.assign((size_t)db.n_jobs * NVL * AR, 0ull);
+    for (int64_t c = 0; c < L.n; ++c) {
+      if (!L.alive.data()[c]) continue;
+      const DFS *cc = L.c(c);
+      const bool at1 = cc[1].from == 1;
+      const int centre = at1 ? cc[0].tolabel : cc[0].fromlabel;
+      const int arm1 = cc[0].elabel * NVL + (at1 ? cc[0].fromlabel : cc[0].tolabel);
+      const int arm2 = cc[1].elabel * NVL + cc[1].tolabel;
+      uint64_t *row = &t2[((size_t)L.job.data()[c] * NVL + centre) * AR];
+      row[arm1] |= 1ull << arm2;
+      row[arm2] |= 1ull << arm1;
+    }
+    t2_ready = true;
+  };
   bool counters_fresh = true;  // the counter block must be zeroed (first level, or it moved)
   bool counters_clear = false;  // the level's counters are zero (k_cursors of the level before cleared them)
 
@@ -1000,7 +1008,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     uint64_t key_next = 0;   // first key (relative to p_next) not written: a pattern split over pieces
     int64_t p_counted = 0;   // patterns whose candidates are in e_cand
     int64_t p_end_next = 0;  // > 0: the next piece ends there (its children were measured)
-    int32_t nom = 0;         // compact levels: nominal rows of a chunk
+    int blocks = 2;          // compact levels: blocks of a chunk
     int32_t meta_stride = 0; // bytes of a pattern's metadata
   };
   std::deque<Frame> frames(1);
@@ -1010,12 +1018,101 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   auto compact_words = [](uint64_t rows) { return std::max<uint64_t>(1, 7 * rows); };
   frames.back().list_cap =
       compact ? compact_words((uint64_t)db.n_vertices) : (uint64_t)std::max<int64_t>(db.n_adj, 1);  // root lists: 2E
-  frames.back().nom = db.root_nom;
   const int64_t budget = w.arena ? 0 : opt.mem_budget;
   double piece_bytes_per_row = 0;  // child bytes per parent row of the last piece (estimate)
   // device bytes a level's rows take (rows with their counts) and a list entry
   auto rows_bytes = [&](int64_t rows, int S_) { return (int64_t)rows * ((compact ? 4 : 22) + S_); };
   int64_t pool_units = 0;  // compact: list pool of the level step (grown when a level overflows it)
+  // compact: blocks of a chunk, as many as leave enough chunks (at most four)
+  auto blocks_for = [&](int64_t rows) {
+    int blocks = std::max(1, std::min(4, max_chunk_rows / 64));
+    while (blocks > 1 && rows / (62 * blocks) < kLevelWaves) blocks /= 2;
+    return blocks;
+  };
+  // Children chosen on the device (k_cselect, k_cchildren): the host launches
+  // the next level from four totals and builds the level's codes, and reports
+  // them, while the device works.  `pend` is what it still has to build the
+  // newest frame's patterns from; their parents are in PL.
+  struct Pending {
+    bool on = false;
+    const Freq *rec = nullptr;  // the level's frequent records, in key order (mapped memory)
+    int64_t F = 0, K = 0;
+    int S = 0, blocks = 1;
+    bool root = false;
+  } pend;
+  Level PL;
+  Arr<int64_t> pidx;          // per child: its record
+  bool dev_select_off = false;  // a level had codes beyond the device check
+  bool dev_t2 = false;          // the path table is on the device
+  int step = 0;
+  auto finish_pending = [&]() {
+    if (!pend.on) return;
+    pend.on = false;
+    Level &L = frames.back().L;
+    const int len = L.len;
+    const Freq *rec = pend.rec;
+    int64_t c = 0, run = 0, chunks = 0;
+    pidx.resize(L.n);
+    for (int64_t i = 0; i < pend.F && c < L.n; ++i) {
+      const uint64_t sup = rec[i].sup, proj = rec[i].proj;
+      if (!pend.root && (sup >> 32) != (uint64_t)kCanonMin + 1) continue;
+      pidx[c] = i;
+      L.row0[c] = run;
+      L.chunk0[c] = chunks;
+      run += (int64_t)proj;
+      chunks += chunk_count((uint32_t)proj, chunk_nominal((uint32_t)pend.blocks, (uint32_t)proj, (uint32_t)sup));
+      ++c;
+    }
+    if (c != L.n || run != L.row0[L.n] || chunks != L.chunk0[L.n])
+      throw Error(GM_E_DEVICE, "internal: children chosen on the device differ from their records");
+    const FastDiv fdK((uint64_t)pend.K), fdNEL((uint64_t)NEL), fdNVL((uint64_t)NVL);
+    Pool::get().run(L.n, threads, [&](int64_t ci) {
+      const Freq &f = rec[pidx[ci]];
+      const uint64_t p = fdK.div(f.key), x = f.key - p * (uint64_t)pend.K;
+      DFS *cc = L.c(ci);
+      uint8_t *cv = L.vl(ci);
+      int nv = 2;
+      if (pend.root) {
+        const uint64_t x1 = fdNVL.div(x), fl = fdNEL.div(x1);
+        cc[0] = DFS{0, 1, (int)fl, (int)(x1 - fl * NEL), (int)(x - x1 * NVL)};
+        cv[0] = (uint8_t)cc[0].fromlabel;
+        cv[1] = (uint8_t)cc[0].tolabel;
+        L.job[ci] = (int32_t)p;
+      } else {
+        const uint8_t *pv = PL.vl((int64_t)p);
+        nv = PL.nv[(int64_t)p];
+        std::memcpy(cc, PL.c((int64_t)p), sizeof(DFS) * PL.len);
+        std::memcpy(cv, pv, (size_t)nv);
+        DFS &t = cc[len - 1];
+        const uint64_t sb = (uint64_t)pend.S * NEL;
+        if (x < sb) {
+          const uint64_t to = fdNEL.div(x);
+          t = DFS{nv - 1, (int)to, pv[nv - 1], (int)(x - to * NEL), pv[to]};
+        } else {
+          const uint64_t y = x - sb, y1 = fdNVL.div(y), fv = fdNEL.div(y1);
+          t = DFS{(int)fv, nv, pv[fv], (int)(y1 - fv * NEL), (int)(y - y1 * NVL)};
+          cv[nv] = (uint8_t)t.tolabel;
+          ++nv;
+        }
+        L.job[ci] = PL.job[(int64_t)p];
+      }
+      L.nv[ci] = (uint8_t)nv;
+      L.sup[ci] = (uint32_t)f.sup;
+      L.node[ci] = 0;
+      L.alive[ci] = 1;
+    }, 2048);
+    if (len == 2 && prune && !t2_partial) build_t2(L);
+    if (!report) return;
+    orig.resize(len);
+    for (int64_t ci = 0; ci < L.n && !stopped; ++ci) {
+      const DFS *cc = L.c(ci);
+      st.n_patterns++;
+      for (int k = 0; k < len; ++k)
+        orig[k] = DFS{cc[k].from, cc[k].to, db.vl_values[cc[k].fromlabel], db.el_values[cc[k].elabel],
+                      db.vl_values[cc[k].tolabel]};
+      if (!report(L.job[ci], orig.data(), len, L.sup[ci], opt.collect_proj ? rec[pidx[ci]].proj : 0)) stopped = true;
+    }
+  };
 
   for (;;) {
     if (frames.empty()) break;
@@ -1075,6 +1172,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     }
     // the counters cover the piece's keys only: (p - p_begin) * K + key,
     // at most kPieceKeys of them (a level with more is cut into pieces)
+    if (P * K > kPieceKeys) finish_pending();  // (pieces need the patterns' first rows)
+    if (stopped) break;
     p_end = std::min<int64_t>(p_end, p_begin + std::max<int64_t>(1, kPieceKeys / K));
     const int64_t nkeys = (p_end - p_begin) * K;
     const FastDiv fdK((uint64_t)K), fdNEL((uint64_t)NEL), fdNVL((uint64_t)NVL);
@@ -1104,7 +1203,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     grow(w.tiles, sizeof(uint32_t) * kReduceTiles, s);
     grow_zero(w.acc, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
     // compact: a page of 256 list entries per 64 nominal rows, records included
-    const uint32_t page = 256u * (uint32_t)std::max(1, (Fr.nom + 63) / 64);
+    const uint32_t page = 256u * (uint32_t)Fr.blocks;
     if (compact) {
       grow(w.chunks, sizeof(CChunk) * std::max<int64_t>(total_chunks, 1), s);
     } else {
@@ -1126,8 +1225,24 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     // device when asked to, or when the host would check them before the
     // write (no speculation: the check is then on the critical path)
     const bool spec_wanted = opt.speculate == 2 || (opt.speculate == 0 && dead_share <= 0.3);
+    // children chosen on the device: whole levels, unless the caller placed
+    // the check or the write otherwise.  The device check and the choice take
+    // 20-50 us however few the keys (a code's steps are a serial chain); the
+    // host does a level of some 50 keys in less, so levels are left to it
+    // whose predecessor had fewer (the root: databases of fewer vertices than
+    // usually give more).  1,000 random graphs: 185 us by the host, 195 us by
+    // the device; 10,000 transactions 1.29 and 1.20 ms.
+    constexpr uint32_t kDevSelectKeys = 48;
+    constexpr int64_t kDevSelectVertices = 100000;
+    const bool dev_select = compact && want_codes && !past_max && budget == 0 && opt.speculate != 2 && !dev_select_off &&
+                            p_begin == 0 && p_end == P &&
+                            (root ? rows_now >= kDevSelectVertices
+                                  : codes_ready && L.len + 1 <= kCanonE && last_fcount >= kDevSelectKeys);
     const bool canon_dev = !root && want_codes && codes_ready && !past_max &&
-                           (opt.canon_mode == 2 || (opt.canon_mode == 0 && !spec_wanted));
+                           (dev_select || opt.canon_mode == 2 || (opt.canon_mode == 0 && !spec_wanted));
+    HostBuf &down = compact && (step++ & 1) ? w.down2 : w.down;
+    CSelect sel;
+    std::memset(&sel, 0, sizeof(sel));
     Counters *dctr = nullptr;
     Counters cnt;
     const char *hbuf = nullptr;
@@ -1150,7 +1265,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         a.crow = root ? db.rrows.as<uint32_t>() : w.row(cur).vt.as<uint32_t>();
         a.ctab = root ? nullptr : w.row(cur).ctab.as<uint2>();
         a.tab0 = ctab0;
-        a.nom = Fr.nom;
+        a.nom = db.root_nom;
       }
       const size_t freq_bytes = sizeof(Counters) + sizeof(Freq) * fcap;
       {
@@ -1195,11 +1310,12 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.tile_keys = reduce_tile_keys(nkeys, rep);
       // counters and (most often all of) the frequent keys come down with
       // the list pass: into the mapped buffer
-      guess = std::min<uint32_t>(fcap, std::max<uint32_t>(1024, 2 * last_fcount));
+      guess = std::min<uint32_t>(fcap, dev_select ? std::max<uint32_t>(16384, 8 * last_fcount)
+                                                  : std::max<uint32_t>(1024, 2 * last_fcount));
       const size_t head = sizeof(Counters) + sizeof(Freq) * guess;
-      hbuf = static_cast<const char *>(w.down.ensure(head));
+      hbuf = static_cast<const char *>(down.ensure(head));
       a.counters = reinterpret_cast<const unsigned long long *>(dctr);
-      a.down = w.arena ? nullptr : static_cast<unsigned long long *>(w.down.dev);
+      a.down = w.arena ? nullptr : static_cast<unsigned long long *>(down.dev);
       a.down_cap = guess;
       a.pid = root ? nullptr : w.row(cur).pid.as<int32_t>();
       a.rgraph = root ? nullptr : w.row(cur).rgraph.as<int32_t>();
@@ -1252,6 +1368,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         c.freq_cap = fcap;
         c.down = a.down ? a.down + kCounterWords : nullptr;
         c.down_cap = a.down_cap;
+        c.spread = dev_select ? a.spread : nullptr;
         c.meta = a.meta;
         c.meta_stride = a.meta_stride;
         c.p_base = (int32_t)p_begin;
@@ -1263,11 +1380,22 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         c.NEL = NEL;
         c.NVL = NVL;
         // one wave per record; the grid loops over however many there are
-        const int64_t grid = std::min<int64_t>(fcap, std::max<int64_t>(256, std::min<int64_t>(8192, 2 * (int64_t)last_fcount)));
+        const int64_t grid = std::min<int64_t>(fcap, std::max<int64_t>(1024, std::min<int64_t>(8192, 4 * (int64_t)last_fcount)));
         hip_check(launch_canon_level(c, (int)grid, s), "k_canon_level");
       }
-      if (!a.down) stage_down(w, w.down, dctr, head, s);
+      if (dev_select) {
+        a.child_blocks = blocks_for(prow_hi - prow_lo);
+        char *b = static_cast<char *>(grow(w.sel, (size_t)fcap * 20, s));
+        sel.row_base = reinterpret_cast<unsigned long long *>(b);
+        sel.fchild = reinterpret_cast<int32_t *>(b + (size_t)fcap * 8);
+        sel.crec = reinterpret_cast<uint32_t *>(b + (size_t)fcap * 12);
+        sel.chunk_base = reinterpret_cast<uint32_t *>(b + (size_t)fcap * 16);
+        hip_check(launch_cselect(a, sel, root, std::max<uint32_t>(4096, 2 * last_fcount), s), "k_cselect");
+      }
+      if (!a.down) stage_down(w, down, dctr, head, s);
+      finish_pending();  // the last level's patterns, while the device works
       hip_check(hipStreamSynchronize(s), "k_level");
+      if (stopped) break;
       std::memcpy(&cnt, hbuf, sizeof(cnt));
       if (cnt.err == kErrListPool) {
         // the lists outgrew the pool: the stage is run again with a larger
@@ -1310,6 +1438,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       hip_check(launch_fill8(w.acc.p, w.acc.cap, s), "clear counters");
       if (!compact) hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");
     }
+    if (stopped) break;
     if (!root) {
       ext_ms += ms;
       ext_launches++;
@@ -1318,14 +1447,123 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     if (failed * 64 > (unsigned long long)total_chunks && table_bits < 11 && opt.table_bits == 0) ++table_bits;
     last_fcount = cnt.fcount;
     const int64_t F = cnt.fcount;
+    // ---- children chosen on the device
+    const uint32_t undecided = (uint32_t)(cnt.pad[kTotChildren - 2] >> 32);
+    const int sel_nv = (int)(cnt.pad[kTotChunks - 2] >> 32);
+    if (dev_select && undecided) dev_select_off = true;
+    if (dev_select && !undecided && F <= (int64_t)guess && sel_nv <= kMaxPatV) {
+      const int64_t C = (int64_t)(uint32_t)cnt.pad[kTotChildren - 2], child_rows = (int64_t)cnt.pad[kTotRows - 2];
+      const int64_t chunks = (int64_t)(uint32_t)cnt.pad[kTotChunks - 2], dropped = (int64_t)cnt.pad[kTotDropped - 2];
+      const int new_len = root ? 1 : L.len + 1;
+      const int CS = tuple_stride(std::max(2, sel_nv)), child_stride = cmeta_bytes(std::max(2, sel_nv));
+      if (!root) st.e_cand += ecand;
+      st.pruned += pruned;
+      st.max_table_fill = std::max<uint64_t>(st.max_table_fill, max_fill);
+      st.n_candidates += root ? 0 : F;
+      (root ? st.e_root : st.e_child) += (uint64_t)child_rows;
+      if (!report) st.n_patterns += (uint64_t)C;
+      st.n_levels++;
+      dead_share = (double)dropped / (double)std::max<int64_t>(1, child_rows + dropped);
+      if (chunks > INT32_MAX) throw Error(GM_E_OOM, "more than 2^31 chunks of rows");
+      int nxt = 0;
+      while (nxt == cur) ++nxt;
+      const size_t codes_off = ((size_t)child_stride * C + 7) & ~size_t(7);
+      const size_t cvl_off = (codes_off + sizeof(uint32_t) * new_len * C + 7) & ~size_t(7);
+      CMetaArgs m;
+      std::memset(&m, 0, sizeof(m));
+      if (C > 0) {
+        char *du = static_cast<char *>(grow(w.row(nxt).upl, cvl_off + (size_t)CS * C, s));
+        grow(w.row(nxt).vt, (size_t)(4 + CS) * child_rows, s);
+        grow(w.row(nxt).ctab, sizeof(uint2) * chunks, s);
+        grow(w.cursor, sizeof(unsigned long long) * C * rep, s);
+        a.crow_out = w.row(nxt).vt.as<uint32_t>();
+        a.child_tab = w.row(nxt).ctab.as<uint2>();
+        a.cursor = w.cursor.as<unsigned long long>();
+        a.ccap = child_rows;
+        a.CS = CS;
+        m.pcode = root ? nullptr : reinterpret_cast<const uint32_t *>(w.row(cur).upl.as<char>() + code_off);
+        m.pvlab = root ? nullptr : reinterpret_cast<const uint8_t *>(w.row(cur).upl.as<char>() + vlab_off);
+        m.len = new_len - 1;
+        m.crec = sel.crec;
+        m.C = C;
+        m.meta = du;
+        m.meta_stride = child_stride;
+        m.code = reinterpret_cast<uint32_t *>(du + codes_off);
+        m.vlab = reinterpret_cast<uint8_t *>(du + cvl_off);
+        if (prune && !t2_partial && (new_len == 2 || (new_len > 2 && (dev_t2 || t2_ready)))) {
+          const size_t bytes = sizeof(uint64_t) * (size_t)db.n_jobs * NVL * AR;
+          m.t2 = static_cast<unsigned long long *>(grow(w.t2, bytes, s));
+          m.masks = 1;
+          if (new_len == 2) {
+            hip_check(launch_fill8(m.t2, bytes, s), "path table");
+            hip_check(launch_ct2(a, m, s), "k_ct2");
+          } else if (!dev_t2) {  // an earlier level's, built by the host
+            hip_check(hipMemcpyAsync(m.t2, t2.data(), bytes, hipMemcpyHostToDevice, s), "path table");
+            hip_check(hipStreamSynchronize(s), "path table");
+          }
+          dev_t2 = true;
+        }
+      }
+      hip_check(launch_cchildren(a, sel, m, root, F, s), "k_cchildren");
+      if (F > 0) counters_clear = true;
+      if (C > 0) {
+        hip_check(launch_cwrite(a, root, s), "k_cwrite");
+        written_expect += (unsigned long long)child_rows;
+        written_pending = true;
+      }
+      dev_sec += tdev.sec();
+      size_t live = db.bytes + w.sup.cap + w.tiles.cap + w.acc.cap + w.freq.cap + w.cand.cap + w.chunks.cap +
+                    w.cursor.cap + w.sel.cap + w.t2.cap;
+      for (const RowSet &rs : w.rows) live += rs.bytes();
+      peak = std::max(peak, live);
+      if (trace_levels)
+        fprintf(stderr,
+                "[gm level %d] device-chosen: patterns %lld rows %lld K %lld chunks %lld stage_us %.1f candidates %llu "
+                "pruned %llu frequent %u children %lld child_rows %lld max_fill %llu\n",
+                level, (long long)P, (long long)rows_now, (long long)K, (long long)total_chunks, ms * 1e3, ecand, pruned,
+                cnt.fcount, (long long)C, (long long)child_rows, max_fill);
+      pend.rec = reinterpret_cast<const Freq *>(hbuf + sizeof(Counters));
+      pend.F = F;
+      pend.K = K;
+      pend.S = S;
+      pend.blocks = a.child_blocks;
+      pend.root = root;
+      pend.on = C > 0;
+      std::swap(PL, L);  // (L is left with a spare level's arrays)
+      Level spare;
+      std::swap(spare, L);
+      frames.pop_back();
+      if (C > 0) {
+        frames.emplace_back();
+        Frame &cf = frames.back();
+        std::swap(cf.L, N);
+        cf.L.resize(C, new_len);
+        cf.L.max_nv = sel_nv;
+        cf.L.row0[0] = cf.L.chunk0[0] = 0;
+        cf.L.row0[C] = child_rows;
+        cf.L.chunk0[C] = chunks;
+        cf.level = level + 1;
+        cf.buf = nxt;
+        cf.S = CS;
+        cf.n_rows = child_rows;
+        cf.list_cap = compact_words((uint64_t)child_rows);
+        cf.blocks = pend.blocks;
+        cf.meta_stride = child_stride;
+        cf.code_off = codes_off;
+        cf.vlab_off = cvl_off;
+        cf.codes_ready = true;
+      }
+      std::swap(N, spare);
+      continue;
+    }
     if (F) {
       const Freq *src = reinterpret_cast<const Freq *>(hbuf + sizeof(Counters));
       if (F > (int64_t)guess) {  // the rest of the list, after the part downloaded
         frall.resize(F);
         std::memcpy(frall.data(), src, sizeof(Freq) * guess);
         const size_t rest = sizeof(Freq) * (F - guess);
-        char *h2 = static_cast<char *>(w.down.ensure(rest));
-        stage_down(w, w.down, reinterpret_cast<const char *>(a.freq) + sizeof(Freq) * guess, rest, s);
+        char *h2 = static_cast<char *>(down.ensure(rest));
+        stage_down(w, down, reinterpret_cast<const char *>(a.freq) + sizeof(Freq) * guess, rest, s);
         hip_check(hipStreamSynchronize(s), "download frequent keys");
         std::memcpy(frall.data() + guess, h2, rest);
         src = frall.data();
@@ -1535,27 +1773,19 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     st.n_candidates += root ? 0 : F;
 
     // children in key order; child c's rows are [row0[c], row0[c + 1])
-    int64_t C = 0, child_rows = 0, child_segs = 0;
+    int64_t C = 0, child_rows = 0;
     int max_nv = 0;
     for (int64_t i = 0; i < F; ++i) {
       if (kidx[i] < 0) continue;
       kidx[i] = C++;
       child_rows += (int64_t)fr[i].proj;
-      child_segs += (int64_t)(fr[i].sup & 0xFFFFFFFFull);  // (bits 32-39 hold the device check's answer)
       if (!late_decode) max_nv = std::max(max_nv, (int)knv[i]);
     }
     if (late_decode) max_nv = max_nv_exact;
     const int CS = C > 0 ? tuple_stride(max_nv) : 4;  // the children's tuple stride
     const bool wide = CS > kNarrowPatV;                 // and metadata layout
     const int child_stride = compact ? cmeta_bytes(std::max(max_nv, 1)) : meta_bytes(CS);
-    // compact: blocks of a chunk, as many as leave enough chunks (at most four)
-    int child_nom = 0;
-    if (compact) {
-      const double seg = (double)child_rows / (double)std::max<int64_t>(1, child_segs);
-      int blocks = std::max(1, std::min(4, max_chunk_rows / 64));
-      while (blocks > 1 && child_rows / chunk_nominal(blocks, seg) < kLevelWaves) blocks /= 2;
-      child_nom = chunk_nominal(blocks, seg);
-    }
+    const int child_blocks = blocks_for(child_rows);
     N.resize(C, new_len);
     nproj.resize(C);
     double us_host = 0, us_overlap = 0;
@@ -1605,7 +1835,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         if (compact) {
           hcb[c] = (uint32_t)chunks;
           N.chunk0[c] = chunks;
-          chunks += ceil_div((int64_t)fr[i].proj, child_nom);
+          chunks += chunk_count((uint32_t)fr[i].proj,
+                                chunk_nominal((uint32_t)child_blocks, (uint32_t)fr[i].proj, (uint32_t)fr[i].sup));
         } else {
           hlb[c] = (unsigned long long)child_items;
           child_items += fr[i].items;
@@ -1654,7 +1885,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         grow(w.row(nxt).ctab, sizeof(uint2) * std::max<int64_t>(N.chunk0[C], 1), s);
         a.crow_out = w.row(nxt).vt.as<uint32_t>();
         a.child_tab = w.row(nxt).ctab.as<uint2>();
-        a.child_nom = child_nom;
+        a.child_blocks = child_blocks;
       } else {
         grow(w.row(nxt).pid, sizeof(int32_t) * std::max<int64_t>(child_rows, 1), s);
         grow(w.row(nxt).rgraph, sizeof(int32_t) * std::max<int64_t>(child_rows, 1), s);
@@ -1725,7 +1956,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         nproj[c] = fr[i].proj;
         if (compact) {
           make_cmeta(hu + (size_t)c * child_stride, cc, new_len, cv, cnv, N.job[c], (uint64_t)N.row0[c], fr[i].proj,
-                     !kalive[i], CS, rules, opt.queries ? &opt.queries->nodes[knode[i]].kids : nullptr);
+                     chunk_nominal((uint32_t)child_blocks, (uint32_t)fr[i].proj, (uint32_t)fr[i].sup), !kalive[i], CS, rules, opt.queries ? &opt.queries->nodes[knode[i]].kids : nullptr);
         } else if (wide) {
           hmw[c] = make_meta<kMaxPatV>(cc, new_len, cv, cnv, N.job[c]);
           if (!kalive[i]) hmw[c].flags |= kPatDead;
@@ -1808,21 +2039,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
           });
         Pool::get().run(F, threads, build_child, 4096);
         if (new_len == 2) {
-          // the job's frequent 2-edge patterns: (0,1,a,e1,b) then
-          // (1,2,b,e2,c) (centre b) or (0,2,a,e2,c) (centre a)
-          t2.assign((size_t)db.n_jobs * NVL * AR, 0ull);
-          for (int64_t c = 0; c < C; ++c) {
-            if (!N.alive[c]) continue;
-            const DFS *cc = N.c(c);
-            const bool at1 = cc[1].from == 1;
-            const int centre = at1 ? cc[0].tolabel : cc[0].fromlabel;
-            const int arm1 = cc[0].elabel * NVL + (at1 ? cc[0].fromlabel : cc[0].tolabel);
-            const int arm2 = cc[1].elabel * NVL + cc[1].tolabel;
-            uint64_t *row = &t2[((size_t)N.job[c] * NVL + centre) * AR];
-            row[arm1] |= 1ull << arm2;
-            row[arm2] |= 1ull << arm1;
-          }
-          t2_ready = true;
+          build_t2(N);
         }
         if (t2_ready) Pool::get().run(C, threads, mask_child, 4096);
       }
@@ -1931,7 +2148,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       cf.S = CS;
       cf.n_rows = child_rows;
       cf.list_cap = std::max<uint64_t>(child_items, 1);  // the children's lists: exactly their item counts
-      cf.nom = child_nom;
+      cf.blocks = child_blocks;
       cf.meta_stride = child_stride;
       cf.mask_off = child_mask_off;
       cf.mask_stride = child_mask_stride;
@@ -1952,7 +2169,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
                                    ") differ from the embedding counts (" + std::to_string(written_expect) + ")");
   }
   hip_check(hipStreamSynchronize(s), "mining");
-  w.acc_zero = true;
+  w.acc_zero = !stopped;  // (a sink may stop the run while the next level's counts are taken)
   st.seconds_total = total.sec();
   st.seconds_device = dev_sec;
   st.seconds_canon = canon_sec;

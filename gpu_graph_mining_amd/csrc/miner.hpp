@@ -98,6 +98,11 @@ struct Workspace {
     return rows[(size_t)i];
   }
   HostBuf up, down;
+  // compact levels: a second download buffer (the host reads one level's
+  // records while the next level's are written), the children chosen on the
+  // device and the 2-edge path table
+  HostBuf down2;
+  DevBuf sel, t2;
   hipEvent_t ev[2] = {nullptr, nullptr};  // stage timing (MineOptions::stage_events)
   // the children's upload runs on a copy engine beside the write pass:
   // its stream (default priority) and the event the next level waits on

@@ -103,3 +103,36 @@ def test_subsets_of_a_compact_database():
         arrays = gm.GraphDB.from_graphs([graphs[i] for i in ids]).arrays() if ids else None
         opats = po.mine_arrays(arrays, minsup)[0] if ids else []
         assert {po.normalize(c): (s, n) for c, s, n in pats} == {po.normalize(c): (s, n) for c, s, n in opats}
+
+
+@pytest.mark.parametrize("sink", [False, True])
+def test_children_chosen_on_the_device(sink):
+    """Levels of hundreds of keys, chosen on the device, with symmetric codes
+    (stars of five and six equal leaves) that its check leaves to the host
+    half way; with a sink, the patterns of every level are reported in key
+    order, and a sink that stops the run is heard."""
+    rng = random.Random(11)
+    graphs = []
+    for _ in range(30):
+        labels, edges = tree(rng, 24, 3, 2, 3)
+        n = len(labels)
+        graphs.append((labels + [0] * 8, edges + [(n, n + i, 0) for i in range(1, 8)]))
+    db = gm.GraphDB.from_graphs(graphs)
+    opats, ost = po.mine_arrays(db.arrays(), 4, max_edges=6)
+    want = {po.normalize(c): (s, n) for c, s, n in opats}
+    print(len(want), "patterns", flush=True)
+    if not sink:
+        pats, st = gm.mine(db, 4, max_edges=6, collect_proj=True)
+        assert {po.normalize(c): (s, n) for c, s, n in pats} == want and len(pats) == len(want)
+        assert (st["e_child"], st["e_cand"]) == (ost["e_child"], ost["e_cand"])
+        assert st["canon_host_keys"] > 0
+        return
+    seen = []
+    gm.mine(db, 4, max_edges=6, on_pattern=lambda c, s, n: seen.append((c, s)))
+    assert {po.normalize(c): s for c, s in seen} == {c: s for c, (s, _) in want.items()}
+    assert [len(c) for c, _ in seen] == sorted(len(c) for c, _ in seen)
+    for stop_at in (1, len(seen) // 2, len(seen)):
+        got = []
+        with pytest.raises(gm.GMError) as e:
+            gm.mine(db, 4, max_edges=6, on_pattern=lambda c, s, n: (got.append((c, s)), len(got) < stop_at)[1])
+        assert e.value.code == gm.GM_E_CALLBACK and got == seen[:stop_at]
