@@ -6,37 +6,43 @@
 // sizes.  The kernels of kernels.hip mine the others, and all databases under
 // the entry point that allocates nothing.
 //
-// Layout.  A vertex is one 8-byte *group* at vgrp[g + u] (g the graph's first
-// group, u the local id): four items (neighbour 6 bits, label pair
-// edge label * NVL + neighbour label 6 bits) of 12 bits, two per word, and in
-// the top byte of the first word the place (relative to g) of a further group
-// when the vertex has more than four neighbours.  One gather per rightmost-path
-// source fetches all of the common vertices' neighbours; nothing depends on an
-// offset read first.  (With a 4-byte offset and 4-byte entries a row's sources
-// touched 4-5 lines of 128 bytes per segment, in two dependent steps.)
+// Layout.  A vertex is one 8-byte *group* (g the graph's first group, u the
+// vertex's local id: group g + u): four 12-bit items (neighbour 6 bits, label
+// pair edge label * NVL + neighbour label 6 bits) and, in bits 48-55, the place
+// (relative to g) of a further group when the vertex has more than four
+// neighbours.  One gather per rightmost-path source fetches all of the common
+// vertices' neighbours; nothing depends on an offset read first.  (With a
+// 4-byte offset and 4-byte entries a row's sources touched 4-5 lines of 128
+// bytes per segment, in two dependent steps.)
 //
-// Rows are {g, tuple} of 1 + TW words (tuple bytes past the pattern's vertices
-// repeat vertex 0's, so that the visited set is an OR over all bytes),
-// pattern-major; a chunk is a run of
-// whole segments (rows of one graph) of ONE pattern, so everything about the
-// pattern is wave-uniform: the sources are walked in a scalar loop, and the
-// label rules of a source (order rule, minimum label, 2-edge path masks) are a
-// 64-bit mask over label pairs that the host prepares.  An item is tested with
-// two shifts: its label pair against the mask, its neighbour against the
-// row's visited set.
+// Rows are {8 g, tuple} of 1 + TW words (tuple bytes past the pattern's
+// vertices repeat vertex 0's, so that the visited set is an OR over all bytes),
+// pattern-major; a chunk is a run of whole segments (rows of one graph) of ONE
+// pattern, so everything about the pattern is wave-uniform: the sources are
+// walked in a scalar loop, and the label rules of a source (order rule,
+// minimum label, 2-edge path masks) are a 64-bit mask over label pairs.  An
+// item is tested with two shifts: its label pair against the mask, its
+// neighbour against the row's visited set.
 //
 // Per block of up to 64 rows and per source, the passing items are counted,
 // ranked over the wave and appended to the chunk's dense list
-//   key << 20 | neighbour << 14 | row of the chunk
-// (4 bytes a candidate; entry key 0xFFF moves the row base on by kMarkRows).
-// Counts live in LDS tables indexed by the key itself (K <= 4032; no hashing,
-// no overflow).  A key names its source, and within a source the list is in
-// row order, so every key's entries are in row order: k_cwrite can place the
-// children's rows graph-contiguously in list order.
+//   source << 25 | item << 13 | row of the chunk
+// (4 bytes a candidate; backward targets are sources 64 on, with the edge
+// label in the label pair's place; source 127 moves the row base on by
+// kMarkRows).  Counts live in LDS records indexed by the key itself (K <=
+// 4032; no hashing, no overflow).  A key names its source, and within a source
+// the list is in row order, so every key's entries are in row order: k_cwrite
+// can place the children's rows graph-contiguously in list order.
 //
-// What bounds them: vector instruction issue and the group gathers' latency;
-// k_level of kernels.hip spends about 2,500 vector instructions on a 64-row
-// block of 8-byte tuples with half of its lanes idle.
+// What bounds k_clevel: the gathers.  A load of one group a lane touches 13
+// lines, nearly all of them misses in a 32 KB L1 that 28 waves share, so a
+// block of 64 rows asks L2 for some 170 lines; with an average of 51 of them in
+// flight a CU's L1 waits on pending lines for 70% of the kernel's time (100,000
+// transactions: 2.5e8 lines and 3.25 ms for the levels of 8-byte tuples, 2.3 ms
+// with the loads alone).  Vector issue comes next (1,000 instructions a block,
+// 68% of the time at 3.3 cycles each) and is hidden behind it: 6% fewer
+// instructions gave 1%.  Items at bit offsets that one shift reaches and 16-byte
+// counter records took that case from 5.15 ms to 4.75 over all levels.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,8 +57,9 @@ namespace gm {
 namespace {
 
 constexpr uint32_t kNone32 = 0xFFFFFFFFu;
-constexpr uint32_t kMarkKey = 0xFFFu;
-constexpr int kMarkRows = 8192;
+constexpr uint32_t kMarkSource = 127u;
+constexpr uint32_t kBackSource = 64u;  // source number of backward target 0
+constexpr int kMarkRows = 4096;        // (rows of a block stay below kMarkRows + 64 < 2^13)
 
 // (lambdas used several times must not become calls: a call needs scratch)
 #define GM_INLINE __attribute__((always_inline))
@@ -91,48 +98,101 @@ __device__ __forceinline__ uint32_t below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+// Pointers read from the argument segment are generic; these make the
+// accesses global ones (a flat access also waits on the LDS counter).
+#define GM_GLOBAL __attribute__((address_space(1)))
+template <class T>
+__device__ __forceinline__ GM_GLOBAL T *as_global(T *p) {
+  return (GM_GLOBAL T *)(uintptr_t)p;
+}
+
 template <int TW>
 struct CRow {
   uint32_t x[1 + TW];
 };
 
-// The graph vertex at pattern vertex i (wave-uniform).  Masks, not selects:
-// the compiler turns a chain of selects into an indexed array in scratch.
+// The graph vertex at pattern vertex i (wave-uniform), in byte 0 (image) or in
+// all four (image4): one byte permute of the two words that can hold it; past
+// eight vertices the words are picked by masks (selects would become an
+// indexed array in scratch).
+template <int TW>
+__device__ __forceinline__ uint32_t image_of(const CRow<TW> &t, int i, uint32_t sel) {
+  uint32_t lo = t.x[1], hi = TW > 1 ? t.x[TW > 1 ? 2 : 1] : 0u;
+  if constexpr (TW > 2) {
+    lo = hi = 0;
+#pragma unroll
+    for (int q = 0; q < TW; q += 2) {
+      const uint32_t m = 0u - (uint32_t)((i >> 3) == q / 2);
+      lo |= t.x[1 + q] & m;
+      if (q + 1 < TW) hi |= t.x[q + 1 < TW ? 2 + q : 1] & m;
+    }
+  }
+  return __builtin_amdgcn_perm(hi, lo, sel);
+}
 template <int TW>
 __device__ __forceinline__ uint32_t image(const CRow<TW> &t, int i) {
-  uint32_t x = 0;
-#pragma unroll
-  for (int q = 0; q < TW; ++q) x |= t.x[1 + q] & (0u - (uint32_t)((i >> 2) == q));
-  return (x >> ((i & 3) * 8)) & 0xFFu;
+  return image_of<TW>(t, i, 0x0C0C0C00u | (uint32_t)(i & 7));
+}
+template <int TW>
+__device__ __forceinline__ uint32_t image4(const CRow<TW> &t, int i) {
+  return image_of<TW>(t, i, 0x01010101u * (uint32_t)(i & 7));
 }
 
-// Groups are held as 64-bit values: items at bits 0, 12, 32 and 44, the next
-// group's place at bits 24-31.
+// A group: items at bits 0, 12, 24 and 36 (unused ones all ones), the next
+// group's place at bits 48-55.
 typedef unsigned long long Group;
-constexpr Group kEmptyGroup = (Group)(kEmptyItem | kEmptyItem << 12) << 32 | (kEmptyItem | kEmptyItem << 12);
-__device__ __forceinline__ uint32_t next_of(Group g) { return (uint32_t)g >> 24; }
-// item i (0..7) of a vertex's first two groups
-__device__ __forceinline__ uint32_t item(Group p, Group o, int i) {
-  const Group g = (i & 4) ? o : p;
-  return (uint32_t)(g >> ((i & 1) * 12 + (i & 2) * 16)) & 0xFFFu;
+__device__ __forceinline__ uint32_t next_of(Group g) { return (uint32_t)(g >> 32) >> 16; }
+__device__ __forceinline__ uint32_t item(Group g, int i) { return (uint32_t)(g >> (12 * i)) & 0xFFFu; }
+// the items' neighbours, a byte each
+__device__ __forceinline__ uint32_t neighbours(Group g) {
+  return item(g, 0) % 64 | (item(g, 1) % 64) << 8 | (item(g, 2) % 64) << 16 | (item(g, 3) % 64) << 24;
 }
+// 0x80 in the lowest byte of x that is zero, if any (and perhaps above it)
+__device__ __forceinline__ uint32_t zero_bytes(uint32_t x) { return (x - 0x01010101u) & ~x & 0x80808080u; }
+
+// Inclusive sum over the wave in data-parallel primitives (six adds; the
+// shuffle scan goes through LDS).
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp_from(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRows, 0xF, kRows == 0xF);
+}
+__device__ __forceinline__ uint32_t wave_incl(uint32_t x) {
+  x += dpp_from<0x111, 0xF>(x);  // row_shr:1
+  x += dpp_from<0x112, 0xF>(x);  // row_shr:2
+  x += dpp_from<0x114, 0xF>(x);  // row_shr:4
+  x += dpp_from<0x118, 0xF>(x);  // row_shr:8
+  x += dpp_from<0x142, 0xA>(x);  // row_bcast:15 to rows 1 and 3
+  x += dpp_from<0x143, 0xC>(x);  // row_bcast:31 to rows 2 and 3
+  // (kept whole: taken apart by a caller's difference, the partial sums keep
+  // the adds from becoming single add-with-shift instructions)
+  asm("" : "+v"(x));
+  return x;
+}
+
+// A key's counts in the chunk: the block's segments that hold it (by head
+// lane), its support (bit 31: the mask's bit 0 is a carried segment, counted
+// already) and its embeddings.
+struct alignas(16) KeyCount {
+  unsigned long long mask;
+  uint32_t sup, emb;
+};
 
 // The chunk's candidate list: extents of entries, the first at
 // chunk * page, further ones from the pool (64 slices with a cursor each on a
 // line of its own).  An extent starts with {entries, next extent or kNone32};
 // extents are named in units of kListUnit entries.
 struct ListOut {
-  uint32_t *ext;
+  GM_GLOBAL uint32_t *ext;
   uint32_t used, cap;
   bool off;  // the pool ran out: the stage runs again with a larger one
 };
 
 template <bool ROOT, int TW, bool M32>
-__global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_clevel(StepArgs) {
+__global__ void __launch_bounds__(64, (M32 ? (TW <= 8 ? 7 : 6) : TW <= 3 ? 6 : 5)) k_clevel(StepArgs) {
   extern __shared__ __attribute__((aligned(16))) uint32_t dyn[];
   const int K = (int)GM_ARG(K);
-  unsigned long long *const kmask = reinterpret_cast<unsigned long long *>(dyn);  // segments of the block, by head lane
-  uint32_t *const ksup = dyn + 2 * K, *const kemb = dyn + 3 * K;
+  KeyCount *const kc = reinterpret_cast<KeyCount *>(dyn);
+  __shared__ uint32_t stage[64];  // a source's items on their way to the list
   const int lane = threadIdx.x;
   const uint32_t gci = blockIdx.x;
   if (gci < (uint32_t)kSpread) stamp_start(GM_ARG(spread), gci);
@@ -165,7 +225,7 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
     nom0 = (uint32_t)uniform((int)ct.y) * nom;
   }
   const uint32_t nom1 = pend - nom0 <= nom ? pend : nom0 + nom;
-  const uint32_t *const rows = GM_ARG(crow) + first * RW;
+  GM_GLOBAL const uint32_t *const rows = as_global(GM_ARG(crow) + first * RW);
   uint32_t b = nom0;
   bool empty = !ROOT && (H.flags & kPatDead);
   if (!empty && nom0 > 0) {
@@ -189,15 +249,11 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
     return;
   }
   const uint32_t start = b;
-  for (int i = lane; i < K; i += 64) {
-    kmask[i] = 0;
-    ksup[i] = 0;
-    kemb[i] = 0;
-  }
+  for (int i = lane; i < K; i += 64) kc[i] = KeyCount{0, 0, 0};
   wave_sync();
 
   const uint32_t page = GM_ARG(page);
-  ListOut L{GM_ARG(clist) + (uint64_t)gci * page, 2u, page, false};
+  ListOut L{as_global(GM_ARG(clist)) + (uint64_t)gci * page, 2u, page, false};
   // room for n entries in one extent: their place in it
   auto reserve = [&](uint32_t n) GM_INLINE -> uint32_t {
     if (L.used + n > L.cap) {
@@ -217,7 +273,7 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
       }
       at = (uint32_t)uniform((int)at);
       L.off = L.off || at == kNone32;
-      if (!L.off) L.ext = GM_ARG(clist) + (uint64_t)at * kListUnit;
+      if (!L.off) L.ext = as_global(GM_ARG(clist)) + (uint64_t)at * kListUnit;
       L.used = 2u;
       L.cap = L.off ? kNone32 - 1u : units * kListUnit;
     }
@@ -235,16 +291,17 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
     const int ws = (int)min(64u, pend - b);
     CRow<TW> t;
     {
-      const uint32_t *src = rows + ((uint64_t)b + (uint32_t)min(lane, ws - 1)) * RW;
-      __builtin_memcpy(&t, src, sizeof(t));
+      GM_GLOBAL const uint32_t *src = rows + ((uint64_t)b + (uint32_t)min(lane, ws - 1)) * RW;
+#pragma unroll
+      for (int q = 0; q < RW; ++q) t.x[q] = src[q];
     }
     const uint32_t g = t.x[0];
     const uint32_t pg = __shfl_up(g, 1, 64);
     const uint64_t diff = __ballot(lane < ws && (lane == 0 ? !carry || g != carry_g : pg != g));
     if (carry && (diff & 1ull)) {  // it ended with the last block: its keys' marks are done with
       for (int i = lane; i < K; i += 64) {
-        ksup[i] &= 0x7FFFFFFFu;
-        kmask[i] = 0;
+        kc[i].sup &= 0x7FFFFFFFu;
+        kc[i].mask = 0;
       }
       wave_sync();
     }
@@ -274,15 +331,17 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
     }
     const bool live = lane < nb;
     const uint64_t starts = nb == 64 ? diff : diff & ((1ull << nb) - 1ull);
-    const unsigned long long hbit = 1ull << head_lane(starts, lane);
-    while (b - start - rowbase >= (uint32_t)kMarkRows) {  // (rows of a block stay below kMarkRows + 64 < 2^14)
+    const uint32_t head = (uint32_t)head_lane(starts, lane);
+    const uint32_t who = (uint32_t)lane << 12 | head << 18;
+    while (b - start - rowbase >= (uint32_t)kMarkRows) {
       const uint32_t pos = reserve(1);
-      if (lane == 0 && !L.off) L.ext[pos] = kMarkKey << 20;
+      if (lane == 0 && !L.off) L.ext[pos] = kMarkSource << 25;
       rowbase += kMarkRows;
     }
-    const uint32_t rowrel = b - start - rowbase + (uint32_t)lane;
+    const uint32_t row0 = b - start - rowbase, rowrel = row0 + (uint32_t)lane;
 
-    // the row's visited vertices
+    // the row's visited vertices (all of them for lanes past the block, whose
+    // items then never pass)
     unsigned long long used = 0;
     if constexpr (ROOT) {
       used = 1ull << (t.x[1] & 63u);
@@ -291,13 +350,14 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
       for (int i = 0; i < 4 * TW; ++i)
         used |= 1ull << ((t.x[1 + i / 4] >> ((i & 3) * 8)) & 63u);
     }
+    if (!live) used = ~0ull;
 
-    const Group *const vgrp = GM_ARG(vgrp);
-    auto load_group = [&](uint32_t off) GM_INLINE -> Group { return vgrp[(uint64_t)g + off]; };
+    GM_GLOBAL const char *const vgrp = (GM_GLOBAL const char *)as_global(GM_ARG(vgrp));
+    auto load_group = [&](uint32_t u) GM_INLINE -> Group { return *(GM_GLOBAL const Group *)(vgrp + (g + u * 8u)); };
     const int nsrc = ROOT ? 1 : H.nsrc;
     const char *srcs = meta + sizeof(CMetaHead);
+    // (lanes past the block load too: their rows are the window's)
     auto load_src = [&](int j) GM_INLINE -> Group {
-      if (!live) return kEmptyGroup;
       if constexpr (ROOT) return load_group(t.x[1] & 63u);
       return load_group(image<TW>(t, cload<int>(srcs + j * (int)sizeof(CSource) + 16)));
     };
@@ -311,14 +371,17 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
       uint32_t nx = next_of(o);
       while (nx) {
         const Group c = load_group(nx);
-        for (int i = 0; i < 4; ++i) fn(item(c, c, i));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fn(item(c, i));
         nx = next_of(c);
       }
     };
-    auto emit = [&](uint32_t pos, uint32_t key, uint32_t w) GM_INLINE {
-      if (!L.off) L.ext[pos] = key << 20 | w << 14 | rowrel;
-      atomicOr(&kmask[key], hbit);
-      atomicAdd(&kemb[key], 1u);
+    // count key for the segment of head lane h, list the entry at byte `at`
+    // of the extent
+    auto emit = [&](uint32_t at, uint32_t key, uint32_t entry, uint32_t h) GM_INLINE {
+      if (!L.off) *(GM_GLOBAL uint32_t *)((GM_GLOBAL char *)L.ext + at) = entry;
+      atomicOr(&kc[key].mask, 1ull << h);
+      atomicAdd(&kc[key].emb, 1u);
     };
 
     Group P = load_src(0), Pn = nsrc > 1 ? load_src(1) : kEmptyGroup;
@@ -328,39 +391,33 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
       // items are tested
       const Group Pnn = j + 2 < nsrc ? load_src(j + 2) : kEmptyGroup;
       const Group On = j + 1 < nsrc ? load_next(Pn) : kEmptyGroup;
-      const bool deep = __ballot(next_of(O) != 0) != 0;  // some vertex has more than eight neighbours
+      const bool more = __ballot(next_of(P) != 0) != 0;          // some vertex has more than four neighbours
+      const bool deep = more && __ballot(next_of(O) != 0) != 0;  // more than eight
 
       // backward: from the rightmost vertex (source 0) to the images of the
-      // path vertices the host lists
+      // path vertices that the pattern lists, a byte compare each against all
+      // neighbours
       if constexpr (!ROOT) {
         if (j == 0 && H.nback) {
           const char *backs = srcs + nsrc * (int)sizeof(CSource);
-          unsigned long long bset = 0;
-          for (int q = 0; q < H.nback; ++q)
-            bset |= 1ull << image<TW>(t, cload<int>(backs + q * (int)sizeof(CSource) + 16));
-          uint32_t hit = 0;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint32_t x = item(P, O, i);
-            hit |= (uint32_t)(bset >> (x & 63u)) & (x >> 6 != 63u ? 1u : 0u);
-          }
-          if (deep || __ballot(hit != 0)) {
-            for (int q = 0; q < H.nback; ++q) {
-              const CSource bk = cload<CSource>(backs + q * (int)sizeof(CSource));
-              const uint32_t v = image<TW>(t, bk.from);
-              uint32_t lab = 63;
-              auto match = [&](uint32_t x) GM_INLINE { lab = (x & 63u) == v ? min(lab, x >> 6) : lab; };
-#pragma unroll
-              for (int i = 0; i < 8; ++i) match(item(P, O, i));
-              walk_on(O, match);
-              const bool ok = live && ((bk.rule >> lab) & 1ull), kept = ok && ((bk.keep >> lab) & 1ull);
-              n_pruned += ok && !kept ? 1u : 0u;
-              const uint64_t m = __ballot(kept);
-              if (m) {
-                const uint32_t pos = reserve((uint32_t)__popcll(m)) + below(m);
-                listed += (unsigned long long)__popcll(m);
-                if (kept) emit(pos, (uint32_t)bk.kbase + ((lab * GM_ARG(inv_nvl)) >> 16), 0u);
-              }
+          const uint32_t np = neighbours(P), no = neighbours(O);
+          for (int q = 0; q < H.nback; ++q) {
+            const int f = cload<int>(backs + q * (int)sizeof(CSource) + 16);
+            const uint32_t v4 = image4<TW>(t, f);
+            const uint32_t zp = zero_bytes(np ^ v4), zo = more ? zero_bytes(no ^ v4) : 0u;
+            if (!deep && !__ballot((zp | zo) != 0)) continue;
+            const CSource bk = cload<CSource>(backs + q * (int)sizeof(CSource));
+            uint32_t lab = 63;
+            if (zp | zo) lab = item(zp ? P : O, __builtin_ctz(zp ? zp : zo) >> 3) >> 6;
+            if (deep) walk_on(O, [&](uint32_t x) GM_INLINE { lab = (x & 63u) == (v4 & 63u) ? min(lab, x >> 6) : lab; });
+            const bool ok = live && ((bk.rule >> lab) & 1ull), kept = ok && ((bk.keep >> lab) & 1ull);
+            n_pruned += ok && !kept ? 1u : 0u;
+            const uint64_t m = __ballot(kept);
+            if (m) {
+              const uint32_t pos = reserve((uint32_t)__popcll(m)) + below(m);
+              listed += (unsigned long long)__popcll(m);
+              const uint32_t el = (lab * GM_ARG(inv_nvl)) >> 16;
+              if (kept) emit(pos * 4u, (uint32_t)bk.kbase + el, (kBackSource + (uint32_t)q) << 25 | el << 19 | rowrel, head);
             }
           }
         }
@@ -370,68 +427,93 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
       // lets through
       typedef typename std::conditional<M32, uint32_t, unsigned long long>::type Mask;
       Mask rule, keep;
-      uint32_t kbase;
-      bool masked = false;
+      uint32_t kbase, source = (uint32_t)j << 25;
       if constexpr (ROOT) {
-        // from a vertex to neighbours of its label or a larger one
+        // from a vertex to neighbours of its label or a larger one; the
+        // source's number is the label
         const uint32_t lu = (t.x[1] >> 8) & 0xFFu;
         const unsigned long long nl = ((1ull << GM_ARG(NVL)) - 1ull) & (~0ull << lu);
         rule = keep = (Mask)(nl * GM_ARG(lab_rep));
         kbase = lu * (uint32_t)GM_ARG(AR);
+        source = lu << 25;
       } else {
         const CSource sc = cload<CSource>(srcs + j * (int)sizeof(CSource));
         rule = (Mask)sc.rule;
         keep = (Mask)sc.keep;
-        masked = sc.keep != sc.rule;
         kbase = (uint32_t)sc.kbase;
       }
-      auto passes = [&](uint32_t x) GM_INLINE -> uint32_t {
-        return (uint32_t)(rule >> (x >> 6 & (M32 ? 31u : 63u))) & ~(uint32_t)(used >> (x & 63u)) & 1u;
-      };
-      auto keeps = [&](uint32_t x) GM_INLINE -> uint32_t { return (uint32_t)(keep >> (x >> 6 & (M32 ? 31u : 63u))) & 1u; };
-      uint32_t m = 0;
+      auto label_bit = [&](Mask x, uint32_t it) GM_INLINE -> uint32_t { return (uint32_t)(x >> (it >> 6 & (M32 ? 31u : 63u))); };
+      auto bit = [&](Mask x, uint32_t it) GM_INLINE -> uint32_t { return label_bit(x, it) & ~(uint32_t)(used >> (it & 63u)) & 1u; };
+      const Mask cut = (Mask)(rule & ~keep);
+      uint32_t p[8], c = 0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) m |= passes(item(P, O, i)) << i;
-      if (__ballot(next_of(P) != 0)) {
+      for (int i = 0; i < 8; ++i) p[i] = 0;
 #pragma unroll
-        for (int i = 4; i < 8; ++i) m |= passes(item(P, O, i)) << i;
+      for (int i = 0; i < 4; ++i) p[i] = bit(keep, item(P, i));
+      c = p[0] + p[1] + p[2] + p[3];
+      if (cut) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) n_pruned += bit(cut, item(P, i));
       }
-      if (masked) {
-        uint32_t k = 0;
+      if (more) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) k |= keeps(item(P, O, i)) << i;
-        n_pruned += (uint32_t)__popc(m & ~k);
-        m &= k;
+        for (int i = 0; i < 4; ++i) p[4 + i] = bit(keep, item(O, i));
+        c += p[4] + p[5] + p[6] + p[7];
+        if (cut) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) n_pruned += bit(cut, item(O, i));
+        }
       }
-      uint32_t total, off;
-      if (!deep) {
-        const uint32_t c = (uint32_t)__popc(m);
-        const uint64_t b0 = __ballot(c & 1u), b1 = __ballot(c & 2u), b2 = __ballot(c & 4u), b3 = __ballot(c & 8u);
-        total = (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2) + 8 * __popcll(b3));
-        off = below(b0) + 2u * below(b1) + 4u * below(b2) + 8u * below(b3);
-      } else {
-        uint32_t c = (uint32_t)__popc(m);
+      if (deep)
         walk_on(O, [&](uint32_t x) GM_INLINE {
-          const uint32_t ok = passes(x), kp = ok & keeps(x);
-          n_pruned += ok & ~kp;
-          c += kp;
+          n_pruned += bit(cut, x);
+          c += bit(keep, x);
         });
-        off = wave_exclusive_scan<uint32_t>(c, total);
-        total = (uint32_t)uniform((int)total);
-      }
+      const uint32_t incl = wave_incl(c), total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
       if (total) {
         listed += total;
-        uint32_t pos = reserve(total) + off;
-        while (m) {
-          const int i = __ffs((int)m) - 1;
-          m &= m - 1;
-          const uint32_t x = item(P, O, i);
-          emit(pos++, kbase + (x >> 6), x & 63u);
+        const uint32_t pos = reserve(total);
+        uint32_t at = incl - c;
+        if (!ROOT && total <= 64 && !deep) {
+          // Through LDS, so that the list store and the two counter updates
+          // are one instruction each for the whole source: a lane's items one
+          // at a time were three to four of each, a sixth of the lanes busy.
+          // (The root writes directly, 134 us against 145 this way for a batch
+          // of 64 databases: its entries' sources and keys differ by lane.)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (p[i]) stage[at] = item(P, i) | who;
+            at += p[i];
+          }
+          if (more) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              if (p[4 + i]) stage[at] = item(O, i) | who;
+              at += p[4 + i];
+            }
+          }
+          wave_sync();
+          const uint32_t x = stage[lane], r = x >> 12 & 63u;  // (lanes past the items: stale, unused)
+          if ((uint32_t)lane < total)
+            emit((pos + (uint32_t)lane) * 4u, kbase + (x >> 6 & 63u), source | (x & 0xFFFu) << 13 | (row0 + r), x >> 18);
+          wave_sync();
+        } else {
+          at = (at + pos) * 4u;
+          const uint32_t tag = source | rowrel;
+          auto put = [&](uint32_t x, uint32_t ok) GM_INLINE {
+            if (ok) emit(at, kbase + (x >> 6), tag | x << 13, head);
+            at += 4u * ok;
+          };
+          uint32_t m = 0;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) m |= p[i] << i;
+          while (m) {
+            const int i = __builtin_ctz(m);
+            m &= m - 1;
+            put(item(i & 4 ? O : P, i & 3), 1u);
+          }
+          if (deep) walk_on(O, [&](uint32_t x) GM_INLINE { put(x, bit(keep, x)); });
         }
-        if (deep)
-          walk_on(O, [&](uint32_t x) GM_INLINE {
-            if (passes(x) & keeps(x)) emit(pos++, kbase + (x >> 6), x & 63u);
-          });
       }
       P = Pn;
       O = On;
@@ -442,12 +524,12 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
     // segment carried in; a carried-out segment keeps its bit (head lane 0)
     // and is marked as counted in bit 31
     for (int i = lane; i < K; i += 64) {
-      const unsigned long long m = kmask[i];
+      const unsigned long long m = kc[i].mask;
       if (m) {
-        const uint32_t sv = ksup[i];
+        const uint32_t sv = kc[i].sup;
         const uint32_t kp = carry_out ? (uint32_t)(m & 1ull) : 0u;
-        ksup[i] = ((sv & 0x7FFFFFFFu) + (uint32_t)__popcll(m) - (sv >> 31)) | (kp << 31);
-        kmask[i] = kp;
+        kc[i].sup = ((sv & 0x7FFFFFFFu) + (uint32_t)__popcll(m) - (sv >> 31)) | (kp << 31);
+        kc[i].mask = kp;
       }
     }
     wave_sync();
@@ -459,8 +541,8 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
   // close the list, commit the counts to the chunk's replica and keep the
   // chunk's {key, embeddings} records behind the list
   uint32_t nrec = 0;
-  for (int i0 = 0; i0 < K; i0 += 64) nrec += (uint32_t)__popcll(__ballot(i0 + lane < K && kemb[min(i0 + lane, K - 1)] != 0));
-  uint32_t *const ext0 = L.ext;
+  for (int i0 = 0; i0 < K; i0 += 64) nrec += (uint32_t)__popcll(__ballot(i0 + lane < K && kc[min(i0 + lane, K - 1)].emb != 0));
+  GM_GLOBAL uint32_t *const ext0 = L.ext;
   const uint32_t n0 = L.used - 2u;
   uint32_t at = 0;
   if (nrec) {
@@ -476,10 +558,10 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
   uint32_t w = at;
   for (int i0 = 0; i0 < K; i0 += 64) {
     const int i = i0 + lane;
-    const uint32_t e = i < K ? kemb[i] : 0u;
+    const uint32_t e = i < K ? kc[i].emb : 0u;
     const uint64_t m = __ballot(e != 0);
     if (e) {
-      atomicAdd(&acc[i], ((unsigned long long)ksup[i] << kSupShift) | (unsigned long long)e);
+      atomicAdd(&acc[i], ((unsigned long long)kc[i].sup << kSupShift) | (unsigned long long)e);
       if (!L.off) {
         const uint32_t q = w + 2u * below(m);
         L.ext[q] = (uint32_t)i;
@@ -490,7 +572,7 @@ __global__ void __launch_bounds__(64, (TW <= 2 && M32 ? 6 : TW <= 8 ? 5 : 4)) k_
   }
   const unsigned long long w_pruned = wave_sum((unsigned long long)n_pruned);
   if (lane == 0) {
-    GM_ARG(cchunks)[gci] = CChunk{(int64_t)(first + start), (uint64_t)(L.ext - GM_ARG(clist)) + at, L.off ? 0u : nrec};
+    GM_ARG(cchunks)[gci] = CChunk{(int64_t)(first + start), (uint64_t)(L.ext - as_global(GM_ARG(clist))) + at, L.off ? 0u : nrec};
     unsigned long long *const spread = GM_ARG(spread), *const line = spread + (gci & (kSpread - 1)) * kSpreadStride;
     if (listed + w_pruned) atomicAdd(&line[kSpreadCand], listed + w_pruned);
     if (w_pruned) atomicAdd(&line[kSpreadPruned], w_pruned);
@@ -516,7 +598,8 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
   const int K = (int)a.K;
   unsigned long long *const cbase = reinterpret_cast<unsigned long long *>(dyn);
   uint32_t *const crun = dyn + 2 * K;
-  uint16_t *const cmap = reinterpret_cast<uint16_t *>(dyn + 3 * K);
+  uint32_t *const skey = dyn + 3 * K;  // first key of every source number
+  uint16_t *const cmap = reinterpret_cast<uint16_t *>(skey + 128);
   const int lane = threadIdx.x;
   const uint32_t gci = blockIdx.x;
   const CChunk c = cload<CChunk>(a.cchunks + gci);
@@ -547,12 +630,21 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
     nchild += __popcll(m);
   }
   if (nchild == 0) return;
-  wave_sync();
   const int bits = nchild > 1 ? 32 - __clz(nchild - 1) : 0;
   constexpr int RW = 1 + TW;
   const int CW = a.CS >> 2;
-  const int nvp = ROOT ? 1 : (int)cload<CMetaHead>(reinterpret_cast<const char *>(a.meta) + (int64_t)p * a.meta_stride).nv;
-  const uint32_t SB = (uint32_t)(a.S * a.NEL);  // first forward key
+  int nvp = 1;
+  if constexpr (ROOT) {
+    skey[lane] = (uint32_t)(lane * a.AR);
+  } else {
+    const char *meta = reinterpret_cast<const char *>(a.meta) + (int64_t)p * a.meta_stride;
+    const CMetaHead H = cload<CMetaHead>(meta);
+    const CSource *src = reinterpret_cast<const CSource *>(meta + sizeof(CMetaHead));
+    nvp = H.nv;
+    if (lane < H.nsrc) skey[lane] = (uint32_t)src[lane].kbase;
+    if (lane < H.nback) skey[kBackSource + lane] = (uint32_t)src[H.nsrc + lane].kbase;
+  }
+  wave_sync();
   unsigned long long written = 0;
   uint32_t rowbase = 0;
   for (const uint32_t *ext = a.clist + (uint64_t)gci * a.page;;) {
@@ -569,15 +661,15 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
       }
 #pragma unroll
       for (int u = 0; u < kWinUnroll; ++u) {
-        const uint32_t key = e[u] >> 20;
+        const uint32_t sid = e[u] >> 25;
         // entries past the end read as marks too, at the lanes behind all others
-        const uint64_t marks = __ballot(key == kMarkKey);
-        uint32_t row = rowbase + (e[u] & 0x3FFFu);
+        const uint64_t marks = __ballot(sid == kMarkSource);
+        uint32_t row = rowbase + (e[u] & 0x1FFFu);
         if (marks) {
           row += (uint32_t)kMarkRows * below(marks);
-          rowbase += (uint32_t)kMarkRows * (uint32_t)__popcll(__ballot(key == kMarkKey && e[u] != kNone32));
+          rowbase += (uint32_t)kMarkRows * (uint32_t)__popcll(__ballot(sid == kMarkSource && e[u] != kNone32));
         }
-        ix[u] = key < (uint32_t)K ? (int)cmap[key] - 1 : -1;
+        ix[u] = sid != kMarkSource ? (int)cmap[skey[sid] + (e[u] >> 19 & 63u)] - 1 : -1;
         if (ix[u] >= 0) {
           const uint32_t *src = a.crow + (c.start + (int64_t)row) * RW;
           __builtin_memcpy(&t[u], src, sizeof(t[u]));
@@ -603,7 +695,8 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
         wave_sync();
         if (sel) {
           const unsigned long long pos = cbase[h] + (unsigned long long)run + rank;
-          const uint32_t key = e[u] >> 20, w = (e[u] >> 14) & 63u;
+          const uint32_t w = (e[u] >> 13) & 63u;
+          const bool forward = e[u] >> 25 < kBackSource;
           if ((int64_t)pos < a.ccap) {
             uint32_t out[2 + TW];
             out[0] = t[u].x[0];
@@ -617,7 +710,7 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
 #pragma unroll
               for (int q = 0; q <= TW; ++q) {
                 const uint32_t word = q < TW ? t[u].x[q < TW ? 1 + q : 1] : fill;
-                out[1 + q] = key >= SB && (nvp >> 2) == q ? (word & clear) | put : word;
+                out[1 + q] = forward && (nvp >> 2) == q ? (word & clear) | put : word;
               }
             }
             uint32_t *dst = a.crow_out + pos * (unsigned long long)(1 + CW);
@@ -950,7 +1043,7 @@ __global__ void __launch_bounds__(64) k_cgather(CGatherArgs g) {
   const int32_t v0 = g.gvbase[src], nv = g.gvbase[src + 1] - v0, dv = g.dvb[t];
   for (uint32_t i = threadIdx.x; i < nb; i += blockDim.x) g.out_vgrp[d0 + i] = g.vgrp[b0 + i];
   for (int32_t i = threadIdx.x; i < nv; i += blockDim.x)
-    g.out_rrows[dv + i] = make_uint2(d0, g.rrows[v0 + i].y);
+    g.out_rrows[dv + i] = make_uint2(d0 * 8u, g.rrows[v0 + i].y);
 }
 
 template <bool ROOT, int TW>
@@ -965,7 +1058,7 @@ hipError_t level_of(const StepArgs &a, hipStream_t s) {
 
 template <bool ROOT, int TW>
 hipError_t write_of(const StepArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL((k_cwrite<ROOT, TW>), dim3((unsigned)a.n_chunks), dim3(64), (size_t)a.K * 14 + 16, s, a);
+  hipLaunchKernelGGL((k_cwrite<ROOT, TW>), dim3((unsigned)a.n_chunks), dim3(64), (size_t)a.K * 14 + 512 + 16, s, a);
   return hipGetLastError();
 }
 

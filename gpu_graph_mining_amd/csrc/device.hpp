@@ -97,18 +97,19 @@ struct KeySpace {
 // kCompactLabels and a graph needs at most 255 groups:
 //   vgrp[g + u]   vertex u of the graph whose first group is g: four 12-bit
 //                 items (neighbour | label pair << 6; label pair = edge label *
-//                 NVL + neighbour's label), two per 32-bit word, unused ones
-//                 kEmptyItem; bits 24-31 of the first word: the place,
-//                 relative to g, of the vertex's next group (0: none), after
-//                 the graph's vertices
-//   rrows[v]      the root level's row of global vertex v: {g, local id |
+//                 NVL + neighbour's label) from bit 0 on, unused ones all ones;
+//                 bits 48-55: the place, relative to g, of the vertex's next
+//                 group (0: none), after the graph's vertices
+//   rrows[v]      the root level's row of global vertex v: {8 g, local id |
 //                 label << 8}
 //   rtab[c]       the root level's chunk c: {job, chunk of the job, the job's
 //                 first vertex, its vertices}
-// Rows of later levels are {g, tuple} of 1 + S / 4 words.
+// Rows of later levels are {8 g, tuple} of 1 + S / 4 words (8 g: the byte offset
+// of the graph's groups, below 2^32).
 constexpr int kCompactV = 64;
 constexpr int kCompactLabels = 63;  // label pairs stay below 63 and keys at 64 vertices below 4096
-constexpr uint32_t kEmptyItem = 63u << 6;
+constexpr unsigned long long kEmptyGroup = 0x0000FFFFFFFFFFFFull;
+constexpr int64_t kCompactGroups = 1ll << 29;  // groups of a database at most
 
 // A pattern of a compact level: the head, then nsrc sources (the rightmost
 // vertex first), then nback backward targets.  A source's rule has the bits

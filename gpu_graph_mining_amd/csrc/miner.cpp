@@ -131,29 +131,29 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // The compact layout's groups of one graph (vertices [v0, v0 + n) of the
 // packed adjacency), appended to pk; false when they do not fit 255.
 bool pack_groups(PackedDB &pk, int32_t v0, int32_t n, int32_t a_end, int32_t NVL) {
-  constexpr unsigned long long kEmpty =
-      (unsigned long long)(kEmptyItem | kEmptyItem << 12) << 32 | (kEmptyItem | kEmptyItem << 12);
   const size_t base = pk.vgrp.size();
-  pk.vgrp.resize(base + n, kEmpty);
+  int32_t next = n;  // further groups after the vertices
+  pk.vgrp.resize(base + (size_t)n, kEmptyGroup);
   for (int32_t v = 0; v < n; ++v) {
-    const int32_t a0 = pk.vadj[v0 + v], a1 = v + 1 < n ? pk.vadj[v0 + v + 1] : a_end;
-    size_t at = base + v;
-    for (int32_t x = a0; x < a1; ++x) {
-      const int i = (x - a0) & 3;
-      if (i == 0 && x > a0) {  // a further group, linked from the last one
-        const size_t next = pk.vgrp.size() - base;
-        if (next > 255) return false;
-        pk.vgrp[at] |= (unsigned long long)next << 24;
-        pk.vgrp.push_back(kEmpty);
-        at = base + next;
+    const int32_t x0 = pk.vadj[v0 + v], x1 = v + 1 < n ? pk.vadj[v0 + v + 1] : a_end;
+    int32_t at = v;
+    for (int32_t x = x0; x < x1; ++x) {
+      const int i = (x - x0) & 3;
+      if (i == 0 && x > x0) {  // a further group, linked from the last one
+        if (next >= 255) return false;
+        pk.vgrp[base + at] |= (unsigned long long)next << 48;
+        at = next++;
+        pk.vgrp.push_back(kEmptyGroup);
       }
       const uint32_t e = pk.adj[x], lab = ((e >> 8) & 0xFF) * (uint32_t)NVL + ((e >> 16) & 0xFF);
-      const int sh = (i & 1) * 12 + (i & 2) * 16;
-      pk.vgrp[at] = (pk.vgrp[at] & ~(0xFFFull << sh)) | (unsigned long long)((e & 0xFF) | lab << 6) << sh;
+      const int sh = 12 * i;
+      unsigned long long &g = pk.vgrp[base + at];
+      g = (g & ~(0xFFFull << sh)) | (unsigned long long)((e & 0xFF) | lab << 6) << sh;
     }
   }
-  for (int32_t v = 0; v < n; ++v) pk.rrows.push_back(make_uint2((uint32_t)base, (uint32_t)v | (uint32_t)pk.vlab[v0 + v] << 8));
-  return true;
+  for (int32_t v = 0; v < n; ++v)
+    pk.rrows.push_back(make_uint2((uint32_t)base * 8u, (uint32_t)v | (uint32_t)pk.vlab[v0 + v] << 8));
+  return (int64_t)pk.vgrp.size() < kCompactGroups;
 }
 
 // The root level's chunks of every job (a compact database's rows are its
@@ -384,7 +384,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
   if (n_jobs < 1 || begin[0] != 0) throw Error(GM_E_ARG, "job ranges must start at 0");
   const int32_t n_sel = begin[n_jobs];
   std::vector<int32_t> sel(n_sel), dvb(n_sel), dab(n_sel), djob(n_sel);
-  std::vector<uint32_t> dgb(src.compact ? n_sel : 0);
+  std::vector<uint64_t> dgb(src.compact ? n_sel : 0);
   int64_t nv = 0, na = 0, ngr = 0;
   int32_t max_v = 0, max_a = 0;
   out.n_jobs = n_jobs;
@@ -401,7 +401,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
       dab[t] = (int32_t)na;
       djob[t] = j;
       if (src.compact) {
-        dgb[t] = (uint32_t)ngr;
+        dgb[t] = (uint64_t)ngr;
         ngr += src.ggb[g + 1] - src.ggb[g];
       }
       nv += n;
@@ -422,12 +422,12 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
   out.NEL = src.NEL;
   out.vl_values = src.vl_values;
   out.el_values = src.el_values;
-  if (src.compact) {
+  if (src.compact && ngr < kCompactGroups) {
     // only the compact layout: a gathered database is mined by gm_batch_mine
     // alone, which takes it
-    if (nv > INT32_MAX - 1 || ngr >= (1ll << 32)) throw Error(GM_E_UNSUPPORTED, "database too large for 32-bit offsets");
     out.compact = true;
     out.n_groups = ngr;
+    const std::vector<uint32_t> first(dgb.begin(), dgb.end());
     std::vector<uint4> tab;
     root_chunks(out, tab);
     upload(out.rtab, tab, s);
@@ -440,7 +440,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
     if (n_sel > 0) {
       hip_check(hipMemcpyAsync(d, sel.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
       hip_check(hipMemcpyAsync(d + n_sel, dvb.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
-      hip_check(hipMemcpyAsync(d + 2 * (size_t)n_sel, dgb.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
+      hip_check(hipMemcpyAsync(d + 2 * (size_t)n_sel, first.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
     }
     CGatherArgs g;
     g.vgrp = src.vgrp.as<unsigned long long>();
