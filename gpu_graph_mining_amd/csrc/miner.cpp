@@ -87,7 +87,12 @@ void *DevBuf::ensure(size_t bytes) {
   }
   const size_t want = (std::max<size_t>({bytes, cap + cap / 2, 256}) + 255) & ~size_t(255);  // fills take 8-byte words
   release();
-  hip_check(hipMalloc(&p, want), "hipMalloc");
+  hipError_t e = hipMalloc(&p, want);
+  if (e == hipErrorOutOfMemory && release_spares()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, want);
+  }
+  hip_check(e, "hipMalloc");
   cap = want;
   return p;
 }
@@ -382,6 +387,7 @@ void upload_db(const PackedDB &pk, DeviceDB &out, hipStream_t s) {
 void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32_t *begin, const int32_t *ids,
                DeviceDB &out, hipStream_t s) {
   if (n_jobs < 1 || begin[0] != 0) throw Error(GM_E_ARG, "job ranges must start at 0");
+  out.compact = false;
   const int32_t n_sel = begin[n_jobs];
   std::vector<int32_t> sel(n_sel), dvb(n_sel), dab(n_sel), djob(n_sel);
   std::vector<uint64_t> dgb(src.compact ? n_sel : 0);
@@ -434,7 +440,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
     out.vgrp.ensure(8 * (size_t)std::max<int64_t>(ngr, 1));
     out.rrows.ensure(8 * (size_t)std::max<int64_t>(nv, 1));
     out.bytes = 8 * (size_t)ngr + 8 * (size_t)nv + 16 * tab.size();
-    DevBuf idx;  // sel, dvb, dgb
+    DevBuf &idx = out.gidx;  // sel, dvb, dgb
     idx.ensure(12 * (size_t)std::max<int32_t>(n_sel, 1));
     int32_t *d = idx.as<int32_t>();
     if (n_sel > 0) {
@@ -454,7 +460,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
     g.out_vgrp = out.vgrp.as<unsigned long long>();
     g.out_rrows = out.rrows.as<uint2>();
     hip_check(launch_cgather(g, s), "k_cgather");
-    hip_check(hipStreamSynchronize(s), "k_cgather");  // before the index buffer is freed
+    hip_check(hipStreamSynchronize(s), "k_cgather");  // before the host's index arrays go
     return;
   }
   out.gvbase.ensure(4 * (size_t)(n_sel + 1));
@@ -472,7 +478,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
     hip_check(hipStreamSynchronize(s), "gather");
     return;
   }
-  DevBuf idx;  // sel, dvb, dab, djob
+  DevBuf &idx = out.gidx;  // sel, dvb, dab, djob
   idx.ensure(16 * (size_t)n_sel);
   int32_t *d = idx.as<int32_t>();
   hip_check(hipMemcpyAsync(d, sel.data(), 4 * (size_t)n_sel, hipMemcpyHostToDevice, s), "gather");
@@ -496,7 +502,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
   g.out_adj = out.adj.as<uint32_t>();
   g.out_vlab = out.vlab.as<uint8_t>();
   hip_check(launch_gather_graphs(g, s), "k_gather_graphs");
-  hip_check(hipStreamSynchronize(s), "k_gather_graphs");  // before the index buffer is freed
+  hip_check(hipStreamSynchronize(s), "k_gather_graphs");  // before the host's index arrays go
 }
 
 namespace {

@@ -16,6 +16,10 @@ namespace gm {
 
 void hip_check(hipError_t e, const char *what);
 
+// Free what is kept for later subset batches (capi.cpp), when an allocation
+// failed; whether anything was.
+bool release_spares();
+
 // A fixed device region (the static workspace of the entry point that
 // allocates nothing) used as two stacks: side 0 grows up from the bottom,
 // side 1 down from the top.  The rows of a level live on side (level id
@@ -149,6 +153,12 @@ struct Workspace {
     return {&sup, &acc, &accb, &freq, &tiles, &rccnt, &cur_rows, &cur_list, &cursor, &fail, &chunks, &chunk_keys, &cand};
   }
   std::vector<DevBuf *> row_bufs(int i) { return row(i).bufs(); }
+  size_t held() {  // device and pinned bytes
+    size_t n = up.cap + down.cap + down2.cap + minsup.cap + sel.cap + t2.cap;
+    for (DevBuf *b : scratch_bufs()) n += b->cap;
+    for (RowSet &r : rows) n += r.bytes();
+    return n;
+  }
   ~Workspace() {
     for (hipEvent_t e : ev)
       if (e) (void)hipEventDestroy(e);
@@ -174,7 +184,13 @@ struct DeviceDB {
   std::vector<uint32_t> ggb;         // first group of each graph, n_graphs + 1
   std::vector<int64_t> root_chunk0;  // n_jobs + 1: first root chunk of each job
   DevBuf vgrp, rrows, rtab, dggb;
+  DevBuf gidx;  // a gathered database's index arrays
   size_t bytes = 0;
+  size_t held() const {  // device and pinned bytes, the workspace's included
+    size_t n = ws ? ws->held() : 0;
+    for (const DevBuf *b : {&gvbase, &vadj, &adj, &vlab, &gjob, &vgraph, &vgrp, &rrows, &rtab, &dggb, &gidx}) n += b->cap;
+    return n;
+  }
   // mining state; one mining call at a time per database
   std::unique_ptr<Workspace> ws;
   std::mutex mu;
@@ -200,7 +216,8 @@ void upload_db(const PackedDB &pk, DeviceDB &out, hipStream_t s);
 // A database of jobs whose graphs are subsets of a resident one, built on
 // the device (no host packing, no upload of graph data): job j holds graphs
 // ids[begin[j] .. begin[j+1]) of `src` (whose host copy gives their sizes),
-// in that order, with src's dense labels.
+// in that order, with src's dense labels.  `out` may hold an earlier gathered
+// database of the same source, whose buffers it then takes.
 void gather_db(const DeviceDB &src, const HostDB &src_host, int32_t n_jobs, const int32_t *begin, const int32_t *ids,
                DeviceDB &out, hipStream_t s);
 

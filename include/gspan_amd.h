@@ -225,7 +225,9 @@ int gm_batch_create(int32_t n_jobs, gm_db *const *dbs, gm_batch **out);
  * graph data): job j holds graphs graph_ids[job_begin[j] ..
  * job_begin[j+1]) of db, in that order (job_begin[0] = 0; subsets may
  * overlap).  Mining it gives each job the results of mining its subset on
- * its own.  No reference counterpart (serving). */
+ * its own.  No reference counterpart (serving).  When such a batch is
+ * destroyed its device memory may be kept for the next one of the same db (at
+ * most two batches of 1 GiB; freed with db, or when an allocation fails). */
 int gm_batch_create_subsets(gm_db *db, int32_t n_jobs, const int32_t *job_begin, const int32_t *graph_ids,
                             gm_batch **out);
 /* Mine every job of the batch in one schedule with per-job min supports;

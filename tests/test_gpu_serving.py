@@ -45,6 +45,53 @@ def test_subset_batch_equals_each_subset_alone():
         assert sorted((tuple(c), s, n) for c, s, n in got) == sorted((tuple(c), s, n) for c, s, n in want)
 
 
+@pytest.mark.parametrize("vlabels", [5, 90])  # the compact layout's alphabets, and beyond them
+def test_subset_batches_take_over_buffers(vlabels):
+    """Subset batches made one after the other from one database (larger,
+    smaller, empty, duplicated graphs), two at a time, after a run that its
+    sink stopped, and after more of them than are kept: each one's own
+    results; a batch outlives its source."""
+    db = gm.GraphDB.random(3, 400, 5, 9, 1.2, vlabels, 2)
+    db.upload()
+
+    def want(ids, minsup):
+        sub = db.subset(ids)
+        pats, st = gm.mine(sub, minsup, collect_proj=True)
+        sub.close()
+        return sorted((tuple(c), s, n) for c, s, n in pats), st["e_cand"]
+
+    def check(batch, ids, minsup):
+        res, st = batch.mine([minsup], collect_proj=True)
+        got = sorted((tuple(c), s, n) for c, s, n in res[0])
+        assert (got, st["e_cand"]) == (want(ids, minsup) if ids else ([], 0))
+
+    jobs = [(list(range(40)), 6), (list(range(400)), 40), (list(range(0, 400, 7)), 6), ([], 1), ([9] * 12, 12),
+            (list(range(399, 0, -2)), 20)]
+    for ids, minsup in jobs + jobs[::-1]:
+        print("alone", len(ids), flush=True)
+        batch = gm.Batch.from_subsets(db, [ids])
+        check(batch, ids, minsup)
+        batch.close()
+    live = [gm.Batch.from_subsets(db, [ids]) for ids, _ in jobs]
+    for batch, (ids, minsup) in zip(live, jobs):
+        print("among others", len(ids), flush=True)
+        check(batch, ids, minsup)
+    for batch in live:
+        batch.close()
+    lib = gm.load_library()
+    batch = gm.Batch.from_subsets(db, [jobs[1][0]])
+    stop = gm.JOB_PATTERN_CB(lambda *_: 1)
+    assert lib.gm_batch_mine(batch._h, (gm.C.c_int32 * 1)(1), None, stop, None, None) != 0
+    batch.close()
+    wants = [want(*jobs[0]), want(*jobs[5])]
+    last = [gm.Batch.from_subsets(db, [jobs[0][0]]), gm.Batch.from_subsets(db, [jobs[5][0]])]
+    db.close()
+    for batch, (_, minsup), w in zip(last, (jobs[0], jobs[5]), wants):
+        res, st = batch.mine([minsup], collect_proj=True)
+        assert (sorted((tuple(c), s, n) for c, s, n in res[0]), st["e_cand"]) == w
+        batch.close()
+
+
 def test_served_results_equal_alone_on_the_full_database():
     """The 50,000-graph molecule database: queries and mining jobs admitted
     into concurrent slots under a small memory budget (requests queue for
