@@ -86,6 +86,12 @@ bool Spares::release(bool close) {
   return !gone.empty();
 }
 
+struct gm_patterns {
+  std::vector<int32_t> dfs5, n_edges, job;
+  std::vector<uint32_t> support;
+  std::vector<uint64_t> n_proj;
+};
+
 namespace {
 
 thread_local std::string g_last_error;
@@ -547,6 +553,40 @@ void gm_batch_destroy(gm_batch *batch) {
   if (!b) return;
   if (std::shared_ptr<Spares> home = std::move(b->home)) home->give(std::move(b));
 }
+
+gm_patterns *gm_patterns_create(void) { return new (std::nothrow) gm_patterns(); }
+
+int gm_patterns_add_job(void *patterns, int32_t job, const int32_t *dfs5, int32_t n_edges, uint32_t support,
+                        uint64_t n_proj) {
+  gm_patterns *p = static_cast<gm_patterns *>(patterns);
+  try {
+    p->dfs5.insert(p->dfs5.end(), dfs5, dfs5 + 5 * (size_t)n_edges);
+    p->n_edges.push_back(n_edges);
+    p->job.push_back(job);
+    p->support.push_back(support);
+    p->n_proj.push_back(n_proj);
+  } catch (...) {
+    return 1;  // out of memory: stops the run
+  }
+  return 0;
+}
+
+int gm_patterns_add(void *patterns, const int32_t *dfs5, int32_t n_edges, uint32_t support, uint64_t n_proj) {
+  return gm_patterns_add_job(patterns, 0, dfs5, n_edges, support, n_proj);
+}
+
+int64_t gm_patterns_get(const gm_patterns *p, const int32_t **dfs5, const int32_t **n_edges, const int32_t **job,
+                        const uint32_t **support, const uint64_t **n_proj) {
+  if (!p) return 0;
+  if (dfs5) *dfs5 = p->dfs5.data();
+  if (n_edges) *n_edges = p->n_edges.data();
+  if (job) *job = p->job.data();
+  if (support) *support = p->support.data();
+  if (n_proj) *n_proj = p->n_proj.data();
+  return (int64_t)p->n_proj.size();
+}
+
+void gm_patterns_destroy(gm_patterns *patterns) { delete patterns; }
 
 int gm_mine_batch(int32_t n_jobs, gm_db *const *dbs, const int32_t *abs_minsup, const gm_cfg *cfg,
                   gm_job_pattern_cb cb, void *user, gm_stats *stats) {

@@ -236,6 +236,20 @@ int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg,
                   gm_stats *stats);
 void gm_batch_destroy(gm_batch *batch);
 
+/* A sink that keeps the patterns: pass gm_patterns_add (or gm_patterns_add_job)
+ * as the callback and the gm_patterns as `user`, and read them in emission
+ * order afterwards.  gm_patterns_get returns how many there are; pattern i
+ * has n_edges[i] tuples, which follow those of the patterns before it in dfs5.
+ * The arrays belong to `patterns` and hold until the next one is added. */
+typedef struct gm_patterns gm_patterns;
+gm_patterns *gm_patterns_create(void); /* NULL: out of memory */
+int gm_patterns_add(void *patterns, const int32_t *dfs5, int32_t n_edges, uint32_t support, uint64_t n_proj);
+int gm_patterns_add_job(void *patterns, int32_t job, const int32_t *dfs5, int32_t n_edges, uint32_t support,
+                        uint64_t n_proj);
+int64_t gm_patterns_get(const gm_patterns *patterns, const int32_t **dfs5, const int32_t **n_edges,
+                        const int32_t **job, const uint32_t **support, const uint64_t **n_proj);
+void gm_patterns_destroy(gm_patterns *patterns);
+
 /* ---- pattern-support queries ------------------------------------------ */
 /* Support (number of database graphs containing the pattern) of each of
  * n_queries patterns, given as DFS codes: query q has n_edges[q] rows of

@@ -317,3 +317,26 @@ def test_callback_guard_keeps_the_exception():
     with pytest.raises(ValueError):
         g.raise_pending()
     assert gm._Guard(lambda *a: 0)(1) == 0
+
+
+@pytest.mark.parametrize("n_patterns,n_jobs", [(0, 1), (0, 3), (1, 1), (300, 1), (300, 4)])
+def test_listing_returns_what_the_sink_was_given(n_patterns, n_jobs):
+    """The library's own sink: codes, supports and embedding counts up to the
+    ends of their ranges, in emission order, a list per job."""
+    rng = random.Random(n_patterns + n_jobs)
+    want = [[] for _ in range(n_jobs)]
+    with gm._Listing() as listing:
+        for _ in range(n_patterns):
+            n, job = rng.choice([1, 2, 13, 63]), rng.randrange(n_jobs)
+            flat = [rng.choice([0, 1, 254, -1, 2**31 - 1, -2**31]) for _ in range(5 * n)]
+            sup, proj = rng.choice([1, 2**32 - 1]), rng.choice([0, 2**32, 2**64 - 1])
+            dfs = (gm.C.c_int32 * (5 * n))(*flat)
+            lib = gm.load_library()
+            if n_jobs == 1:
+                assert lib.add_pattern(listing.user, dfs, n, sup, proj) == 0
+            else:
+                assert lib.add_job_pattern(listing.user, job, dfs, n, sup, proj) == 0
+            want[job].append((gm.DFSCode(flat[5 * i:5 * i + 5] for i in range(n)), sup, proj))
+        got = listing.patterns(n_jobs)
+    assert got == want
+    assert all(type(c) is gm.DFSCode and type(t) is gm.DFS for pats in got for c, _, _ in pats for t in c)
