@@ -164,7 +164,7 @@ bool pack_groups(PackedDB &pk, int32_t v0, int32_t n, int32_t a_end, int32_t NVL
 // The root level's chunks of every job (a compact database's rows are its
 // vertices).
 void root_chunks(DeviceDB &out, std::vector<uint4> &tab) {
-  out.root_nom = (int32_t)chunk_nominal(2, (uint32_t)out.n_vertices, (uint32_t)out.n_graphs);
+  out.root_nom = (int32_t)chunk_nominal((uint32_t)compact_blocks(out.n_vertices), (uint32_t)out.n_vertices, (uint32_t)out.n_graphs);
   out.root_chunk0.assign(1, 0);
   for (int32_t j = 0; j < out.n_jobs; ++j) {
     const int64_t v0 = out.job_first_vertex[j], n = out.job_first_vertex[j + 1] - v0;
@@ -1014,7 +1014,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     uint64_t key_next = 0;   // first key (relative to p_next) not written: a pattern split over pieces
     int64_t p_counted = 0;   // patterns whose candidates are in e_cand
     int64_t p_end_next = 0;  // > 0: the next piece ends there (its children were measured)
-    int blocks = 2;          // compact levels: blocks of a chunk
+    int blocks = 1;          // compact levels after the root: blocks of a chunk
     int32_t meta_stride = 0; // bytes of a pattern's metadata
   };
   std::deque<Frame> frames(1);
@@ -1029,11 +1029,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   // device bytes a level's rows take (rows with their counts) and a list entry
   auto rows_bytes = [&](int64_t rows, int S_) { return (int64_t)rows * ((compact ? 4 : 22) + S_); };
   int64_t pool_units = 0;  // compact: list pool of the level step (grown when a level overflows it)
-  // compact: blocks of a chunk, as many as leave enough chunks (at most four)
+  // compact: blocks of a chunk
   auto blocks_for = [&](int64_t rows) {
-    int blocks = std::max(1, std::min(4, max_chunk_rows / 64));
-    while (blocks > 1 && rows / (62 * blocks) < kLevelWaves) blocks /= 2;
-    return blocks;
+    return compact_blocks(rows, std::max(1, std::min(kCompactBlocks, max_chunk_rows / 64)));
   };
   // Children chosen on the device (k_cselect, k_cchildren): the host launches
   // the next level from four totals and builds the level's codes, and reports
@@ -1187,7 +1185,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     const int64_t prow_lo = prow(p_begin), prow_hi = prow(p_end);
     // chunk length: kChunkRows, or shorter so that the piece has about
     // kLevelWaves chunks (a power of two, at least one block)
-    // (compact levels: their chunk table was laid out with the rows)
+    // (compact levels: compact_blocks(); their chunk table was laid out with the rows)
     int chunk_rows = max_chunk_rows;
     while (chunk_rows > kMinChunkRows && (prow_hi - prow_lo) / chunk_rows < kLevelWaves) chunk_rows /= 2;
     int64_t total_chunks = 0;
@@ -1209,7 +1207,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     grow(w.tiles, sizeof(uint32_t) * kReduceTiles, s);
     grow_zero(w.acc, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
     // compact: a page of 256 list entries per 64 nominal rows, records included
-    const uint32_t page = 256u * (uint32_t)Fr.blocks;
+    const uint32_t page = 256u * (uint32_t)(root ? compact_blocks(db.n_vertices) : Fr.blocks);
     if (compact) {
       grow(w.chunks, sizeof(CChunk) * std::max<int64_t>(total_chunks, 1), s);
     } else {
