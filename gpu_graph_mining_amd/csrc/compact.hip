@@ -798,17 +798,25 @@ struct SelSums {
   }
 };
 
+struct SelRec {
+  unsigned long long w, rows;
+};
+__device__ __forceinline__ SelRec sel_load(const StepArgs &a, uint32_t i) {
+  return SelRec{a.freq[4ull * i + 1], a.freq[4ull * i + 2]};
+}
 template <bool ROOT>
-__device__ __forceinline__ SelSums sel_of(const StepArgs &a, uint32_t i) {
-  const unsigned long long w = a.freq[4ull * i + 1], rows = a.freq[4ull * i + 2];
+__device__ __forceinline__ SelSums sel_of(const StepArgs &a, const SelRec &r) {
+  const unsigned long long w = r.w, rows = r.rows;
   const uint32_t answer = (uint32_t)(w >> 32) & 0xFFu;  // k_canon_level's, + 1
   const bool sel = ROOT || answer == kCanonMin + 1;
   SelSums s;
   s.n = sel ? 1u : 0u;
   s.rows = sel ? rows : 0ull;
   s.dropped = sel ? 0ull : rows;
-  s.chunks =
-      sel ? chunk_count((uint32_t)rows, chunk_nominal((uint32_t)a.child_blocks, (uint32_t)rows, (uint32_t)w)) : 0u;
+  uint32_t chunks = ROOT ? kChunksMany : (uint32_t)(w >> 40);  // k_canon_level's
+  if (chunks == kChunksMany && sel)
+    chunks = chunk_count((uint32_t)rows, chunk_nominal((uint32_t)a.child_blocks, (uint32_t)rows, (uint32_t)w));
+  s.chunks = sel ? chunks : 0u;
   s.undecided = !ROOT && answer != kCanonMin + 1 && answer != kCanonNotMin + 1 ? 1u : 0u;
   return s;
 }
@@ -826,9 +834,17 @@ __global__ void __launch_bounds__(kSelThreads) k_cselect(StepArgs a, CSelect c) 
   const uint32_t tiles = F > 0 ? (F + kSelThreads - 1) / kSelThreads : 1u;
   for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
     SelSums b{0, 0, 0, 0, 0};  // the lane's share of the records before the tile
-    for (uint32_t i = threadIdx.x; i < tile * kSelThreads; i += kSelThreads) b.add(sel_of<ROOT>(a, i));
+    uint32_t q0 = 0;
+    for (; q0 + 4 <= tile; q0 += 4) {  // four records' loads in flight
+      SelRec r[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) r[u] = sel_load(a, (q0 + (uint32_t)u) * kSelThreads + threadIdx.x);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b.add(sel_of<ROOT>(a, r[u]));
+    }
+    for (; q0 < tile; ++q0) b.add(sel_of<ROOT>(a, sel_load(a, q0 * kSelThreads + threadIdx.x)));
     const uint32_t i = tile * kSelThreads + threadIdx.x;
-    const SelSums x = i < F ? sel_of<ROOT>(a, i) : SelSums{0, 0, 0, 0, 0};
+    const SelSums x = i < F ? sel_of<ROOT>(a, sel_load(a, i)) : SelSums{0, 0, 0, 0, 0};
     const SelSums wb = wave_total(b), wx = wave_total(x);
     if (lane == 0) {
       s_before[wave] = wb;

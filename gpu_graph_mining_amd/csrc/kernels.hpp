@@ -283,9 +283,11 @@ constexpr int kCanonV = 40;     // pattern vertices (+1 for the grown code's nex
 constexpr int kCanonE = 64;     // pattern edges (64-bit used-edge masks)
 constexpr int kCanonCap = 64;   // embeddings of the grown code held at once
 constexpr int kCanonNotMin = 0, kCanonMin = 1, kCanonHost = 2, kCanonBad = 3;
+constexpr uint32_t kChunksMany = 0xFFFFFFu;
 struct CanonArgs {
   // a later level's frequent records (key, support, embeddings, item sum):
-  // the answer + 1 for record i goes to bits 32-39 of its support word
+  // the answer + 1 for record i goes to bits 32-39 of its support word (and
+  // with spread its chunks, at most kChunksMany, to bits 40-63)
   unsigned long long *freq;
   const uint32_t *freq_count;
   uint32_t freq_cap;
@@ -304,7 +306,9 @@ struct CanonArgs {
   int32_t len;
   int64_t K;
   int32_t S, NEL, NVL;
-  unsigned long long *spread;  // (level check) kSpreadNv lines; null: not wanted
+  // children chosen on the device: kSpreadNv lines and blocks of a child's chunk; null: not
+  unsigned long long *spread;
+  int32_t child_blocks;
   // explicit codes: n codes of len (from, to, fromlabel, elabel, tolabel)
   // tuples; out[i] gets the answer (kCanonBad: a malformed tuple)
   const int32_t *codes;

@@ -1059,7 +1059,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     pidx.resize(L.n);
     for (int64_t i = 0; i < pend.F && c < L.n; ++i) {
       const uint64_t sup = rec[i].sup, proj = rec[i].proj;
-      if (!pend.root && (sup >> 32) != (uint64_t)kCanonMin + 1) continue;
+      if (!pend.root && ((sup >> 32) & 0xFF) != (uint64_t)kCanonMin + 1) continue;
       pidx[c] = i;
       L.row0[c] = run;
       L.chunk0[c] = chunks;
@@ -1314,7 +1314,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       a.tile_keys = reduce_tile_keys(nkeys, rep);
       // counters and (most often all of) the frequent keys come down with
       // the list pass: into the mapped buffer
-      guess = std::min<uint32_t>(fcap, dev_select ? std::max<uint32_t>(16384, 8 * last_fcount)
+      guess = std::min<uint32_t>(fcap, dev_select ? std::max<uint32_t>(16384, 16 * last_fcount)
                                                   : std::max<uint32_t>(1024, 2 * last_fcount));
       const size_t head = sizeof(Counters) + sizeof(Freq) * guess;
       hbuf = static_cast<const char *>(down.ensure(head));
@@ -1373,6 +1373,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         c.down = a.down ? a.down + kCounterWords : nullptr;
         c.down_cap = a.down_cap;
         c.spread = dev_select ? a.spread : nullptr;
+        c.child_blocks = blocks_for(prow_hi - prow_lo);
         c.meta = a.meta;
         c.meta_stride = a.meta_stride;
         c.p_base = (int32_t)p_begin;

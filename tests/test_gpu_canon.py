@@ -141,3 +141,15 @@ def test_mining_with_keys_left_to_the_host():
     opats, ost = po.mine_arrays(db.arrays(), n)
     assert sorted((po.normalize(c), s, p) for c, s, p in pats) == sorted((c, s, p) for c, s, p in opats)
     assert st["e_child"] == ost["e_child"] and st["n_patterns"] == leaves
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 36])
+def test_device_check_with_many_images_of_the_root(n):
+    """A path of n equal edges: its root tuple has 2 n images, up to and past
+    the 64 embeddings the device holds (more are left to the host)."""
+    path = [(i, i + 1, 0, 0, 0) for i in range(n)]
+    # the same path grown from its second vertex: not minimal
+    other = [(0, 1, 0, 0, 0)] + [(i, i + 1, 0, 0, 0) for i in range(1, n - 1)] + [(0, n, 0, 0, 0)]
+    want = [gm.DFSCode(c).is_min() for c in (path, other)]
+    assert want == [True, False]
+    assert gm.codes_are_min([path, other]) == want
