@@ -353,7 +353,7 @@ __device__ __forceinline__ int canon_core(CanonLds &L, int n, int nv, int lane) 
 // bounds it is a code's chain of LDS reads.  With a lane per embedding walking
 // the path, 64-bit minima through LDS and one lane finding the rightmost path
 // again for every tuple, a level of 23,000 2-edge codes took 73 us and the
-// twelve levels of 100,000 transactions 550 us; now 35 and 288 us.
+// twelve levels of 100,000 transactions 550 us; now 46 and 288 us.
 //
 // Sizes for codes of n edges: VS bytes of vertex map (the code's vertices and
 // the next one, whole words of 8).

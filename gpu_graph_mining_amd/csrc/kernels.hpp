@@ -237,6 +237,12 @@ hipError_t launch_level_fix(const StepArgs &a, bool root, hipStream_t s);
 // adds their counts up), each a whole number of the workgroup's steps.
 constexpr int64_t kReduceTiles = 1024;
 constexpr int kReduceSplitRep = 8;  // replicas from which four lane groups share a key's
+// Keys and counters up to which one workgroup reduces a level (k_reduce_small):
+// 4-5 us below the line against 9 and a launch for k_reduce and k_reduce_list;
+// past it, at 3,240 keys of 8 replicas or 8,000 of 2, 11 us against 7-9, and at
+// 130,000 counters 16 against 9.
+constexpr int64_t kSmallKeys = 2048, kSmallCounters = 16384;
+inline bool reduce_small(int64_t nkeys, int rep) { return nkeys <= kSmallKeys && nkeys * rep <= kSmallCounters; }
 inline int64_t reduce_tile_keys(int64_t nkeys, int rep) {
   const int64_t step = rep >= kReduceSplitRep ? 64 : 256;
   const int64_t steps = (nkeys + step * kReduceTiles - 1) / (step * kReduceTiles);

@@ -1395,7 +1395,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         sel.fchild = reinterpret_cast<int32_t *>(b + (size_t)fcap * 8);
         sel.crec = reinterpret_cast<uint32_t *>(b + (size_t)fcap * 12);
         sel.chunk_base = reinterpret_cast<uint32_t *>(b + (size_t)fcap * 16);
-        hip_check(launch_cselect(a, sel, root, std::max<uint32_t>(4096, 2 * last_fcount), s), "k_cselect");
+        hip_check(launch_cselect(a, sel, root, guess, s), "k_cselect");
       }
       if (!a.down) stage_down(w, down, dctr, head, s);
       finish_pending();  // the last level's patterns, while the device works

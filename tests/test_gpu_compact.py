@@ -136,3 +136,23 @@ def test_children_chosen_on_the_device(sink):
         with pytest.raises(gm.GMError) as e:
             gm.mine(db, 4, max_edges=6, on_pattern=lambda c, s, n: (got.append((c, s)), len(got) < stop_at)[1])
         assert e.value.code == gm.GM_E_CALLBACK and got == seen[:stop_at]
+
+
+@pytest.mark.parametrize("graphs,nvl,nel,minsup", [(40, 16, 8, 3), (40, 16, 9, 3), (40, 3, 2, 12), (6000, 3, 2, 2400),
+                                                   (6000, 6, 1, 1500), (6000, 7, 5, 600)])
+def test_reductions_of_few_and_many_counters(graphs, nvl, nel, minsup):
+    """Root keys at and past the 2,048 that one workgroup reduces (general
+    kernels, with item sums), and databases of enough chunks for counter
+    replicas: patterns and counts equal those of the entry point whose buffers
+    and kernels are the general ones with one replica, and the oracle's."""
+    db = gm.GraphDB.random(graphs, graphs, 8, 14, 1.1, nvl, nel)
+    db.upload()
+    key = lambda pats: sorted((tuple(c), s, n) for c, s, n in pats)
+    pats, st = gm.mine(db, minsup, collect_proj=True)
+    other, so = gm.mine_noalloc(db, minsup, collect_proj=True)
+    assert pats and key(pats) == key(other)
+    assert all(st[k] == so[k] for k in ("n_patterns", "e_root", "e_child", "e_cand"))
+    if graphs == 40:
+        opats, ost = po.mine_arrays(db.arrays(), minsup)
+        assert sorted((po.normalize(c), s, n) for c, s, n in pats) == sorted((c, s, n) for c, s, n in opats)
+        assert (st["e_child"], st["e_cand"]) == (ost["e_child"], ost["e_cand"])
