@@ -940,7 +940,16 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   unsigned long long written_expect = 0;  // child rows asked of every k_write so far
   bool written_pending = false;           // the last k_write's rows are not compared with it yet
   uint32_t last_fcount = 0;
-  int table_bits = opt.table_bits > 0 ? opt.table_bits : 8;
+  // The count table of the general kernels' root: a chunk is 64 rows or one
+  // graph, and about half of its adjacency entries are candidates.  256
+  // entries hold 224 keys; from 96 expected on a tenth of the chunks and more
+  // were recounted (40 x 6 labels, graphs of 100 to 256 vertices: 767 us, with
+  // 512 entries 729; 100 x 2 labels at degree 6: 1653 and 1379), below it 512
+  // cost 2 to 7 % (16 x 8 labels: 404 and 434 us).
+  const double root_keys = db.n_vertices > 0 && db.n_graphs > 0
+                               ? 0.5 * std::max(64.0, (double)db.n_vertices / db.n_graphs) * (double)db.n_adj / (double)db.n_vertices
+                               : 0.0;
+  int table_bits = opt.table_bits > 0 ? opt.table_bits : root_keys > 96.0 && (int64_t)NVL * NEL * NVL > 224 && !w.arena ? 9 : 8;
   const int max_chunk_rows = opt.chunk_rows > 0 ? opt.chunk_rows : kChunkRows;
   const Counters *dctr_last = nullptr;
   // Path pruning: t2[((job * NVL) + centre label) * AR + arm] is the mask of
