@@ -939,6 +939,7 @@ __global__ void __launch_bounds__(256) k_ct2(StepArgs a, CMetaArgs m) {
 // make_cmeta.
 struct ChildLds {
   unsigned long long vm[kCompactV];  // arms that go with every pattern edge at a vertex (path rule)
+  unsigned long long fm[kCompactV];  // label pairs the parent extends by to a frequent pattern (sibling rule)
   unsigned long long bwd;            // vertices the rightmost one has an edge to
   uint32_t code[64];
   uint8_t lab[kCompactV], found[kCompactV], path[kCompactV];  // label; its forward tuple; rightmost path's tuples
@@ -1006,6 +1007,33 @@ __global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaA
     v = (int)(L.code[k] & 0xFF);
   }
   wave_sync();
+  // Sibling rule: an extension of the child at a vertex that the parent has on
+  // its rightmost path was one of the parent's too (the same path edge there,
+  // or an order rule that only got stricter), and its pattern contains the
+  // parent's: it must have been frequent.  (The root's children: the edge must
+  // be a frequent one.)
+  L.fm[lane] = m.siblings && (ROOT || !t.forward || lane < nv) ? 0ull : ~0ull;
+  wave_sync();
+  auto frequent = [&](int64_t k) GM_INLINE -> bool {
+    const int32_t s = a.sup[k];  // (negative: chosen, its id)
+    return s < 0 || (s > 0 && s >= (a.minsup_job ? a.minsup_job[job] : a.minsup_one));
+  };
+  if (m.siblings) {
+    // a lane per (vertex, label pair): the rightmost vertex, then the path's
+    const int pairs = (nrm + 1) * a.AR;
+    for (int x = lane; x < pairs; x += 64) {
+      const int q = x / a.AR, b = x - q * a.AR, v = q ? (int)(L.code[L.path[q - 1]] & 0xFFu) : cnv - 1;
+      bool ok = false;
+      if constexpr (ROOT) {
+        const int el = b / a.NVL, l = b - el * a.NVL, lv = L.lab[v];
+        ok = frequent((int64_t)p * a.K + (min(lv, l) * a.NEL + el) * a.NVL + max(lv, l));
+      } else if (v < nv) {
+        ok = frequent((int64_t)p * a.K + a.S * a.NEL + v * a.AR + b);
+      }
+      if (ok) atomicOr(&L.fm[v], 1ull << b);
+    }
+  }
+  wave_sync();
   // lane q: the rightmost path's edge q and its from vertex f
   const uint32_t w = lane < nrm ? L.code[L.path[lane]] : 0u;
   const int fv = (int)(w & 0xFF), e1 = (int)(w >> 16 & 0xFF), l1 = lane < nrm ? (int)L.lab[w >> 8 & 0xFF] : 0;
@@ -1039,13 +1067,17 @@ __global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaA
     h.nom = chunk_nominal((uint32_t)a.child_blocks, (uint32_t)f[2], (uint32_t)f[1]);
     h.pad = 0;
     *reinterpret_cast<CMetaHead *>(out) = h;
-    if (has_own) src[0] = CSource{own, own & L.vm[rv], rv, SB + rv * a.AR};
+    if (has_own) src[0] = CSource{own, own & L.vm[rv] & L.fm[rv], rv, SB + rv * a.AR};
   }
-  if (fr) src[has_own + (int)below(mf)] = CSource{fr, fr & L.vm[fv], fv, SB + fv * a.AR};
+  if (fr) src[has_own + (int)below(mf)] = CSource{fr, fr & L.vm[fv] & L.fm[fv], fv, SB + fv * a.AR};
   if (br) {
     // a new arm at both ends: (e, label of f) at the rightmost vertex, (e, its label) at f
     const unsigned long long both = (L.vm[rv] >> lf) & (L.vm[fv] >> maxlabel) & a.lab_rep;
-    src[nsrc + (int)below(mb)] = CSource{br, m.masks ? br & (both << lf) : br, fv, fv * a.NEL};
+    unsigned long long keep = m.masks ? br & (both << lf) : br;
+    if (!ROOT && m.siblings && !t.forward)
+      for (int el = 0; el < a.NEL; ++el)
+        if (!frequent((int64_t)p * a.K + fv * a.NEL + el)) keep &= ~(1ull << (el * a.NVL + lf));
+    src[nsrc + (int)below(mb)] = CSource{br, keep, fv, fv * a.NEL};
   }
 }
 

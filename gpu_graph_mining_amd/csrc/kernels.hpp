@@ -183,6 +183,7 @@ struct CMetaArgs {
   // path rule: arms t2[(job * NVL + centre) * AR + arm]; null: none
   unsigned long long *t2;
   int32_t masks;         // the table is complete: the sources' keep masks follow it
+  int32_t siblings;      // and they follow the parents' frequent extensions
   char *meta;            // out: meta_stride bytes a child
   int32_t meta_stride;
   uint32_t *code;        // out: len + 1 tuples a child

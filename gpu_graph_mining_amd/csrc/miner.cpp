@@ -963,6 +963,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   // only) and when NEL * NVL > 64 (the masks are 64-bit).
   const int AR = NEL * NVL;
   const bool prune = opt.path_pruning && !opt.queries && AR <= 64;
+  const bool siblings = compact && prune;  // the sibling rule beside it
+  std::vector<uint64_t> edge_ok;           // per job and label: the label pairs of its frequent edges
   std::vector<uint64_t> t2;
   bool t2_ready = false;
   bool t2_partial = false;  // the 2-edge level was written in pieces: no path table
@@ -1511,6 +1513,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         m.pvlab = root ? nullptr : reinterpret_cast<const uint8_t *>(w.row(cur).upl.as<char>() + vlab_off);
         m.len = new_len - 1;
         m.crec = sel.crec;
+        m.siblings = siblings;
         m.C = C;
         m.meta = du;
         m.meta_stride = child_stride;
@@ -1950,6 +1953,55 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       counters_clear = true;
       us_host = t_host.sec() * 1e6;
 
+      // The sibling rule (k_cchildren has the reason): what a child's sources
+      // let through at vertices of its parent must have been frequent there.
+      // Records are in key order, a parent's side by side; at the root a
+      // job's frequent edges make a mask per label.
+      if (siblings && root) {
+        edge_ok.assign((size_t)db.n_jobs * NVL, 0);
+        for (int64_t i = 0; i < F; ++i) {
+          const int64_t p = parent_of(fr[i].key);
+          const DFS &t = ktup[i];
+          edge_ok[(size_t)p * NVL + t.fromlabel] |= 1ull << (t.elabel * NVL + t.tolabel);
+          edge_ok[(size_t)p * NVL + t.tolabel] |= 1ull << (t.elabel * NVL + t.fromlabel);
+        }
+      }
+      auto sibling_child = [&](int64_t i, char *meta) {
+        const CMetaHead *h = reinterpret_cast<const CMetaHead *>(meta);
+        CSource *src = reinterpret_cast<CSource *>(meta + sizeof(CMetaHead));
+        const int64_t p = parent_of(fr[i].key);
+        const DFS &t = ktup[i];
+        if (root) {
+          for (int k = 0; k < h->nsrc; ++k)
+            src[k].keep &= edge_ok[(size_t)p * NVL + (src[k].from ? t.tolabel : t.fromlabel)];
+          return;
+        }
+        const bool forward = t.from < t.to;
+        uint64_t fwd[kMaxPatV] = {}, bwd[kMaxPatV] = {};  // label pairs per source, edge labels per target
+        const uint64_t k0 = fr[i].key - fdK.mod(fr[i].key), SB = (uint64_t)S * NEL;
+        auto take = [&](int64_t j) {
+          const uint64_t x = fr[j].key - k0;
+          if (x >= SB) {
+            const uint64_t y = x - SB, v = y / (uint64_t)AR;
+            fwd[v] |= 1ull << (y - v * AR);
+          } else {
+            bwd[x / (uint64_t)NEL] |= 1ull << (x % (uint64_t)NEL);
+          }
+        };
+        for (int64_t j = i; j >= 0 && fr[j].key >= k0; --j) take(j);
+        for (int64_t j = i + 1; j < F && fr[j].key < k0 + (uint64_t)K; ++j) take(j);
+        for (int k = 0; k < h->nsrc; ++k, ++src)
+          if (!forward || src->from != t.to) src->keep &= fwd[src->from];
+        if (forward) return;  // (targets from the new vertex)
+        const uint8_t *pv = L.vl(p);
+        for (int k = 0; k < h->nback; ++k, ++src) {
+          uint64_t b = 0;
+          for (int el = 0; el < NEL; ++el)
+            if ((bwd[src->from] >> el) & 1) b |= 1ull << (el * NVL + pv[src->from]);
+          src->keep &= b;
+        }
+      };
+
       // while the device writes the children: the canonical check of the
       // speculative children, their codes and metadata, the path masks
       Timer t_over;
@@ -1982,6 +2034,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         if (compact) {
           make_cmeta(hu + (size_t)c * child_stride, cc, new_len, cv, cnv, N.job[c], (uint64_t)N.row0[c], fr[i].proj,
                      chunk_nominal((uint32_t)child_blocks, (uint32_t)fr[i].proj, (uint32_t)fr[i].sup), !kalive[i], CS, rules, opt.queries ? &opt.queries->nodes[knode[i]].kids : nullptr);
+          if (siblings) sibling_child(i, hu + (size_t)c * child_stride);
         } else if (wide) {
           hmw[c] = make_meta<kMaxPatV>(cc, new_len, cv, cnv, N.job[c]);
           if (!kalive[i]) hmw[c].flags |= kPatDead;
@@ -2016,14 +2069,14 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         if (compact) {
           const CMetaHead *h = reinterpret_cast<const CMetaHead *>(hu + (size_t)c * child_stride);
           CSource *src = reinterpret_cast<CSource *>(hu + (size_t)c * child_stride + sizeof(CMetaHead));
-          for (int k = 0; k < h->nsrc; ++k, ++src) src->keep = src->rule & vm[src->from];
+          for (int k = 0; k < h->nsrc; ++k, ++src) src->keep &= vm[src->from];
           // backward rv -> t (a pair's label is t's): a new arm at both ends
           for (int k = 0; k < h->nback; ++k, ++src) {
             const int t = src->from;
             uint64_t b = 0;
             for (int el = 0; el < NEL; ++el)
               b |= ((vm[rv] >> (el * NVL + cv[t])) & (vm[t] >> (el * NVL + cv[rv])) & 1ull) << (el * NVL + cv[t]);
-            src->keep = src->rule & b;
+            src->keep &= b;
           }
           return;
         }

@@ -99,7 +99,7 @@ typedef struct gm_stats {
   uint64_t split_passes;   /* chunks recounted because their LDS count table filled */
   uint64_t max_graph_rows; /* unused (0) */
   uint64_t max_table_fill; /* most distinct keys one chunk's count table held */
-  uint64_t pruned;         /* candidates dropped by the 2-edge path rule (counted in e_cand) */
+  uint64_t pruned;         /* candidates dropped by the path and sibling rules (counted in e_cand) */
   double seconds_stage_events; /* extension + support stages timed by HIP events (cfg.stage_events) */
   uint64_t canon_host_keys;    /* frequent keys the device check left to the host (beyond its capacity) */
 } gm_stats;

@@ -156,3 +156,29 @@ def test_reductions_of_few_and_many_counters(graphs, nvl, nel, minsup):
         opats, ost = po.mine_arrays(db.arrays(), minsup)
         assert sorted((po.normalize(c), s, n) for c, s, n in pats) == sorted((c, s, n) for c, s, n in opats)
         assert (st["e_child"], st["e_cand"]) == (ost["e_child"], ost["e_cand"])
+
+
+@pytest.mark.parametrize("graphs,nvl,nel,factor,minsup", [(12000, 3, 2, 1.4, 240), (12000, 2, 1, 1.7, 1800), (300, 3, 1, 1.6, 30)])
+def test_extensions_infrequent_at_the_parent_are_not_listed(graphs, nvl, nel, factor, minsup):
+    """The sibling rule drops only what cannot be frequent, forward and backward
+    (cycles), with children chosen on the device (12,000 graphs) and on the
+    host, checked there or written ahead, in pieces and by job: patterns,
+    supports, |Proj| and E_cand are those of a run without path pruning."""
+    db = gm.GraphDB.random(5, graphs, 6, 12, factor, nvl, nel)
+    db.upload()
+    key = lambda pats: sorted((tuple(c), s, n) for c, s, n in pats)
+    want, so = gm.mine(db, minsup, collect_proj=True, path_pruning=False)
+    assert any(t[0] > t[1] for c, _, _ in want for t in c) and so["pruned"] == 0
+    for kw in ({}, {"canon_host": 1}, {"canon_host": 2}, {"speculate": 2}, {"mem_budget": 6 << 20}):
+        print("options", kw, flush=True)
+        pats, st = gm.mine(db, minsup, collect_proj=True, **kw)
+        assert key(pats) == key(want)
+        assert all(st[k] == so[k] for k in ("n_patterns", "e_root", "e_child", "e_cand"))
+        assert st["pruned"] > 0
+    ids = [list(range(0, graphs, 2)), list(range(graphs))]
+    batch = gm.Batch.from_subsets(db, ids)
+    res, _ = batch.mine([minsup, minsup], collect_proj=True)
+    assert key(res[1]) == key(want)
+    half = db.subset(ids[0])
+    assert key(res[0]) == key(gm.mine(half, minsup, collect_proj=True, path_pruning=False)[0])
+    batch.close()
