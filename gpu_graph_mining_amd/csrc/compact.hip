@@ -988,6 +988,7 @@ __global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaA
                                     : (uint32_t)t.from | (uint32_t)t.to << 8 | (uint32_t)t.el << 16 | (uint32_t)tl << 24;
     L.code[lane] = w;
     m.code[ci * n + lane] = w;
+    if (lane == 0) m.key[ci] = key;
     const int u = (int)(w & 0xFF), v = (int)(w >> 8 & 0xFF);
     if (u < v) L.found[v] = (uint8_t)lane;
     else if (u == cnv - 1) atomicOr(&L.bwd, 1ull << v);
@@ -1034,6 +1035,26 @@ __global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaA
     }
   }
   wave_sync();
+  // The same at a new vertex, by another pattern of the level: when the parent
+  // is G + g and the child's new edge n starts at a vertex of G, G + n is in
+  // the child too; if it is a pattern of this level (its code is minimal), what
+  // it extends its last vertex by must have been frequent.
+  int64_t cousin = -1;
+  if constexpr (!ROOT) {
+    if (m.pkey && t.forward) {
+      const uint32_t pk = m.pkey[p], g = pk / m.pK;
+      const int nvg = pk - g * m.pK >= (uint32_t)(m.pS * a.NEL) ? nv - 1 : nv;  // G's vertices
+      if (t.from < nvg) {
+        const int32_t r = m.psup[(int64_t)g * m.pK + m.pS * a.NEL + (t.from * a.NEL + t.el) * a.NVL + t.tl];
+        if (r < 0) cousin = (int64_t)(-(r + 1)) * a.K;
+      }
+      if (cousin >= 0) {
+        const uint64_t ok = __ballot(lane < a.AR && frequent(cousin + a.S * a.NEL + nvg * a.AR + lane));
+        if (lane == 0) L.fm[cnv - 1] = ok;
+      }
+      wave_sync();
+    }
+  }
   // lane q: the rightmost path's edge q and its from vertex f
   const uint32_t w = lane < nrm ? L.code[L.path[lane]] : 0u;
   const int fv = (int)(w & 0xFF), e1 = (int)(w >> 16 & 0xFF), l1 = lane < nrm ? (int)L.lab[w >> 8 & 0xFF] : 0;
@@ -1074,9 +1095,11 @@ __global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaA
     // a new arm at both ends: (e, label of f) at the rightmost vertex, (e, its label) at f
     const unsigned long long both = (L.vm[rv] >> lf) & (L.vm[fv] >> maxlabel) & a.lab_rep;
     unsigned long long keep = m.masks ? br & (both << lf) : br;
-    if (!ROOT && m.siblings && !t.forward)
+    if (!ROOT && m.siblings && (!t.forward || cousin >= 0)) {
+      const int64_t at = t.forward ? cousin : (int64_t)p * a.K;
       for (int el = 0; el < a.NEL; ++el)
-        if (!frequent((int64_t)p * a.K + fv * a.NEL + el)) keep &= ~(1ull << (el * a.NVL + lf));
+        if (!frequent(at + fv * a.NEL + el)) keep &= ~(1ull << (el * a.NVL + lf));
+    }
     src[nsrc + (int)below(mb)] = CSource{br, keep, fv, fv * a.NEL};
   }
 }

@@ -184,6 +184,13 @@ struct CMetaArgs {
   unsigned long long *t2;
   int32_t masks;         // the table is complete: the sources' keep masks follow it
   int32_t siblings;      // and they follow the parents' frequent extensions
+  // the level's patterns as the level before chose them: their keys there and
+  // its support table (chosen keys: -(pattern + 1)); null: not known
+  const uint32_t *pkey;
+  const int32_t *psup;
+  uint32_t pK;
+  int32_t pS;
+  uint32_t *key;         // out: the children's keys
   char *meta;            // out: meta_stride bytes a child
   int32_t meta_stride;
   uint32_t *code;        // out: len + 1 tuples a child

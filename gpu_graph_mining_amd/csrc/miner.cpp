@@ -1021,6 +1021,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     int mask_stride = 0;
     size_t code_off = 0, vlab_off = 0;  // packed codes and vertex labels for the device check
     bool codes_ready = false;
+    // patterns chosen on the device after the root: their keys in the upload
+    // (0: none), and the key space of the support table in sup2
+    size_t key_off = 0;
+    uint32_t pK = 0;
+    int pS = 0;
     int64_t p_next = 0;      // first pattern whose children are not all written
     uint64_t key_next = 0;   // first key (relative to p_next) not written: a pattern split over pieces
     int64_t p_counted = 0;   // patterns whose candidates are in e_cand
@@ -1497,10 +1502,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       while (nxt == cur) ++nxt;
       const size_t codes_off = ((size_t)child_stride * C + 7) & ~size_t(7);
       const size_t cvl_off = (codes_off + sizeof(uint32_t) * new_len * C + 7) & ~size_t(7);
+      const size_t key_off = (cvl_off + (size_t)CS * C + 3) & ~size_t(3);
       CMetaArgs m;
       std::memset(&m, 0, sizeof(m));
       if (C > 0) {
-        char *du = static_cast<char *>(grow(w.row(nxt).upl, cvl_off + (size_t)CS * C, s));
+        char *du = static_cast<char *>(grow(w.row(nxt).upl, key_off + sizeof(uint32_t) * C, s));
         grow(w.row(nxt).vt, (size_t)(4 + CS) * child_rows, s);
         grow(w.row(nxt).ctab, sizeof(uint2) * chunks, s);
         grow(w.cursor, sizeof(unsigned long long) * C * rep, s);
@@ -1514,6 +1520,13 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         m.len = new_len - 1;
         m.crec = sel.crec;
         m.siblings = siblings;
+        m.key = reinterpret_cast<uint32_t *>(du + key_off);
+        if (siblings && Fr.key_off > 0) {
+          m.pkey = reinterpret_cast<const uint32_t *>(w.row(cur).upl.as<char>() + Fr.key_off);
+          m.psup = w.sup2.as<int32_t>();
+          m.pK = Fr.pK;
+          m.pS = Fr.pS;
+        }
         m.C = C;
         m.meta = du;
         m.meta_stride = child_stride;
@@ -1542,7 +1555,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       }
       dev_sec += tdev.sec();
       size_t live = db.bytes + w.sup.cap + w.tiles.cap + w.acc.cap + w.freq.cap + w.cand.cap + w.chunks.cap +
-                    w.cursor.cap + w.sel.cap + w.t2.cap;
+                    w.cursor.cap + w.sel.cap + w.t2.cap + w.sup2.cap;
       for (const RowSet &rs : w.rows) live += rs.bytes();
       peak = std::max(peak, live);
       if (trace_levels)
@@ -1581,6 +1594,13 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         cf.code_off = codes_off;
         cf.vlab_off = cvl_off;
         cf.codes_ready = true;
+        if (siblings && !root) {  // the choice's support table and keys, for the next one
+          std::swap(w.sup.p, w.sup2.p);
+          std::swap(w.sup.cap, w.sup2.cap);
+          cf.key_off = key_off;
+          cf.pK = (uint32_t)K;
+          cf.pS = S;
+        }
       }
       std::swap(N, spare);
       continue;

@@ -106,7 +106,7 @@ struct Workspace {
   // records while the next level's are written), the children chosen on the
   // device and the 2-edge path table
   HostBuf down2;
-  DevBuf sel, t2;
+  DevBuf sel, t2, sup2;  // sup2: the level before's support table
   hipEvent_t ev[2] = {nullptr, nullptr};  // stage timing (MineOptions::stage_events)
   // the children's upload runs on a copy engine beside the write pass:
   // its stream (default priority) and the event the next level waits on
@@ -154,7 +154,7 @@ struct Workspace {
   }
   std::vector<DevBuf *> row_bufs(int i) { return row(i).bufs(); }
   size_t held() {  // device and pinned bytes
-    size_t n = up.cap + down.cap + down2.cap + minsup.cap + sel.cap + t2.cap;
+    size_t n = up.cap + down.cap + down2.cap + minsup.cap + sel.cap + t2.cap + sup2.cap;
     for (DevBuf *b : scratch_bufs()) n += b->cap;
     for (RowSet &r : rows) n += r.bytes();
     return n;
