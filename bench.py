@@ -269,7 +269,7 @@ def _main_section(args) -> dict:
 
     roof = {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None,
             "traffic": _traffic("stage", config["workload"]),
-            "kernel": "k_level (+ k_level_fix): extension enumeration and support counting of one level step",
+            "kernel": "k_clevel, or k_level (+ k_level_fix): extension enumeration and support counting of one level step",
             "traffic_unit": "HBM bytes per launch (one level step's k_level + k_level_fix)",
             "launches_per_step": launches / args.steps,
             "avg_launch_ms": (ev_s / launches * 1e3) if launches else None}
