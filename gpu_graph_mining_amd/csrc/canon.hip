@@ -21,7 +21,8 @@
 // LDS; the lanes take the embeddings, and each step's smallest tuple is a
 // wave-wide minimum.  A code beyond the LDS capacity (more than kCanonE
 // edges, kCanonV - 1 vertices, kCanonCap embeddings, or a repeated edge)
-// is left undecided (kCanonHost) for the host check.
+// is left undecided (kCanonHost) for the host check.  Explicit codes (any
+// labels) take canon_core; a level's own codes, with dense labels, canon_level.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -36,13 +36,14 @@
 //
 // What bounds k_clevel: the gathers.  A load of one group a lane touches 13
 // lines, nearly all of them misses in a 32 KB L1 that 28 waves share, so a
-// block of 64 rows asks L2 for some 170 lines; with an average of 51 of them in
-// flight a CU's L1 waits on pending lines for 70% of the kernel's time (100,000
-// transactions: 2.5e8 lines and 3.25 ms for the levels of 8-byte tuples, 2.3 ms
-// with the loads alone).  Vector issue comes next (1,000 instructions a block,
-// 68% of the time at 3.3 cycles each) and is hidden behind it: 6% fewer
-// instructions gave 1%.  Items at bit offsets that one shift reaches and 16-byte
-// counter records took that case from 5.15 ms to 4.75 over all levels.
+// block of 64 rows asks L2 for some 170 lines.  The address units are 80-85 %
+// busy and L1 waits on pending lines for 75 % of the time (100,000
+// transactions: 2.85 ms for the levels of 8-byte tuples, 2.3 ms with the loads
+// alone); neither more waves, loads further ahead nor lines kept in an XCD's
+// L2 change it.  Vector issue comes next (850 instructions a block) and is
+// hidden behind it.  Items at bit offsets that one shift reaches and 16-byte
+// counter records took all levels of that case from 5.15 ms to 4.75, the
+// sibling rules (k_cchildren), which leave fewer candidates to list, to 4.2.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -6,24 +6,24 @@
 // This driver grows it level by level instead: one level step extends the
 // embeddings of *every* pattern of the current size in the same launches,
 // so each step costs a fixed number of kernels and one host round trip
-// (the frequent-key list down, the chosen children up) no matter how many
-// patterns the level holds.  Patterns are independent subtrees, so the
+// (the frequent-key list down, the chosen children up when the host chose them)
+// no matter how many patterns the level holds.  Patterns are independent subtrees, so the
 // set of reported (code, support) pairs is the one the depth-first oracle
 // reports (src/gspan/gspan.cpp:172-274); only the emission order differs.
 //
-// Level step for patterns P_1..P_n with embeddings in graph-major rows:
-//   1. k_expand    : every row's extension candidates, listed (row-parallel);
-//      k_support   : distinct-graph support and embedding count of every
-//                    (pattern, extension key), one workgroup per graph;
-//      k_reduce    : the keys whose support reached their job's min support;
-//   2. host        : decode each frequent key into a child code, keep the
-//                    minimal ones (canonical.cpp; on speculative levels every
-//                    frequent key becomes a child and the check runs while
-//                    the device writes), number the children in key order;
-//   3. children    : count, place and write the child rows (row-parallel
-//                    passes where every candidate is listed, per-graph passes
-//                    otherwise), sized exactly by the embedding counts
-//                    k_support gathered.
+// A level step, for patterns with pattern-major rows (their embeddings):
+//   1. k_level and k_level_fix, or k_clevel on compact databases: every row's
+//      extension candidates, listed and counted per (pattern, extension key);
+//      k_reduce, k_reduce_list: the keys whose support reached their job's
+//      min support, in key order;
+//   2. the children: k_canon_level, k_cselect and k_cchildren check, number
+//      and describe them on the device; or the host decodes each frequent key
+//      into a child code, keeps the minimal ones (canonical.cpp or
+//      k_canon_level; on speculative levels every frequent key becomes a child
+//      and the check runs while the device writes) and numbers them in key
+//      order, and k_cursors or k_ccursors sets their row cursors;
+//   3. k_write or k_cwrite: the child rows, sized exactly by the embedding
+//      counts.
 #include "miner.hpp"
 
 #include <algorithm>
