@@ -81,7 +81,9 @@ constexpr uint32_t kEmpty32 = 0xFFFFFFFFu;
 constexpr int kWriteTableBits = 6;
 // The root level's chunks span many graphs and every label triple: there a
 // chunk often holds more than 64 frequent children, and a 256-entry table
-// (5 waves per SIMD) beats the residue passes.
+// (5 waves per SIMD) beats the residue passes.  Where k_level's root took a
+// table of 512 entries or more, so does the write (18 KB of LDS a wave): 3,000
+// graphs of 100 to 256 vertices with 40 x 6 labels 257 -> 84 us.
 constexpr int kWriteTableBitsRoot = 8;
 constexpr int kFixTableBits = 11;   // k_level_fix: (segment, key) pairs per pass
 
@@ -1015,9 +1017,8 @@ __global__ void __launch_bounds__(256) k_cursors(StepArgs a, const int32_t *fchi
 // child residue before anything is reserved.
 constexpr int kWriteUnroll = 2;  // candidate windows whose loads are issued together
 
-template <bool ROOT, int TW>
-__global__ void __launch_bounds__(64, (ROOT ? 5 : TW <= 8 ? 8 : 6)) k_write(StepArgs a) {
-  constexpr int kBits = ROOT ? kWriteTableBitsRoot : kWriteTableBits;
+template <bool ROOT, int TW, int kBits = kWriteTableBits>
+__global__ void __launch_bounds__(64, (kBits > 8 ? 2 : ROOT ? 5 : TW <= 8 ? 8 : 6)) k_write(StepArgs a) {
   constexpr uint32_t cap = 1u << kBits;
   // keyed by the candidate's key relative to the chunk's first pattern
   // (which names one child), with that child's id in cch
@@ -1409,7 +1410,10 @@ hipError_t launch_write(const StepArgs &a, bool root, hipStream_t s) {
   if (a.n_chunks <= 0) return hipSuccess;
   const unsigned grid = (unsigned)a.n_chunks;
   if (root) {
-    hipLaunchKernelGGL((k_write<true, 0>), dim3(grid), dim3(64), 0, s, a);
+    if (a.table_bits > kWriteTableBitsRoot)
+      hipLaunchKernelGGL((k_write<true, 0, kWriteTableBitsRoot + 1>), dim3(grid), dim3(64), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_write<true, 0, kWriteTableBitsRoot>), dim3(grid), dim3(64), 0, s, a);
     return hipGetLastError();
   }
   switch (a.S >> 2) {

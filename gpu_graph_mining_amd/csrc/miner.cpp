@@ -943,9 +943,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   // The count table of the general kernels' root: a chunk is 64 rows or one
   // graph, and about half of its adjacency entries are candidates.  256
   // entries hold 224 keys; from 96 expected on a tenth of the chunks and more
-  // were recounted (40 x 6 labels, graphs of 100 to 256 vertices: 767 us, with
-  // 512 entries 729; 100 x 2 labels at degree 6: 1653 and 1379), below it 512
-  // cost 2 to 7 % (16 x 8 labels: 404 and 434 us).
+  // were recounted, by the write too (40 x 6 labels, graphs of 100 to 256
+  // vertices: 767 us, with 512 entries 604; 100 x 2 labels at degree 6: 1656 and
+  // 1243), below it 512 cost 2 to 10 % (16 x 8 labels: 392 and 434 us).
   const double root_keys = db.n_vertices > 0 && db.n_graphs > 0
                                ? 0.5 * std::max(64.0, (double)db.n_vertices / db.n_graphs) * (double)db.n_adj / (double)db.n_vertices
                                : 0.0;

@@ -272,3 +272,16 @@ def test_gpu_candidate_counts_closed_form():
     db = gm.GraphDB.from_arrays([0, 3], [0, 0, 0], [0, 3], [0, 1, 0], [1, 2, 2], [0, 0, 0])
     pats, st = gm.mine(db, 1)
     assert len(pats) == 3 and (st["e_cand"], st["e_child"], st["e_root"]) == (18, 12, 6)
+
+
+@pytest.mark.parametrize("table_bits", [0, 8, 9, 10])
+def test_root_chunks_of_many_keys(table_bits):
+    """Graphs of 200 to 256 vertices with 40 x 6 labels: a root chunk (one
+    graph) holds more keys than the 224 of the smallest count table and the 256
+    of the smaller write table, whichever tables are taken."""
+    db = gm.GraphDB.random(2, 60, 200, 256, 1.6, 40, 6)
+    pats, st = gm.mine(db, 6, max_edges=2, collect_proj=True, table_bits=table_bits)
+    opats, ost = po.mine_arrays(db.arrays(), 6, max_edges=2)
+    assert sorted((po.normalize(c), s, p) for c, s, p in pats) == sorted((c, s, p) for c, s, p in opats)
+    assert (st["e_root"], st["e_child"], st["e_cand"]) == (ost["e_root"], ost["e_child"], ost["e_cand"])
+    assert st["max_table_fill"] > (256 if table_bits != 8 else 0)
