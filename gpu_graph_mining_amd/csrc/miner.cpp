@@ -1343,7 +1343,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       // counters and (most often all of) the frequent keys come down with
       // the list pass: into the mapped buffer
       guess = std::min<uint32_t>(fcap, dev_select ? std::max<uint32_t>(16384, 16 * last_fcount)
-                                                  : std::max<uint32_t>(1024, 2 * last_fcount));
+                                                  : std::max<uint32_t>(root ? 8192 : 1024, 2 * last_fcount));
       const size_t head = sizeof(Counters) + sizeof(Freq) * guess;
       hbuf = static_cast<const char *>(down.ensure(head));
       a.counters = reinterpret_cast<const unsigned long long *>(dctr);
@@ -1772,7 +1772,6 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     }
     const bool spec = want_spec && max_nv_exact <= kMaxPatV;
     const bool late_decode = spec;
-    if (!spec) Pool::get().run(F, threads, decode, 4096);
     // the device's answer for frequent key i (written by k_canon_level as
     // answer + 1 in bits 32-39 of the support word); undecided keys are
     // checked here
@@ -1789,7 +1788,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     };
     if (!spec) {
       std::atomic<bool> too_big(false);
+      // (the root's edges need no check: waking the pool costs more than 2,000 of them)
       Pool::get().run(F, threads, [&](int64_t i) {
+        decode(i);
         const uint32_t sup = (uint32_t)fr[i].sup;
         const int cnv = knv[i];
         bool keep = false;
@@ -1810,7 +1811,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         }
         kidx[i] = keep ? 0 : -1;
         kalive[i] = keep ? 1 : 0;
-      });
+      }, root ? 2048 : 64);
       if (too_big) throw Error(GM_E_UNSUPPORTED, "pattern with more than 64 vertices is frequent");
     } else {
       for (int64_t i = 0; i < F; ++i) kidx[i] = in_piece(i) ? 0 : -1;  // decoded while the device writes
