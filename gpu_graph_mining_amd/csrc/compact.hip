@@ -846,17 +846,25 @@ __global__ void __launch_bounds__(kSelThreads) k_cselect(StepArgs a, CSelect c) 
     for (; q0 < tile; ++q0) b.add(sel_of<ROOT>(a, sel_load(a, q0 * kSelThreads + threadIdx.x)));
     const uint32_t i = tile * kSelThreads + threadIdx.x;
     const SelSums x = i < F ? sel_of<ROOT>(a, sel_load(a, i)) : SelSums{0, 0, 0, 0, 0};
-    const SelSums wb = wave_total(b), wx = wave_total(x);
-    if (lane == 0) {
-      s_before[wave] = wb;
-      s_own[wave] = wx;
+    // the wave's own sums: counts by ballot, the others with their scans
+    unsigned long long tr;
+    const unsigned long long er = wave_exclusive_scan<unsigned long long>(x.rows, tr);
+    const uint64_t chosen = __ballot(x.n != 0);
+    const uint32_t en = below(chosen), ic = wave_incl(x.chunks), ec = ic - x.chunks;
+    const SelSums wx{tr, wave_sum(x.dropped), (uint32_t)__popcll(chosen), (uint32_t)__builtin_amdgcn_readlane((int)ic, 63),
+                     (uint32_t)__popcll(__ballot(x.undecided != 0))};
+    if (tile > 0) {
+      const SelSums wb = wave_total(b);
+      if (lane == 0) s_before[wave] = wb;
     }
+    if (lane == 0) s_own[wave] = wx;
     __syncthreads();
     SelSums base{0, 0, 0, 0, 0};  // everything before this wave's records
-#pragma unroll 1
-    for (int q = 0; q < kWaves; ++q) {
-      base.add(s_before[q]);
-      if (q < wave) base.add(s_own[q]);
+#pragma unroll 4
+    for (int q = 0; q < wave; ++q) base.add(s_own[q]);
+    if (tile > 0) {
+#pragma unroll 4
+      for (int q = 0; q < kWaves; ++q) base.add(s_before[q]);
     }
     if (tile == tiles - 1 && wave == kWaves - 1) {  // base and this wave's own: the totals
       unsigned long long nv = 2;
@@ -871,10 +879,6 @@ __global__ void __launch_bounds__(kSelThreads) k_cselect(StepArgs a, CSelect c) 
         a.down[kTotDropped] = base.dropped + wx.dropped;
       }
     }
-    unsigned long long tr;
-    uint32_t tn, tc;
-    const unsigned long long er = wave_exclusive_scan<unsigned long long>(x.rows, tr);
-    const uint32_t en = wave_exclusive_scan<uint32_t>(x.n, tn), ec = wave_exclusive_scan<uint32_t>(x.chunks, tc);
     if (i < F) c.fchild[i] = x.n ? (int32_t)(base.n + en) : -1;
     if (x.n) {
       const uint32_t ch = base.n + en;
