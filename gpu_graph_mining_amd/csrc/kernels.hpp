@@ -63,7 +63,7 @@ struct alignas(16) ChunkInfo {
   int32_t p_lo;    // their keys are (pattern - p_lo) * K + key
   uint32_t pad;
 };
-// A chunk of a compact level: its first row and its {key, embeddings}
+// A chunk of a compact level: its first row and its {key, first place}
 // records, nrec of them at entry rec of the list buffer.
 struct alignas(16) CChunk {
   int64_t start;
