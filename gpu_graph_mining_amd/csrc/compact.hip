@@ -823,7 +823,8 @@ __device__ __forceinline__ SelSums sel_of(const StepArgs &a, const SelRec &r) {
   if (chunks == kChunksMany && sel)
     chunks = chunk_count((uint32_t)rows, chunk_nominal((uint32_t)a.child_blocks, (uint32_t)rows, (uint32_t)w));
   s.chunks = sel ? chunks : 0u;
-  s.undecided = !ROOT && answer != kCanonMin + 1 && answer != kCanonNotMin + 1 ? 1u : 0u;
+  // (2^32 rows and more: for the host, which refuses them)
+  s.undecided = (!ROOT && answer != kCanonMin + 1 && answer != kCanonNotMin + 1) || (sel && rows >> 32) ? 1u : 0u;
   return s;
 }
 
