@@ -746,6 +746,9 @@ __global__ void __launch_bounds__(64, (TW <= 4 ? 8 : 5)) k_cwrite(StepArgs a) {
 // cursor starts at its first row, and the children's chunk table is filled
 // ({child, chunk of the child}).  `rep` lanes take one frequent key; t is the
 // lane's index over all of them.
+// With kByRecord the bases are the host's, in its mapped memory, per record and
+// not per child: they are read beside the ids, a trip over the bus less.
+template <bool kByRecord>
 __device__ __forceinline__ void cursors_of(const StepArgs &a, int64_t t, const int32_t *fchild,
                                            const unsigned long long *row_base, const uint32_t *chunk_base, int64_t F) {
   const int64_t i = t / a.rep;
@@ -753,11 +756,16 @@ __device__ __forceinline__ void cursors_of(const StepArgs &a, int64_t t, const i
   const bool ok = i < F;
   int64_t key = 0, at = 0;
   int32_t ch = -1;
-  unsigned long long rows = 0;
+  unsigned long long rows = 0, row0 = 0;
+  uint32_t chunk0 = 0;
   if (ok) {
+    ch = fchild[i];
+    if (kByRecord && row_base) {  // (none: no child is written)
+      row0 = row_base[i];
+      chunk0 = chunk_base[i];
+    }
     key = (int64_t)a.freq[4 * i];
     at = (int64_t)r * a.nkeys + key;
-    ch = fchild[i];
     rows = a.acc[at] & ((1ull << kSupShift) - 1);
   }
   unsigned long long sr = rows;  // inclusive scan over the key's replicas
@@ -769,18 +777,22 @@ __device__ __forceinline__ void cursors_of(const StepArgs &a, int64_t t, const i
   a.acc[at] = 0;
   if (ch < 0) return;
   if (r == 0) a.sup[key] = -(ch + 1);
-  a.cursor[(int64_t)ch * a.rep + r] = row_base[ch] + (sr - rows);
+  if (!kByRecord) {
+    row0 = row_base[ch];
+    chunk0 = chunk_base[ch];
+  }
+  a.cursor[(int64_t)ch * a.rep + r] = row0 + (sr - rows);
   const unsigned long long all = a.freq[4 * i + 2];
   const uint32_t n =
       chunk_count((uint32_t)all, chunk_nominal((uint32_t)a.child_blocks, (uint32_t)all, (uint32_t)a.freq[4 * i + 1]));
-  uint2 *tab = a.child_tab + chunk_base[ch];
+  uint2 *tab = a.child_tab + chunk0;
   for (uint32_t k = (uint32_t)r; k < n; k += (uint32_t)a.rep) tab[k] = make_uint2((uint32_t)ch, k);
 }
 
 __global__ void __launch_bounds__(256) k_ccursors(StepArgs a, const int32_t *fchild, const unsigned long long *row_base,
                                                   const uint32_t *chunk_base, int64_t F) {
   if (blockIdx.x == 0) clear_counters(a);
-  cursors_of(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, fchild, row_base, chunk_base, F);
+  cursors_of<true>(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, fchild, row_base, chunk_base, F);
 }
 
 // The children, chosen on the device: a tile of 1,024 records per workgroup,
@@ -961,7 +973,7 @@ __global__ void __launch_bounds__(256) k_cchildren(StepArgs a, CSelect c, CMetaA
   __shared__ ChildLds lds[4];
   if ((int64_t)blockIdx.x < cursor_blocks) {
     if (blockIdx.x == 0) clear_counters(a);
-    cursors_of(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, c.fchild, c.row_base, c.chunk_base, F);
+    cursors_of<false>(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, c.fchild, c.row_base, c.chunk_base, F);
     return;
   }
   const int lane = threadIdx.x & 63;

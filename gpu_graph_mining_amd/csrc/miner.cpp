@@ -1850,7 +1850,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     const size_t meta_all = (size_t)child_stride * C;
     const size_t fc_off = (meta_all + 7) & ~size_t(7);
     const size_t rb_off = (fc_off + sizeof(int32_t) * F + 7) & ~size_t(7);
-    const size_t lb_off = rb_off + sizeof(unsigned long long) * C;
+    const int64_t bases = compact ? F : C;  // (compact: per record, see cursors_of)
+    const size_t lb_off = rb_off + sizeof(unsigned long long) * bases;
     // path masks of the children with >= 2 edges: a forward and a
     // backward word per rightmost-path vertex (at most max_nv of them)
     // (a 2-edge level written in pieces leaves no complete path table, nor
@@ -1860,7 +1861,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     if ((new_len == 1 && !keys_whole) || (new_len == 2 && !(p_begin == 0 && p_end == P && keys_whole))) t2_partial = true;
     const bool masks = prune && !t2_partial && new_len >= 2 && C > 0;
     const int mstride = masks && !compact ? max_nv : 0;  // (compact: the masks are in the metadata)
-    const size_t masks_off = lb_off + sizeof(unsigned long long) * C;
+    const size_t masks_off = lb_off + sizeof(unsigned long long) * bases;
     // then per child its packed code (from | to << 8 | elabel << 16 |
     // tolabel << 24 per tuple) and its vertex labels, for the next level's
     // minimum-code check on the device
@@ -1878,11 +1879,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         const int64_t c = kidx[i];
         hfc[i] = (int32_t)c;
         if (c < 0) continue;
-        hrb[c] = (unsigned long long)run;
+        hrb[compact ? i : c] = (unsigned long long)run;
         N.row0[c] = run;
         run += (int64_t)fr[i].proj;
         if (compact) {
-          hcb[c] = (uint32_t)chunks;
+          hcb[i] = (uint32_t)chunks;
           N.chunk0[c] = chunks;
           chunks += chunk_count((uint32_t)fr[i].proj,
                                 chunk_nominal((uint32_t)child_blocks, (uint32_t)fr[i].proj, (uint32_t)fr[i].sup));
