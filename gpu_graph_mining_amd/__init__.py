@@ -49,6 +49,7 @@ EXPORTED_SYMBOLS = (
     "gm_batch_create", "gm_batch_mine", "gm_batch_destroy", "gm_support_queries", "gm_support_query",
     "gm_db_write", "gm_db_load_part", "gm_mine_noalloc", "gm_dfs_codes_are_min", "gm_batch_create_subsets",
     "gm_patterns_create", "gm_patterns_add", "gm_patterns_add_job", "gm_patterns_get", "gm_patterns_destroy",
+    "gm_db_set_limits", "gm_batch_set_limits",
 )
 
 
@@ -106,6 +107,7 @@ def load_library(path: Optional[os.PathLike] = None) -> C.CDLL:
         "gm_db_counts": (C.c_int, [dbp, P(C.c_int64)]),
         "gm_db_export": (C.c_int, [dbp, i32p, i32p, i32p, i32p, i32p, i32p]),
         "gm_db_upload": (C.c_int, [dbp]),
+        "gm_db_set_limits": (C.c_int, [dbp, C.c_int64, C.c_int64]),
         "gm_db_destroy": (None, [dbp]),
         "gm_mine": (C.c_int, [dbp, C.c_int32, P(gm_cfg), PATTERN_CB, C.c_void_p, P(gm_stats)]),
         "gm_mine_noalloc": (C.c_int, [dbp, C.c_int32, P(gm_cfg), PATTERN_CB, C.c_void_p, P(gm_stats)]),
@@ -122,6 +124,7 @@ def load_library(path: Optional[os.PathLike] = None) -> C.CDLL:
         "gm_batch_create": (C.c_int, [C.c_int32, P(dbp), P(dbp)]),
         "gm_batch_create_subsets": (C.c_int, [dbp, C.c_int32, i32p, i32p, P(dbp)]),
         "gm_batch_mine": (C.c_int, [dbp, i32p, P(gm_cfg), JOB_PATTERN_CB, C.c_void_p, P(gm_stats)]),
+        "gm_batch_set_limits": (C.c_int, [dbp, C.c_int64, C.c_int64]),
         "gm_batch_destroy": (None, [dbp]),
         "gm_patterns_create": (C.c_void_p, []),
         "gm_patterns_get": (C.c_int64, [C.c_void_p, P(i32p), P(i32p), P(i32p), P(P(C.c_uint32)), P(P(C.c_uint64))]),
@@ -457,6 +460,11 @@ class GraphDB:
     def upload(self) -> None:
         _check(load_library().gm_db_upload(self._h))
 
+    def set_limits(self, piece_keys: int = 0, list_units: int = 0) -> None:
+        """Where the level steps on this handle are cut (gm_db_set_limits;
+        0 = the default)."""
+        _check(load_library().gm_db_set_limits(self._h, piece_keys, list_units))
+
     def close(self) -> None:
         if self._h and self._h.value:
             load_library().gm_db_destroy(self._h)
@@ -720,6 +728,10 @@ class Batch:
             cb = JOB_PATTERN_CB() if count_only else lib.add_job_pattern
             _check(lib.gm_batch_mine(self._h, _ptr(ms), C.byref(cfg), cb, listing.user, C.byref(st)))
             return listing.patterns(self.n_jobs), st.as_dict()
+
+    def set_limits(self, piece_keys: int = 0, list_units: int = 0) -> None:
+        """GraphDB.set_limits for the batch."""
+        _check(load_library().gm_batch_set_limits(self._h, piece_keys, list_units))
 
     def close(self) -> None:
         if self._h and self._h.value:

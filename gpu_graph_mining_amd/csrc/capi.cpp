@@ -214,6 +214,16 @@ gm::MineOptions options(const gm_cfg *cfg) {
   return o;
 }
 
+void set_limits(gm::DeviceDB &d, int64_t piece_keys, int64_t list_units) {
+  if (piece_keys < 0 || piece_keys > gm::kPieceKeys) throw gm::Error(GM_E_ARG, "piece_keys must be in [0, 2^26]");
+  if (list_units < 0 || list_units > (1ll << 31)) throw gm::Error(GM_E_ARG, "list_units must be in [0, 2^31]");
+  gm::Limits l;
+  if (piece_keys > 0) l.piece_keys = piece_keys;
+  l.list_units = list_units;
+  std::lock_guard<std::mutex> lock(d.mu);
+  d.limits = l;
+}
+
 }  // namespace
 
 extern "C" {
@@ -345,6 +355,14 @@ int gm_db_upload(gm_db *db) {
   return guard([&]() {
     if (!db) throw gm::Error(GM_E_ARG, "null argument");
     ensure_device(db);
+  });
+}
+
+int gm_db_set_limits(gm_db *db, int64_t piece_keys, int64_t list_units) {
+  return guard([&]() {
+    if (!db) throw gm::Error(GM_E_ARG, "null argument");
+    ensure_device(db);
+    set_limits(*db->dev, piece_keys, list_units);
   });
 }
 
@@ -545,6 +563,13 @@ int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg,
       };
     if (!gm::mine(batch->dev, o, rep, stats, batch->stream))
       throw gm::Error(GM_E_CALLBACK, "callback stopped mining");
+  });
+}
+
+int gm_batch_set_limits(gm_batch *batch, int64_t piece_keys, int64_t list_units) {
+  return guard([&]() {
+    if (!batch) throw gm::Error(GM_E_ARG, "null batch");
+    set_limits(batch->dev, piece_keys, list_units);
   });
 }
 

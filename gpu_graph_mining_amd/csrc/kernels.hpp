@@ -30,10 +30,6 @@ inline int compact_blocks(int64_t rows, int most = kCompactBlocks) {
   while (blocks > 1 && rows / (62 * blocks) < kCompactWaves) blocks /= 2;
   return blocks;
 }
-// Counter keys of one level piece at most (16 bytes per key and replica): a
-// level with more patterns x keys per pattern is mined in pieces.
-constexpr int64_t kPieceKeys = 1ll << 26;
-
 // Statistics counters that every wave bumps are spread over kSpread cache
 // lines: atomics on one address serialise across the device.
 constexpr int kSpread = 64;

@@ -388,6 +388,7 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
                DeviceDB &out, hipStream_t s) {
   if (n_jobs < 1 || begin[0] != 0) throw Error(GM_E_ARG, "job ranges must start at 0");
   out.compact = false;
+  out.limits = Limits();
   const int32_t n_sel = begin[n_jobs];
   std::vector<int32_t> sel(n_sel), dvb(n_sel), dab(n_sel), djob(n_sel);
   std::vector<uint64_t> dgb(src.compact ? n_sel : 0);
@@ -880,6 +881,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
           Workspace *ws) {
   std::lock_guard<std::mutex> lock(db.mu);
   Timer total;
+  const Limits limits = db.limits;
   const int32_t NEL = db.NEL, NVL = db.NVL;
   int threads = opt.canon_threads > 0 ? opt.canon_threads
                                       : (int)std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
@@ -1034,6 +1036,19 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     int32_t meta_stride = 0; // bytes of a pattern's metadata
   };
   std::deque<Frame> frames(1);
+  // A row set for a level's children: one that no level on the stack holds.
+  // The current level's is read by the write; a level cut into pieces waits
+  // below it, also without a budget (limits.piece_keys).
+  auto free_row_set = [&]() {
+    auto held = [&](int b) {
+      for (const Frame &f : frames)
+        if (f.buf == b) return true;
+      return false;
+    };
+    int b = 0;
+    while (held(b)) ++b;
+    return b;
+  };
   // Compact lists are written as they come (4 bytes a candidate), not sized
   // exactly beforehand: seven 8-byte words a row stand for them in the budget
   // (pages of a little over 4 entries a row and a pool of 8).
@@ -1203,10 +1218,10 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       p_end = lo;
     }
     // the counters cover the piece's keys only: (p - p_begin) * K + key,
-    // at most kPieceKeys of them (a level with more is cut into pieces)
-    if (P * K > kPieceKeys) finish_pending();  // (pieces need the patterns' first rows)
+    // at most limits.piece_keys of them (a level with more is cut into pieces)
+    if (P * K > limits.piece_keys) finish_pending();  // (pieces need the patterns' first rows)
     if (stopped) break;
-    p_end = std::min<int64_t>(p_end, p_begin + std::max<int64_t>(1, kPieceKeys / K));
+    p_end = std::min<int64_t>(p_end, p_begin + std::max<int64_t>(1, limits.piece_keys / K));
     const int64_t nkeys = (p_end - p_begin) * K;
     const FastDiv fdK((uint64_t)K), fdNEL((uint64_t)NEL), fdNVL((uint64_t)NVL);
     auto parent_of = [&](uint64_t key) { return (int64_t)fdK.div(key) + p_begin; };
@@ -1249,7 +1264,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     // the pool of further list extents: eight entries a row (the levels
     // measured list 2 to 6), at least 512 units (8,192 entries, more than one
     // source of a block can list) a slice
-    pool_units = std::max<int64_t>(kSpread * 512, (prow_hi - prow_lo) * 8 / kListUnit);
+    pool_units = limits.list_units > 0 ? limits.list_units
+                                       : std::max<int64_t>(kSpread * 512, (prow_hi - prow_lo) * 8 / kListUnit);
     uint32_t fcap = (uint32_t)std::min<int64_t>(std::max<int64_t>(nkeys, 1), std::max<int64_t>(1 << 16, (p_end - p_begin) * 64));
     // the children would pass max_edges: none is kept
     const bool past_max = opt.max_edges > 0 && (root ? 1 : L.len + 1) > opt.max_edges;
@@ -1498,8 +1514,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       st.n_levels++;
       dead_share = (double)dropped / (double)std::max<int64_t>(1, child_rows + dropped);
       if (chunks > INT32_MAX) throw Error(GM_E_OOM, "more than 2^31 chunks of rows");
-      int nxt = 0;
-      while (nxt == cur) ++nxt;
+      const int nxt = free_row_set();
       const size_t codes_off = ((size_t)child_stride * C + 7) & ~size_t(7);
       const size_t cvl_off = (codes_off + sizeof(uint32_t) * new_len * C + 7) & ~size_t(7);
       const size_t key_off = (cvl_off + (size_t)CS * C + 3) & ~size_t(3);
@@ -1916,14 +1931,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       // starts; the children's metadata (the next level's) follows in one
       // upload.
       Timer tdev2;
-      // a row set no level on the stack holds (this one's is read by the write)
-      auto held_by_stack = [&](int b) {
-        for (const Frame &f : frames)
-          if (f.buf == b) return true;
-        return false;
-      };
-      int nxt = 0;
-      while (held_by_stack(nxt)) ++nxt;
+      const int nxt = free_row_set();
       if (w.arena && nxt > 1) throw Error(GM_E_DEVICE, "internal: row set beyond the static workspace's two");
       child_buf = nxt;
       PatMeta *hm = reinterpret_cast<PatMeta *>(hu);  // narrow layout (else hmw)

@@ -167,6 +167,17 @@ struct Workspace {
   }
 };
 
+// Counter keys of one level piece at most (16 bytes per key and replica): a
+// level with more patterns x keys per pattern is mined in pieces.
+constexpr int64_t kPieceKeys = 1ll << 26;
+
+// Where the level steps on a database stop working on a whole level at once
+// (gm_db_set_limits).
+struct Limits {
+  int64_t piece_keys = kPieceKeys;
+  int64_t list_units = 0;  // compact: the list pool of a level's first try (0: by its rows)
+};
+
 // The packed database of device.hpp on the GPU, for one or more jobs.
 struct DeviceDB {
   int32_t n_graphs = 0, n_jobs = 1;
@@ -186,6 +197,7 @@ struct DeviceDB {
   DevBuf vgrp, rrows, rtab, dggb;
   DevBuf gidx;  // a gathered database's index arrays
   size_t bytes = 0;
+  Limits limits;
   size_t held() const {  // device and pinned bytes, the workspace's included
     size_t n = ws ? ws->held() : 0;
     for (const DevBuf *b : {&gvbase, &vadj, &adj, &vlab, &gjob, &vgraph, &vgrp, &rrows, &rtab, &dggb, &gidx}) n += b->cap;

@@ -176,6 +176,18 @@ int gm_db_export(const gm_db *db, int32_t *graph_vbegin, int32_t *vlabels, int32
  * (src/globals/cuda_graph_types.cpp:130-153). */
 int gm_db_upload(gm_db *db);
 
+/* Limits of the level steps on this handle (they change how a run is cut, not
+ * what it finds; tests lower them to cut small databases):
+ *   piece_keys  counter keys of a level step at most, 16 bytes each and per
+ *               replica; a level of more patterns x keys per pattern is mined
+ *               in pieces (1 to 2^26; 0 = the default, 2^26)
+ *   list_units  compact databases: units of 64 bytes of the candidate lists'
+ *               common pool when a level's lists are first written; a level
+ *               that needs more writes them again into a larger one (0 = the
+ *               default, by the level's rows)
+ * Makes the device copy if there is none.  GM_E_ARG outside the ranges. */
+int gm_db_set_limits(gm_db *db, int64_t piece_keys, int64_t list_units);
+
 /* Release host and device memory.  Replaces
  * gspan_cuda::delete_database_from_device (src/gspan_cuda/gspan_cuda.hpp:286)
  * and the destructor (gspan_cuda.cpp:52-64). */
@@ -234,6 +246,8 @@ int gm_batch_create_subsets(gm_db *db, int32_t n_jobs, const int32_t *job_begin,
  * identical per-job results to gm_mine on each database. */
 int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg, gm_job_pattern_cb cb, void *user,
                   gm_stats *stats);
+/* gm_db_set_limits for a batch. */
+int gm_batch_set_limits(gm_batch *batch, int64_t piece_keys, int64_t list_units);
 void gm_batch_destroy(gm_batch *batch);
 
 /* A sink that keeps the patterns: pass gm_patterns_add (or gm_patterns_add_job)

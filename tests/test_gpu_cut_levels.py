@@ -1,0 +1,80 @@
+"""Levels cut into pieces without a memory budget (more counter keys than a
+level step takes, GraphDB.set_limits), on compact databases: a piece's
+children, chosen on the device, and their children are mined while the cut
+level's rows wait for its next piece.  Patterns, supports, |Proj(P)|, E_child
+and E_cand are the oracle's, for one database and for the jobs of a batch."""
+import re
+
+import pytest
+
+import gpu_graph_mining_amd as gm
+from oracle import py_oracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+def _key(pats):
+    return sorted((po.normalize(c), s, n) for c, s, n in pats)
+
+
+def _chosen_under_a_cut_level(trace):
+    """Levels whose children the device chose while an earlier level had
+    pieces to come."""
+    cut, n = set(), 0
+    for line in trace.splitlines():
+        level = int(re.search(r"^\[gm level (\d+)\]", line)[1])
+        cut = {x for x in cut if x < level}
+        piece = re.search(r"piece \d+-(\d+) of (\d+)", line)
+        if piece and int(piece[1]) < int(piece[2]):
+            cut.add(level)
+        elif not piece and cut and int(re.search(r"children (\d+)", line)[1]):
+            n += 1
+    return n
+
+
+@pytest.fixture
+def trace(monkeypatch, capfd):
+    monkeypatch.setenv("GM_LEVEL_TRACE", "1")
+
+    def read():
+        return capfd.readouterr().err
+
+    return read
+
+
+@pytest.mark.parametrize("piece_keys", [8000, 16000, 64000])
+def test_a_cut_level_keeps_its_rows(trace, piece_keys):
+    db = gm.GraphDB.molecule(3, 100)
+    opats, ost = po.mine_arrays(db.arrays(), 4, max_edges=8)
+    db.set_limits(piece_keys=piece_keys)
+    trace()
+    pats, st = gm.mine(db, 4, max_edges=8, collect_proj=True)
+    assert _chosen_under_a_cut_level(trace()) > 0
+    assert _key(pats) == _key(opats)
+    assert (st["e_child"], st["e_cand"]) == (ost["e_child"], ost["e_cand"])
+
+
+def test_a_cut_level_of_a_batch_keeps_its_rows(trace):
+    db = gm.GraphDB.molecule(3, 100)
+    jobs = [(list(range(100)), 8), (list(range(1, 100, 2)), 5), (list(range(30)), 6)]
+    batch = gm.Batch.from_subsets(db, [ids for ids, _ in jobs])
+    batch.set_limits(piece_keys=16000)
+    trace()
+    res, _ = batch.mine([minsup for _, minsup in jobs], collect_proj=True)
+    assert _chosen_under_a_cut_level(trace()) > 0
+    for (ids, minsup), pats in zip(jobs, res):
+        assert _key(pats) == _key(po.mine_arrays(db.subset(ids).arrays(), minsup)[0])
+    batch.close()
+    # a batch that takes over the buffers has the default limits again
+    batch = gm.Batch.from_subsets(db, [ids for ids, _ in jobs])
+    assert [_key(pats) for pats in batch.mine([minsup for _, minsup in jobs], collect_proj=True)[0]] == [_key(p) for p in res]
+    assert not re.search(r"piece 0-(?!(\d+) of \1 )", trace())
+    batch.close()
+
+
+@pytest.mark.parametrize("limits", [(-1, 0), ((1 << 26) + 1, 0), (0, -1)])
+def test_limits_outside_their_range_are_refused(limits):
+    db = gm.GraphDB.molecule(3, 5)
+    with pytest.raises(gm.GMError) as e:
+        db.set_limits(*limits)
+    assert e.value.code == gm.GM_E_ARG
