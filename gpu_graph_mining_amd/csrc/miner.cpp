@@ -2148,6 +2148,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         Pool::get().run(F, threads, build_child, 4096);
         if (new_len == 2) {
           build_t2(N);
+          dev_t2 = false;  // the device's, if any, is an earlier root piece's
         }
         if (t2_ready) Pool::get().run(C, threads, mask_child, 4096);
       }

@@ -3,12 +3,15 @@ level step takes, GraphDB.set_limits), on compact databases: a piece's
 children, chosen on the device, and their children are mined while the cut
 level's rows wait for its next piece.  Patterns, supports, |Proj(P)|, E_child
 and E_cand are the oracle's, for one database and for the jobs of a batch."""
+import random
 import re
 
 import pytest
 
 import gpu_graph_mining_amd as gm
 from oracle import py_oracle as po
+
+from test_gpu_compact import all_labels, tree
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +81,27 @@ def test_limits_outside_their_range_are_refused(limits):
     with pytest.raises(gm.GMError) as e:
         db.set_limits(*limits)
     assert e.value.code == gm.GM_E_ARG
+
+
+def test_the_path_table_is_the_root_pieces_own(trace):
+    """A root level cut by jobs: the first piece's 2-edge level is chosen on the
+    device, the second piece's (few edges) on the host and its 3-edge level on
+    the device again, which takes the second piece's 2-edge paths."""
+    rng = random.Random(5)
+    rich = [gm.GraphDB.from_graphs([all_labels(3, 2)] + [tree(rng, 16, 3, 2, 2) for _ in range(12)]) for _ in range(7)]
+    single = gm.GraphDB.from_graphs([([0, 0], [(0, 1, 0)])])
+    # 18 root keys a job: 222 jobs in the first piece
+    dbs = rich[:6] + [single] * 220 + rich[6:]
+    minsups = [4] * 6 + [2] * 220 + [2]
+    batch = gm.Batch(dbs)
+    batch.set_limits(piece_keys=4000)
+    trace()
+    res, _ = batch.mine(minsups, collect_proj=True)
+    lines = trace().splitlines()
+    second = [i for i, line in enumerate(lines) if line.startswith("[gm level 0]")][1]
+    assert any(line.startswith("[gm level 1] device-chosen") for line in lines[:second])
+    assert lines[second + 1].startswith("[gm level 1] piece")
+    assert lines[second + 2].startswith("[gm level 2] device-chosen")
+    for i, (db, minsup, pats) in enumerate(zip(dbs, minsups, res)):
+        assert _key(pats) == (_key(po.mine_arrays(db.arrays(), minsup)[0]) if db is not single else []), i
+    batch.close()
