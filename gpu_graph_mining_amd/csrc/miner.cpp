@@ -1049,16 +1049,24 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     while (held(b)) ++b;
     return b;
   };
-  // Compact lists are written as they come (4 bytes a candidate), not sized
-  // exactly beforehand: seven 8-byte words a row stand for them in the budget
-  // (pages of a little over 4 entries a row and a pool of 8).
-  auto compact_words = [](uint64_t rows) { return std::max<uint64_t>(1, 7 * rows); };
-  frames.back().list_cap =
-      compact ? compact_words((uint64_t)db.n_vertices) : (uint64_t)std::max<int64_t>(db.n_adj, 1);  // root lists: 2E
+  // (compact lists are written as they come: a page a chunk and a pool, see list_units)
+  frames.back().list_cap = compact ? 1 : (uint64_t)std::max<int64_t>(db.n_adj, 1);  // root lists: 2E
   const int64_t budget = w.arena ? 0 : opt.mem_budget;
   double piece_bytes_per_row = 0;  // child bytes per parent row of the last piece (estimate)
   // device bytes a level's rows take (rows with their counts) and a list entry
   auto rows_bytes = [&](int64_t rows, int S_) { return (int64_t)rows * ((compact ? 4 : 22) + S_); };
+  // Compact lists of a piece of `chunks` chunks and `rows` rows, in units: a
+  // page of 256 entries a block for every chunk, records included, and a pool
+  // of further extents, eight entries a row (the levels measured list 2 to 6).
+  // The pool has at least 512 units (8,192 entries, more than one source of a
+  // block can list) a slice; under a budget an eighth of it, but not below 64
+  // units a slice (what those do not hold is written again into a larger one).
+  const int64_t pool_least =
+      budget > 0 ? std::min<int64_t>(kSpread * 512, std::max<int64_t>(kSpread * 64, budget / 8 / (4 * kListUnit))) : kSpread * 512;
+  auto pool_for = [&](int64_t rows) {
+    return limits.list_units > 0 ? limits.list_units : std::max<int64_t>(pool_least, rows * 8 / kListUnit);
+  };
+  auto list_units = [&](int64_t chunks, uint32_t page, int64_t rows) { return chunks * (int64_t)(page / kListUnit) + pool_for(rows); };
   int64_t pool_units = 0;  // compact: list pool of the level step (grown when a level overflows it)
   // compact: blocks of a chunk
   auto blocks_for = [&](int64_t rows) {
@@ -1183,14 +1191,15 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     int64_t p_end = P;
     const int64_t p_end_measured = Fr.p_end_next;
     Fr.p_end_next = 0;
+    const uint32_t page = 256u * (uint32_t)(root ? compact_blocks(db.n_vertices) : Fr.blocks);  // compact: list entries a chunk
     int64_t held = 0;  // rows of the levels on the stack, and this level's lists
     for (const Frame &f : frames) held += rows_bytes(f.n_rows, f.S);
     if (!compact) held += (int64_t)list_cap * 8;
-    // Compact lists are the piece's alone (56 bytes a row of it, in one buffer
-    // that every piece uses): of what the rows on the stack leave, the
-    // children's rows get a fifth and the piece's lists the rest.  The share
-    // is small because the children need 56 bytes in turn for each 8 to 20 of
-    // their own; it measured best of 0.08-0.4 over five databases and budgets
+    // Compact lists are the piece's alone (some 50 bytes a row of it, 1,024 and
+    // more a pattern of few rows, in one buffer that every piece uses): of what
+    // the rows on the stack leave, the children's rows get a fifth and the
+    // piece's lists the rest.  The share is small because the children need
+    // those lists in turn for each 8 to 20 bytes of their own; it measured best of 0.08-0.4 over five databases and budgets
     // (30,000 transactions under 64 MiB: 3.8 ms at 0.08, 2.4 at 0.2, 2.9 at
     // 0.4).  With the whole level's lists and the children's counted at once
     // it took 64 level steps and 4.2 ms, now 36 steps.
@@ -1205,12 +1214,18 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     } else if (p_end_measured > 0) {
       p_end = p_end_measured;
     } else if (budget > 0 && (compact || piece_bytes_per_row > 0)) {
-      double rows_fit = piece_bytes_per_row > 0 ? std::max(0.0, (double)avail / piece_bytes_per_row) : 1e18;
-      if (compact) rows_fit = std::min(rows_fit, (double)(free_now - avail) / (8.0 * (double)compact_words(1)));
+      const double rows_fit = piece_bytes_per_row > 0 ? std::max(0.0, (double)avail / piece_bytes_per_row) : 1e18;
+      const std::vector<int64_t> &root0 = db.root_chunk0;
+      auto fits = [&](int64_t end) {
+        const int64_t rows = prow(end) - prow(p_begin);
+        if ((double)rows > rows_fit) return false;
+        const int64_t chunks = !compact ? 0 : root ? root0[end] - root0[p_begin] : L.chunk0[end] - L.chunk0[p_begin];
+        return !compact || list_units(chunks, page, rows) * 4 * kListUnit <= free_now - avail;
+      };
       int64_t lo = p_begin + 1, hi = P;  // the last p_end whose rows fit, at least p_begin + 1
       while (lo < hi) {
         const int64_t mid = (lo + hi + 1) / 2;
-        if ((double)(prow(mid) - prow(p_begin)) <= rows_fit)
+        if (fits(mid))
           lo = mid;
         else
           hi = mid - 1;
@@ -1243,14 +1258,15 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     // on one address serialise at ~100 ns each); up to 64 MB of them
     // (one replica in the static workspace of the entry point that
     // allocates nothing)
+    // (compact chunks are of one pattern: under a budget the replicas follow
+    // the rows, or patterns of few rows would hold most in counters: 28 MB
+    // beside 5 MB of lists for 3,000 patterns of 6 rows)
+    const int64_t shared = budget > 0 ? std::min(total_chunks, (prow_hi - prow_lo) / 64) : total_chunks;
     int rep = 1;
-    while (!w.arena && rep < 64 && (int64_t)rep * 2 * nkeys * 16 <= (64ll << 20) && (int64_t)rep * 2 * 32 <= total_chunks)
-      rep *= 2;
+    while (!w.arena && rep < 64 && (int64_t)rep * 2 * nkeys * 16 <= (64ll << 20) && (int64_t)rep * 2 * 32 <= shared) rep *= 2;
     grow(w.sup, sizeof(int32_t) * std::max<int64_t>(nkeys, 1), s);
     grow(w.tiles, sizeof(uint32_t) * kReduceTiles, s);
     grow_zero(w.acc, sizeof(unsigned long long) * std::max<int64_t>(nkeys * rep, 1), s);
-    // compact: a page of 256 list entries per 64 nominal rows, records included
-    const uint32_t page = 256u * (uint32_t)(root ? compact_blocks(db.n_vertices) : Fr.blocks);
     if (compact) {
       grow(w.chunks, sizeof(CChunk) * std::max<int64_t>(total_chunks, 1), s);
     } else {
@@ -1261,11 +1277,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       grow(w.rccnt, sizeof(uint16_t) * std::max<int64_t>(rows_now, 1), s);
       grow(w.cand, sizeof(uint2) * std::max<uint64_t>(list_cap, 1), s);
     }
-    // the pool of further list extents: eight entries a row (the levels
-    // measured list 2 to 6), at least 512 units (8,192 entries, more than one
-    // source of a block can list) a slice
-    pool_units = limits.list_units > 0 ? limits.list_units
-                                       : std::max<int64_t>(kSpread * 512, (prow_hi - prow_lo) * 8 / kListUnit);
+    pool_units = pool_for(prow_hi - prow_lo);
     uint32_t fcap = (uint32_t)std::min<int64_t>(std::max<int64_t>(nkeys, 1), std::max<int64_t>(1 << 16, (p_end - p_begin) * 64));
     // the children would pass max_edges: none is kept
     const bool past_max = opt.max_edges > 0 && (root ? 1 : L.len + 1) > opt.max_edges;
@@ -1603,7 +1615,6 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         cf.buf = nxt;
         cf.S = CS;
         cf.n_rows = child_rows;
-        cf.list_cap = compact_words((uint64_t)child_rows);
         cf.blocks = pend.blocks;
         cf.meta_stride = child_stride;
         cf.code_off = codes_off;
@@ -1912,7 +1923,6 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       }
       N.row0[C] = run;
       N.chunk0[C] = chunks;
-      if (compact) child_items = compact_words((uint64_t)child_rows);
       if (chunks > INT32_MAX) throw Error(GM_E_OOM, "more than 2^31 chunks of rows");
     }
     if (F > 0) stage_up(w, w.up, fc_off, masks_off - fc_off, s);  // child ids, bases

@@ -65,3 +65,21 @@ def test_negative_budget_is_rejected():
     db, _ = wl.config0(n_graphs=20)
     with pytest.raises(gm.GMError):
         gm.mine(db, 5, mem_budget=-1)
+
+
+@pytest.mark.parametrize("budget", [1 << 20, 2 << 20, 4 << 20])
+def test_budget_covers_patterns_of_few_rows(budget):
+    """Thousands of patterns of a few embeddings each, where a pattern's
+    candidate lists (1 KiB at least) weigh more than its rows: the run's peak
+    stays near the budget.  Beside the rows and lists (with the buffers' growth
+    by half, 1.5 budgets) it holds the database (under 1 MiB), the frequent-key
+    list (2 MiB, or 2 KiB a pattern and so twice the lists), the counters of
+    one replica (72 keys of 8 bytes a pattern, half of the lists) and the
+    children's upload (under 1 KiB a pattern)."""
+    db = gm.GraphDB.random(7, 400, 10, 30, 1.2, 5, 3)
+    full, s0 = gm.mine(db, 4, collect_proj=True, max_edges=4)
+    db = gm.GraphDB.random(7, 400, 10, 30, 1.2, 5, 3)  # (a new workspace)
+    part, sb = gm.mine(db, 4, collect_proj=True, max_edges=4, mem_budget=budget)
+    assert _key(part) == _key(full) and all(sb[k] == s0[k] for k in ("n_patterns", "e_child", "e_root", "e_cand"))
+    print("peak", sb["peak_device_bytes"], "levels", sb["n_levels"], flush=True)
+    assert sb["peak_device_bytes"] <= 3 * (1 << 20) + 6 * budget
