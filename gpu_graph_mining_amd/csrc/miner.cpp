@@ -71,6 +71,20 @@ void *Arena::take(int side, size_t bytes) {
   return base + at;
 }
 
+namespace {
+
+// An allocation that fails for want of memory is tried again when subset
+// batches kept for later (device and pinned memory) could be freed.
+template <class Take>
+hipError_t take_or_release(Take &&take) {
+  const hipError_t e = take();
+  if (e != hipErrorOutOfMemory || !release_spares()) return e;
+  (void)hipGetLastError();
+  return take();
+}
+
+}  // namespace
+
 void DevBuf::release() {
   if (p && !arena) (void)hipFree(p);
   p = nullptr;
@@ -87,12 +101,7 @@ void *DevBuf::ensure(size_t bytes) {
   }
   const size_t want = (std::max<size_t>({bytes, cap + cap / 2, 256}) + 255) & ~size_t(255);  // fills take 8-byte words
   release();
-  hipError_t e = hipMalloc(&p, want);
-  if (e == hipErrorOutOfMemory && release_spares()) {
-    (void)hipGetLastError();
-    e = hipMalloc(&p, want);
-  }
-  hip_check(e, "hipMalloc");
+  hip_check(take_or_release([&]() { return hipMalloc(&p, want); }), "hipMalloc");
   cap = want;
   return p;
 }
@@ -115,7 +124,8 @@ void *HostBuf::ensure(size_t bytes) {
   p = nullptr;
   dev = nullptr;
   cap = 0;
-  hip_check(hipHostMalloc(&p, want, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
+  hip_check(take_or_release([&]() { return hipHostMalloc(&p, want, hipHostMallocMapped | hipHostMallocCoherent); }),
+            "hipHostMalloc");
   cap = want;
   hip_check(hipHostGetDevicePointer(&dev, p, 0), "hipHostGetDevicePointer");
   return p;

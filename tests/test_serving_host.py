@@ -1,10 +1,16 @@
 """Admission control of the serving loop, host side (no GPU): the memory
 gate admits a batch while the running estimates fit the budget (any batch
 on an idle device), and the estimator follows measured bytes per unit."""
+import subprocess
 import threading
 import time
+from pathlib import Path
 
+import gpu_graph_mining_amd as gm
+from gpu_graph_mining_amd import build as gbuild
 from gpu_graph_mining_amd import serving
+
+ROOT = Path(__file__).resolve().parent.parent
 
 
 def test_gate_admits_within_budget_and_waits_for_memory():
@@ -54,3 +60,74 @@ def test_estimator_follows_measurements():
     assert abs(e.per_unit - 64.0) < 1.0
     e.observe(0, 5)                            # nothing measured: unchanged
     assert abs(e.per_unit - 64.0) < 1.0
+
+
+def test_failed_allocations_free_the_kept_batches_and_try_again(tmp_path):
+    """Device and pinned buffers alike: an allocation that fails for want of
+    memory frees what is kept for later subset batches and is tried once more;
+    any other failure, or nothing kept, is the caller's error.  (No GPU: the
+    program's own allocators stand before the runtime's.)"""
+    src = tmp_path / "alloc.cpp"
+    src.write_text('''#include <cstdio>
+#include <cstdlib>
+#include "miner.hpp"
+static int fails, calls, freed;
+static bool kept;
+static hipError_t error;
+static hipError_t take(void **p, size_t n) {
+  ++calls;
+  if (fails-- > 0) return error;
+  *p = std::malloc(n);
+  return hipSuccess;
+}
+bool gm::release_spares() {
+  ++freed;
+  return kept;
+}
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n); }
+hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
+hipError_t hipHostFree(void *p) { std::free(p); return hipSuccess; }
+hipError_t hipHostGetDevicePointer(void **d, void *p, unsigned) { *d = p; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+}
+template <class Buf>
+void run(const char *name) {
+  for (int f = 0; f < 3; ++f)
+    for (int k = 0; k < 2; ++k)
+      for (hipError_t e : {hipErrorOutOfMemory, hipErrorInvalidValue}) {
+        fails = f;
+        kept = k;
+        error = e;
+        calls = freed = 0;
+        int code = 0;
+        Buf b;
+        try {
+          b.ensure(100);
+        } catch (const gm::Error &x) {
+          code = x.code;
+        }
+        std::printf("%s %d %d %d : %d %d %d\\n", name, f, k, (int)(e == hipErrorOutOfMemory), calls, freed, code);
+      }
+}
+int main() {
+  run<gm::DevBuf>("dev");
+  run<gm::HostBuf>("host");
+}
+''')
+    exe = tmp_path / "alloc"
+    subprocess.run(["g++", "-std=c++17", "-rdynamic", "-D__HIP_PLATFORM_AMD__", f"-I{ROOT / 'include'}",
+                    f"-I{ROOT / 'gpu_graph_mining_amd' / 'csrc'}", "-I/opt/rocm/include", str(src), f"-L{gbuild.LIB_DIR}",
+                    "-lgspan_amd", f"-Wl,-rpath,{gbuild.LIB_DIR}", "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True, timeout=60).stdout.split("\n")
+    want = []
+    for name in ("dev", "host"):
+        for fails in range(3):
+            for kept in range(2):
+                for oom in (1, 0):
+                    again = fails > 0 and oom and kept
+                    calls = 2 if again else 1
+                    code = 0 if fails < calls else gm.GM_E_OOM if oom else gm.GM_E_DEVICE
+                    want.append(f"{name} {fails} {kept} {oom} : {calls} {int(fails > 0 and oom)} {code}")
+    assert out[:-1] == want
