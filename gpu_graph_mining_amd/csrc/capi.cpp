@@ -65,6 +65,7 @@ std::unique_ptr<gm_batch> Spares::take(int device) {
     if (kept[i]->device == device) {
       b = std::move(kept[i]);
       kept.erase(kept.begin() + (std::ptrdiff_t)i);
+      if (b->dev.ws) b->dev.ws->taken_over();
     }
   return b;
 }

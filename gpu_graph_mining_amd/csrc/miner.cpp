@@ -92,6 +92,9 @@ void DevBuf::release() {
 }
 
 void *DevBuf::ensure(size_t bytes) {
+  // (fills take 8-byte words)
+  auto grown = [&](size_t from) { return (std::max<size_t>({bytes, from + from / 2, 256}) + 255) & ~size_t(255); };
+  if (bytes > asked || asked == 0) asked = grown(asked);
   if (bytes <= cap && p) return p;
   if (arena) {  // exact sizes (whole 256-byte blocks); the stacks are emptied level by level
     release();
@@ -99,7 +102,7 @@ void *DevBuf::ensure(size_t bytes) {
     p = arena->take(side, cap);
     return p;
   }
-  const size_t want = (std::max<size_t>({bytes, cap + cap / 2, 256}) + 255) & ~size_t(255);  // fills take 8-byte words
+  const size_t want = grown(cap);
   release();
   hip_check(take_or_release([&]() { return hipMalloc(&p, want); }), "hipMalloc");
   cap = want;
@@ -829,7 +832,7 @@ static_assert(sizeof(Counters) == 8 * kCounterWords, "counter block layout");
 // Grow a workspace buffer; the stream is drained first because the old
 // allocation may still be in use by queued kernels.
 void *grow(DevBuf &b, size_t bytes, hipStream_t s) {
-  if (bytes <= b.cap && b.p) return b.p;
+  if (bytes <= b.cap && b.p) return b.ensure(bytes);
   // (arena regions are only reused by work queued later on the stream)
   if (!b.arena) hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
   return b.ensure(bytes);
@@ -839,8 +842,9 @@ void *grow(DevBuf &b, size_t bytes, hipStream_t s) {
 // of the buffer); a fill kernel, not hipMemsetAsync (which graph capture
 // does not replay reliably).
 void grow_zero(DevBuf &b, size_t bytes, hipStream_t s) {
-  if (bytes <= b.cap && b.p) return;
+  const bool held = bytes <= b.cap && b.p;
   grow(b, bytes, s);
+  if (held) return;
   hip_check(launch_fill8(b.p, b.cap, s), "clear counters");
 }
 
@@ -1591,9 +1595,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         written_pending = true;
       }
       dev_sec += tdev.sec();
-      size_t live = db.bytes + w.sup.cap + w.tiles.cap + w.acc.cap + w.freq.cap + w.cand.cap + w.chunks.cap +
-                    w.cursor.cap + w.sel.cap + w.t2.cap + w.sup2.cap;
-      for (const RowSet &rs : w.rows) live += rs.bytes();
+      size_t live = db.bytes + w.sup.asked + w.tiles.asked + w.acc.asked + w.freq.asked + w.cand.asked + w.chunks.asked +
+                    w.cursor.asked + w.sel.asked + w.t2.asked + w.sup2.asked;
+      for (const RowSet &rs : w.rows) live += rs.asked();
       peak = std::max(peak, live);
       if (trace_levels)
         fprintf(stderr,
@@ -1633,6 +1637,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         if (siblings && !root) {  // the choice's support table and keys, for the next one
           std::swap(w.sup.p, w.sup2.p);
           std::swap(w.sup.cap, w.sup2.cap);
+          std::swap(w.sup.asked, w.sup2.asked);
           cf.key_off = key_off;
           cf.pK = (uint32_t)K;
           cf.pS = S;
@@ -2214,9 +2219,10 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       }
       us_overlap = t_over.sec() * 1e6;
       dev_sec += tdev2.sec();
-      size_t live = db.bytes + w.sup.cap + w.tiles.cap + w.acc.cap + w.accb.cap + w.freq.cap + w.rccnt.cap + w.cand.cap +
-                    w.chunks.cap + w.fail.cap + w.cur_rows.cap + w.cur_list.cap + w.cursor.cap + w.chunk_keys.cap;
-      for (const RowSet &rs : w.rows) live += rs.bytes();
+      size_t live = db.bytes + w.sup.asked + w.tiles.asked + w.acc.asked + w.accb.asked + w.freq.asked + w.rccnt.asked +
+                    w.cand.asked + w.chunks.asked + w.fail.asked + w.cur_rows.asked + w.cur_list.asked + w.cursor.asked +
+                    w.chunk_keys.asked;
+      for (const RowSet &rs : w.rows) live += rs.asked();
       peak = std::max(peak, live);
       child_mask_off = masks_off;
       child_code_off = codes_off;

@@ -49,6 +49,7 @@ struct Arena {
 struct DevBuf {
   void *p = nullptr;
   size_t cap = 0;
+  size_t asked = 0;  // what cap would be had the owner started without memory (Workspace::taken_over)
   Arena *arena = nullptr;
   int side = -1;
   DevBuf() = default;
@@ -87,6 +88,9 @@ struct RowSet {
   DevBuf ctab;  // compact levels: the chunk table (their rows, {graph, tuple}, are in vt)
   std::vector<DevBuf *> bufs() { return {&pid, &rgraph, &vt, &rbound, &rlist, &upl, &ctab}; }
   size_t bytes() const { return pid.cap + rgraph.cap + vt.cap + rbound.cap + rlist.cap + upl.cap + ctab.cap; }
+  size_t asked() const {
+    return pid.asked + rgraph.asked + vt.asked + rbound.asked + rlist.asked + upl.asked + ctab.asked;
+  }
 };
 
 // Device buffers of the level steps, kept across mining calls on one
@@ -158,6 +162,14 @@ struct Workspace {
     for (DevBuf *b : scratch_bufs()) n += b->cap;
     for (RowSet &r : rows) n += r.bytes();
     return n;
+  }
+  // Another owner takes the buffers over: peak_device_bytes counts what its
+  // calls ask for, not what they find.
+  void taken_over() {
+    for (DevBuf *b : scratch_bufs()) b->asked = 0;
+    for (DevBuf *b : {&minsup, &sel, &t2, &sup2}) b->asked = 0;
+    for (RowSet &r : rows)
+      for (DevBuf *b : r.bufs()) b->asked = 0;
   }
   ~Workspace() {
     for (hipEvent_t e : ev)

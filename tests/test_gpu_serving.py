@@ -105,3 +105,28 @@ def test_served_results_equal_alone_on_the_full_database():
         print("request", r.rid, r.kind, flush=True)
         assert r.result == serving.run_alone(db, r)
     assert out["bytes_per_unit"][serving.QUERY] > 0 and out["bytes_per_unit"][serving.MINING] > 0
+
+
+@pytest.mark.parametrize("vlabels,minsups,least", [(5, [8, 4, 8], 20), (90, [2, 3, 2], 2)])  # compact and general kernels
+def test_a_taken_over_batch_reports_its_own_memory(vlabels, minsups, least):
+    """A small subset mined after a large one reports the peaks, call by call,
+    that it has on a database that mined nothing before."""
+
+    def fresh():
+        db = gm.GraphDB.random(3, 400, 5, 9, 1.2, vlabels, 2)
+        db.upload()
+        return db
+
+    def peaks(db, ids, minsups):
+        batch = gm.Batch.from_subsets(db, [ids])
+        got = [batch.mine([m])[1]["peak_device_bytes"] for m in minsups]
+        batch.close()
+        return got
+
+    small, large = list(range(60)), list(range(400))
+    want = peaks(fresh(), small, minsups)
+    db = fresh()
+    first = peaks(db, large, [least])
+    assert first[0] > want[0]
+    assert peaks(db, small, minsups) == want
+    assert peaks(db, large, [least]) == first
