@@ -49,7 +49,7 @@ EXPORTED_SYMBOLS = (
     "gm_batch_create", "gm_batch_mine", "gm_batch_destroy", "gm_support_queries", "gm_support_query",
     "gm_db_write", "gm_db_load_part", "gm_mine_noalloc", "gm_dfs_codes_are_min", "gm_batch_create_subsets",
     "gm_patterns_create", "gm_patterns_add", "gm_patterns_add_job", "gm_patterns_get", "gm_patterns_destroy",
-    "gm_db_set_limits", "gm_batch_set_limits",
+    "gm_db_set_limits", "gm_batch_set_limits", "gm_db_spare_limit",
 )
 
 
@@ -125,6 +125,7 @@ def load_library(path: Optional[os.PathLike] = None) -> C.CDLL:
         "gm_batch_create_subsets": (C.c_int, [dbp, C.c_int32, i32p, i32p, P(dbp)]),
         "gm_batch_mine": (C.c_int, [dbp, i32p, P(gm_cfg), JOB_PATTERN_CB, C.c_void_p, P(gm_stats)]),
         "gm_batch_set_limits": (C.c_int, [dbp, C.c_int64, C.c_int64]),
+        "gm_db_spare_limit": (C.c_int, [dbp, C.c_int64]),
         "gm_batch_destroy": (None, [dbp]),
         "gm_patterns_create": (C.c_void_p, []),
         "gm_patterns_get": (C.c_int64, [C.c_void_p, P(i32p), P(i32p), P(i32p), P(P(C.c_uint32)), P(P(C.c_uint64))]),
@@ -464,6 +465,12 @@ class GraphDB:
         """Where the level steps on this handle are cut (gm_db_set_limits;
         0 = the default)."""
         _check(load_library().gm_db_set_limits(self._h, piece_keys, list_units))
+
+    def spare_limit(self, n_bytes: int = -1) -> None:
+        """Bytes up to which a closed Batch.from_subsets() of this database
+        is kept for the next one (gm_db_spare_limit; 0: none is kept; < 0: the
+        default, 1 GiB)."""
+        _check(load_library().gm_db_spare_limit(self._h, n_bytes))
 
     def close(self) -> None:
         if self._h and self._h.value:

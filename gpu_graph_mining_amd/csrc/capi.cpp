@@ -23,17 +23,20 @@
 // resident database: their buffers, workspace and stream.  A mining request
 // on 5,000 molecules made and freed some 70 of them, 6.5 of its 8.7 ms; with
 // them kept it takes 1.8 ms.  At most kSpares batches of at most
-// kSpareBytes each, all freed with the database or when an allocation fails.
+// kSpareBytes (gm_db_spare_limit) each, all freed with the database or when an
+// allocation fails.
 constexpr size_t kSpares = 2;
 constexpr size_t kSpareBytes = 1ull << 30;
 struct Spares {
   std::mutex mu;
   bool closed = false;  // the database is gone
+  size_t limit = kSpareBytes;
   std::vector<std::unique_ptr<gm_batch>> kept;
   Spares() { kept.reserve(kSpares); }
   std::unique_ptr<gm_batch> take(int device);
   void give(std::unique_ptr<gm_batch> b);  // keeps it or frees it
   bool release(bool close);                // frees what is kept
+  void set_limit(size_t bytes);            // and frees what is over it
 };
 
 struct gm_db {
@@ -74,9 +77,20 @@ void Spares::give(std::unique_ptr<gm_batch> b) {
   // A call that did not end normally may have left work on the stream (and
   // counters that are not zero).
   const bool idle = !b->dev.ws || b->dev.ws->acc_zero;
-  if (!idle || b->dev.held() > kSpareBytes) return;
+  const size_t held = b->dev.held();
   std::lock_guard<std::mutex> lock(mu);
-  if (!closed && kept.size() < kSpares) kept.push_back(std::move(b));
+  if (idle && limit > 0 && held <= limit && !closed && kept.size() < kSpares) kept.push_back(std::move(b));
+}
+
+void Spares::set_limit(size_t bytes) {
+  std::vector<std::unique_ptr<gm_batch>> gone;
+  std::lock_guard<std::mutex> lock(mu);
+  limit = bytes;
+  for (size_t i = kept.size(); i-- > 0;)
+    if (kept[i]->dev.held() > limit || limit == 0) {
+      gone.push_back(std::move(kept[i]));
+      kept.erase(kept.begin() + (std::ptrdiff_t)i);
+    }
 }
 
 bool Spares::release(bool close) {
@@ -564,6 +578,13 @@ int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg,
       };
     if (!gm::mine(batch->dev, o, rep, stats, batch->stream))
       throw gm::Error(GM_E_CALLBACK, "callback stopped mining");
+  });
+}
+
+int gm_db_spare_limit(gm_db *db, int64_t bytes) {
+  return guard([&]() {
+    if (!db) throw gm::Error(GM_E_ARG, "null argument");
+    spares_of(db)->set_limit(bytes < 0 ? kSpareBytes : (size_t)bytes);
   });
 }
 

@@ -25,7 +25,9 @@ its subset) times the device bytes per unit measured on the requests of its
 kind completed so far (peak device bytes of the run less the resident
 database), starting from a fixed guess; a batch is admitted while the
 estimates of everything running fit the budget (a request that would not
-fit on an idle device runs alone).  Latency = completion - arrival.
+fit on an idle device runs alone).  The memory that closed subset batches keep
+for the next ones comes out of the budget first.  Latency = completion -
+arrival.
 """
 from __future__ import annotations
 
@@ -178,6 +180,24 @@ class MemoryGate:
             self.cv.notify_all()
 
 
+# A mining request's buffers are kept for the next one up to a share of the
+# budget: a request on 10,000 molecules holds 220 MiB, so that budgets whose
+# share is far below that keep none.
+SPARE_SHARE = 32
+SPARE_LEAST = 128 << 20
+
+
+def spare_bytes(budget: int, mining_slots: int) -> Tuple[int, int]:
+    """The most a kept subset batch may hold under a budget, and what all of
+    them together come to: two are kept at once, and each slot's running batch
+    may have taken one over."""
+    limit = budget // SPARE_SHARE
+    if limit < SPARE_LEAST:
+        return 0, 0
+    limit = min(limit, 1 << 30)
+    return limit, (mining_slots + 2) * limit
+
+
 class Estimator:
     """Device bytes per unit of a request kind, learned from completed
     batches (peak device bytes less the resident database)."""
@@ -214,7 +234,10 @@ class Server:
         self.copies = [db] + [db.subset(list(range(self.n_graphs))) for _ in range(max(0, query_slots - 1))]
         for d in self.copies:
             d.upload()
-        self.gate = MemoryGate(budget_bytes)
+        self.query_slots, self.mining_slots = max(1, query_slots), max(1, mining_slots)
+        limit, reserve = spare_bytes(budget_bytes, self.mining_slots)
+        db.spare_limit(limit)
+        self.gate = MemoryGate(budget_bytes - reserve)
         self.est = {QUERY: Estimator(16.0), MINING: Estimator(4096.0)}
         self.max_q = max_query_batch
         self.max_m = max_mining_batch
@@ -224,7 +247,6 @@ class Server:
         self._lock = threading.Lock()
         self._stop = threading.Event()
         self._errors: List[BaseException] = []
-        self.query_slots, self.mining_slots = max(1, query_slots), max(1, mining_slots)
         self._workers = [threading.Thread(target=self._query_loop, args=(self.copies[i],), daemon=True)
                          for i in range(self.query_slots)]
         self._workers += [threading.Thread(target=self._mining_loop, daemon=True) for _ in range(self.mining_slots)]
@@ -318,6 +340,7 @@ class Server:
         self._stop.set()
         for w in self._workers:
             w.join()
+        self.copies[0].spare_limit()
         for d in self.copies[1:]:
             d.close()
         if self._errors:

@@ -239,13 +239,18 @@ int gm_batch_create(int32_t n_jobs, gm_db *const *dbs, gm_batch **out);
  * overlap).  Mining it gives each job the results of mining its subset on
  * its own.  No reference counterpart (serving).  When such a batch is
  * destroyed its device memory may be kept for the next one of the same db (at
- * most two batches of 1 GiB; freed with db, or when an allocation fails). */
+ * most two batches of 1 GiB; freed with db, or when an allocation fails; see
+ * gm_db_spare_limit). */
 int gm_batch_create_subsets(gm_db *db, int32_t n_jobs, const int32_t *job_begin, const int32_t *graph_ids,
                             gm_batch **out);
 /* Mine every job of the batch in one schedule with per-job min supports;
  * identical per-job results to gm_mine on each database. */
 int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg, gm_job_pattern_cb cb, void *user,
                   gm_stats *stats);
+/* Keep a destroyed subset batch of db only up to this many bytes of device and
+ * pinned memory (0: keep none; < 0: the default, 1 GiB).  Kept ones over it are
+ * freed now.  For callers that bound the device memory they use. */
+int gm_db_spare_limit(gm_db *db, int64_t bytes);
 /* gm_db_set_limits for a batch. */
 int gm_batch_set_limits(gm_batch *batch, int64_t piece_keys, int64_t list_units);
 void gm_batch_destroy(gm_batch *batch);

@@ -1,6 +1,9 @@
 """Serving on the GPU: every request answered by the continuously batched
 server (queries and mining jobs overlapping on the device) equals the same
 request run alone -- exactly (integer supports and pattern sets)."""
+import ctypes
+import time
+
 import pytest
 
 import gpu_graph_mining_amd as gm
@@ -130,3 +133,43 @@ def test_a_taken_over_batch_reports_its_own_memory(vlabels, minsups, least):
     assert first[0] > want[0]
     assert peaks(db, small, minsups) == want
     assert peaks(db, large, [least]) == first
+
+
+@pytest.mark.parametrize("budget", [64 << 20, 8 << 30])
+def test_kept_batches_stay_within_the_servers_budget(budget):
+    """Mining requests of 10,000 molecules (some 220 MiB of buffers each): what
+    the device holds when they are done is at most what the budget sets aside
+    for the next ones (nothing of 64 MiB), and the handle's own limit is back
+    after the server."""
+    hip = gm.load_library()  # (the runtime that the library is linked with)
+    db = gm.GraphDB.molecule(3, 30000)
+    db.upload()
+
+    def free():
+        now, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(now), ctypes.byref(total)) == 0
+        return now.value
+
+    server = serving.Server(db, budget_bytes=budget, query_slots=1)
+    before = free()
+    requests = [serving.Request(serving.MINING, i, graphs=list(range(i, 30000, 3)), minsup=2000 - i, units=100000)
+                for i in range(3)]
+    for i, r in enumerate(requests):  # (one at a time: a batch of them holds more)
+        server.submit(r)
+        while len(server.finished) <= i and not server._errors:
+            time.sleep(0.01)
+    limit, reserve = serving.spare_bytes(budget, server.mining_slots)
+    held = before - free()
+    server.close()
+    print("budget", budget, "held", held, "limit", limit, flush=True)
+    assert held <= reserve and (held > 0) == (reserve > 0) and server.gate.budget + reserve == budget
+    for r in requests:
+        assert r.result == serving.run_alone(db, r)
+    batch = gm.Batch.from_subsets(db, [requests[0].graphs])
+    batch.mine([2000], count_only=True)
+    used = before - free()
+    batch.close()
+    assert used > 100 << 20 and before - free() >= used  # kept: the default limit
+    db.spare_limit(0)
+    assert before - free() < used
+    db.close()

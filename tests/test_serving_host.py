@@ -131,3 +131,12 @@ int main() {
                     code = 0 if fails < calls else gm.GM_E_OOM if oom else gm.GM_E_DEVICE
                     want.append(f"{name} {fails} {kept} {oom} : {calls} {int(fails > 0 and oom)} {code}")
     assert out[:-1] == want
+
+
+def test_kept_batches_take_a_small_share_of_the_budget():
+    for budget in (0, 1, 256 << 20, 4 << 30, 8 << 30, 64 << 30, 1 << 40):
+        for slots in (1, 2, 4):
+            limit, reserve = serving.spare_bytes(budget, slots)
+            assert reserve == (slots + 2) * limit <= budget * (slots + 2) // 32
+            assert limit == 0 or 128 << 20 <= limit <= 1 << 30
+            assert (limit > 0) == (budget >= 4 << 30)
