@@ -49,7 +49,8 @@ EXPORTED_SYMBOLS = (
     "gm_batch_create", "gm_batch_mine", "gm_batch_destroy", "gm_support_queries", "gm_support_query",
     "gm_db_write", "gm_db_load_part", "gm_mine_noalloc", "gm_dfs_codes_are_min", "gm_batch_create_subsets",
     "gm_patterns_create", "gm_patterns_add", "gm_patterns_add_job", "gm_patterns_get", "gm_patterns_destroy",
-    "gm_db_set_limits", "gm_batch_set_limits", "gm_db_spare_limit",
+    "gm_db_set_limits", "gm_batch_set_limits", "gm_db_spare_limit", "gm_db_device_bytes",
+    "gm_batch_device_bytes",
 )
 
 
@@ -125,6 +126,8 @@ def load_library(path: Optional[os.PathLike] = None) -> C.CDLL:
         "gm_batch_create_subsets": (C.c_int, [dbp, C.c_int32, i32p, i32p, P(dbp)]),
         "gm_batch_mine": (C.c_int, [dbp, i32p, P(gm_cfg), JOB_PATTERN_CB, C.c_void_p, P(gm_stats)]),
         "gm_batch_set_limits": (C.c_int, [dbp, C.c_int64, C.c_int64]),
+        "gm_db_device_bytes": (C.c_int64, [dbp]),
+        "gm_batch_device_bytes": (C.c_int64, [dbp]),
         "gm_db_spare_limit": (C.c_int, [dbp, C.c_int64]),
         "gm_batch_destroy": (None, [dbp]),
         "gm_patterns_create": (C.c_void_p, []),
@@ -461,6 +464,10 @@ class GraphDB:
     def upload(self) -> None:
         _check(load_library().gm_db_upload(self._h))
 
+    def device_bytes(self) -> int:
+        """Bytes of the device copy (gm_db_device_bytes)."""
+        return load_library().gm_db_device_bytes(self._h)
+
     def set_limits(self, piece_keys: int = 0, list_units: int = 0) -> None:
         """Where the level steps on this handle are cut (gm_db_set_limits;
         0 = the default)."""
@@ -735,6 +742,10 @@ class Batch:
             cb = JOB_PATTERN_CB() if count_only else lib.add_job_pattern
             _check(lib.gm_batch_mine(self._h, _ptr(ms), C.byref(cfg), cb, listing.user, C.byref(st)))
             return listing.patterns(self.n_jobs), st.as_dict()
+
+    def device_bytes(self) -> int:
+        """Bytes of the jobs' graphs on the device (gm_batch_device_bytes)."""
+        return load_library().gm_batch_device_bytes(self._h)
 
     def set_limits(self, piece_keys: int = 0, list_units: int = 0) -> None:
         """GraphDB.set_limits for the batch."""

@@ -373,6 +373,8 @@ int gm_db_upload(gm_db *db) {
   });
 }
 
+int64_t gm_db_device_bytes(const gm_db *db) { return db && db->dev ? (int64_t)db->dev->bytes : 0; }
+
 int gm_db_set_limits(gm_db *db, int64_t piece_keys, int64_t list_units) {
   return guard([&]() {
     if (!db) throw gm::Error(GM_E_ARG, "null argument");
@@ -580,6 +582,8 @@ int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg,
       throw gm::Error(GM_E_CALLBACK, "callback stopped mining");
   });
 }
+
+int64_t gm_batch_device_bytes(const gm_batch *batch) { return batch ? (int64_t)batch->dev.bytes : 0; }
 
 int gm_db_spare_limit(gm_db *db, int64_t bytes) {
   return guard([&]() {

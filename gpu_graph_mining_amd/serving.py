@@ -128,8 +128,9 @@ def make_requests(db: GraphDB, n: int, seed: int = 4, query_frac: float = 0.9,
 
 
 def db_bytes(n_graphs: int, n_vertices: int, n_edges: int) -> int:
-    """Device bytes of a packed database (graph and vertex offsets, packed
-    adjacency, labels, job and graph ids)."""
+    """Device bytes of a packed database in the general layout alone (graph and
+    vertex offsets, packed adjacency, labels, job and graph ids); a resident
+    one's are GraphDB.device_bytes()."""
     return 4 * (n_graphs + 1) + 4 * (n_vertices + 1) + 8 * n_edges + n_vertices + 4 * n_graphs + 4 * n_vertices
 
 
@@ -226,9 +227,8 @@ class Server:
     def __init__(self, db: GraphDB, budget_bytes: int = 8 << 30, max_query_batch: int = 4096,
                  max_mining_batch: int = 8, query_slots: int = 2, mining_slots: int = 2):
         db.upload()
-        c = db.counts()
-        self.n_graphs = c["n_graphs"]
-        self.resident_bytes = db_bytes(c["n_graphs"], c["n_vertices"], c["n_edges"])
+        self.n_graphs = len(db)
+        self.resident_bytes = db.device_bytes()
         # one resident copy per query slot (a handle runs one call at a
         # time); mining slots gather their subsets from the first
         self.copies = [db] + [db.subset(list(range(self.n_graphs))) for _ in range(max(0, query_slots - 1))]
@@ -323,12 +323,12 @@ class Server:
                 try:
                     b = Batch.from_subsets(self.copies[0], [r.graphs for r in batch])
                     try:
+                        sub_bytes = b.device_bytes()
                         res, st = b.mine([r.minsup for r in batch])
                     finally:
                         b.close()
                 finally:
                     self.gate.release(used)
-                sub_bytes = sum(db_bytes(len(r.graphs), r.n_vertices, r.n_edges) for r in batch)
                 self.est[MINING].observe(sum(r.units for r in batch), st["peak_device_bytes"] - sub_bytes)
                 for r, pats in zip(batch, res):
                     r.result = sorted((tuple(c), s) for c, s, _ in pats)

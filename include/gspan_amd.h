@@ -176,6 +176,14 @@ int gm_db_export(const gm_db *db, int32_t *graph_vbegin, int32_t *vlabels, int32
  * (src/globals/cuda_graph_types.cpp:130-153). */
 int gm_db_upload(gm_db *db);
 
+/* Device bytes of the database's resident copy, the part of
+ * gm_stats.peak_device_bytes that is there before a run (0: not uploaded).  A
+ * database of graphs of at most 64 vertices and few labels (edge labels x
+ * (vertex labels + 1) <= 63) is held in two layouts: 8-byte vertex groups,
+ * which gm_mine, gm_support_queries and the subset batches read, and the packed
+ * adjacency of all others, which gm_mine_noalloc reads. */
+int64_t gm_db_device_bytes(const gm_db *db);
+
 /* Limits of the level steps on this handle (they change how a run is cut, not
  * what it finds; tests lower them to cut small databases):
  *   piece_keys  counter keys of a level step at most, 16 bytes each and per
@@ -247,6 +255,8 @@ int gm_batch_create_subsets(gm_db *db, int32_t n_jobs, const int32_t *job_begin,
  * identical per-job results to gm_mine on each database. */
 int gm_batch_mine(gm_batch *batch, const int32_t *abs_minsup, const gm_cfg *cfg, gm_job_pattern_cb cb, void *user,
                   gm_stats *stats);
+/* gm_db_device_bytes for a batch. */
+int64_t gm_batch_device_bytes(const gm_batch *batch);
 /* Keep a destroyed subset batch of db only up to this many bytes of device and
  * pinned memory (0: keep none; < 0: the default, 1 GiB).  Kept ones over it are
  * freed now.  For callers that bound the device memory they use. */

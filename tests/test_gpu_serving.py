@@ -173,3 +173,19 @@ def test_kept_batches_stay_within_the_servers_budget(budget):
     db.spare_limit(0)
     assert before - free() < used
     db.close()
+
+
+@pytest.mark.parametrize("vlabels", [5, 90])  # two layouts on the device, and one
+def test_the_server_knows_what_is_resident(vlabels):
+    """What the estimates of a request's memory subtract from a run's peak is
+    what the run finds on the device: a run that keeps no pattern has that
+    peak, on the database and on a batch of its graphs."""
+    db = gm.GraphDB.random(3, 400, 5, 9, 1.2, vlabels, 2)
+    assert db.device_bytes() == 0
+    server = serving.Server(db)
+    resident = server.resident_bytes
+    server.close()
+    assert resident == db.device_bytes() == gm.mine(db, 401)[1]["peak_device_bytes"] > 0
+    batch = gm.Batch.from_subsets(db, [list(range(100)), [7, 7]])
+    assert batch.device_bytes() == batch.mine([101, 3])[1]["peak_device_bytes"] > 0
+    batch.close()
