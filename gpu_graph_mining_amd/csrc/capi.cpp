@@ -105,6 +105,9 @@ struct gm_patterns {
   std::vector<int32_t> dfs5, n_edges, job;
   std::vector<uint32_t> support;
   std::vector<uint64_t> n_proj;
+  int32_t every = 0;  // gm_patterns_poll
+  int (*poll)(void *) = nullptr;
+  void *user = nullptr;
 };
 
 namespace {
@@ -619,7 +622,14 @@ int gm_patterns_add_job(void *patterns, int32_t job, const int32_t *dfs5, int32_
   } catch (...) {
     return 1;  // out of memory: stops the run
   }
-  return 0;
+  return p->every > 0 && p->n_proj.size() % (size_t)p->every == 0 ? p->poll(p->user) : 0;
+}
+
+void gm_patterns_poll(gm_patterns *p, int32_t every, int (*poll)(void *user), void *user) {
+  if (!p) return;
+  p->every = poll ? every : 0;
+  p->poll = poll;
+  p->user = user;
 }
 
 int gm_patterns_add(void *patterns, const int32_t *dfs5, int32_t n_edges, uint32_t support, uint64_t n_proj) {

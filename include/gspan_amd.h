@@ -277,6 +277,9 @@ int gm_patterns_add_job(void *patterns, int32_t job, const int32_t *dfs5, int32_
                         uint64_t n_proj);
 int64_t gm_patterns_get(const gm_patterns *patterns, const int32_t **dfs5, const int32_t **n_edges,
                         const int32_t **job, const uint32_t **support, const uint64_t **n_proj);
+/* After every `every` patterns added ask poll(user), whose non-zero answer stops
+ * the run like a callback's (every <= 0 or poll NULL: never). */
+void gm_patterns_poll(gm_patterns *patterns, int32_t every, int (*poll)(void *user), void *user);
 void gm_patterns_destroy(gm_patterns *patterns);
 
 /* ---- pattern-support queries ------------------------------------------ */

@@ -1,9 +1,14 @@
 """Host-side tests of the product library (no GPU needed): the C ABI loads
 and exports every declared symbol, readers, generators, the canonical check
 and the error paths that fire before any device work."""
+import ctypes
+import os
 import random
 import re
+import signal
 import struct
+import subprocess
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -340,3 +345,48 @@ def test_listing_returns_what_the_sink_was_given(n_patterns, n_jobs):
         got = listing.patterns(n_jobs)
     assert got == want
     assert all(type(c) is gm.DFSCode and type(t) is gm.DFS for pats in got for c, _, _ in pats for t in c)
+
+
+def test_a_long_listing_is_interrupted_between_patterns(tmp_path):
+    """A signal that arrives while the library adds patterns is handled before
+    the call has ended: its handler's exception stops the run and is raised
+    (a C function that adds a pattern every 20 us stands for the run)."""
+    src = tmp_path / "run.c"
+    src.write_text('''#include <stdint.h>
+#include <unistd.h>
+typedef int (*add_fn)(void *, const int32_t *, int32_t, uint32_t, uint64_t);
+int run(add_fn add, void *patterns, int32_t n) {
+  const int32_t code[5] = {0, 1, 0, 0, 0};
+  for (int32_t i = 0; i < n; ++i) {
+    if (add(patterns, code, 1, 1, 1)) return i + 1;
+    usleep(20);
+  }
+  return -n;
+}
+''')
+    lib = tmp_path / "run.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+    run = ctypes.CDLL(str(lib)).run
+    run.argtypes = [gm.PATTERN_CB, ctypes.c_void_p, ctypes.c_int32]
+    add = gm.load_library().add_pattern
+    with gm._Listing() as listing:  # no signal: the run ends by itself
+        assert run(add, listing.user, 3000) == -3000
+        listing.check(gm.GM_OK)
+        assert len(listing.patterns()[0]) == 3000
+    handled = []
+    old = signal.signal(signal.SIGUSR1, lambda *_: handled.append(1))
+    timers = [threading.Timer(t, os.kill, (os.getpid(), s)) for t, s in ((0.05, signal.SIGUSR1), (0.2, signal.SIGINT))]
+    try:
+        with gm._Listing() as listing:
+            for t in timers:
+                t.start()
+            n = run(add, listing.user, 100000)
+            assert 0 < n < 100000 and n % 1024 == 0 and handled == [1]
+            with pytest.raises(KeyboardInterrupt):
+                listing.check(gm.GM_E_CALLBACK)
+            with pytest.raises(gm.GMError):  # raised once; the call's own error otherwise
+                listing.check(gm.GM_E_CALLBACK)
+    finally:
+        for t in timers:
+            t.join()
+        signal.signal(signal.SIGUSR1, old)
