@@ -1323,6 +1323,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     double ms = 0;
     unsigned long long ecand = 0, max_fill = 0, pruned = 0, failed = 0;
     uint32_t guess = 0;  // frequent keys in the first download
+    int lists_again = 0;  // runs whose list pool was too small
     // the stage; rerun with a longer frequent-key list when it overflowed
     for (int attempt = 0;; ++attempt) {
       if (compact) {
@@ -1476,6 +1477,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
         // the lists outgrew the pool: the stage is run again with a larger
         // one, from cleared counters
         pool_units = std::max<int64_t>(pool_units * 4, kSpread * 512);
+        ++lists_again;
         hip_check(launch_fill8(w.acc.p, w.acc.cap, s), "clear counters");
         attempt = -1;
         continue;
@@ -1602,9 +1604,9 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       if (trace_levels)
         fprintf(stderr,
                 "[gm level %d] device-chosen: patterns %lld rows %lld K %lld chunks %lld stage_us %.1f candidates %llu "
-                "pruned %llu frequent %u children %lld child_rows %lld max_fill %llu\n",
+                "pruned %llu frequent %u children %lld child_rows %lld max_fill %llu lists_again %d\n",
                 level, (long long)P, (long long)rows_now, (long long)K, (long long)total_chunks, ms * 1e3, ecand, pruned,
-                cnt.fcount, (long long)C, (long long)child_rows, max_fill);
+                cnt.fcount, (long long)C, (long long)child_rows, max_fill, lists_again);
       pend.rec = reinterpret_cast<const Freq *>(hbuf + sizeof(Counters));
       pend.F = F;
       pend.K = K;
@@ -2253,11 +2255,11 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
       fprintf(stderr,
               "[gm level %d] piece %lld-%lld of %lld patterns, rows %lld of %lld K %lld chunks %lld table_bits %d stage_us %.1f "
               "candidates %llu pruned %llu frequent %u children %lld child_rows %lld minimal %lld spec %d "
-              "failed %llu max_fill %llu list_cap %llu canon_dev %d host_us canon %.1f host %.1f overlap %.1f\n",
+              "failed %llu max_fill %llu list_cap %llu lists_again %d canon_dev %d host_us canon %.1f host %.1f overlap %.1f\n",
               level, (long long)p_begin, (long long)p_end, (long long)P, (long long)(prow_hi - prow_lo), (long long)rows_now,
               (long long)K, (long long)total_chunks, table_bits, ms * 1e3,
               ecand, pruned, cnt.fcount, (long long)C, (long long)child_rows, (long long)alive, spec ? 1 : 0, failed,
-              max_fill, (unsigned long long)list_cap, canon_dev ? 1 : 0, us_canon, us_host, us_overlap);
+              max_fill, (unsigned long long)list_cap, lists_again, canon_dev ? 1 : 0, us_canon, us_host, us_overlap);
     st.n_levels++;
     if (stopped) break;
     // the piece is written: the level continues after it, or is done (its

@@ -1,8 +1,12 @@
-"""Levels cut into pieces without a memory budget (more counter keys than a
+"""Levels that do not go through in one piece or at the first try.
+
+Levels cut into pieces without a memory budget (more counter keys than a
 level step takes, GraphDB.set_limits), on compact databases: a piece's
 children, chosen on the device, and their children are mined while the cut
 level's rows wait for its next piece.  Patterns, supports, |Proj(P)|, E_child
-and E_cand are the oracle's, for one database and for the jobs of a batch."""
+and E_cand are the oracle's, for one database and for the jobs of a batch.  Levels whose candidate lists
+outgrow their pool (set small here) are listed again into a larger one, with
+the same results."""
 import random
 import re
 
@@ -11,7 +15,7 @@ import pytest
 import gpu_graph_mining_amd as gm
 from oracle import py_oracle as po
 
-from test_gpu_compact import all_labels, tree
+from test_gpu_compact import all_labels, clique, star, tree
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +109,41 @@ def test_the_path_table_is_the_root_pieces_own(trace):
     for i, (db, minsup, pats) in enumerate(zip(dbs, minsups, res)):
         assert _key(pats) == (_key(po.mine_arrays(db.arrays(), minsup)[0]) if db is not single else []), i
     batch.close()
+
+
+def _bushy(n, seed=11):
+    """Trees with a star of seven equal leaves each: many candidates a row."""
+    rng = random.Random(seed)
+    graphs = []
+    for _ in range(n):
+        labels, edges = tree(rng, 24, 3, 2, 3)
+        k = len(labels)
+        graphs.append((labels + [0] * 8, edges + [(k, k + i, 0) for i in range(1, 8)]))
+    return graphs
+
+
+LISTS = {
+    "stars": ([star(n) for n in (1, 3, 9, 12, 12)], 1, 4, False),
+    "cliques": ([clique(n) for n in (3, 5, 6, 9, 10)], 1, 3, False),
+    "largest_star": ([star(63), star(40), clique(14)], 1, 2, False),
+    "chosen_on_the_device": (_bushy(60), 6, 6, True),
+}
+
+
+@pytest.mark.parametrize("list_units", [1, 1200])  # no extent fits; a few do
+@pytest.mark.parametrize("name", list(LISTS))
+def test_lists_that_outgrow_their_pool(trace, name, list_units):
+    graphs, minsup, max_edges, device = LISTS[name]
+    db = gm.GraphDB.from_graphs(graphs)
+    opats, ost = po.mine_arrays(db.arrays(), minsup, max_edges=max_edges)
+    db.set_limits(list_units=list_units)
+    for kw in ({}, {"canon_host": 2}, {"speculate": 2}):
+        trace()
+        pats, st = gm.mine(db, minsup, max_edges=max_edges, collect_proj=True, **kw)
+        lines = trace().splitlines()
+        again = [line for line in lines if int(re.search(r"lists_again (\d+)", line)[1]) > 0]
+        assert again or (list_units > 1 and name == "stars")
+        if device and "speculate" not in kw:
+            assert any("device-chosen" in line for line in again)
+        assert _key(pats) == _key(opats)
+        assert (st["e_child"], st["e_cand"]) == (ost["e_child"], ost["e_cand"])
