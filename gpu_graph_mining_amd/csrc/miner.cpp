@@ -477,6 +477,8 @@ void gather_db(const DeviceDB &src, const HostDB &h, int32_t n_jobs, const int32
     hip_check(hipStreamSynchronize(s), "k_cgather");  // before the host's index arrays go
     return;
   }
+  // (pack_db's limit; graphs may be selected several times)
+  if (nv > INT32_MAX - 1 || na > INT32_MAX - 1) throw Error(GM_E_UNSUPPORTED, "subsets too large for 32-bit offsets");
   out.gvbase.ensure(4 * (size_t)(n_sel + 1));
   out.vadj.ensure(4 * (size_t)(nv + 1));
   out.adj.ensure(4 * (size_t)std::max<int64_t>(na, 1));

@@ -189,3 +189,16 @@ def test_the_server_knows_what_is_resident(vlabels):
     batch = gm.Batch.from_subsets(db, [list(range(100)), [7, 7]])
     assert batch.device_bytes() == batch.mine([101, 3])[1]["peak_device_bytes"] > 0
     batch.close()
+
+
+def test_subsets_past_32_bit_offsets_are_refused():
+    """One graph selected so often that the gathered adjacency (65,280 entries
+    a time) passes 2^31: refused before anything is gathered."""
+    n = 256
+    db = gm.GraphDB.from_graphs([([0] * n, [(a, b, 0) for a in range(n) for b in range(a + 1, n)])])
+    with pytest.raises(gm.GMError) as e:
+        gm.Batch.from_subsets(db, [[0] * 33000])
+    assert e.value.code == gm.GM_E_UNSUPPORTED
+    batch = gm.Batch.from_subsets(db, [[0] * 3])
+    assert batch.mine([4])[0] == [[]]
+    batch.close()
