@@ -64,6 +64,29 @@ def _traffic(kernel: str, workload: str):
         return None
 
 
+def _roofline(traffic, algorithmic, stage_s: float, launches: float) -> dict:
+    """The extension + support stage against the HBM peak: `traffic` bytes a
+    launch (one level step's stage) as the counters measured them, in stage_s
+    seconds of `launches` launches per step.  The algorithmic bytes of a step
+    count a layout that re-reads pattern metadata and edge labels item by item;
+    the compact kernels move about half of them, so their rate is no share of
+    the peak and is given under its own name."""
+    roof = {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None,
+            "traffic": traffic,
+            "kernel": "k_clevel, or k_level (+ k_level_fix): extension enumeration and support counting of one level step",
+            "traffic_unit": "HBM bytes per launch (the kernels of one level step's stage)",
+            "launches_per_step": launches,
+            "avg_launch_ms": (stage_s / launches * 1e3) if launches else None}
+    if traffic and launches and stage_s > 0:
+        roof["achieved"] = traffic * launches / stage_s / 1e9
+        roof["frac"] = roof["achieved"] / HBM_PEAK_GBS
+    if algorithmic and launches and stage_s > 0:
+        roof["algorithmic_bytes_per_step"] = algorithmic
+        roof["algorithmic_bytes_per_launch"] = algorithmic / launches
+        roof["algorithmic_rate"] = algorithmic / stage_s / 1e9
+    return roof
+
+
 def _golden_case(cfg: int):
     """The reference's listing of the workload (tests/golden/golden.json):
     sha256 and count of its sorted "code<TAB>support" lines, plus the
@@ -267,12 +290,6 @@ def _main_section(args) -> dict:
         "max_table_fill": st["max_table_fill"],
     }
 
-    roof = {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None,
-            "traffic": _traffic("stage", config["workload"]),
-            "kernel": "k_clevel, or k_level (+ k_level_fix): extension enumeration and support counting of one level step",
-            "traffic_unit": "HBM bytes per launch (one level step's k_level + k_level_fix)",
-            "launches_per_step": launches / args.steps,
-            "avg_launch_ms": (ev_s / launches * 1e3) if launches else None}
     # parity: the reference's listing (sha256 + count), the oracle's counts
     ok = True
     if golden is not None:
@@ -300,18 +317,13 @@ def _main_section(args) -> dict:
                "sample": sample, "seconds": ost["seconds"], "patterns": ost["n_patterns"], "cpu": _cpu_model()}
     if oracle is not None:
         ok = ok and oracle["e_child"] == e_child and oracle["e_cand"] == st["e_cand"]
-        # algorithmic bytes of the extension + support stage over the whole
-        # run (formula in oracle/cpu_gspan.cpp), per launch = per level step
-        b = oracle["b_ext"] + oracle["b_sup"]
-        per_launch = b / (launches / args.steps)
-        roof["algorithmic_bytes_per_step"] = b
-        roof["algorithmic_bytes_per_launch"] = per_launch
-        roof["achieved"] = b / (ev_s / args.steps) / 1e9
-        roof["frac"] = roof["achieved"] / HBM_PEAK_GBS
     line["parity"] = ("identical" if ok else "MISMATCH") if (golden is not None or oracle is not None) else None
     if cpu is not None:
         line["cpu_baseline"] = cpu
-    line["roofline"] = roof
+    # algorithmic bytes of the extension + support stage over the whole run
+    # (formula in oracle/cpu_gspan.cpp)
+    line["roofline"] = _roofline(_traffic("stage", config["workload"]), oracle and oracle["b_ext"] + oracle["b_sup"],
+                                 ev_s / args.steps, launches / args.steps)
     return line
 
 
