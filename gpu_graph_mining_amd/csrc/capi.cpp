@@ -22,7 +22,7 @@
 // Subset batches that were destroyed and wait for the next one of the same
 // resident database: their buffers, workspace and stream.  A mining request
 // on 5,000 molecules made and freed some 70 of them, 6.5 of its 8.7 ms; with
-// them kept it takes 1.8 ms.  At most kSpares batches of at most
+// them kept it took 2.0 ms.  At most kSpares batches of at most
 // kSpareBytes (gm_db_spare_limit) each, all freed with the database or when an
 // allocation fails.
 constexpr size_t kSpares = 2;

@@ -34,9 +34,10 @@
 // the list is in row order, so every key's entries are in row order: k_cwrite
 // can place the children's rows graph-contiguously in list order.
 //
-// What bounds k_clevel: the gathers.  A load of one group a lane touches 13
-// lines, nearly all of them misses in a 32 KB L1 that 28 waves share, so a
-// block of 64 rows asks L2 for some 170 lines.  The address units are 80-85 %
+// What bounds k_clevel: the gathers.  64 rows lie in some 40 graphs, so a load
+// of one group a lane touches about as many lines; a block's 20 vector memory
+// instructions touch 300 lines in all, of which 170 miss the 32 KB L1 that 28
+// waves share and are asked of L2.  The address units are 80-85 %
 // busy and L1 waits on pending lines for 75 % of the time (100,000
 // transactions: 2.85 ms for the levels of 8-byte tuples, 2.3 ms with the loads
 // alone); neither more waves, loads further ahead nor lines kept in an XCD's

@@ -1218,7 +1218,7 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     // those lists in turn for each 8 to 20 bytes of their own; it measured best of 0.08-0.4 over five databases and budgets
     // (30,000 transactions under 64 MiB: 3.8 ms at 0.08, 2.4 at 0.2, 2.9 at
     // 0.4).  With the whole level's lists and the children's counted at once
-    // it took 64 level steps and 4.2 ms, now 36 steps.
+    // it took 64 level steps and 4.2 ms, now 30 steps and 2.2 ms.
     constexpr double kShare = 0.2;
     const int64_t child_row = rows_bytes(1, tuple_stride(root ? 2 : std::min(L.max_nv + 1, kMaxPatV)));
     const int64_t free_now = std::max<int64_t>(0, budget - held);
@@ -1305,9 +1305,12 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
     // the check or the write otherwise.  The device check and the choice take
     // 20-50 us however few the keys (a code's steps are a serial chain); the
     // host does a level of some 50 keys in less, so levels are left to it
-    // whose predecessor had fewer (the root: databases of fewer vertices than
-    // usually give more).  1,000 random graphs: 185 us by the host, 195 us by
-    // the device; 10,000 transactions 1.29 and 1.20 ms.
+    // whose predecessor had fewer.  1,000 random graphs: 185 us by the host,
+    // 195 us by the device; 10,000 transactions 1.29 and 1.20 ms.  The root has
+    // no predecessor: its vertices stand for its keys, a poor stand-in.  From
+    // 1,000 to 20,000 graphs the device was 0-4 % slower with 6 to 63 frequent
+    // edges (278 against 267 us for 10,000 random graphs) and 10-30 % faster
+    // with 216 (124 against 148), whatever the size.
     constexpr uint32_t kDevSelectKeys = 48;
     constexpr int64_t kDevSelectVertices = 100000;
     const bool dev_select = compact && want_codes && !past_max && budget == 0 && opt.speculate != 2 && !dev_select_off &&
