@@ -897,7 +897,6 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
           Workspace *ws) {
   std::lock_guard<std::mutex> lock(db.mu);
   Timer total;
-  const Limits limits = db.limits;
   const int32_t NEL = db.NEL, NVL = db.NVL;
   int threads = opt.canon_threads > 0 ? opt.canon_threads
                                       : (int)std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
@@ -905,6 +904,8 @@ bool mine(DeviceDB &db, const MineOptions &opt, const ReportFn &report, gm_stats
   std::memset(&st, 0, sizeof(st));
   if (!ws && !db.ws) db.ws.reset(new Workspace());
   Workspace &w = ws ? *ws : *db.ws;
+  // (the static workspace has two row sets: its levels are never cut)
+  const Limits limits = w.arena ? Limits() : db.limits;
   if (!w.acc_zero) {
     if (w.acc.p) hip_check(launch_fill8(w.acc.p, w.acc.cap, s), "clear counters");
     if (w.accb.p) hip_check(launch_fill8(w.accb.p, w.accb.cap, s), "clear counters");

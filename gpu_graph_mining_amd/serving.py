@@ -222,7 +222,8 @@ class Estimator:
 
 class Server:
     """query_slots + mining_slots workers over resident handles of one
-    database; submit() enqueues, results land on the Request objects."""
+    database; submit() enqueues, results land on the Request objects.  From
+    its start to close(), db's spare limit is the server's."""
 
     def __init__(self, db: GraphDB, budget_bytes: int = 8 << 30, max_query_batch: int = 4096,
                  max_mining_batch: int = 8, query_slots: int = 2, mining_slots: int = 2):

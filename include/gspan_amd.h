@@ -193,7 +193,8 @@ int64_t gm_db_device_bytes(const gm_db *db);
  *               common pool when a level's lists are first written; a level
  *               that needs more writes them again into a larger one (0 = the
  *               default, by the level's rows)
- * Makes the device copy if there is none.  GM_E_ARG outside the ranges. */
+ * Makes the device copy if there is none.  GM_E_ARG outside the ranges.
+ * Ignored by gm_mine_noalloc. */
 int gm_db_set_limits(gm_db *db, int64_t piece_keys, int64_t list_units);
 
 /* Release host and device memory.  Replaces

@@ -111,6 +111,15 @@ def test_the_path_table_is_the_root_pieces_own(trace):
     batch.close()
 
 
+def test_the_static_workspace_ignores_the_limits():
+    """Its levels hold two row sets and cannot wait for pieces."""
+    db = gm.GraphDB.molecule(3, 100)
+    db.upload()
+    want = _key(gm.mine_noalloc(db, 20, collect_proj=True)[0])
+    db.set_limits(piece_keys=500, list_units=1)
+    assert _key(gm.mine_noalloc(db, 20, collect_proj=True)[0]) == want == _key(gm.mine(db, 20, collect_proj=True)[0])
+
+
 def _bushy(n, seed=11):
     """Trees with a star of seven equal leaves each: many candidates a row."""
     rng = random.Random(seed)
